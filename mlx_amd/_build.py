@@ -82,6 +82,36 @@ def build_glue_gpu_test(verbose: bool = False) -> str:
     return GLUE_GPU_TEST
 
 
+NATIVE = os.path.join(HERE, "native")
+FAST_OPS = os.path.join(LIB_DIR, "fast_ops.so")
+
+
+def build_fast_ops(verbose: bool = False) -> str:
+    """The CPython extension with the operators' host path (host code only:
+    libtorch's headers, no kernels; it is handed the HIP library's entry points
+    at run time)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    os.makedirs(LIB_DIR, exist_ok=True)
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", INCLUDE,
+           "-I", sysconfig.get_paths()["include"]]
+    for path in cpp_extension.include_paths(device_type="cuda"):
+        cmd += ["-isystem", path]
+    cmd += [os.path.join(NATIVE, "fast_ops.cpp"), "-o", FAST_OPS]
+    for path in cpp_extension.library_paths(device_type="cuda"):
+        cmd += ["-L", path]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building fast_ops failed:\n{proc.stdout}\n{proc.stderr}")
+    if verbose:
+        print("built", FAST_OPS)
+    return FAST_OPS
+
+
 PROBE_DIR = os.path.join(HERE, "probe")
 READ_PROBE = os.path.join(LIB_DIR, "read_probe")
 
@@ -103,6 +133,7 @@ def build_read_probe(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     build(verbose=True)
+    build_fast_ops(verbose=True)
     build_glue_gpu_test(verbose=True)
     build_read_probe(verbose=True)
     sys.exit(0)

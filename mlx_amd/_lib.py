@@ -141,6 +141,36 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+FAST_OPS_PATH = os.path.join(HERE, "lib", "fast_ops.so")
+_fast = None
+
+
+def load_fast():
+    """The extension with the operators' host path (native/fast_ops.cpp), bound
+    to the entry points of the loaded HIP library; raises if it is not built."""
+    global _fast
+    if _fast is not None:
+        return _fast
+    import importlib.machinery
+    import importlib.util
+
+    import torch  # noqa: F401  (the extension resolves libtorch's symbols in this process)
+
+    lib = load()
+    if not os.path.isfile(FAST_OPS_PATH):
+        raise ImportError(
+            f"{FAST_OPS_PATH} not found: build it with `python -m mlx_amd._build`."
+        )
+    loader = importlib.machinery.ExtensionFileLoader("mlx_amd.fast_ops", FAST_OPS_PATH)
+    spec = importlib.util.spec_from_loader("mlx_amd.fast_ops", loader)
+    module = importlib.util.module_from_spec(spec)
+    loader.exec_module(module)
+    module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                 for name in SIGNATURES})
+    _fast = module
+    return module
+
+
 def qmm_plan(M, N, K, L=1, batched_weights=False, group_size=64, bits=4, dtype=BFLOAT16,
              transpose=True, workspace_bytes=None):
     """(status, record) of a rehearsed mlxrocm_qmm call: the dispatch rules it

@@ -34,6 +34,16 @@ def _defaults_for_mode(mode: str, group_size: Optional[int], bits: Optional[int]
     return group_size or default_group_size, bits or default_bits
 
 
+def _held(layer: torch.nn.Module, *names: str):
+    """Buffers of a layer, straight from their dict: torch.nn.Module's attribute
+    lookup takes longer than the operator's own host path."""
+    buffers = layer._buffers
+    try:
+        return [buffers[name] for name in names]
+    except KeyError:  # held some other way (as a Parameter, say)
+        return [getattr(layer, name) for name in names]
+
+
 class QuantizedLinear(torch.nn.Module):
     """``y = quantized_matmul(x, weight, scales, biases, transpose=True) + bias``."""
 
@@ -76,18 +86,16 @@ class QuantizedLinear(torch.nn.Module):
         return self
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        image = getattr(self, "_sb_image", None)
+        weight, scales, biases, bias = _held(self, "weight", "scales", "biases", "bias")
+        image = self.__dict__.get("_sb_image")
         if image is not None and (
-                self.biases is None
-                or self._sb_image_of != (self.scales.data_ptr(), self.biases.data_ptr())
-                or torch.promote_types(x.dtype, self.scales.dtype) != image.dtype):
+                biases is None
+                or self._sb_image_of != (scales.data_ptr(), biases.data_ptr())
+                or torch.promote_types(x.dtype, scales.dtype) != image.dtype):
             image = None  # weights replaced, or a product in another type
-        y = ops.quantized_matmul(x, self.weight, self.scales, self.biases, transpose=True,
-                                 group_size=self.group_size, bits=self.bits, mode=self.mode,
-                                 sb_image=image)
-        if self.bias is not None:
-            y = y + self.bias
-        return y
+        y = ops.quantized_matmul(x, weight, scales, biases, True,
+                                 self.group_size, self.bits, self.mode, sb_image=image)
+        return y if bias is None else y + bias
 
     @classmethod
     def from_linear(cls, linear_layer, group_size: Optional[int] = None,
@@ -228,17 +236,19 @@ class SwiGLU(torch.nn.Module):
         self.down_proj = QuantizedLinear(hidden_dims, input_dims, **kw)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        g, u = self.gate_proj, self.up_proj
+        modules = self._modules
+        g, u = modules["gate_proj"], modules["up_proj"]
         rows = x.numel() // max(x.shape[-1], 1)
-        fused = (0 < rows <= 8 and g.bias is None and u.bias is None
+        *g_triplet, g_bias = _held(g, "weight", "scales", "biases", "bias")
+        *u_triplet, u_bias = _held(u, "weight", "scales", "biases", "bias")
+        fused = (0 < rows <= 8 and g_bias is None and u_bias is None
                  and (g.group_size, g.bits, g.mode) == (u.group_size, u.bits, "affine")
                  and u.mode == "affine")
         if fused:
-            h = ops.quantized_swiglu(x, (g.weight, g.scales, g.biases),
-                                     (u.weight, u.scales, u.biases), g.group_size, g.bits)
+            h = ops.quantized_swiglu(x, tuple(g_triplet), tuple(u_triplet), g.group_size, g.bits)
         else:
             h = torch.nn.functional.silu(g(x)) * u(x)
-        return self.down_proj(h)
+        return modules["down_proj"](h)
 
 
 class QuantizedSwitchLinear(torch.nn.Module):

@@ -33,6 +33,26 @@ _INTEGER = (
 )
 
 
+class _FastOps:
+    """Stands in for the extension of native/fast_ops.cpp until an operator is
+    called with a tensor on the GPU.  Its functions take an operator's arguments
+    and return the result, or None where the operator's own body has to run
+    (anything that is not a plain call)."""
+
+    def __getattr__(self, name):
+        def first_call(*args):
+            if not (isinstance(args[0], torch.Tensor) and args[0].is_cuda):
+                return None
+            global _fast
+            _fast = _lib.load_fast()
+            return getattr(_fast, name)(*args)
+
+        return first_call
+
+
+_fast = _FastOps()
+
+
 def _stream_ptr(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
@@ -201,6 +221,10 @@ def quantize(
     ``mode="affine"`` (mlx/ops.cpp:5208-5246 -> affine_quantize :5035-5099) and
     ``(w_q uint32, scales uint8)`` for the floating-point modes (fp_quantize
     :5101-5205)."""
+    if global_scale is None:
+        out = _fast.quantize(w, group_size, bits, mode)
+        if out is not None:
+            return out
     mode = _mode("quantize", mode)
     group_size, bits = _params_from_mode(mode, group_size, bits)
     if w.dtype not in _FLOATING:
@@ -271,6 +295,10 @@ def dequantize(
 ):
     """``mx.dequantize`` (mlx/ops.cpp:5465-5517 -> affine_dequantize :5248-5340,
     fp_dequantize :5342-5462)."""
+    if global_scale is None:
+        out = _fast.dequantize(w, scales, biases, group_size, bits, mode, dtype)
+        if out is not None:
+            return out
     out_type, mode = _validate_mode_with_type("dequantize", scales, biases, dtype, mode)
     group_size, bits = _params_from_mode(mode, group_size, bits)
     gscale = _global_scale("dequantize", mode, global_scale, w)
@@ -392,6 +420,9 @@ def quantized_swiglu(
     ``nn.QuantizedLinear`` holds them (python/mlx/nn/layers/quantized.py:205-307);
     the reference has no fused primitive for the gated MLP, so more rows of x, or
     a device other than the GPU, raise instead of taking another route."""
+    out = _fast.quantized_swiglu(x, gate, up, group_size, bits)
+    if out is not None:
+        return out
     wg, sg, bg = gate
     wu, su, bu = up
     dtype, mode = _validate_mode_with_type("quantized_swiglu", sg, bg, None, "affine")
@@ -441,14 +472,17 @@ class _QuantizedMatmulVjp(torch.autograd.Function):
     def forward(ctx, x, w, scales, biases, transpose, group_size, bits, mode, sb_image):
         ctx.save_for_backward(w, scales, biases if biases is not None else scales)
         ctx.args = (bool(transpose), group_size, bits, mode, biases is None, x.shape, x.dtype)
-        return _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, sb_image)
+        # gradient recording is off in here
+        return quantized_matmul(
+            x, w, scales, biases, transpose, group_size, bits, mode, sb_image=sb_image)
 
     @staticmethod
     def backward(ctx, cotangent):
         w, scales, biases = ctx.saved_tensors
         transpose, group_size, bits, mode, no_biases, x_shape, x_dtype = ctx.args
-        dx = _quantized_matmul(cotangent, w, scales, None if no_biases else biases,
-                               not transpose, group_size, bits, mode, None)
+        with torch.no_grad():  # (as before under create_graph: no second derivative)
+            dx = quantized_matmul(cotangent, w, scales, None if no_biases else biases,
+                                  not transpose, group_size, bits, mode)
         if tuple(dx.shape) != tuple(x_shape):
             raise NotImplementedError(
                 "[QuantizedMatmul::vjp] x was broadcast against a batched weight: "
@@ -475,6 +509,10 @@ def quantized_matmul(
     results do not depend on it.  Under autograd the gradient with respect to x
     is the reference's (QuantizedMatmul::vjp, mlx/primitives.cpp:3532-3555);
     gradients with respect to scales and biases are not provided."""
+    out = _fast.quantized_matmul(
+        x, w, scales, biases, transpose, group_size, bits, mode, sb_image)
+    if out is not None:
+        return out
     if torch.is_grad_enabled():
         wants = [t is not None and t.requires_grad for t in (scales, biases)]
         if any(wants):
@@ -827,6 +865,10 @@ def qqmm(
     quantized w; unlike it, any number of rows of x.  A floating-point w, which
     the CPU backend does not take either, is quantized first as the CUDA backend
     does (mlx/backend/cuda/quantized/qqmm.cpp)."""
+    if global_scale_x is None and global_scale_w is None:
+        out = _fast.qqmm(x, w, scales, group_size, bits, mode)
+        if out is not None:
+            return out
     mode = _mode("qqmm", mode)
     group_size, bits = _params_from_mode(mode, group_size, bits)
     in_shape = tuple(x.shape)

@@ -209,6 +209,32 @@ int mlxrocm_fp_qmm(
     mlxrocm_stream_t stream);
 
 /*
+ * mlxrocm_qmm_rows for the floating-point modes (2..64 rows per problem; 9..64 in
+ * float16, whose range the scales could leave; K a multiple of 128).
+ */
+int mlxrocm_fp_qmm_rows_supported(
+    int M, int N, int K, int L, int mode, int dtype);
+size_t mlxrocm_fp_qmm_rows_workspace_size(
+    int M, int N, int K, int L, int mode, int dtype);
+int mlxrocm_fp_qmm_rows(
+    const void* x,
+    const uint32_t* wq,
+    const uint8_t* scales,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t scales_batch_stride,
+    int mode,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream);
+
+/*
  * qqmm with a quantized second operand (mlx/ops.cpp:4926-4990; CPU:
  * QQMatmul::eval_cpu, mlx/backend/cpu/quantized.cpp:1322-1360, which takes one
  * row of x): y = quantize_dequantize(x) . dequantize(w)^T.  x [M, K] and out
@@ -515,6 +541,38 @@ int mlxrocm_qmm(
     int bits,
     int dtype,
     int transpose,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream);
+
+/*
+ * mlxrocm_qmm with transpose != 0 for the rows of a decode step of some sequences
+ * (3..64 rows per problem, 16-bit types, every width), on the kernel that walks x
+ * through LDS: one pass over W whatever the rows, nothing rounded before the
+ * result.  _supported: 1 where it takes a call and is ahead of mlxrocm_qmm, else 0;
+ * it looks at shapes only.  workspace: device scratch used only during the call,
+ * 16-byte aligned, of _workspace_size bytes (mostly 0, and then it may be NULL).
+ */
+int mlxrocm_qmm_rows_supported(
+    int M, int N, int K, int L, int group_size, int bits, int dtype);
+size_t mlxrocm_qmm_rows_workspace_size(
+    int M, int N, int K, int L, int group_size, int bits, int dtype);
+int mlxrocm_qmm_rows(
+    const void* x,
+    const uint32_t* wq,
+    const void* scales,
+    const void* biases,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t sb_batch_stride,
+    int group_size,
+    int bits,
+    int dtype,
     void* workspace,
     size_t workspace_bytes,
     mlxrocm_stream_t stream);

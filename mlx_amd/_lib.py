@@ -36,6 +36,9 @@ SIGNATURES = {
         _i,
         [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _i, _p, _sz, _p],
     ),
+    "mlxrocm_qmm_rows_supported": (_i, [_i] * 7),
+    "mlxrocm_qmm_rows_workspace_size": (_sz, [_i] * 7),
+    "mlxrocm_qmm_rows": (_i, [_p] * 5 + [_i] * 4 + [_i64] * 3 + [_i] * 3 + [_p, _sz, _p]),
     "mlxrocm_qmm_sb_image_size": (_sz, [_i] * 5),
     "mlxrocm_qmm_sb_image": (_i, [_p, _p, _p, _i, _i, _i, _i64, _i, _i, _p]),
     "mlxrocm_qmm_prepacked": (
@@ -58,6 +61,9 @@ SIGNATURES = {
     "mlxrocm_fp_quantize_dequantize": (_i, [_p, _p, _sz, _i, _i, _p]),
     "mlxrocm_fp_qmm_workspace_size": (_sz, [_i] * 8),
     "mlxrocm_fp_qmm": (_i, [_p] * 4 + [_i] * 4 + [_i64] * 3 + [_i] * 3 + [_p, _sz, _p]),
+    "mlxrocm_fp_qmm_rows_supported": (_i, [_i] * 6),
+    "mlxrocm_fp_qmm_rows_workspace_size": (_sz, [_i] * 6),
+    "mlxrocm_fp_qmm_rows": (_i, [_p] * 4 + [_i] * 4 + [_i64] * 3 + [_i] * 2 + [_p, _sz, _p]),
     "mlxrocm_fp_qqmm_workspace_size": (_sz, [_i] * 5),
     "mlxrocm_fp_qqmm": (_i, [_p] * 4 + [_i] * 5 + [_p, _sz, _p]),
     "mlxrocm_fp_qmm_plan": (_i, [_i] * 8 + [_sz, ctypes.c_char_p, _sz]),

@@ -578,6 +578,17 @@ bool fp_tile_applies(int M, int N, int K, int L, int mode, int dtype, bool trans
       static_cast<uint64_t>(N) * (K / 32) * 4 < limit;
 }
 
+// 2..64 rows (9.. in f16, whose range the scales may leave: below, the streaming
+// kernel applies them in fp32) on the kernel of qmm_walk.h.  Graph replays, bf16
+// [M, 4096] x [14336, 4096], mxfp4 / mxfp8 / nvfp4 against the kernels below: 2
+// rows 10.7 / 16.8 / 13.8 us against 13.0 / 15.9 / 15.4 (mxfp8 from 3 rows on), 8
+// rows 11.1 / 16.8 / 13.9 against 31.9 / 38.4 / 37.2, 32 rows 15.8 / 22.5 / 19.0
+// against 31.5 / 34.2 / 33.1, 64 rows 21.6 / 25.8 / 25 against 32.9 / 36.0 / 34.7.
+bool fp_walk_applies(const QmmArgs& a, int mode, int dtype) {
+  const int least = dtype != MLXROCM_BFLOAT16 ? 9 : mode == MLXROCM_MXFP8 ? 3 : 2;
+  return a.M >= least && a.K >= 1024 && qmm_walk_fp_supported(a, mode, dtype);
+}
+
 size_t fp_image_bytes(int N, int K, int batches) {
   return (static_cast<size_t>(batches) * N * (K / 32) * 4 + 255) / 256 * 256;
 }
@@ -667,6 +678,15 @@ int fp_launch(const QmmArgs& a, int mode, int dtype, bool transpose, hipStream_t
   });
 }
 
+QmmArgs fp_shape(int M, int N, int K, int L) {
+  QmmArgs a{};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.L = L;
+  return a;
+}
+
 bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
@@ -697,7 +717,8 @@ int fp_qmm_entry(
     void* workspace,
     size_t workspace_bytes,
     mlxrocm_stream_t stream,
-    const float* out_scale = nullptr) {
+    const float* out_scale = nullptr,
+    bool rows = false) { // a call that fp_walk_applies() to
   int rc = fp_check("quantized_matmul", M, N, K, L, mode, dtype, transpose);
   if (rc != MLXROCM_OK) {
     return rc;
@@ -744,6 +765,19 @@ int fp_qmm_entry(
   a.x_batches = L;
   a.n_experts = L;
   a.out_scale = out_scale;
+  if (rows) {
+    const size_t need = qmm_walk_fp_plane_bytes(a, mode);
+    if (need != 0 &&
+        (workspace == nullptr || workspace_bytes < need ||
+         (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0)) {
+      return fail(
+          MLXROCM_INVALID_ARGUMENT,
+          "[quantized_matmul] this shape needs a 16-byte aligned workspace of %zu bytes "
+          "(mlxrocm_fp_qmm_rows_workspace_size); got %zu",
+          need, workspace_bytes);
+    }
+    return launch_qmm_walk_fp(a, mode, dtype, workspace, s);
+  }
   if (fp_tile_applies(M, N, K, L, mode, dtype, transpose != 0)) {
     const int batches = scales_batch_stride != 0 ? L : 1;
     const size_t need = fp_tile_workspace(M, N, K, L, batches);
@@ -827,6 +861,46 @@ extern "C" int mlxrocm_fp_qmm(
       dtype, transpose, workspace, workspace_bytes, stream);
 }
 
+extern "C" int mlxrocm_fp_qmm_rows_supported(int M, int N, int K, int L, int mode, int dtype) {
+  return M >= 2 && fp_check("quantized_matmul", M, N, K, L, mode, dtype, 1) == MLXROCM_OK &&
+      N > 0 && L > 0 && fp_walk_applies(fp_shape(M, N, K, L), mode, dtype);
+}
+
+extern "C" size_t mlxrocm_fp_qmm_rows_workspace_size(
+    int M, int N, int K, int L, int mode, int dtype) {
+  return mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)
+      ? qmm_walk_fp_plane_bytes(fp_shape(M, N, K, L), mode)
+      : 0;
+}
+
+extern "C" int mlxrocm_fp_qmm_rows(
+    const void* x,
+    const uint32_t* wq,
+    const uint8_t* scales,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t scales_batch_stride,
+    int mode,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream) {
+  mlxrocm::ApiRange api_range("mlxrocm_fp_qmm_rows");
+  if (!mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)) {
+    return fail(
+        MLXROCM_UNSUPPORTED, "[quantized_matmul] M=%d N=%d K=%d: not a shape of the few-row kernel",
+        M, N, K);
+  }
+  return fp_qmm_entry(
+      x, wq, scales, out, M, N, K, L, x_batch_stride, w_batch_stride, scales_batch_stride, mode,
+      dtype, 1, workspace, workspace_bytes, stream, nullptr, true);
+}
+
 extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, int dtype) {
   if (fp_check("qqmm", M, N, K, 1, mode, dtype, 1) != MLXROCM_OK ||
       static_cast<int64_t>(M) * N == 0 || K == 0) {
@@ -837,7 +911,9 @@ extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, 
     return round256(static_cast<size_t>(M) * K * bits / 8) + round256(static_cast<size_t>(M) * K / 32);
   }
   return round256(static_cast<size_t>(M) * K * dtype_size(dtype)) +
-      mlxrocm_fp_qmm_workspace_size(M, N, K, 1, 0, mode, dtype, 1);
+      (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)
+           ? mlxrocm_fp_qmm_rows_workspace_size(M, N, K, 1, mode, dtype)
+           : mlxrocm_fp_qmm_workspace_size(M, N, K, 1, 0, mode, dtype, 1));
 }
 
 extern "C" int mlxrocm_fp_qqmm(
@@ -899,7 +975,8 @@ extern "C" int mlxrocm_fp_qqmm(
   const size_t xhat_bytes = round256(n_elems * dtype_size(dtype));
   return fp_qmm_entry(
       workspace, wq, scales, out, M, N, K, 1, 0, 0, 0, mode, dtype, 1,
-      static_cast<char*>(workspace) + xhat_bytes, workspace_bytes - xhat_bytes, stream);
+      static_cast<char*>(workspace) + xhat_bytes, workspace_bytes - xhat_bytes, stream, nullptr,
+      mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype) != 0);
 }
 
 namespace {
@@ -1339,5 +1416,5 @@ extern "C" int mlxrocm_nvfp4_qqmm_global(
   return fp_qmm_entry(
       workspace, wq, scales, out, M, N, K, 1, 0, 0, 0, mode, dtype, 1,
       static_cast<char*>(workspace) + xhat_bytes, workspace_bytes - xhat_bytes, stream,
-      global_scale_w);
+      global_scale_w, mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype) != 0);
 }

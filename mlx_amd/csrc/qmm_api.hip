@@ -573,6 +573,41 @@ int two_passes(const Call& c, const QmmArgs& head, const QmmArgs& tail) {
   return run(tail, c.gs, c.bits, c.dtype, c.transpose, c.sc, c.s);
 }
 
+// 3..64 rows of x (mlxrocm_qmm_rows), whatever regime of the table below they
+// belong to: where the kernel of qmm_walk.h (rows of W dealt out evenly to the compute units, the whole of K
+// each, x walking through LDS) is ahead of that regime's own.  Graph replays over
+// 15 shapes from 1024 x 1024 to 128256 x 4096, us against the regime's kernel: 4-bit
+// g64 14336 x 4096 16 rows 13.8 against 16.6, 48 rows 21.5 against 33.7, 4096 x 4096
+// 32 rows 9.8 against 14.7, 4096 x 14336 8 rows 13.9 against 15.6; 8-bit 14336 x 4096
+// 8 rows 16.6 against 23.1, 8192 x 8192 8 rows 18.7 against 35.0; 6-bit 14336 x 4096
+// 16 rows 19.1 against 28.7.  It is not where K is short (8-bit 4096 x 2048, 16 rows:
+// 6.5 against 5.8), nor, at 4 bits, where the kernels that keep x in LDS stage it less
+// often: many rounds of workgroups (32000 x 4096, 32 rows: 35.8 against 30.8) or a
+// long K with 9..32 rows (4096 x 14336, 32 rows: 20.6 against 19.5).
+bool walk_pays(const QmmArgs& a, int gs, int bits) {
+  const long per_cu = (static_cast<long>(a.N) * a.L + compute_units() - 1) / compute_units();
+  if (a.M < 3) {
+    return false;
+  }
+  if (a.M > 32) {
+    return true; // everything else takes two passes or a 256-row tile
+  }
+  if (bits != 4) {
+    return a.M <= 8 ? a.K >= (bits == 8 ? 1024 : 2048)
+                    : a.K >= 4096 || (a.K >= 2048 && (bits != 8 || (a.M <= 16 && per_cu > 16)));
+  }
+  if (a.M <= 4) {
+    return false;
+  }
+  if (a.M <= 8) {
+    return per_cu < 56 && a.K >= 1024 && (gs != 32 || a.K < 8192);
+  }
+  if (a.M <= 16) {
+    return per_cu <= 64 && a.K >= 3072 && a.K < (gs == 32 ? 8192 : 11008);
+  }
+  return per_cu <= 64 && a.K >= 2048 && (gs == 32 || a.K < 8192 || per_cu <= 8);
+}
+
 int slab_launch(const Call& c, const QmmArgs& a, void* region) {
   return MLXROCM_LAUNCH(c.sc, launch_qmm_slab(a, c.gs, c.bits, c.dtype, region, c.s));
 }
@@ -1011,6 +1046,10 @@ extern "C" int mlxrocm_qmm_swiglu(
     if (qmv_stream_glu_supported(one, group_size, bits, dtype)) {
       return launch_qmv_stream_glu(one, group_size, bits, dtype, s);
     }
+    // likewise with a few rows where both products would run on the walking kernel
+    if (walk_pays(a, group_size, bits) && qmm_walk_glu_supported(one, group_size, bits, dtype)) {
+      return launch_qmm_walk_glu(one, group_size, bits, dtype, s);
+    }
   }
   Scratch none; // decode shapes with transpose != 0 claim no scratch
   rc = run(a, group_size, bits, dtype, true, none, s);
@@ -1155,6 +1194,94 @@ extern "C" int mlxrocm_qmm(
       x, wq, scales, biases, out, M, N, K, L, x_batch_stride, w_batch_stride,
       sb_batch_stride, group_size, bits, dtype, transpose, sc,
       static_cast<hipStream_t>(stream));
+}
+
+namespace {
+
+QmmArgs rows_shape(int M, int N, int K, int L) {
+  QmmArgs a{};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.L = L;
+  return a;
+}
+
+} // namespace
+
+extern "C" int mlxrocm_qmm_rows_supported(
+    int M, int N, int K, int L, int group_size, int bits, int dtype) {
+  if (M <= 0 || N <= 0 || L <= 0 ||
+      check_shape("quantized_matmul", M, N, K, L, group_size, bits, dtype, 1) != MLXROCM_OK) {
+    return 0;
+  }
+  const QmmArgs a = rows_shape(M, N, K, L);
+  return walk_pays(a, group_size, bits) && qmm_walk_supported(a, group_size, bits, dtype, true);
+}
+
+extern "C" size_t mlxrocm_qmm_rows_workspace_size(
+    int M, int N, int K, int L, int group_size, int bits, int dtype) {
+  return mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)
+      ? qmm_walk_plane_bytes(rows_shape(M, N, K, L), group_size, bits)
+      : 0;
+}
+
+extern "C" int mlxrocm_qmm_rows(
+    const void* x,
+    const uint32_t* wq,
+    const void* scales,
+    const void* biases,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t sb_batch_stride,
+    int group_size,
+    int bits,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream) {
+  mlxrocm::ApiRange api_range("mlxrocm_qmm_rows");
+  if (!mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)) {
+    return fail(
+        MLXROCM_UNSUPPORTED, "[quantized_matmul] M=%d N=%d K=%d: not a shape of the few-row kernel",
+        M, N, K);
+  }
+  if (!x || !wq || !scales || !biases || !out) {
+    return fail(MLXROCM_INVALID_ARGUMENT, "[quantized_matmul] null device pointer");
+  }
+  if (x_batch_stride < 0 || w_batch_stride < 0 || sb_batch_stride < 0) {
+    return fail(MLXROCM_INVALID_ARGUMENT, "[quantized_matmul] negative stride");
+  }
+  QmmArgs a = rows_shape(M, N, K, L);
+  a.x = x;
+  a.w = wq;
+  a.scales = scales;
+  a.biases = biases;
+  a.out = out;
+  a.x_batch_stride = x_batch_stride;
+  a.w_batch_stride = w_batch_stride;
+  a.sb_batch_stride = sb_batch_stride;
+  a.x_batches = L;
+  a.n_experts = L;
+  const int rc = check_alignment("quantized_matmul", a, dtype, true, bits);
+  if (rc != MLXROCM_OK) {
+    return rc;
+  }
+  const size_t need = qmm_walk_plane_bytes(a, group_size, bits);
+  if (need != 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {
+    return fail(
+        MLXROCM_INVALID_ARGUMENT,
+        "[quantized_matmul] this shape needs a 16-byte aligned workspace of %zu bytes "
+        "(mlxrocm_qmm_rows_workspace_size); got %zu",
+        need, workspace_bytes);
+  }
+  return launch_qmm_walk(
+      a, group_size, bits, dtype, workspace, static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t mlxrocm_qmm_sb_image_size(int N, int K, int batches, int group_size, int dtype) {

@@ -164,6 +164,19 @@ bool qmm_skinny_supported(const QmmArgs& a, int gs, int bits, int dtype, bool tr
 int launch_qmm_skinny(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 int launch_zero_fill(void* p, size_t bytes, hipStream_t s);
 
+// 2..64 rows of x walking through LDS (qmm_walk.h); `planes` of
+// qmm_walk_plane_bytes() where K is cut into ranges.
+bool qmm_walk_supported(const QmmArgs& a, int gs, int bits, int dtype, bool transpose);
+size_t qmm_walk_plane_bytes(const QmmArgs& a, int gs, int bits);
+int launch_qmm_walk(const QmmArgs& a, int gs, int bits, int dtype, void* planes, hipStream_t s);
+// floating-point modes
+bool qmm_walk_fp_supported(const QmmArgs& a, int mode, int dtype);
+size_t qmm_walk_fp_plane_bytes(const QmmArgs& a, int mode);
+int launch_qmm_walk_fp(const QmmArgs& a, int mode, int dtype, void* planes, hipStream_t s);
+// silu(w . x) * (w_alt . x) in one launch (L = 1)
+bool qmm_walk_glu_supported(const QmmArgs& a, int gs, int bits, int dtype);
+int launch_qmm_walk_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
+
 // Grouping of gathered index pairs by expert (gather_group.hip) and the grouped
 // launch of the matrix-core GEMM over its tiles (qmm_mfma.hip).
 constexpr int kGroupLargeTile = 256; // rows per tile of the tile GEMM

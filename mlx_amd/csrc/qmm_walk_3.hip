@@ -1,0 +1,12 @@
+// qmm_walk_3.hip -- the kernel of qmm_walk.h for 3-bit codes.
+#include "qmm_walk.h"
+
+namespace mlxrocm {
+
+int launch_walk_3(
+    const WalkArgs& wa, const WalkPlan& pl, int gs, int dtype, int table_groups, const dim3& grid,
+    hipStream_t s) {
+  return launch_walk_bits<3>(wa, pl, gs, dtype, table_groups, grid, s);
+}
+
+} // namespace mlxrocm

@@ -38,8 +38,14 @@ struct Abi {
   decltype(&mlxrocm_qmm_workspace_size) qmm_workspace_size;
   decltype(&mlxrocm_qmm_prepacked) qmm_prepacked;
   decltype(&mlxrocm_qmm_sb_image_size) qmm_sb_image_size;
+  decltype(&mlxrocm_qmm_rows_supported) rows_supported;
+  decltype(&mlxrocm_qmm_rows_workspace_size) rows_workspace_size;
+  decltype(&mlxrocm_qmm_rows) rows;
   decltype(&mlxrocm_fp_qmm_workspace_size) fp_qmm_workspace_size;
   decltype(&mlxrocm_fp_qmm) fp_qmm;
+  decltype(&mlxrocm_fp_qmm_rows_supported) fp_rows_supported;
+  decltype(&mlxrocm_fp_qmm_rows_workspace_size) fp_rows_workspace_size;
+  decltype(&mlxrocm_fp_qmm_rows) fp_rows;
   decltype(&mlxrocm_qmm_swiglu_workspace_size) swiglu_workspace_size;
   decltype(&mlxrocm_qmm_swiglu) swiglu;
   decltype(&mlxrocm_fp_qqmm_workspace_size) fp_qqmm_workspace_size;
@@ -267,7 +273,15 @@ PyObject* quantized_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor out = new_tensor(with_last(*x, N), x->scalar_type(), device);
   void* stream = stream_of(device);
   int rc = 0;
-  if (mode == kAffine) {
+  if (mode == kAffine && transpose && abi.rows_supported(M, N, K, 1, gs, bits, code)) {
+    const Workspace ws(abi.rows_workspace_size(M, N, K, 1, gs, bits, code), device);
+    Py_BEGIN_ALLOW_THREADS;
+    rc = abi.rows(
+        x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
+        biases->data_ptr(), out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code, ws.ptr(),
+        ws.bytes, stream);
+    Py_END_ALLOW_THREADS;
+  } else if (mode == kAffine) {
     const Workspace ws(
         abi.qmm_workspace_size(M, N, K, 1, 0, gs, bits, code, transpose), device);
     Py_BEGIN_ALLOW_THREADS;
@@ -275,6 +289,14 @@ PyObject* quantized_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
         x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
         biases->data_ptr(), image, out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code,
         transpose, ws.ptr(), ws.bytes, stream);
+    Py_END_ALLOW_THREADS;
+  } else if (transpose && abi.fp_rows_supported(M, N, K, 1, mode, code)) {
+    const Workspace ws(abi.fp_rows_workspace_size(M, N, K, 1, mode, code), device);
+    Py_BEGIN_ALLOW_THREADS;
+    rc = abi.fp_rows(
+        x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()),
+        static_cast<const uint8_t*>(scales->data_ptr()), out.data_ptr(), M, N, K, 1, M * K, 0, 0,
+        mode, code, ws.ptr(), ws.bytes, stream);
     Py_END_ALLOW_THREADS;
   } else {
     const Workspace ws(abi.fp_qmm_workspace_size(M, N, K, 1, 0, mode, code, transpose), device);
@@ -556,8 +578,14 @@ PyObject* bind(PyObject*, PyObject* table) {
   bound = take("mlxrocm_qmm_workspace_size", abi.qmm_workspace_size) &&
       take("mlxrocm_qmm_prepacked", abi.qmm_prepacked) &&
       take("mlxrocm_qmm_sb_image_size", abi.qmm_sb_image_size) &&
+      take("mlxrocm_qmm_rows_supported", abi.rows_supported) &&
+      take("mlxrocm_qmm_rows_workspace_size", abi.rows_workspace_size) &&
+      take("mlxrocm_qmm_rows", abi.rows) &&
       take("mlxrocm_fp_qmm_workspace_size", abi.fp_qmm_workspace_size) &&
       take("mlxrocm_fp_qmm", abi.fp_qmm) &&
+      take("mlxrocm_fp_qmm_rows_supported", abi.fp_rows_supported) &&
+      take("mlxrocm_fp_qmm_rows_workspace_size", abi.fp_rows_workspace_size) &&
+      take("mlxrocm_fp_qmm_rows", abi.fp_rows) &&
       take("mlxrocm_qmm_swiglu_workspace_size", abi.swiglu_workspace_size) &&
       take("mlxrocm_qmm_swiglu", abi.swiglu) &&
       take("mlxrocm_fp_qqmm_workspace_size", abi.fp_qqmm_workspace_size) &&

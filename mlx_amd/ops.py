@@ -587,6 +587,19 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
     out = torch.empty(out_shape, dtype=dtype, device=x.device)
     code = _DTYPE_CODE[dtype]
     if not affine:
+        fp = _MODE_CODE[mode]
+        if transpose and lib.mlxrocm_fp_qmm_rows_supported(M, w_outer, K, L, fp, code):
+            # the rows of a decode step of some sequences
+            ws_bytes = lib.mlxrocm_fp_qmm_rows_workspace_size(M, w_outer, K, L, fp, code)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+            _lib.check(
+                lib.mlxrocm_fp_qmm_rows(
+                    xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), out.data_ptr(),
+                    M, w_outer, K, L, M * K, w_stride, sb_stride, fp, code,
+                    ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(x),
+                )
+            )
+            return out
         ws_bytes = lib.mlxrocm_fp_qmm_workspace_size(
             M, w_outer, K, L, int(sb_stride != 0), _MODE_CODE[mode], code, int(bool(transpose)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
@@ -600,6 +613,18 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
         )
         return out
     bb, _ = _dense_batches(biases, batch_shape)
+    if transpose and sb_image is None and lib.mlxrocm_qmm_rows_supported(
+            M, w_outer, K, L, group_size, bits, code):
+        ws_bytes = lib.mlxrocm_qmm_rows_workspace_size(M, w_outer, K, L, group_size, bits, code)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+        _lib.check(
+            lib.mlxrocm_qmm_rows(
+                xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(), out.data_ptr(),
+                M, w_outer, K, L, M * K, w_stride, sb_stride, group_size, bits, code,
+                ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(x),
+            )
+        )
+        return out
     ws_bytes = lib.mlxrocm_qmm_workspace_size(
         M, w_outer, K, L, int(w_stride != 0), group_size, bits, code, int(bool(transpose))
     )

@@ -160,13 +160,36 @@ void QuantizedMatmul::eval_gpu(const std::vector<array>& inputs, array& out) {
   if (!affine) {
     // inputs are {x, w, scales}: no biases (mlx/ops.cpp:4816-4821)
     const int mode = fp_mode_code(mode_);
-    const size_t ws_bytes = mlxrocm_fp_qmm_workspace_size(
-        M, N, K, L, w.ndim() > 2, mode, dt, transpose_ ? 1 : 0);
+    // the rows of a decode step of some sequences have a kernel of their own
+    const bool rows = transpose_ && mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dt) != 0;
+    const size_t ws_bytes = rows
+        ? mlxrocm_fp_qmm_rows_workspace_size(M, N, K, L, mode, dt)
+        : mlxrocm_fp_qmm_workspace_size(M, N, K, L, w.ndim() > 2, mode, dt, transpose_ ? 1 : 0);
     void* ws_ptr = nullptr;
     if (ws_bytes > 0) {
       array ws = workspace_array(ws_bytes);
       enc.add_temporary(ws);
       ws_ptr = rocm::gpu_ptr<void>(ws, enc.stream());
+    }
+    if (rows) {
+      rocm::check(mlxrocm_fp_qmm_rows(
+          rocm::gpu_ptr<void>(x, enc.stream()),
+          rocm::gpu_ptr<uint32_t>(w, enc.stream()),
+          rocm::gpu_ptr<uint8_t>(scales, enc.stream()),
+          rocm::gpu_ptr<void>(out, enc.stream()),
+          M,
+          N,
+          K,
+          L,
+          int64_t(M) * K,
+          w_stride,
+          sb_stride,
+          mode,
+          dt,
+          ws_ptr,
+          ws_bytes,
+          enc.stream()));
+      return;
     }
     rocm::check(mlxrocm_fp_qmm(
         rocm::gpu_ptr<void>(x, enc.stream()),
@@ -190,9 +213,14 @@ void QuantizedMatmul::eval_gpu(const std::vector<array>& inputs, array& out) {
   }
   array biases = ensure_row_contiguous(inputs[3], enc, s);
 
+  // the rows of a decode step of some sequences have a kernel of their own
+  const bool rows = transpose_ &&
+      mlxrocm_qmm_rows_supported(M, N, K, L, group_size_, bits_, dt) != 0;
   // device scratch of the call: a temporary like any other
-  const size_t ws_bytes = mlxrocm_qmm_workspace_size(
-      M, N, K, L, w.ndim() > 2, group_size_, bits_, dt, transpose_ ? 1 : 0);
+  const size_t ws_bytes = rows
+      ? mlxrocm_qmm_rows_workspace_size(M, N, K, L, group_size_, bits_, dt)
+      : mlxrocm_qmm_workspace_size(
+            M, N, K, L, w.ndim() > 2, group_size_, bits_, dt, transpose_ ? 1 : 0);
   void* ws_ptr = nullptr;
   if (ws_bytes > 0) {
     array ws = workspace_array(ws_bytes);
@@ -200,6 +228,28 @@ void QuantizedMatmul::eval_gpu(const std::vector<array>& inputs, array& out) {
     ws_ptr = rocm::gpu_ptr<void>(ws, enc.stream());
   }
 
+  if (rows) {
+    rocm::check(mlxrocm_qmm_rows(
+        rocm::gpu_ptr<void>(x, enc.stream()),
+        rocm::gpu_ptr<uint32_t>(w, enc.stream()),
+        rocm::gpu_ptr<void>(scales, enc.stream()),
+        rocm::gpu_ptr<void>(biases, enc.stream()),
+        rocm::gpu_ptr<void>(out, enc.stream()),
+        M,
+        N,
+        K,
+        L,
+        int64_t(M) * K,
+        w_stride,
+        sb_stride,
+        group_size_,
+        bits_,
+        dt,
+        ws_ptr,
+        ws_bytes,
+        enc.stream()));
+    return;
+  }
   rocm::check(mlxrocm_qmm(
       rocm::gpu_ptr<void>(x, enc.stream()),
       rocm::gpu_ptr<uint32_t>(w, enc.stream()),

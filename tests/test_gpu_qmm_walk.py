@@ -1,0 +1,121 @@
+"""The few-row kernel whose x walks through LDS: the edges of its tiles of rows of
+W and x, its 128-code chunks and stages, K ranges, every width, group and mode,
+against the exact product of the dequantized weights."""
+import pytest
+import torch
+
+import mlx_amd
+from mlx_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (2, 3, 5, 8, 9, 16, 17, 31, 33, 48, 49, 64)
+# N and K: less than a tile, ragged tiles, a ragged last chunk (K % 128), a last
+# stage of one chunk, one and several rounds of workgroups, K in ranges
+SHAPES = ((4, 1024), (67, 1120), (1000, 2080), (4096, 4096), (5001, 1152), (33000, 1024),
+          (512, 14336))
+
+
+def _check(x, q, group, bits, mode, y):
+    # bf16 / f16 products are exact in fp32; sums are fp32 over K terms: the result
+    # is within half an ulp of its type of the exact sum, plus the sums' own 2e-6
+    if mode == "affine":
+        w = mlx_amd.dequantize(q[0], q[1].float(), q[2].float(), group, bits).double()
+    else:
+        w = mlx_amd.dequantize(q[0], q[1], mode=mode, dtype=torch.float32).double()
+    want = x.double() @ w.T
+    size = x.double().abs() @ w.abs().T
+    # (codes are multiplied with an offset of at most 1024 that the biases take back,
+    # in fp32: 1024 / (2^bits - 1) times the size of the product at worst)
+    sums = 2e-6 * (1 if mode != "affine" else 1 + 1024 / (2 ** bits - 1) / 8)
+    half = 2.0 ** -8 if x.dtype == torch.bfloat16 else 2.0 ** -11
+    err = (y.double() - want).abs()
+    ok = bool((err <= half * want.abs() + sums * size).all())
+    assert ok, (tuple(x.shape), tuple(q[0].shape), group, bits, mode, float((err / size).max()))
+
+
+def _inputs(M, N, K, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((N, K), generator=g, device="cuda") * K ** -0.5).to(dtype)
+    return x, w
+
+
+@pytest.mark.parametrize("bits", (2, 3, 4, 5, 6, 8))
+@pytest.mark.parametrize("group", (32, 64, 128))
+def test_affine(bits, group):
+    taken = 0
+    for i, (N, K) in enumerate(SHAPES):
+        K = K // group * group
+        dtype = (torch.bfloat16, torch.float16)[(i + bits) % 2]
+        for M in ROWS[(i + bits) % 2::2]:
+            if not _lib.load().mlxrocm_qmm_rows_supported(
+                    M, N, K, 1, group, bits, 2 if dtype == torch.bfloat16 else 1):
+                continue  # (kernels that round the weights to the type: another bound)
+            taken += 1
+            x, w = _inputs(M, N, K, dtype, M + N)
+            q = mlx_amd.quantize(w, group, bits)
+            y = mlx_amd.quantized_matmul(x, *q, group_size=group, bits=bits)
+            _check(x, q, group, bits, "affine", y)
+    assert taken >= 18, taken
+
+
+@pytest.mark.parametrize("mode", ("mxfp4", "mxfp8", "nvfp4"))
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+def test_fp_modes(mode, dtype):
+    taken = 0
+    for N, K in SHAPES:
+        K = K // 32 * 32
+        for M in ROWS:
+            x, w = _inputs(M, N, K, dtype, M + N)
+            q = mlx_amd.quantize(w, mode=mode)
+            taken += _lib.load().mlxrocm_fp_qmm_rows_supported(
+                M, N, K, 1, _lib.MXFP4 + ("mxfp4", "mxfp8", "nvfp4").index(mode),
+                2 if dtype == torch.bfloat16 else 1)
+            _check(x, q, None, None, mode, mlx_amd.quantized_matmul(x, *q, mode=mode))
+    assert taken >= 30
+
+
+def test_fp8_codes_that_no_quantizer_writes():
+    # 0x7f and 0xff stand for +-480, not NaN
+    x, w = _inputs(8, 96, 1024, torch.bfloat16, 3)
+    wq, scales = mlx_amd.quantize(w, mode="mxfp8")
+    codes = wq.view(torch.uint8).clone()
+    codes[::7, ::97] = 0x7F
+    codes[3::11, 5::64] = 0xFF
+    q = (codes.view(torch.uint32), scales)
+    _check(x, q, None, None, "mxfp8", mlx_amd.quantized_matmul(x, *q, mode="mxfp8"))
+
+
+def test_stacks_of_weights_and_the_tensor_wide_scale():
+    x, w = _inputs(24, 640, 4096, torch.bfloat16, 5)
+    q = mlx_amd.quantize(w.reshape(2, 320, 4096), 64, 8)
+    y = mlx_amd.quantized_matmul(x.reshape(2, 12, 4096), *q, group_size=64, bits=8)
+    for i in range(2):
+        _check(x.reshape(2, 12, 4096)[i], [t[i] for t in q], 64, 8, "affine", y[i])
+    qf = mlx_amd.quantize(w.reshape(2, 320, 4096), mode="mxfp4")
+    y = mlx_amd.quantized_matmul(x.reshape(2, 12, 4096), *qf, mode="mxfp4")
+    for i in range(2):
+        _check(x.reshape(2, 12, 4096)[i], [t[i] for t in qf], None, None, "mxfp4", y[i])
+    # nvfp4 with global scales goes through qqmm: 24 rows against one row at a time
+    one = torch.ones((), device="cuda")
+    g = w.abs().max().float()
+    qn = mlx_amd.quantize(w, mode="nvfp4", global_scale=g)
+    kw = dict(mode="nvfp4", global_scale_x=one, global_scale_w=g)
+    y = mlx_amd.qqmm(x, *qn, **kw)
+    rows = torch.cat([mlx_amd.qqmm(x[i:i + 1], *qn, **kw) for i in range(24)])
+    assert float((y.double() - rows.double()).norm() / rows.double().norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("bits,group,N,K", ((8, 128, 18944, 3584), (8, 64, 4099, 1024),
+                                            (4, 32, 5504, 2048), (6, 64, 9000, 2048)))
+def test_gated_form(bits, group, N, K):
+    for M in (3, 5, 8):
+        x, gate = _inputs(M, N, K, torch.bfloat16, 1)
+        _, up = _inputs(M, N, K, torch.bfloat16, 2)
+        g, u = mlx_amd.quantize(gate, group, bits), mlx_amd.quantize(up, group, bits)
+        y = mlx_amd.quantized_swiglu(x, g, u, group, bits).double()
+        a, b = (mlx_amd.quantized_matmul(x, *q, group_size=group, bits=bits) for q in (g, u))
+        want = ((a.float() * torch.sigmoid(a.float()).bfloat16()).bfloat16() * b).double()
+        # same sums in another order, then the same four roundings: a few last places
+        assert float((y - want).norm() / want.norm()) < 2.0 ** -7

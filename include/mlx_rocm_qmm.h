@@ -663,6 +663,44 @@ int mlxrocm_qmm_static(
     mlxrocm_stream_t stream);
 
 /*
+ * The expert-routed gated MLP: out[t, j] = h W_down[e]^T with
+ * h = silu(x[t] W_gate[e]^T) * (x[t] W_up[e]^T) and e = indices[t, j] -- three
+ * mlxrocm_gather_qmm calls and the arithmetic between them (each product, the
+ * activation and h rounded to dtype) as one.  x [tokens, D], indices [tokens, top]
+ * of 4 or 8 bytes (index_bytes), gate and up [n_experts, F, D], down [n_experts, D, F]
+ * (dense stacks), out [tokens, top, D]; 16-bit dtypes.  Rows whose index is out of
+ * range are zero.  workspace: 16-byte aligned, mlxrocm_switch_glu_workspace_size
+ * bytes (0: not a shape of this call), used only during the call.
+ */
+size_t mlxrocm_switch_glu_workspace_size(
+    int tokens, int top, int D, int F, int n_experts, int group_size, int bits, int dtype);
+int mlxrocm_switch_glu(
+    const void* x,
+    const void* indices,
+    int index_bytes,
+    const uint32_t* gate_w,
+    const void* gate_scales,
+    const void* gate_biases,
+    const uint32_t* up_w,
+    const void* up_scales,
+    const void* up_biases,
+    const uint32_t* down_w,
+    const void* down_scales,
+    const void* down_biases,
+    void* out,
+    int tokens,
+    int top,
+    int D,
+    int F,
+    int n_experts,
+    int group_size,
+    int bits,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream);
+
+/*
  * Gated-MLP decode: out = silu(x @ dequant(w_gate).T) * (x @ dequant(w_up).T),
  * both projections in one launch over the shared x, then one elementwise pass.
  * No single primitive of the reference corresponds to it: it fuses the two

@@ -49,6 +49,8 @@ SIGNATURES = {
         _i,
         [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _i, _p],
     ),
+    "mlxrocm_switch_glu_workspace_size": (_sz, [_i] * 8),
+    "mlxrocm_switch_glu": (_i, [_p] * 2 + [_i] + [_p] * 10 + [_i] * 8 + [_p, _sz, _p]),
     "mlxrocm_qmm_swiglu_workspace_size": (_sz, [_i, _i, _i]),
     "mlxrocm_qmm_swiglu": (_i, [_p] * 9 + [_i] * 6 + [_p]),
     "mlxrocm_gather_qmm": (

@@ -148,6 +148,29 @@ __global__ __launch_bounds__(256) void group_scatter_kernel(
 constexpr int kFusedThreads = 1024;
 constexpr int kFusedMaxPairs = 16384;
 
+// counter[key] += 1 for every lane with `live`; returns the lane's old value.  The
+// lanes of a wavefront that share a key find each other by ballots over the key's
+// bits and go together: one atomic instruction per wavefront, an address per key.
+// (One per lane serializes on the counters of a few experts.)
+__device__ __forceinline__ int wave_counter_add(
+    int32_t* counter, uint32_t key, bool live, int key_bits) {
+  const int lane = threadIdx.x & 63;
+  uint64_t same = __ballot(live);
+  for (int b = 0; b < key_bits; ++b) {
+    const uint64_t ones = __ballot((key >> b) & 1u);
+    same &= (key >> b) & 1u ? ones : ~ones;
+  }
+  const int leader = __ffsll(static_cast<unsigned long long>(same)) - 1;
+  int base = 0;
+  if (live && lane == leader) {
+    base = atomicAdd(&counter[key], __popcll(same));
+  }
+  base = __shfl(base, leader < 0 ? 0 : leader, 64);
+  return base + __popcll(same & ((uint64_t{1} << lane) - 1));
+}
+
+// (every pair's expert stays in a register between the two passes: the loads of all
+// of them are in flight together)
 template <typename T>
 __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     const uint32_t* lhs,
@@ -155,6 +178,7 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     int n_indices,
     int x_batches,
     int n_experts,
+    int key_bits,
     int tile_rows,
     int32_t* offsets,
     int32_t* tiles,
@@ -162,22 +186,36 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     int32_t* perm,
     T* out,
     int N) {
+  constexpr int kPer = kFusedMaxPairs / kFusedThreads;
+  constexpr uint32_t kNone = 0xffffffffu;
   __shared__ int32_t cnt[kMaxExperts];
   __shared__ int32_t first_pos[kMaxExperts];
   __shared__ int32_t first_tile[kMaxExperts]; // later: the scatter cursor
+  uint32_t key[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int l = i * kFusedThreads + threadIdx.x;
+    key[i] = kNone;
+    if (l < n_indices) {
+      const uint32_t xi = lhs[l];
+      const uint32_t wi = rhs[l];
+      key[i] = xi < static_cast<uint32_t>(x_batches) && wi < static_cast<uint32_t>(n_experts)
+          ? wi : kNone - 1;
+    }
+  }
   for (int e = threadIdx.x; e < n_experts; e += kFusedThreads) {
     cnt[e] = 0;
   }
   __syncthreads();
-  for (int l = threadIdx.x; l < n_indices; l += kFusedThreads) {
-    const uint32_t xi = lhs[l];
-    const uint32_t wi = rhs[l];
-    if (xi < static_cast<uint32_t>(x_batches) && wi < static_cast<uint32_t>(n_experts)) {
-      atomicAdd(&cnt[wi], 1);
-    } else {
-      T* row = out + static_cast<size_t>(l) * N;
-      for (int n = 0; n < N; ++n) {
-        row[n] = static_cast<T>(0.0f);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i * kFusedThreads < n_indices) { // (uniform: whole wavefronts stay together)
+      wave_counter_add(cnt, key[i], key[i] < static_cast<uint32_t>(n_experts), key_bits);
+      if (key[i] == kNone - 1) {
+        T* row = out + static_cast<size_t>(i * kFusedThreads + threadIdx.x) * N;
+        for (int n = 0; n < N; ++n) {
+          row[n] = static_cast<T>(0.0f);
+        }
       }
     }
   }
@@ -207,15 +245,17 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
   }
   __syncthreads();
   for (int e = threadIdx.x; e < n_experts; e += kFusedThreads) {
-    first_tile[e] = 0;
+    first_tile[e] = first_pos[e];
   }
   __syncthreads();
-  for (int l = threadIdx.x; l < n_indices; l += kFusedThreads) {
-    const uint32_t xi = lhs[l];
-    const uint32_t wi = rhs[l];
-    if (xi < static_cast<uint32_t>(x_batches) && wi < static_cast<uint32_t>(n_experts)) {
-      const int rank = atomicAdd(&first_tile[wi], 1);
-      perm[first_pos[wi] + rank] = l;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i * kFusedThreads < n_indices) {
+      const bool live = key[i] < static_cast<uint32_t>(n_experts);
+      const int pos = wave_counter_add(first_tile, key[i], live, key_bits);
+      if (live) {
+        perm[pos] = i * kFusedThreads + threadIdx.x;
+      }
     }
   }
 }
@@ -277,13 +317,17 @@ int launch_gather_group(QmmArgs& a, int dtype, int tile_rows, void* workspace, h
   MLXROCM_REHEARSE(n <= kFusedMaxPairs ? "gather_group(fused)" : "gather_group(3 kernels)");
   a.group_tile_rows = tile_rows;
   if (n <= kFusedMaxPairs) {
+    int key_bits = 1;
+    while ((1 << key_bits) < E) {
+      ++key_bits;
+    }
     if (dtype == MLXROCM_BFLOAT16) {
       group_fused_kernel<bf16_t><<<1, kFusedThreads, 0, s>>>(
-          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, tile_rows, offsets, tiles, n_tiles,
+          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, offsets, tiles, n_tiles,
           perm, static_cast<bf16_t*>(a.out), a.N);
     } else {
       group_fused_kernel<f16_t><<<1, kFusedThreads, 0, s>>>(
-          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, tile_rows, offsets, tiles, n_tiles,
+          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, offsets, tiles, n_tiles,
           perm, static_cast<f16_t*>(a.out), a.N);
     }
     MLXROCM_HIP_TRY(hipGetLastError());

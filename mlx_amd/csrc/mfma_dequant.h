@@ -41,6 +41,19 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, Tx2));
 }
 
+// One of the two T of a dword, as a float.
+template <typename T>
+__device__ __forceinline__ float half_of(uint32_t v, int which) {
+  return to_f32(__builtin_bit_cast(T, static_cast<uint16_t>(which != 0 ? v >> 16 : v)));
+}
+
+// silu(g) * u for values of T: the activation is rounded to T before the product
+// (whose rounding is the caller's), as an elementwise silu followed by a multiply does.
+template <typename T>
+__device__ __forceinline__ float gated(float g, float u) {
+  return round_to<T>(g / (1.0f + __expf(-g))) * u;
+}
+
 // Code i (0..31) of the 32 codes held in BITS consecutive dwords.
 template <int BITS>
 __device__ __forceinline__ uint32_t code32(const uint32_t (&w)[BITS], int i) {

@@ -1,0 +1,56 @@
+// qmm_mfma_experts.hip -- the tile kernel on tiles of rows routed to one expert,
+// with the pair image of scales and biases: the two launches of an expert-routed
+// gated MLP (switch_glu.hip).
+#include "qmm_mfma_tile.h"
+
+namespace mlxrocm {
+
+// Row tiles that a routing of `pairs` rows to `experts` makes: every expert ends
+// on a partial tile, half of one on average.
+int expected_tiles(int pairs, int experts) {
+  return (pairs + kBM - 1) / kBM + experts / 2;
+}
+
+// h = silu(x W_gate^T) * (x W_up^T): a.w / a.scales the gate weights and their pair
+// images, a.w_alt / a.scales_alt the up weights.  256-column tiles, 128 of each.
+int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s) {
+  constexpr int kNT = 8;
+  MLXROCM_REHEARSE("qmm_t_tile_experts_glu(nt=%d)", kNT);
+  const int gs_shift = shift_of(gs);
+  const dim3 grid(
+      (a.N + 16 * kNT - 1) / (16 * kNT), gather_group_max_tiles(a.L, a.n_experts, kGroupLargeTile), 1);
+  auto run = [&](auto tval) -> int {
+    using T = decltype(tval);
+    return dispatch_bits(bits, [&](auto bval) {
+      constexpr int B = decltype(bval)::value;
+      return launch_variant<T, T, T, B, kNT, true, false, true, 0, true>(a, gs_shift, grid, s);
+    });
+  };
+  return dtype == MLXROCM_BFLOAT16 ? run(bf16_t{}) : run(f16_t{});
+}
+
+int launch_qmm_mfma_experts(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s) {
+  const int gs_shift = shift_of(gs);
+  // the tile count is on the device: the width that suits the expected one
+  const int nt = choose_nt(expected_tiles(a.L, a.n_experts) * kBM, a.N, 1);
+  MLXROCM_REHEARSE("qmm_t_tile_experts(nt=%d)", nt);
+  const dim3 grid(
+      (a.N + 32 * nt - 1) / (32 * nt), gather_group_max_tiles(a.L, a.n_experts, kGroupLargeTile), 1);
+  auto run = [&](auto tval) -> int {
+    using T = decltype(tval);
+    return dispatch_bits(bits, [&](auto bval) {
+      constexpr int B = decltype(bval)::value;
+      switch (nt) {
+        case 5:
+          return launch_variant<T, T, T, B, 5, true, false, true>(a, gs_shift, grid, s);
+        case 6:
+          return launch_variant<T, T, T, B, 6, true, false, true>(a, gs_shift, grid, s);
+        default:
+          return launch_variant<T, T, T, B, 7, true, false, true>(a, gs_shift, grid, s);
+      }
+    });
+  };
+  return dtype == MLXROCM_BFLOAT16 ? run(bf16_t{}) : run(f16_t{});
+}
+
+} // namespace mlxrocm

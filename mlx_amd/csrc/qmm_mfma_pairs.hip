@@ -53,6 +53,55 @@ __global__ __launch_bounds__(256) void interleave_sb_kernel(
   }
 }
 
+// The same where a row's groups are whole 16-byte pieces: 64 rows x 64 groups per
+// workgroup, eight groups of both arrays per load, 256 bytes of n per store.
+// (8 x 14336 x 64 pairs: 18.1 -> 11.6 us, a thread of the kernel above loads two bytes
+// at a time.)
+constexpr int kWideRows = 64;
+constexpr int kWideGroups = 64;
+__global__ __launch_bounds__(256) void interleave_sb_wide_kernel(
+    const uint16_t* scales,
+    const uint16_t* biases,
+    uint32_t* out,
+    int N,
+    int G,
+    int64_t src_stride) {
+  __shared__ uint32_t tile[kWideGroups][kWideRows + 1];
+  const int l = blockIdx.z;
+  uint32_t* dst = out + static_cast<size_t>(l) * N * G;
+  const int g0 = blockIdx.x * kWideGroups;
+  const int n0 = blockIdx.y * kWideRows;
+  // eight lanes cover the 64 groups of a row: 128 bytes of each array
+  const int part = threadIdx.x & 7;
+#pragma unroll
+  for (int i = 0; i < kWideRows / 32; ++i) {
+    const int r = i * 32 + (threadIdx.x >> 3);
+    if (n0 + r < N && g0 + part * 8 < G) {
+      const size_t at = l * src_stride + static_cast<size_t>(n0 + r) * G + g0 + part * 8;
+      const uint4 s = *reinterpret_cast<const uint4*>(scales + at);
+      const uint4 b = *reinterpret_cast<const uint4*>(biases + at);
+      const uint32_t sd[4] = {s.x, s.y, s.z, s.w};
+      const uint32_t bd[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        tile[part * 8 + 2 * e][r] = (sd[e] & 0xffffu) | (bd[e] << 16);
+        tile[part * 8 + 2 * e + 1][r] = (sd[e] >> 16) | (bd[e] & 0xffff0000u);
+      }
+    }
+  }
+  __syncthreads();
+  const int n = threadIdx.x & 63;
+  if (n0 + n < N) {
+#pragma unroll
+    for (int i = 0; i < kWideGroups / 4; ++i) {
+      const int g = i * 4 + (threadIdx.x >> 6);
+      if (g0 + g < G) {
+        dst[static_cast<size_t>(g0 + g) * N + n0 + n] = tile[g][n];
+      }
+    }
+  }
+}
+
 } // namespace
 
 int interleave_sb_for_qmm_t(
@@ -69,6 +118,16 @@ int interleave_sb_for_qmm_t(
     return fail(MLXROCM_UNSUPPORTED, "[qmm] N=%d or batch=%d exceed the grid", N, batches);
   }
   MLXROCM_REHEARSE("interleave_sb");
+  if (G % 8 == 0 && src_stride % 8 == 0 &&
+      ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 15u) == 0) {
+    const dim3 wide(
+        (G + kWideGroups - 1) / kWideGroups, (N + kWideRows - 1) / kWideRows, batches);
+    interleave_sb_wide_kernel<<<wide, 256, 0, s>>>(
+        static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),
+        static_cast<uint32_t*>(out), N, G, src_stride);
+    MLXROCM_HIP_TRY(hipGetLastError());
+    return MLXROCM_OK;
+  }
   // the kernel only moves 16-bit patterns: one instantiation serves both types
   interleave_sb_kernel<uint16_t><<<grid, 256, 0, s>>>(
       static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),

@@ -104,8 +104,12 @@ constexpr int wstore_at(int m, int ns) {
 // affine integers; the pair image then holds, per 32 codes, the scale of the
 // first 16 in the low half and of the last 16 in the high half (gs_shift == 5).
 // FP == 3 (nvfp4) also honours QmmArgs::out_scale.
+// GLU (grouped, pair image, 16-bit): the tile's columns are kBN / 2 rows of w and
+// the same rows of w_alt (NT even: each wavefront loads rows of one of them), and
+// what is written is silu(first) * second -- y has half the columns, and neither
+// product passes through memory.
 template <typename T, typename TS, typename TO, int BITS, int NT, bool GROUPED, bool WN = false,
-          bool SBI = false, int FP = 0>
+          bool SBI = false, int FP = 0, bool GLU = false>
 __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
     const QmmArgs a,
     const int gs_shift,
@@ -115,8 +119,8 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
   static_assert(!(WN && kSplit), "[K, N] weights: 16-bit problems only");
   static_assert(!WN || BITS == 4 || BITS == 8, "[K, N] weights: 4- and 8-bit codes");
   static_assert(
-      !SBI || (!WN && !kSplit && sizeof(TS) == 2 && (!GROUPED || FP != 0)),
-      "pair image: plain 16-bit launches, and the grouped gather of the fp modes");
+      !SBI || (!WN && !kSplit && sizeof(TS) == 2), "pair image: transposed 16-bit launches");
+  static_assert(!GLU || (GROUPED && SBI && FP == 0 && NT % 2 == 0), "gated: grouped, pair image");
   static_assert(FP == 0 || (SBI && BITS == (FP == 2 ? 8 : 4)), "fp codes: pair image, 4 or 8 bits");
   using DQ = std::conditional_t<FP != 0, FpPairDequant<T, (FP != 0 ? FP : 1)>, PairDequant<T, BITS>>;
   constexpr int kBN = 32 * NT;
@@ -136,7 +140,8 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
   const int wm = wave >> 1; // which 64 rows (m) of the tile
   const int N = a.N;
   const int K = a.K;
-  const int n0 = blockIdx.x * kBN;
+  constexpr int kCols = GLU ? kBN / 2 : kBN; // columns of y
+  const int n0 = blockIdx.x * kCols;
   int M = a.M;
   int m0 = blockIdx.y * kBM;
   int row0 = 0; // grouped: first sorted position of the tile
@@ -162,6 +167,11 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
     p.w = reinterpret_cast<const uint8_t*>(a.w + static_cast<int64_t>(e) * a.w_batch_stride);
     p.scales = static_cast<const TS*>(a.scales) + static_cast<int64_t>(e) * a.sb_batch_stride;
     p.biases = static_cast<const TS*>(a.biases) + static_cast<int64_t>(e) * a.sb_batch_stride;
+    if (GLU && 32 * wave >= kCols) { // this wavefront's rows of the W tile
+      p.w = reinterpret_cast<const uint8_t*>(
+          a.w_alt + static_cast<int64_t>(e) * a.w_batch_stride);
+      p.scales = static_cast<const TS*>(a.scales_alt) + static_cast<int64_t>(e) * a.sb_batch_stride;
+    }
     p.out = static_cast<TO*>(a.out);
     p.valid = true;
   } else {
@@ -235,7 +245,8 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
     // four rows' values are 8 contiguous bytes
     sb_voff = (static_cast<uint32_t>(ncol >> gs_shift) * K + 4 * kg) * static_cast<uint32_t>(sizeof(TS));
   } else {
-    const int w_row = (n0 + wr < N) ? n0 + wr : N - 1; // clamp: loads stay in bounds
+    const int w_col = n0 + (GLU && wr >= kCols ? wr - kCols : wr);
+    const int w_row = w_col < N ? w_col : N - 1; // clamp: loads stay in bounds
     w_voff = (static_cast<uint32_t>(w_row) * row_words + wh * BITS) * 4u;
     // group g of row w_row: [row][g], or [g][row] in the transposed image
     sb_voff = (a.sb_transposed ? static_cast<uint32_t>(w_row)
@@ -702,7 +713,7 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
       }
     }
     __syncthreads();
-    constexpr int kChunks = kBN / kPiece;        // 16-byte pieces per tile row
+    constexpr int kChunks = kCols / kPiece;      // 16-byte pieces per tile row
     constexpr int kLanesPerRow = 256 / kPiece;   // a power of two >= kChunks
     constexpr int kRowsPerIter = kThreads / kLanesPerRow;
     const int c = tid % kLanesPerRow;
@@ -717,7 +728,21 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
         if (mr >= M - m0 || m >= M || n >= N) {
           continue;
         }
-        const TO* src = ys + r * kOutStride + c * kPiece;
+        TO* src = ys + r * kOutStride + c * kPiece;
+        if constexpr (GLU) { // in place: this thread alone reads and writes the piece
+          const uint4 g4 = *reinterpret_cast<const uint4*>(src);
+          const uint4 u4 = *reinterpret_cast<const uint4*>(src + kCols);
+          const uint32_t gd[4] = {g4.x, g4.y, g4.z, g4.w};
+          const uint32_t ud[4] = {u4.x, u4.y, u4.z, u4.w};
+          uint32_t hd[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            hd[e] = pack2<TO>(
+                gated<TO>(half_of<TO>(gd[e], 0), half_of<TO>(ud[e], 0)),
+                gated<TO>(half_of<TO>(gd[e], 1), half_of<TO>(ud[e], 1)));
+          }
+          *reinterpret_cast<uint4*>(src) = make_uint4(hd[0], hd[1], hd[2], hd[3]);
+        }
         const size_t orow =
             GROUPED ? static_cast<size_t>(a.group_perm[row0 + mr]) : static_cast<size_t>(m);
         TO* dst = p.out + orow * N + n;
@@ -769,13 +794,13 @@ int choose_nt(int M, int N, int L, int min_nt = 5) {
 }
 
 template <typename T, typename TS, typename TO, int BITS, int NT, bool GROUPED, bool WN = false,
-          bool SBI = false, int FP = 0>
+          bool SBI = false, int FP = 0, bool GLU = false>
 int launch_variant(const QmmArgs& a, int gs_shift, dim3 grid, hipStream_t s, int k_splits = 1) {
   constexpr size_t smem = qmm_smem_bytes<NT>();
   if (grid.y > 65535u || grid.z > 65535u) {
     return fail(MLXROCM_UNSUPPORTED, "[qmm] M=%d or batch=%d exceed the grid", a.M, a.L);
   }
-  auto kern = qmm_t_mfma_kernel<T, TS, TO, BITS, NT, GROUPED, WN, SBI, FP>;
+  auto kern = qmm_t_mfma_kernel<T, TS, TO, BITS, NT, GROUPED, WN, SBI, FP, GLU>;
   static bool configured = false; // per instantiation
   if (!configured) {
     MLXROCM_HIP_TRY(hipFuncSetAttribute(

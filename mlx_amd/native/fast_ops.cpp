@@ -50,6 +50,8 @@ struct Abi {
   decltype(&mlxrocm_qmm_swiglu) swiglu;
   decltype(&mlxrocm_fp_qqmm_workspace_size) fp_qqmm_workspace_size;
   decltype(&mlxrocm_fp_qqmm) fp_qqmm;
+  decltype(&mlxrocm_switch_glu_workspace_size) switch_glu_workspace_size;
+  decltype(&mlxrocm_switch_glu) switch_glu;
   decltype(&mlxrocm_affine_quantize) affine_quantize;
   decltype(&mlxrocm_affine_dequantize) affine_dequantize;
   decltype(&mlxrocm_fp_quantize) fp_quantize;
@@ -373,6 +375,93 @@ PyObject* quantized_swiglu(PyObject*, PyObject* const* args, Py_ssize_t n) {
   FAST_CATCH
 }
 
+// switch_glu(x, indices, gate, up, down, group_size, bits): the expert-routed gated
+// MLP of nn.SwitchGLU over three (weight, scales, biases) stacks
+PyObject* switch_glu(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (!bound || n != 7) {
+    NOT_PLAIN;
+  }
+  FAST_TRY
+  const c10::DeviceIndex device = device_of(args[0]);
+  if (device < 0) {
+    NOT_PLAIN;
+  }
+  const at::Tensor* x = tensor_of(args[0], device);
+  const at::Tensor* indices = tensor_of(args[1], device);
+  int gs = 0;
+  int bits = 0;
+  if (x == nullptr || indices == nullptr || x->dim() < 1 || indices->dim() != x->dim() ||
+      !params_of(kAffine, args[5], args[6], &gs, &bits)) {
+    NOT_PLAIN;
+  }
+  const at::ScalarType it = indices->scalar_type();
+  const int index_bytes = it == at::kLong ? 8 : it == at::kInt || it == at::kUInt32 ? 4 : 0;
+  const int code = dtype_code(x->scalar_type());
+  const auto lead = [](const at::Tensor& t) { return t.sizes().slice(0, t.dim() - 1); };
+  if (index_bytes == 0 || code < 0 || code == MLXROCM_FLOAT32 || lead(*x) != lead(*indices)) {
+    NOT_PLAIN;
+  }
+  const int64_t D = x->size(-1);
+  const at::Tensor* t[3][3];
+  for (int i = 0; i < 3; ++i) {
+    PyObject* triplet = args[2 + i];
+    if (!PyTuple_CheckExact(triplet) || PyTuple_GET_SIZE(triplet) != 3) {
+      NOT_PLAIN;
+    }
+    for (int j = 0; j < 3; ++j) {
+      t[i][j] = tensor_of(PyTuple_GET_ITEM(triplet, j), device);
+      if (t[i][j] == nullptr || t[i][j]->dim() != 3 ||
+          t[i][j]->scalar_type() != (j == 0 ? at::kUInt32 : x->scalar_type())) {
+        NOT_PLAIN;
+      }
+    }
+  }
+  const int64_t E = t[0][0]->size(0);
+  const int64_t F = t[0][0]->size(1);
+  for (int i = 0; i < 3; ++i) {
+    const int64_t rows = i < 2 ? F : D;
+    const int64_t inner = i < 2 ? D : F;
+    const at::Tensor& w = *t[i][0];
+    if (w.size(0) != E || w.size(1) != rows || w.size(2) * 32 != inner * bits) {
+      NOT_PLAIN;
+    }
+    for (int j = 1; j < 3; ++j) {
+      const at::Tensor& s = *t[i][j];
+      if (s.size(0) != E || s.size(1) != rows || s.size(2) * gs != inner) {
+        NOT_PLAIN;
+      }
+    }
+  }
+  const int64_t top = indices->size(-1);
+  const int64_t tokens = indices->numel() / top;
+  if (!fits_int(tokens * top) || !fits_int(D) || !fits_int(F) || !fits_int(E)) {
+    NOT_PLAIN;
+  }
+  const size_t need = abi.switch_glu_workspace_size(tokens, top, D, F, E, gs, bits, code);
+  if (need == 0) {
+    NOT_PLAIN;
+  }
+  c10::SmallVector<int64_t, 6> shape(indices->sizes().begin(), indices->sizes().end());
+  shape.push_back(D);
+  at::Tensor out = new_tensor(shape, x->scalar_type(), device);
+  const Workspace ws(need, device);
+  void* stream = stream_of(device);
+  int rc = 0;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = abi.switch_glu(
+      x->data_ptr(), indices->data_ptr(), index_bytes,
+      static_cast<const uint32_t*>(t[0][0]->data_ptr()), t[0][1]->data_ptr(), t[0][2]->data_ptr(),
+      static_cast<const uint32_t*>(t[1][0]->data_ptr()), t[1][1]->data_ptr(), t[1][2]->data_ptr(),
+      static_cast<const uint32_t*>(t[2][0]->data_ptr()), t[2][1]->data_ptr(), t[2][2]->data_ptr(),
+      out.data_ptr(), tokens, top, D, F, E, gs, bits, code, ws.ptr(), ws.bytes, stream);
+  Py_END_ALLOW_THREADS;
+  if (rc != MLXROCM_OK) {
+    NOT_PLAIN;
+  }
+  return wrap(std::move(out));
+  FAST_CATCH
+}
+
 // qqmm(x, w, scales, group_size, bits, mode) with a quantized w
 PyObject* qqmm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!bound || n != 6) {
@@ -590,6 +679,8 @@ PyObject* bind(PyObject*, PyObject* table) {
       take("mlxrocm_qmm_swiglu", abi.swiglu) &&
       take("mlxrocm_fp_qqmm_workspace_size", abi.fp_qqmm_workspace_size) &&
       take("mlxrocm_fp_qqmm", abi.fp_qqmm) &&
+      take("mlxrocm_switch_glu_workspace_size", abi.switch_glu_workspace_size) &&
+      take("mlxrocm_switch_glu", abi.switch_glu) &&
       take("mlxrocm_affine_quantize", abi.affine_quantize) &&
       take("mlxrocm_affine_dequantize", abi.affine_dequantize) &&
       take("mlxrocm_fp_quantize", abi.fp_quantize) &&
@@ -605,6 +696,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 PyMethodDef methods[] = {
     FASTCALL(quantized_matmul),
     FASTCALL(quantized_swiglu),
+    FASTCALL(switch_glu),
     FASTCALL(qqmm),
     FASTCALL(quantize),
     FASTCALL(dequantize),

@@ -295,9 +295,10 @@ class QuantizedSwitchLinear(torch.nn.Module):
 class SwitchGLU(torch.nn.Module):
     """Expert-routed gated MLP: ``down(act(gate(x)) * up(x))`` with every
     projection a :class:`QuantizedSwitchLinear` and token ``t`` sent to the
-    experts ``indices[t, :]``.  From 64 routed rows on, the rows are ordered by
-    expert first (one argsort), so that all three projections run with
-    ``sorted_indices=True``, and put back afterwards."""
+    experts ``indices[t, :]``.  With silu, no additive biases and 16-bit types the
+    whole block is one call of the library, which groups the routed rows by expert
+    once; otherwise the three projections in turn (each groups the rows itself,
+    whatever their order, so ``sort_threshold`` no longer changes anything)."""
 
     def __init__(self, input_dims: int, hidden_dims: int, num_experts: int,
                  activation: Callable[[torch.Tensor], torch.Tensor] = torch.nn.functional.silu,
@@ -311,25 +312,30 @@ class SwitchGLU(torch.nn.Module):
         self.activation = activation
         self.sort_threshold = sort_threshold
 
+    def _in_one_call(self, x: torch.Tensor, indices: torch.Tensor) -> Optional[torch.Tensor]:
+        if self.activation is not torch.nn.functional.silu:
+            return None
+        modules = self._modules
+        layers = [modules[name] for name in ("gate_proj", "up_proj", "down_proj")]
+        first = layers[0]
+        triplets = []
+        for layer in layers:
+            *triplet, bias = _held(layer, "weight", "scales", "biases", "bias")
+            if bias is not None or (layer.group_size, layer.bits, layer.mode) != (
+                    first.group_size, first.bits, "affine"):
+                return None
+            triplets.append(tuple(triplet))
+        return ops._fast.switch_glu(x, indices, *triplets, first.group_size, first.bits)
+
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """x ``[..., D]``, indices ``[..., k]`` -> ``[..., k, D]``."""
-        k = indices.shape[-1]
+        y = self._in_one_call(x, indices)
+        if y is not None:
+            return y
         x = x.unsqueeze(-2).unsqueeze(-3)  # [..., 1, 1, D]
-        do_sort = indices.numel() >= self.sort_threshold
-        idx = indices
-        if do_sort:
-            flat = indices.reshape(-1)
-            order = torch.argsort(flat.long(), stable=True)
-            inverse = torch.argsort(order)
-            x = x.reshape(-1, 1, x.shape[-1])[order // k]  # [n, 1, D]: one row per routed pair
-            # torch cannot index uint32 tensors: reorder through an integer copy
-            idx = flat.long()[order].to(indices.dtype)
-        up = self.up_proj(x, idx, sorted_indices=do_sort)
-        gate = self.gate_proj(x, idx, sorted_indices=do_sort)
-        y = self.down_proj(self.activation(gate) * up, idx, sorted_indices=do_sort)
-        if do_sort:
-            y = y[inverse].reshape(*indices.shape, 1, y.shape[-1])
-        return y.squeeze(-2)
+        up = self.up_proj(x, indices)
+        gate = self.gate_proj(x, indices)
+        return self.down_proj(self.activation(gate) * up, indices).squeeze(-2)
 
 
 def _to_quantized(m, **kwargs):

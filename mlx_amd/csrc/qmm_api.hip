@@ -202,7 +202,7 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
   // few tiles: also cut K (one row block, one batch entry only)
   int k_splits = 1;
   if (rows_per_block == a.M && a.L == 1 && (static_cast<int64_t>(a.M) * a.N) % 4 == 0) {
-    k_splits = qmm_mfma_k_splits(a.M, a.N, a.K, 1);
+    k_splits = qmm_mfma_k_splits(a.M, a.N, a.K, 1, kSplitFp32Width);
   }
   const size_t x_bytes = (split_x_bytes(rows_per_block, a.K) + 255) / 256 * 256;
   const size_t plane = static_cast<size_t>(a.M) * a.N;
@@ -367,10 +367,8 @@ int run_qmv_n(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStr
 int run_qmm_n(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStream_t s) {
   const int G = a.N / gs;
   const int batches = a.sb_batch_stride == 0 ? 1 : a.L;
-  int k_splits = 1;
-  if ((static_cast<int64_t>(a.M) * a.N) % 4 == 0) {
-    k_splits = qmm_mfma_k_splits(a.M, a.N, a.K, a.L);
-  }
+  const TilePlan pl = qmm_n_plan(a.M, a.N, a.K, a.L);
+  const int k_splits = pl.splits;
   const size_t sb_bytes = (qmm_n_sb_bytes(a.K, G, batches, dtype) + 255) / 256 * 256;
   const size_t plane = static_cast<size_t>(a.M) * a.N;
   const size_t partial_bytes = k_splits > 1 ? plane * k_splits * sizeof(float) : 0;
@@ -390,11 +388,11 @@ int run_qmm_n(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStr
   part.biases = static_cast<char*>(region) + image * dtype_size(dtype);
   part.sb_batch_stride = batches == 1 ? 0 : static_cast<int64_t>(2 * image);
   if (k_splits <= 1) {
-    return launch_qmm_mfma_n(part, gs, bits, dtype, 1, s);
+    return launch_qmm_mfma_n(part, gs, bits, dtype, pl, s);
   }
   void* partial = static_cast<char*>(region) + sb_bytes;
   part.out = partial;
-  rc = launch_qmm_mfma_n(part, gs, bits, dtype, k_splits, s);
+  rc = launch_qmm_mfma_n(part, gs, bits, dtype, pl, s);
   if (rc != MLXROCM_OK) {
     return rc;
   }

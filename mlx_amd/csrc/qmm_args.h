@@ -218,11 +218,18 @@ int split_x_for_mfma(const void* x, void* xs, size_t rows, int K, hipStream_t s)
 int launch_qmm_mfma_split(const QmmArgs& a, int gs, int bits, hipStream_t s, int k_splits);
 // Few tiles: K is cut into qmm_mfma_k_splits() ranges whose fp32 partial tiles
 // (k_splits planes of M x N behind a.out) reduce_k_splits() adds up.
-int qmm_mfma_k_splits(int M, int N, int K, int L);
+int qmm_mfma_k_splits(int M, int N, int K, int L, int nt = 7);
+constexpr int kSplitFp32Width = 6; // of launch_qmm_mfma_split's tiles, times 32 columns
 // transpose=false (w [K, N*bits/32]), 4/8-bit, 16-bit types, K % 64 == 0; with
 // k_splits > 1 `a.out` points at k_splits fp32 planes as for the k-split launch.
 // `a.scales` / `a.biases` must point at [group][k] images (transpose_sb_for_qmm_n).
-int launch_qmm_mfma_n(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, hipStream_t s);
+struct TilePlan {
+  int nt;     // tiles of nt x 32 columns
+  int splits; // ranges of K
+};
+TilePlan qmm_n_plan(int M, int N, int K, int L);
+int launch_qmm_mfma_n(
+    const QmmArgs& a, int gs, int bits, int dtype, const TilePlan& pl, hipStream_t s);
 size_t qmm_n_sb_bytes(int K, int G, int batches, int dtype);
 // scales / biases [N][G] (16-bit types) -> per batch entry [G][N] pairs
 // (scale in the low half of a dword, bias in the high half); same size as the

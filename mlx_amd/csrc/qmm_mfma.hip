@@ -110,24 +110,75 @@ int transpose_sb_for_qmm_n(
   return MLXROCM_OK;
 }
 
+// [K, N] weights: the width of the tiles and the number of K ranges that finish
+// first.  What a launch costs, in nanoseconds, from timing every width and number of
+// ranges on eight shapes (errors up to 15 %): a K-step takes longer the wider its
+// tile, and the more compute units work beside it (the clock gives way: 224 columns
+// 1.46 us with 76 of 256 units at work, 1.78 with 228); a tile costs some
+// microseconds before and after its steps; ranges cost the fp32 planes, written and
+// read again.
+TilePlan qmm_n_plan(int M, int N, int K, int L) {
+  const long cus = compute_units();
+  const long mt = (M + kBM - 1) / kBM;
+  const long steps = K / kBK;
+  auto cost = [&](int nt, int splits) -> double {
+    const long wgs = mt * ((N + 32 * nt - 1) / (32 * nt)) * (splits > 1 ? splits : L);
+    const double rounds = static_cast<double>((wgs + cus - 1) / cus);
+    const double busy = static_cast<double>(wgs) / (rounds * cus);
+    const double step = (400.0 + 110.0 * nt) * (1.0 + 0.3 * busy);
+    double ns = rounds * (static_cast<double>((steps + splits - 1) / splits) * step + 4000.0);
+    if (splits > 1) {
+      ns += 3000.0 + static_cast<double>(splits) * M * N * 4.0 / 5000.0; // 5 TB/s
+    }
+    return ns;
+  };
+  TilePlan best = {choose_nt(M, N, L), 1};
+  if (L != 1 || (static_cast<int64_t>(M) * N) % 4 != 0) {
+    return best;
+  }
+  // a margin of 8 % for the plain launch: it needs no planes
+  double best_ns = cost(best.nt, 1) / 1.08;
+  for (int nt = 6; nt <= 7; ++nt) { // the widths built with fp32 planes
+    const long tiles = mt * ((N + 32 * nt - 1) / (32 * nt));
+    for (int splits = 2; splits <= 16 && splits * 8 <= steps && splits * tiles <= 2 * cus;
+         ++splits) {
+      const double ns = cost(nt, splits);
+      if (ns < best_ns) {
+        best = {nt, splits};
+        best_ns = ns;
+      }
+    }
+  }
+  return best;
+}
+
 // transpose=false on the matrix cores: same tiles, column loader for W.  a.scales
 // / a.biases point at the transposed images made by transpose_sb_for_qmm_n.
-int launch_qmm_mfma_n(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, hipStream_t s) {
+// Tiles of 224 columns as for transpose=true (245 registers; 256 columns spill):
+// dy [1024, 14336] x W [14336, 4096] at 4 bits takes 133 us in three K ranges of
+// them (228 workgroups), against 206 in three of 192 columns (264: a second round
+// for eight workgroups) and 157 in two.
+int launch_qmm_mfma_n(
+    const QmmArgs& a, int gs, int bits, int dtype, const TilePlan& pl, hipStream_t s) {
   const int gs_shift = shift_of(gs);
-  MLXROCM_REHEARSE("qmm_n_tile(ksplit=%d)", k_splits);
-  if (k_splits > 1) {
-    const dim3 grid((a.N + 32 * 6 - 1) / (32 * 6), (a.M + kBM - 1) / kBM, k_splits);
-    return dtype == MLXROCM_BFLOAT16
-        ? launch_wn<bf16_t, float, 6>(a, gs_shift, bits, grid, s, k_splits)
-        : launch_wn<f16_t, float, 6>(a, gs_shift, bits, grid, s, k_splits);
-  }
-  int nt = choose_nt(a.M, a.N, a.L);
-  nt = nt > 6 ? 6 : nt; // the column loader's registers leave room for 6 x 32 columns
-  const dim3 grid((a.N + 32 * nt - 1) / (32 * nt), (a.M + kBM - 1) / kBM, a.L);
+  const int nt = pl.nt;
+  MLXROCM_REHEARSE("qmm_n_tile(ksplit=%d)", pl.splits);
+  const dim3 grid(
+      (a.N + 32 * nt - 1) / (32 * nt), (a.M + kBM - 1) / kBM, pl.splits > 1 ? pl.splits : a.L);
   auto run = [&](auto tval) -> int {
     using T = decltype(tval);
-    return nt == 5 ? launch_wn<T, T, 5>(a, gs_shift, bits, grid, s, 1)
-                   : launch_wn<T, T, 6>(a, gs_shift, bits, grid, s, 1);
+    if (pl.splits > 1) {
+      return nt == 6 ? launch_wn<T, float, 6>(a, gs_shift, bits, grid, s, pl.splits)
+                     : launch_wn<T, float, 7>(a, gs_shift, bits, grid, s, pl.splits);
+    }
+    switch (nt) {
+      case 5:
+        return launch_wn<T, T, 5>(a, gs_shift, bits, grid, s, 1);
+      case 6:
+        return launch_wn<T, T, 6>(a, gs_shift, bits, grid, s, 1);
+      default:
+        return launch_wn<T, T, 7>(a, gs_shift, bits, grid, s, 1);
+    }
   };
   return dtype == MLXROCM_BFLOAT16 ? run(bf16_t{}) : run(f16_t{});
 }
@@ -161,13 +212,13 @@ int launch_qmm_mfma(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s
 
 // How many ranges to cut K into so that a launch with few tiles still fills the
 // compute units (1 = no split): only for a single problem, and every range
-// keeps at least eight steps.
-int qmm_mfma_k_splits(int M, int N, int K, int L) {
+// keeps at least eight steps.  nt: the width of the launcher's tiles.
+int qmm_mfma_k_splits(int M, int N, int K, int L, int nt) {
   if (L != 1) {
     return 1;
   }
   const long cus = compute_units();
-  const long tiles = static_cast<long>((M + kBM - 1) / kBM) * ((N + 32 * 7 - 1) / (32 * 7));
+  const long tiles = static_cast<long>((M + kBM - 1) / kBM) * ((N + 32 * nt - 1) / (32 * nt));
   const long steps = K / kBK;
   long s = cus / tiles;
   if (s > steps / 8) {
@@ -272,7 +323,7 @@ int reduce_k_splits(const void* partial, void* out, size_t n, int k_splits, int 
 int launch_qmm_mfma_split(const QmmArgs& a, int gs, int bits, hipStream_t s, int k_splits) {
   // six column blocks: with fp32 scales and the weight split, seven spill
   // registers to scratch memory (measured 620 against 415 us at 1024 x 11008 x 4096)
-  constexpr int kNT = 6;
+  constexpr int kNT = kSplitFp32Width;
   const int gs_shift = shift_of(gs);
   const dim3 grid(
       (a.N + 32 * kNT - 1) / (32 * kNT), (a.M + kBM - 1) / kBM, k_splits > 1 ? k_splits : a.L);

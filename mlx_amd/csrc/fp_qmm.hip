@@ -835,6 +835,15 @@ size_t round256(size_t n) {
   return (n + 255) / 256 * 256;
 }
 
+// Whether the scale bytes of w are rewritten as a step-major image first (a scale
+// dword per row and K-step is a cache line of its own in the caller's layout).  The
+// image of 14336 x 4096 takes 4 us and every 256 rows of x read it once; a call of 512
+// rows takes 100 us or more, one of 100 rows 32 with the caller's layout.
+constexpr int kQqImageMinM = 512;
+bool qq_ws_image(int M) {
+  return M >= kQqImageMinM;
+}
+
 } // namespace
 
 extern "C" int mlxrocm_fp_qmm(
@@ -908,7 +917,9 @@ extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, 
   }
   if (qq_native(M, N, K, mode, dtype)) {
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
-    return round256(static_cast<size_t>(M) * K * bits / 8) + round256(static_cast<size_t>(M) * K / 32);
+    return round256(static_cast<size_t>(M) * K * bits / 8) +
+        round256(static_cast<size_t>(M) * K / 32) +
+        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0);
   }
   return round256(static_cast<size_t>(M) * K * dtype_size(dtype)) +
       (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)
@@ -961,11 +972,21 @@ extern "C" int mlxrocm_fp_qqmm(
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     void* codes = workspace;
     uint8_t* xs = static_cast<uint8_t*>(workspace) + round256(n_elems * bits / 8);
-    rc = fp_quantize_activations(x, codes, xs, n_elems, mode, dtype, s);
+    rc = fp_quantize_activations(x, codes, xs, M, K, mode, dtype, s);
     if (rc != MLXROCM_OK) {
       return rc;
     }
-    return launch_qq_mfma(codes, xs, wq, scales, out, M, N, K, mode, dtype, s);
+    const uint8_t* ws = scales;
+    const bool image = qq_ws_image(M) && (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
+    if (image) {
+      uint8_t* dst = xs + round256(n_elems / 32);
+      rc = launch_mx_scale_image(scales, dst, N, K, s);
+      if (rc != MLXROCM_OK) {
+        return rc;
+      }
+      ws = dst;
+    }
+    return launch_qq_mfma(codes, xs, wq, ws, image, out, M, N, K, mode, dtype, s);
   }
   // x_hat in the element type, then the product with the quantized w
   rc = mlxrocm_fp_quantize_dequantize(x, workspace, n_elems, mode, dtype, stream);

@@ -240,10 +240,13 @@ __global__ __launch_bounds__(kFpBlock) void fp_dequantize_kernel(
 // mlx/backend/cpu/quantized.cpp:1094-1128, fp32 arithmetic throughout.
 // CODES: write the codes and the scale byte (wq, scales) instead of the
 // dequantized elements (out): the operand the block-scaled matrix instruction
-// multiplies as it is.
+// multiplies as it is.  The scale bytes go out as the image that instruction's
+// kernel reads, [K / 128][rows] dwords of four consecutive groups' bytes (`rows`
+// rows of `row_groups` groups each, a multiple of four).
 template <typename T, int GS, int BITS, bool CODES = false>
 __global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
-    const T* w, T* out, size_t n_units, uint8_t* wq = nullptr, uint8_t* scales = nullptr) {
+    const T* w, T* out, size_t n_units, uint8_t* wq = nullptr, uint8_t* scales = nullptr,
+    uint32_t rows = 0, uint32_t row_groups = 1) {
   const size_t u = static_cast<size_t>(blockIdx.x) * kFpBlock + threadIdx.x;
   constexpr int kLanes = GS / 8;
   float v[8];
@@ -335,7 +338,11 @@ __global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
       reinterpret_cast<uint32_t*>(wq)[u] = lo;
     }
     if (u % kLanes == 0) {
-      scales[u / kLanes] = static_cast<uint8_t>(scale_byte);
+      const size_t g = u / kLanes;
+      const uint32_t row = static_cast<uint32_t>(g / row_groups);
+      const uint32_t col = static_cast<uint32_t>(g - static_cast<size_t>(row) * row_groups);
+      scales[(static_cast<size_t>(col / 4) * rows + row) * 4 + col % 4] =
+          static_cast<uint8_t>(scale_byte);
     }
   } else {
     float o[8];
@@ -586,9 +593,10 @@ extern "C" int mlxrocm_fp_dequantize(
 namespace mlxrocm {
 
 // x -> codes and scale bytes by the rules of fp_quantize_dequantize (what qqmm
-// applies to its first operand).  n_elems a multiple of the group size.
+// applies to its first operand), in the MX modes.  x is [M][K], K % 128 == 0.
 int fp_quantize_activations(
-    const void* x, void* codes, uint8_t* scales, size_t n_elems, int mode, int dtype, hipStream_t s) {
+    const void* x, void* codes, uint8_t* scales, int M, int K, int mode, int dtype, hipStream_t s) {
+  const size_t n_elems = static_cast<size_t>(M) * K;
   const size_t n_units = n_elems / 8;
   const size_t blocks = (n_units + kFpBlock - 1) / kFpBlock;
   if (blocks > 0x7fffffffull) {
@@ -601,11 +609,55 @@ int fp_quantize_activations(
       constexpr int G = decltype(gval)::value;
       constexpr int B = decltype(bval)::value;
       fp_quantize_dequantize_kernel<T, G, B, true><<<static_cast<unsigned>(blocks), kFpBlock, 0, s>>>(
-          static_cast<const T*>(x), nullptr, n_units, static_cast<uint8_t*>(codes), scales);
+          static_cast<const T*>(x), nullptr, n_units, static_cast<uint8_t*>(codes), scales,
+          static_cast<uint32_t>(M), static_cast<uint32_t>(K / 32));
       MLXROCM_HIP_TRY(hipGetLastError());
       return static_cast<int>(MLXROCM_OK);
     });
   });
+}
+
+namespace {
+
+// [rows][steps] dwords (four scale bytes of 128 codes) -> [steps][rows]: 64 rows x 32
+// steps per workgroup through LDS.
+__global__ __launch_bounds__(kFpBlock) void mx_scale_image_kernel(
+    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int rows, int steps) {
+  __shared__ uint32_t tile[64][33];
+  const int r0 = blockIdx.y * 64;
+  const int s0 = blockIdx.x * 32;
+  const int sx = threadIdx.x & 31;
+#pragma unroll
+  for (int r = threadIdx.x >> 5; r < 64; r += kFpBlock / 32) {
+    if (r0 + r < rows && s0 + sx < steps) {
+      tile[r][sx] = in[static_cast<size_t>(r0 + r) * steps + s0 + sx];
+    }
+  }
+  __syncthreads();
+  const int rx = threadIdx.x & 63;
+#pragma unroll
+  for (int st = threadIdx.x >> 6; st < 32; st += kFpBlock / 64) {
+    if (r0 + rx < rows && s0 + st < steps) {
+      out[static_cast<size_t>(s0 + st) * rows + r0 + rx] = tile[rx][st];
+    }
+  }
+}
+
+} // namespace
+
+// The scale bytes [rows][K / 32] of an MX weight as the image [K / 128][rows] of
+// dwords; scales 4-byte aligned, K % 128 == 0.
+int launch_mx_scale_image(const uint8_t* scales, void* image, int rows, int K, hipStream_t s) {
+  const int steps = K / 128;
+  const dim3 grid((steps + 31) / 32, (rows + 63) / 64);
+  if (grid.y > 65535u) {
+    return fail(MLXROCM_UNSUPPORTED, "[qqmm] N=%d exceeds the grid", rows);
+  }
+  MLXROCM_REHEARSE("mx_scale_image");
+  mx_scale_image_kernel<<<grid, kFpBlock, 0, s>>>(
+      reinterpret_cast<const uint32_t*>(scales), static_cast<uint32_t*>(image), rows, steps);
+  MLXROCM_HIP_TRY(hipGetLastError());
+  return MLXROCM_OK;
 }
 
 } // namespace mlxrocm

@@ -140,14 +140,16 @@ int launch_qmm_mfma_fp(const QmmArgs& a, int mode, int dtype, int k_splits, hipS
 int launch_qmm_mfma_fp_grouped(const QmmArgs& a, int mode, int dtype, hipStream_t s);
 
 // qqmm in the MX modes on the block-scaled matrix instruction (qq_mfma.hip):
-// x as codes and scale bytes (fp_quantize_activations, fp_quantize.hip) times
-// the quantized w, both [rows][K]; K % 128 == 0.
+// x as codes and an image of scale bytes (fp_quantize_activations, fp_quantize.hip)
+// times the quantized w, both [rows][K]; K % 128 == 0.  ws: the caller's scale bytes
+// [N][K / 32], or (ws_image) their image.
 bool qq_mfma_supported(int M, int N, int K, int mode);
 int launch_qq_mfma(
     const void* xq,
     const uint8_t* xs,
     const uint32_t* wq,
     const uint8_t* ws,
+    bool ws_image,
     void* out,
     int M,
     int N,
@@ -156,7 +158,8 @@ int launch_qq_mfma(
     int dtype,
     hipStream_t s);
 int fp_quantize_activations(
-    const void* x, void* codes, uint8_t* scales, size_t n_elems, int mode, int dtype, hipStream_t s);
+    const void* x, void* codes, uint8_t* scales, int M, int K, int mode, int dtype, hipStream_t s);
+int launch_mx_scale_image(const uint8_t* scales, void* image, int rows, int K, hipStream_t s);
 
 bool qmv_wide_supported(const QmmArgs& a, int gs, int bits, int dtype, bool transpose);
 int launch_qmv_wide(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);

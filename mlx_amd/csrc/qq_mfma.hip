@@ -12,8 +12,15 @@
 //
 // Workgroup: 512 threads, tile 256 (m) x 128 (n), K-step 128 codes.  Both code
 // tiles and their scale dwords go HBM -> LDS by DMA (global_load_lds) into a
-// ring of stages; the only loads of the loop are those, so one vmcnt wait and
-// one barrier per step order everything.  16-byte pieces of a row are
+// ring of stages.  Reading a step's fragments takes about as long as multiplying
+// them (8-bit codes: 128 KB at 128 bytes a clock against 16 instructions of 32 to 40
+// clocks on each wavefront), so the two wavefronts of a SIMD take turns (k_loop):
+// with all eight in step the two phases added up, and the matrix pipe was busy for
+// 35 % of the time.  Scale dwords come from step-major images, [K / 128][rows]: in the
+// caller's layout each is a cache line of its own, as many requests as the codes.
+// x [2048, 4096] x W [14336, 4096], bf16, quantizing x included: mxfp8 172 -> 143 us,
+// mxfp4 102 -> 95; 512 rows, 14336 -> 4096, mxfp8 129 -> 105.
+// 16-byte pieces of a row are
 // XOR-swizzled so that fragment reads hit every bank once.  Wavefront (wm, wn)
 // owns a 64 x 64 block: W fragments are the instruction's A operand, x
 // fragments its B operand, so a lane holds four consecutive n of one row m of y.
@@ -70,11 +77,12 @@ struct QqShape {
 
 struct QqArgs {
   const uint8_t* xq;     // [M][K bits / 8]
-  const uint8_t* xs;     // [M][K / 32]
+  const uint8_t* xs;     // scale bytes of x: image [K / 128][M] of dwords
   const uint8_t* wq;     // [N][K bits / 8]
-  const uint8_t* ws;     // [N][K / 32]
+  const uint8_t* ws;     // the caller's [N][K / 32], or the image [K / 128][N]
   void* out;             // [M][N]
   int M, N, K;
+  uint32_t ws_row, ws_step; // bytes from a row of W, from a step, to the next
 };
 
 // slot of logical piece `piece` of tile row `row`
@@ -109,7 +117,6 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   const int m0 = blockIdx.y * kBM;
   const int nk = K / kQqBK;
   const uint32_t row_bytes = static_cast<uint32_t>(K) * BITS / 8;
-  const uint32_t srow_bytes = static_cast<uint32_t>(K) / 32;
 
   // ---- loader roles.  A DMA instruction of a wavefront moves kRowsPerDma rows
   // of kRowBytes: lane l lands in slot l % kSlots of row l / kSlots and fetches
@@ -117,6 +124,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   const int drow = lane / S::kSlots;
   const int dslot = lane % S::kSlots;
   uint32_t xoff[S::kXDma], woff[S::kWDma], soff[S::kSDma];
+  const uint8_t* sbase[S::kSDma]; // uniform
+  uint32_t sstep[S::kSDma];
 #pragma unroll
   for (int j = 0; j < S::kXDma; ++j) {
     const int r = (wave * S::kXDma + j) * S::kRowsPerDma + drow; // tile row
@@ -137,13 +146,16 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #pragma unroll
   for (int j = 0; j < S::kSDma; ++j) {
     const int d = scale_dword(j);
+    const bool of_x = (j * S::kWaves + wave) * 64 < kBM;
+    sbase[j] = of_x ? a.xs : a.ws;
+    sstep[j] = of_x ? 4u * static_cast<uint32_t>(M) : a.ws_step;
     if (d < kBM) {
       const int m = m0 + d < M ? m0 + d : M - 1;
-      soff[j] = static_cast<uint32_t>(m) * srow_bytes;
+      soff[j] = static_cast<uint32_t>(m) * 4u;
     } else {
       const int r = d - kBM < kBN ? d - kBM : kBN - 1;
       const int n = n0 + r < N ? n0 + r : N - 1;
-      soff[j] = static_cast<uint32_t>(n) * srow_bytes;
+      soff[j] = static_cast<uint32_t>(n) * a.ws_row;
     }
   }
 
@@ -168,10 +180,10 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
                  : "memory");                                                    \
   } while (0)
 
-  // all loads of step t (clamped to the last step: the counts stay the same)
-  auto issue = [&](int t) {
+  // all loads of step t (clamped to the last step: the counts stay the same), into
+  // the stage at byte `stage`
+  auto issue = [&](int t, int stage) {
     const int tc = t < nk ? t : nk - 1;
-    const int stage = (t % S::kStages) * S::kStage;
     const uint8_t* xg = a.xq + static_cast<size_t>(tc) * S::kRowBytes;
     const uint8_t* wg = a.wq + static_cast<size_t>(tc) * S::kRowBytes;
 #pragma unroll
@@ -185,9 +197,82 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #pragma unroll
     for (int j = 0; j < S::kSDma; ++j) {
       const int first = (j * S::kWaves + wave) * 64; // uniform
-      const uint8_t* sg = (first < kBM ? a.xs : a.ws) + static_cast<size_t>(tc) * 4;
-      QQ_DMA4(soff[j], sg, stage + S::kXTile + S::kWTile + first * 4);
+      QQ_DMA4(soff[j], sbase[j] + static_cast<size_t>(tc) * sstep[j],
+              stage + S::kXTile + S::kWTile + first * 4);
     }
+  };
+
+  // The K loop.  The wavefronts w and w + 4 of a SIMD take turns: while one half of
+  // the workgroup reads the fragments of a step from LDS (and requests a later step),
+  // the other half multiplies.  A barrier ends each phase; half B runs one phase
+  // behind A.  In phase 2 t, A reads step t and B multiplies step t - 1; in phase
+  // 2 t + 1, A multiplies step t and B reads it.
+  //   * Step t is in LDS before phase 2 t: each wavefront has waited for its own loads
+  //     of it before the barrier that ends phase 2 t - 1 (steps t + 1 .. t + kS - 2 may
+  //     still be in flight).
+  //   * In its read phase of step t a wavefront requests step t + kS - 1 into the stage
+  //     of step t - 1, whose last reads (B's, phase 2 t - 1) were waited for before the
+  //     barrier that ended them.
+  // Every wavefront passes 2 nk + 2 barriers.
+  constexpr int kS = S::kStages;
+  auto k_loop = [&](auto&& read_step, auto&& settle, auto&& multiply) {
+    auto barrier = [] {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto landed = [] { // all but the newest kS - 2 steps of this wavefront's loads
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kS - 2) * S::kLoads) : "memory");
+    };
+#pragma unroll
+    for (int t = 0; t < kS - 1; ++t) {
+      issue(t, t * S::kStage);
+    }
+    landed();
+    barrier();
+    // (one loop per half: matrix instructions would be moved past a branch that
+    // follows them, and with it past the wait)
+    auto half = [&](auto behind_c) {
+      constexpr bool kBehind = decltype(behind_c)::value;
+      if constexpr (kBehind) {
+        barrier();
+      }
+      int rd = 0;                    // stage of step t
+      int wr = (kS - 1) * S::kStage; // stage of step t + kS - 1
+      for (int t = 0; t < nk; ++t) {
+        read_step(smem + rd);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(t + kS - 1, wr);
+        wr = rd;
+        rd = rd + S::kStage < kS * S::kStage ? rd + S::kStage : 0;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        settle();
+        if constexpr (kBehind) {
+          landed();
+        }
+        barrier();
+        __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (!kBehind) {
+          landed();
+        }
+        barrier();
+      }
+      if constexpr (!kBehind) {
+        barrier();
+      }
+    };
+    if (wave >= S::kWaves / 2) { // uniform
+      half(std::true_type{});
+    } else {
+      half(std::false_type{});
+    }
+    // the clamped extra loads must have landed before the workgroup's LDS is given up
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
 
   if constexpr (BIG) {
@@ -210,24 +295,12 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     }
     const int fr = lane & 31;
     const int kblk = lane >> 5;
-    constexpr int kS = S::kStages;
-#pragma unroll
-    for (int t = 0; t < kS - 1; ++t) {
-      issue(t);
-    }
-    for (int t = 0; t < nk; ++t) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kS - 2) * S::kLoads) : "memory");
-      __syncthreads();
-      issue(t + kS - 1);
-      const uint8_t* st = smem + (t % kS) * S::kStage;
+    qq_i32x4 af[2][NT], bf[2][MT];
+    uint32_t da[NT], db[MT]; // scale dwords as read
+    // scale bytes: register q holds tiles 2 q and 2 q + 1, bytes (tile % 2) 2 + h
+    int sa[(NT + 1) / 2], sb[(MT + 1) / 2];
+    auto read_step = [&](const uint8_t* st) {
       const uint32_t* sc = reinterpret_cast<const uint32_t*>(st + S::kXTile + S::kWTile);
-      qq_i32x4 af[2][NT], bf[2][MT];
-      // scale bytes: register q holds tiles 2 q and 2 q + 1, bytes (tile % 2) 2 + h
-      int sa[(NT + 1) / 2], sb[(MT + 1) / 2];
-      auto two_bytes = [&](uint32_t d) {
-        // the blocks of this lane in the two halves: kblk and 2 + kblk
-        return ((d >> (8 * kblk)) & 0xffu) | (((d >> (8 * (2 + kblk))) & 0xffu) << 8);
-      };
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
         const int xr = wm * 16 * MI + 32 * j + fr;
@@ -237,12 +310,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
           const uint4 v = *reinterpret_cast<const uint4*>(row + qq_slot<4>(xr, 2 * h + kblk) * 16);
           bf[h][j] = qq_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
         }
-        const uint32_t two = two_bytes(sc[xr]);
-        if (j % 2 == 0) {
-          sb[j / 2] = static_cast<int>(two);
-        } else {
-          sb[j / 2] |= static_cast<int>(two << 16);
-        }
+        db[j] = sc[xr];
       }
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
@@ -253,13 +321,26 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
           const uint4 v = *reinterpret_cast<const uint4*>(row + qq_slot<4>(wr, 2 * h + kblk) * 16);
           af[h][i] = qq_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
         }
-        const uint32_t two = two_bytes(sc[kBM + wr]);
-        if (i % 2 == 0) {
-          sa[i / 2] = static_cast<int>(two);
-        } else {
-          sa[i / 2] |= static_cast<int>(two << 16);
-        }
+        da[i] = sc[kBM + wr];
       }
+    };
+    auto settle = [&] {
+      // the blocks of this lane in the two halves: kblk and 2 + kblk
+      auto two_bytes = [&](uint32_t d) {
+        return ((d >> (8 * kblk)) & 0xffu) | (((d >> (8 * (2 + kblk))) & 0xffu) << 8);
+      };
+#pragma unroll
+      for (int j = 0; j < MT; j += 2) {
+        sb[j / 2] = static_cast<int>(two_bytes(db[j]) | (j + 1 < MT ? two_bytes(db[j + 1]) << 16 : 0u));
+        asm volatile("" : "+v"(sb[j / 2])); // (packed here, not among the instructions that use it)
+      }
+#pragma unroll
+      for (int i = 0; i < NT; i += 2) {
+        sa[i / 2] = static_cast<int>(two_bytes(da[i]) | (two_bytes(da[i + 1]) << 16));
+        asm volatile("" : "+v"(sa[i / 2]));
+      }
+    };
+    auto multiply = [&] {
       auto wide = [](const qq_i32x4& f) { return qq_i32x8{f[0], f[1], f[2], f[3], 0, 0, 0, 0}; };
 #define QQ_MMA32(i, j, h)                                                        \
   if constexpr ((i) < NT && (j) < MT) {                                          \
@@ -273,8 +354,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       QQ_MMA32_ROW(0, 1) QQ_MMA32_ROW(1, 1) QQ_MMA32_ROW(2, 1) QQ_MMA32_ROW(3, 1)
 #undef QQ_MMA32_ROW
 #undef QQ_MMA32
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    k_loop(read_step, settle, multiply);
     // D[n][m] 32 x 32: register i of lane (col, half) holds n = 8 (i / 4) + 4 half
     // + i % 4, m = col
     TO* out = static_cast<TO*>(a.out);
@@ -342,6 +423,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   using Frag = std::conditional_t<BITS == 8, qq_i32x8, qq_i32x4>;
   struct Frags {
     Frag af[NI], bf[MI];
+    uint32_t da[NI], db[MI]; // scale dwords as read
     int sa[NI / 4], sb[MI / 4];
   };
   auto fragment = [&](const uint8_t* row_base, int r) -> Frag {
@@ -365,16 +447,9 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       return qq_i32x8{f[0], f[1], f[2], f[3], 0, 0, 0, 0};
     }
   };
-  // byte kb of four rows' scale dwords, packed (row j in byte j)
-  auto pack_scales = [&](const uint32_t* d) {
-    const int sh = 8 * kb;
-    return static_cast<int>(
-        ((d[0] >> sh) & 0xffu) | (((d[16] >> sh) & 0xffu) << 8) | (((d[32] >> sh) & 0xffu) << 16) |
-        ((d[48] >> sh) << 24));
-  };
-  // the fragments and scale bytes of step t, from its stage
-  auto read_step = [&](int t, Frags& f) {
-    const uint8_t* st = smem + (t % S::kStages) * S::kStage;
+  Frags f;
+  // the fragments and scale dwords of a step, from its stage
+  auto read_step = [&](const uint8_t* st) {
     const uint32_t* sc = reinterpret_cast<const uint32_t*>(st + S::kXTile + S::kWTile);
     const int xr0 = wm * 16 * MI + fr; // x tile rows xr0 + 16 j
 #pragma unroll
@@ -382,8 +457,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       f.bf[j] = fragment(st, xr0 + 16 * j);
     }
 #pragma unroll
-    for (int q = 0; q < MI / 4; ++q) {
-      f.sb[q] = pack_scales(sc + xr0 + 64 * q);
+    for (int j = 0; j < MI; ++j) {
+      f.db[j] = sc[xr0 + 16 * j];
     }
     const int wr0 = wn * 16 * NI + fr; // W tile rows wr0 + 16 i
 #pragma unroll
@@ -391,8 +466,27 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       f.af[i] = fragment(st + S::kXTile, wr0 + 16 * i);
     }
 #pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      f.da[i] = sc[kBM + wr0 + 16 * i];
+    }
+  };
+  // byte kb of four rows' scale dwords, packed (row j in byte j)
+  auto settle = [&] {
+    auto pack_scales = [&](const uint32_t* d) {
+      const int sh = 8 * kb;
+      return static_cast<int>(
+          ((d[0] >> sh) & 0xffu) | (((d[1] >> sh) & 0xffu) << 8) | (((d[2] >> sh) & 0xffu) << 16) |
+          ((d[3] >> sh) << 24));
+    };
+#pragma unroll
+    for (int q = 0; q < MI / 4; ++q) {
+      f.sb[q] = pack_scales(f.db + 4 * q);
+      asm volatile("" : "+v"(f.sb[q])); // (packed here, not among the instructions that use it)
+    }
+#pragma unroll
     for (int q = 0; q < NI / 4; ++q) {
-      f.sa[q] = pack_scales(sc + kBM + wr0 + 64 * q);
+      f.sa[q] = pack_scales(f.da + 4 * q);
+      asm volatile("" : "+v"(f.sa[q]));
     }
   };
   // cbsz / blgp: the operand formats (0 = e4m3, 4 = e2m1); op_sel: which byte of
@@ -406,34 +500,14 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #define QQ_MMA_ROW(i)                                                            \
   QQ_MMA(i, 0) QQ_MMA(i, 1) QQ_MMA(i, 2) QQ_MMA(i, 3)                            \
   QQ_MMA(i, 4) QQ_MMA(i, 5) QQ_MMA(i, 6) QQ_MMA(i, 7)
-  auto multiply = [&](const Frags& f) {
+  auto multiply = [&] {
     QQ_MMA_ROW(0) QQ_MMA_ROW(1) QQ_MMA_ROW(2) QQ_MMA_ROW(3)
     QQ_MMA_ROW(4) QQ_MMA_ROW(5) QQ_MMA_ROW(6) QQ_MMA_ROW(7)
   };
 #undef QQ_MMA_ROW
 #undef QQ_MMA
 
-  // Steps 0 .. kStages - 2 are requested up front; iteration t waits for step t,
-  // asks for step t + kStages - 1 (into the stage that iteration t - 1 read) and
-  // multiplies step t.  (Reading the fragments one iteration ahead of their
-  // matrix instructions, from a second register set, changed nothing for the
-  // 4-bit kernel and cost the 8-bit one, with its three stages, a step of lead.)
-  constexpr int kS = S::kStages;
-#pragma unroll
-  for (int t = 0; t < kS - 1; ++t) {
-    issue(t);
-  }
-  for (int t = 0; t < nk; ++t) {
-    // the loads of steps t + 1 .. t + kStages - 2 may still be in flight
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kS - 2) * S::kLoads) : "memory");
-    __syncthreads(); // step t is in LDS for everyone; stage (t - 1) % kStages is free
-    issue(t + kS - 1);
-    Frags f;
-    read_step(t, f);
-    multiply(f);
-  }
-  // the clamped extra loads must have landed before the workgroup's LDS is given up
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  k_loop(read_step, settle, multiply);
 #undef QQ_DMA16
 #undef QQ_DMA4
 
@@ -516,6 +590,7 @@ int launch_qq_mfma(
     const uint8_t* xs,
     const uint32_t* wq,
     const uint8_t* ws,
+    bool ws_image,
     void* out,
     int M,
     int N,
@@ -532,6 +607,8 @@ int launch_qq_mfma(
   a.M = M;
   a.N = N;
   a.K = K;
+  a.ws_row = ws_image ? 4u : static_cast<uint32_t>(K) / 32;
+  a.ws_step = ws_image ? 4u * static_cast<uint32_t>(N) : 4u;
   MLXROCM_REHEARSE("qq_mfma(%s)", mode == MLXROCM_MXFP8 ? "e4m3" : "e2m1");
   return dispatch_dtype(dtype, [&](auto tval) {
     using T = decltype(tval);

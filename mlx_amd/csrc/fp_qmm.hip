@@ -919,7 +919,8 @@ extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, 
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     return round256(static_cast<size_t>(M) * K * bits / 8) +
         round256(static_cast<size_t>(M) * K / 32) +
-        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0);
+        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0) +
+        round256(qq_mfma_plane_bytes(M, N, K, mode));
   }
   return round256(static_cast<size_t>(M) * K * dtype_size(dtype)) +
       (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)
@@ -972,21 +973,17 @@ extern "C" int mlxrocm_fp_qqmm(
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     void* codes = workspace;
     uint8_t* xs = static_cast<uint8_t*>(workspace) + round256(n_elems * bits / 8);
-    rc = fp_quantize_activations(x, codes, xs, M, K, mode, dtype, s);
+    const bool image = qq_ws_image(M) && (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
+    uint8_t* ws = xs + round256(n_elems / 32);
+    rc = fp_quantize_activations(
+        x, codes, xs, M, K, scales, image ? ws : nullptr, N, mode, dtype, s);
     if (rc != MLXROCM_OK) {
       return rc;
     }
-    const uint8_t* ws = scales;
-    const bool image = qq_ws_image(M) && (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
-    if (image) {
-      uint8_t* dst = xs + round256(n_elems / 32);
-      rc = launch_mx_scale_image(scales, dst, N, K, s);
-      if (rc != MLXROCM_OK) {
-        return rc;
-      }
-      ws = dst;
-    }
-    return launch_qq_mfma(codes, xs, wq, ws, image, out, M, N, K, mode, dtype, s);
+    void* planes = xs + round256(n_elems / 32) +
+        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0);
+    return launch_qq_mfma(
+        codes, xs, wq, image ? ws : scales, image, out, M, N, K, mode, dtype, planes, s);
   }
   // x_hat in the element type, then the product with the quantized w
   rc = mlxrocm_fp_quantize_dequantize(x, workspace, n_elems, mode, dtype, stream);

@@ -243,11 +243,10 @@ __global__ __launch_bounds__(kFpBlock) void fp_dequantize_kernel(
 // multiplies as it is.  The scale bytes go out as the image that instruction's
 // kernel reads, [K / 128][rows] dwords of four consecutive groups' bytes (`rows`
 // rows of `row_groups` groups each, a multiple of four).
-template <typename T, int GS, int BITS, bool CODES = false>
-__global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
-    const T* w, T* out, size_t n_units, uint8_t* wq = nullptr, uint8_t* scales = nullptr,
-    uint32_t rows = 0, uint32_t row_groups = 1) {
-  const size_t u = static_cast<size_t>(blockIdx.x) * kFpBlock + threadIdx.x;
+template <typename T, int GS, int BITS, bool CODES>
+__device__ __forceinline__ void quantize_dequantize_unit(
+    const T* w, T* out, size_t u, size_t n_units, uint8_t* wq, uint8_t* scales, uint32_t rows,
+    uint32_t row_groups) {
   constexpr int kLanes = GS / 8;
   float v[8];
   const bool live = u < n_units;
@@ -354,6 +353,50 @@ __global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
       o[i] = scale * val;
     }
     store8<T>(out + u * 8, o);
+  }
+}
+
+template <typename T, int GS, int BITS>
+__global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
+    const T* w, T* out, size_t n_units) {
+  quantize_dequantize_unit<T, GS, BITS, false>(
+      w, out, static_cast<size_t>(blockIdx.x) * kFpBlock + threadIdx.x, n_units, nullptr, nullptr,
+      0, 1);
+}
+
+// The operands of the block-scaled matrix instruction: the first q_blocks workgroups
+// quantize x [rows][32 row_groups]; the rest (if any) rewrite the scale bytes of w, as
+// dwords [w_rows][steps], to [steps][w_rows], 64 rows x 32 steps each through LDS.
+// One launch for both: the second would take as long to start as it runs (4 us).
+template <typename T, int GS, int BITS>
+__global__ __launch_bounds__(kFpBlock) void fp_activations_kernel(
+    const T* x, size_t n_units, uint8_t* xq, uint8_t* xs, uint32_t rows, uint32_t row_groups,
+    unsigned q_blocks, const uint32_t* ws, uint32_t* ws_image, int w_rows, int steps) {
+  __shared__ uint32_t tile[64][33];
+  if (blockIdx.x < q_blocks) { // uniform
+    quantize_dequantize_unit<T, GS, BITS, true>(
+        x, nullptr, static_cast<size_t>(blockIdx.x) * kFpBlock + threadIdx.x, n_units, xq, xs, rows,
+        row_groups);
+    return;
+  }
+  const unsigned t = blockIdx.x - q_blocks;
+  const unsigned across = static_cast<unsigned>(steps + 31) / 32;
+  const int r0 = static_cast<int>(t / across) * 64;
+  const int s0 = static_cast<int>(t % across) * 32;
+  const int sx = threadIdx.x & 31;
+#pragma unroll
+  for (int r = threadIdx.x >> 5; r < 64; r += kFpBlock / 32) {
+    if (r0 + r < w_rows && s0 + sx < steps) {
+      tile[r][sx] = ws[static_cast<size_t>(r0 + r) * steps + s0 + sx];
+    }
+  }
+  __syncthreads();
+  const int rx = threadIdx.x & 63;
+#pragma unroll
+  for (int st = threadIdx.x >> 6; st < 32; st += kFpBlock / 64) {
+    if (r0 + rx < w_rows && s0 + st < steps) {
+      ws_image[static_cast<size_t>(s0 + st) * w_rows + r0 + rx] = tile[rx][st];
+    }
   }
 }
 
@@ -593,71 +636,36 @@ extern "C" int mlxrocm_fp_dequantize(
 namespace mlxrocm {
 
 // x -> codes and scale bytes by the rules of fp_quantize_dequantize (what qqmm
-// applies to its first operand), in the MX modes.  x is [M][K], K % 128 == 0.
+// applies to its first operand), in the MX modes.  x is [M][K], K % 128 == 0.  ws_image
+// not null: also the scale bytes ws of w, [N][K / 32] and 4-byte aligned, as the image
+// [K / 128][N] of dwords.
 int fp_quantize_activations(
-    const void* x, void* codes, uint8_t* scales, int M, int K, int mode, int dtype, hipStream_t s) {
-  const size_t n_elems = static_cast<size_t>(M) * K;
-  const size_t n_units = n_elems / 8;
-  const size_t blocks = (n_units + kFpBlock - 1) / kFpBlock;
+    const void* x, void* codes, uint8_t* scales, int M, int K, const uint8_t* ws, void* ws_image,
+    int N, int mode, int dtype, hipStream_t s) {
+  const size_t n_units = static_cast<size_t>(M) * K / 8;
+  const size_t q_blocks = (n_units + kFpBlock - 1) / kFpBlock;
+  const int steps = K / 128;
+  const size_t image_blocks =
+      ws_image != nullptr ? static_cast<size_t>((N + 63) / 64) * ((steps + 31) / 32) : 0;
+  const size_t blocks = q_blocks + image_blocks;
   if (blocks > 0x7fffffffull) {
-    return fail(MLXROCM_UNSUPPORTED, "[qqmm] %zu elements exceed the grid", n_elems);
+    return fail(
+        MLXROCM_UNSUPPORTED, "[qqmm] %zu elements exceed the grid", static_cast<size_t>(M) * K);
   }
   MLXROCM_REHEARSE("fp_quantize_activations");
   return dispatch_dtype(dtype, [&](auto tval) {
     using T = decltype(tval);
-    return dispatch_mode(mode, [&](auto gval, auto bval) {
-      constexpr int G = decltype(gval)::value;
+    auto run = [&](auto bval) {
       constexpr int B = decltype(bval)::value;
-      fp_quantize_dequantize_kernel<T, G, B, true><<<static_cast<unsigned>(blocks), kFpBlock, 0, s>>>(
-          static_cast<const T*>(x), nullptr, n_units, static_cast<uint8_t*>(codes), scales,
-          static_cast<uint32_t>(M), static_cast<uint32_t>(K / 32));
+      fp_activations_kernel<T, 32, B><<<static_cast<unsigned>(blocks), kFpBlock, 0, s>>>(
+          static_cast<const T*>(x), n_units, static_cast<uint8_t*>(codes), scales,
+          static_cast<uint32_t>(M), static_cast<uint32_t>(K / 32), static_cast<unsigned>(q_blocks),
+          reinterpret_cast<const uint32_t*>(ws), static_cast<uint32_t*>(ws_image), N, steps);
       MLXROCM_HIP_TRY(hipGetLastError());
       return static_cast<int>(MLXROCM_OK);
-    });
+    };
+    return mode == MLXROCM_MXFP8 ? run(IntC<8>{}) : run(IntC<4>{});
   });
-}
-
-namespace {
-
-// [rows][steps] dwords (four scale bytes of 128 codes) -> [steps][rows]: 64 rows x 32
-// steps per workgroup through LDS.
-__global__ __launch_bounds__(kFpBlock) void mx_scale_image_kernel(
-    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int rows, int steps) {
-  __shared__ uint32_t tile[64][33];
-  const int r0 = blockIdx.y * 64;
-  const int s0 = blockIdx.x * 32;
-  const int sx = threadIdx.x & 31;
-#pragma unroll
-  for (int r = threadIdx.x >> 5; r < 64; r += kFpBlock / 32) {
-    if (r0 + r < rows && s0 + sx < steps) {
-      tile[r][sx] = in[static_cast<size_t>(r0 + r) * steps + s0 + sx];
-    }
-  }
-  __syncthreads();
-  const int rx = threadIdx.x & 63;
-#pragma unroll
-  for (int st = threadIdx.x >> 6; st < 32; st += kFpBlock / 64) {
-    if (r0 + rx < rows && s0 + st < steps) {
-      out[static_cast<size_t>(s0 + st) * rows + r0 + rx] = tile[rx][st];
-    }
-  }
-}
-
-} // namespace
-
-// The scale bytes [rows][K / 32] of an MX weight as the image [K / 128][rows] of
-// dwords; scales 4-byte aligned, K % 128 == 0.
-int launch_mx_scale_image(const uint8_t* scales, void* image, int rows, int K, hipStream_t s) {
-  const int steps = K / 128;
-  const dim3 grid((steps + 31) / 32, (rows + 63) / 64);
-  if (grid.y > 65535u) {
-    return fail(MLXROCM_UNSUPPORTED, "[qqmm] N=%d exceeds the grid", rows);
-  }
-  MLXROCM_REHEARSE("mx_scale_image");
-  mx_scale_image_kernel<<<grid, kFpBlock, 0, s>>>(
-      reinterpret_cast<const uint32_t*>(scales), static_cast<uint32_t*>(image), rows, steps);
-  MLXROCM_HIP_TRY(hipGetLastError());
-  return MLXROCM_OK;
 }
 
 } // namespace mlxrocm

@@ -144,6 +144,7 @@ int launch_qmm_mfma_fp_grouped(const QmmArgs& a, int mode, int dtype, hipStream_
 // times the quantized w, both [rows][K]; K % 128 == 0.  ws: the caller's scale bytes
 // [N][K / 32], or (ws_image) their image.
 bool qq_mfma_supported(int M, int N, int K, int mode);
+size_t qq_mfma_plane_bytes(int M, int N, int K, int mode); // scratch for K ranges (planes)
 int launch_qq_mfma(
     const void* xq,
     const uint8_t* xs,
@@ -156,10 +157,11 @@ int launch_qq_mfma(
     int K,
     int mode,
     int dtype,
+    void* planes,
     hipStream_t s);
 int fp_quantize_activations(
-    const void* x, void* codes, uint8_t* scales, int M, int K, int mode, int dtype, hipStream_t s);
-int launch_mx_scale_image(const uint8_t* scales, void* image, int rows, int K, hipStream_t s);
+    const void* x, void* codes, uint8_t* scales, int M, int K, const uint8_t* ws, void* ws_image,
+    int N, int mode, int dtype, hipStream_t s);
 
 bool qmv_wide_supported(const QmmArgs& a, int gs, int bits, int dtype, bool transpose);
 int launch_qmv_wide(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);

@@ -83,6 +83,8 @@ struct QqArgs {
   void* out;             // [M][N]
   int M, N, K;
   uint32_t ws_row, ws_step; // bytes from a row of W, from a step, to the next
+  // K ranges (blockIdx.z): range z writes plane z of `out`, [splits][M][N]
+  int splits;
 };
 
 // slot of logical piece `piece` of tile row `row`
@@ -115,7 +117,16 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   const int M = a.M, N = a.N, K = a.K;
   const int n0 = blockIdx.x * kBN;
   const int m0 = blockIdx.y * kBM;
-  const int nk = K / kQqBK;
+  int k_first = 0;
+  int nk = K / kQqBK;
+  if (a.splits > 1) { // uniform (steps x ranges fits 32 bits: at most 2^24 x 16)
+    const uint32_t steps = static_cast<uint32_t>(nk);
+    const uint32_t splits = static_cast<uint32_t>(a.splits);
+    k_first = static_cast<int>(steps * blockIdx.z / splits);
+    nk = static_cast<int>(steps * (blockIdx.z + 1) / splits) - k_first;
+  }
+  const uint8_t* const xq = a.xq + static_cast<size_t>(k_first) * S::kRowBytes;
+  const uint8_t* const wq = a.wq + static_cast<size_t>(k_first) * S::kRowBytes;
   const uint32_t row_bytes = static_cast<uint32_t>(K) * BITS / 8;
 
   // ---- loader roles.  A DMA instruction of a wavefront moves kRowsPerDma rows
@@ -147,8 +158,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   for (int j = 0; j < S::kSDma; ++j) {
     const int d = scale_dword(j);
     const bool of_x = (j * S::kWaves + wave) * 64 < kBM;
-    sbase[j] = of_x ? a.xs : a.ws;
     sstep[j] = of_x ? 4u * static_cast<uint32_t>(M) : a.ws_step;
+    sbase[j] = (of_x ? a.xs : a.ws) + static_cast<size_t>(k_first) * sstep[j];
     if (d < kBM) {
       const int m = m0 + d < M ? m0 + d : M - 1;
       soff[j] = static_cast<uint32_t>(m) * 4u;
@@ -184,8 +195,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   // the stage at byte `stage`
   auto issue = [&](int t, int stage) {
     const int tc = t < nk ? t : nk - 1;
-    const uint8_t* xg = a.xq + static_cast<size_t>(tc) * S::kRowBytes;
-    const uint8_t* wg = a.wq + static_cast<size_t>(tc) * S::kRowBytes;
+    const uint8_t* xg = xq + static_cast<size_t>(tc) * S::kRowBytes;
+    const uint8_t* wg = wq + static_cast<size_t>(tc) * S::kRowBytes;
 #pragma unroll
     for (int j = 0; j < S::kXDma; ++j) {
       QQ_DMA16(xoff[j], xg, stage + (wave * S::kXDma + j) * 1024);
@@ -358,7 +369,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     k_loop(read_step, settle, multiply);
     // D[n][m] 32 x 32: register i of lane (col, half) holds n = 8 (i / 4) + 4 half
     // + i % 4, m = col
-    TO* out = static_cast<TO*>(a.out);
+    TO* out = static_cast<TO*>(a.out) + static_cast<size_t>(blockIdx.z) * M * N;
     const int col = lane & 31;
     const int half = lane >> 5;
     const bool vec_ok = (N % 4) == 0;
@@ -512,7 +523,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #undef QQ_DMA4
 
   // D[n][m]: register r of lane (col, quad) holds n = 4 quad + r, m = col
-  TO* out = static_cast<TO*>(a.out);
+  TO* out = static_cast<TO*>(a.out) + static_cast<size_t>(blockIdx.z) * M * N;
   const int col = lane & 15;
   const int quad = lane >> 4;
   const bool vec_ok = (N % 4) == 0;
@@ -555,7 +566,7 @@ int launch_qq(const QqArgs& a, hipStream_t s) {
   using S = QqShape<BITS, MI, NI, WM, WN>;
   constexpr size_t smem = static_cast<size_t>(S::kStages) * S::kStage;
   static_assert(smem <= 160 * 1024, "LDS");
-  const dim3 grid((a.N + S::kBN - 1) / S::kBN, (a.M + S::kBM - 1) / S::kBM, 1);
+  const dim3 grid((a.N + S::kBN - 1) / S::kBN, (a.M + S::kBM - 1) / S::kBM, a.splits);
   if (grid.y > 65535u) {
     return fail(MLXROCM_UNSUPPORTED, "[qqmm] M=%d exceeds the grid", a.M);
   }
@@ -585,6 +596,50 @@ bool qq_mfma_supported(int M, int N, int K, int mode) {
       static_cast<uint64_t>(N) * K * bits / 8 < limit;
 }
 
+// Tile width and K ranges of a launch, the ones that finish first.  A step of the
+// 256 x 128 tile takes 0.8..1 us with 8-bit codes and 0.6 with 4-bit ones (256 x 256:
+// 1.2), a tile some 4 us before and after its steps; ranges cost fp32 planes, written
+// and read again at about 5 TB/s, and a launch.  [512, 14336] x [4096, 14336] has 64
+// tiles for 256 compute units: mxfp8 105 -> 53 us in ranges, mxfp4 82 -> 49; 16 rows,
+// 4096 x 4096: 30 -> 14 and 24 -> 14.
+struct QqPlan {
+  bool wide; // 4-bit codes: 256 x 256
+  int splits;
+};
+QqPlan qq_plan(int M, int N, int K, int mode) {
+  const long cus = compute_units();
+  const long mt = (M + 255) / 256;
+  const long steps = K / kQqBK;
+  const long wide_tiles = mt * ((N + 255) / 256);
+  // (4-bit codes: the wide tile where it still fills the chip)
+  QqPlan best = {mode == MLXROCM_MXFP4 && wide_tiles >= cus, 1};
+  if (best.wide || (static_cast<int64_t>(M) * N) % 4 != 0) {
+    return best;
+  }
+  const long tiles = mt * ((N + 127) / 128);
+  const double step = mode == MLXROCM_MXFP8 ? 900.0 : 600.0; // ns
+  auto cost = [&](long splits) -> double {
+    const long rounds = (tiles * splits + cus - 1) / cus;
+    const double ns = static_cast<double>(rounds) *
+        (static_cast<double>((steps + splits - 1) / splits) * step + 4000.0);
+    return splits == 1 ? ns : ns + 4000.0 + static_cast<double>(splits) * M * N * 4.0 / 4000.0;
+  };
+  double best_ns = cost(1) / 1.08;
+  for (long splits = 2; splits <= 16 && splits * 4 <= steps && splits * tiles <= 2 * cus; ++splits) {
+    const double ns = cost(splits);
+    if (ns < best_ns) {
+      best.splits = static_cast<int>(splits);
+      best_ns = ns;
+    }
+  }
+  return best;
+}
+
+size_t qq_mfma_plane_bytes(int M, int N, int K, int mode) {
+  const int splits = qq_plan(M, N, K, mode).splits;
+  return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
+}
+
 int launch_qq_mfma(
     const void* xq,
     const uint8_t* xs,
@@ -597,31 +652,34 @@ int launch_qq_mfma(
     int K,
     int mode,
     int dtype,
+    void* planes,
     hipStream_t s) {
+  const QqPlan pl = qq_plan(M, N, K, mode);
   QqArgs a;
+  a.splits = pl.splits;
   a.xq = static_cast<const uint8_t*>(xq);
   a.xs = xs;
   a.wq = reinterpret_cast<const uint8_t*>(wq);
   a.ws = ws;
-  a.out = out;
+  a.out = pl.splits > 1 ? planes : out;
   a.M = M;
   a.N = N;
   a.K = K;
   a.ws_row = ws_image ? 4u : static_cast<uint32_t>(K) / 32;
   a.ws_step = ws_image ? 4u * static_cast<uint32_t>(N) : 4u;
   MLXROCM_REHEARSE("qq_mfma(%s)", mode == MLXROCM_MXFP8 ? "e4m3" : "e2m1");
-  return dispatch_dtype(dtype, [&](auto tval) {
+  const int rc = dispatch_dtype(pl.splits > 1 ? MLXROCM_FLOAT32 : dtype, [&](auto tval) {
     using T = decltype(tval);
     if (mode == MLXROCM_MXFP8) {
       return launch_qq<T, 8, 4, 4, 4, 2>(a, s);
     }
-    // the wide tile where it still fills the chip
-    const long wide = static_cast<long>((M + 255) / 256) * ((N + 255) / 256);
-    if (wide >= compute_units()) {
-      return launch_qq<T, 4, 4, 8, 4, 2, true>(a, s);
-    }
-    return launch_qq<T, 4, 4, 4, 4, 2, true>(a, s);
+    return pl.wide ? launch_qq<T, 4, 4, 8, 4, 2, true>(a, s)
+                   : launch_qq<T, 4, 4, 4, 4, 2, true>(a, s);
   });
+  if (rc != MLXROCM_OK || pl.splits == 1) {
+    return rc;
+  }
+  return reduce_k_splits(planes, out, static_cast<size_t>(M) * N, pl.splits, dtype, s);
 }
 
 } // namespace mlxrocm

@@ -1,5 +1,6 @@
 """qqmm on the block-scaled matrix instruction: fewer K-steps than LDS stages, one
-more, ragged tiles, scale bytes in the caller's layout and as an image --
+more, ragged tiles, scale bytes in the caller's layout and as an image,
+K ranges --
 against the product of the two dequantized operands in 64 bits."""
 import pytest
 import torch

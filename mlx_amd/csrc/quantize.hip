@@ -1,6 +1,7 @@
 // quantize.hip -- affine group-wise quantize / dequantize for gfx950.
 //
-// Both kernels are HBM-bound streaming kernels.  A lane owns one "unit" of 8
+// Streaming kernels, dequantize bound by HBM and quantize by its vector instructions.
+// A lane owns one "unit" of 8
 // consecutive elements: 8 codes are exactly BITS bytes of the packed stream for
 // every supported width, so a unit never shares a byte with its neighbour even
 // when 3/5/6-bit codes straddle uint32 words.  A quantization group is GS/8
@@ -87,7 +88,7 @@ __device__ __forceinline__ void quantize_unit_exact(
 
 }
 
-// lane ^ OFF of an operand that is the same within aligned runs of OFF lanes: data
+// the value of lane ^ OFF (or one equal to it), of an operand that is the same within aligned runs of OFF lanes: data
 // parallel moves, no LDS (half_mirror and mirror reverse runs of 8 and 16)
 template <int OFF>
 __device__ __forceinline__ float dpp_xor(float x) {

@@ -44,6 +44,16 @@ def _held(layer: torch.nn.Module, *names: str):
         return [getattr(layer, name) for name in names]
 
 
+def _passable(layer: torch.nn.Module, cls: type) -> bool:
+    """Whether calling ``layer`` is ``cls.forward`` over its buffers and nothing more,
+    so that a block may hand those buffers to one call of the library instead: not a
+    wrapper, an adapter on top of ``cls``, or a layer that someone listens to."""
+    return (type(layer) is cls and "forward" not in layer.__dict__
+            and not (layer._forward_hooks or layer._forward_pre_hooks
+                     or layer._backward_hooks or layer._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
 class QuantizedLinear(torch.nn.Module):
     """``y = quantized_matmul(x, weight, scales, biases, transpose=True) + bias``."""
 
@@ -295,10 +305,11 @@ class QuantizedSwitchLinear(torch.nn.Module):
 class SwitchGLU(torch.nn.Module):
     """Expert-routed gated MLP: ``down(act(gate(x)) * up(x))`` with every
     projection a :class:`QuantizedSwitchLinear` and token ``t`` sent to the
-    experts ``indices[t, :]``.  With silu, no additive biases and 16-bit types the
-    whole block is one call of the library, which groups the routed rows by expert
-    once; otherwise the three projections in turn (each groups the rows itself,
-    whatever their order, so ``sort_threshold`` no longer changes anything)."""
+    experts ``indices[t, :]``.  With silu, no additive biases, 16-bit types and
+    projections that are nothing but that (no subclass, no hooks) the whole block is
+    one call of the library, which groups the routed rows by expert once; otherwise
+    the three projections in turn (each groups the rows itself, whatever their order,
+    so ``sort_threshold`` no longer changes anything)."""
 
     def __init__(self, input_dims: int, hidden_dims: int, num_experts: int,
                  activation: Callable[[torch.Tensor], torch.Tensor] = torch.nn.functional.silu,
@@ -317,6 +328,8 @@ class SwitchGLU(torch.nn.Module):
             return None
         modules = self._modules
         layers = [modules[name] for name in ("gate_proj", "up_proj", "down_proj")]
+        if not all(_passable(layer, QuantizedSwitchLinear) for layer in layers):
+            return None
         first = layers[0]
         triplets = []
         for layer in layers:

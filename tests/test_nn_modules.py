@@ -1,0 +1,81 @@
+"""The layer blocks on the host: which projections a block may pass by and hand to
+one call of the library.  No GPU: the operators are stand-ins."""
+import pytest
+import torch
+
+from mlx_amd import nn, ops
+
+D, F, E = 64, 128, 4
+
+
+@pytest.fixture
+def stubs(monkeypatch):
+    """Operators that record their calls; products are ones."""
+    calls = []
+
+    def quantize(w, group_size=None, bits=None, mode="affine"):
+        g, b = group_size or 64, bits or 4
+        s = torch.zeros(w.shape[:-1] + (w.shape[-1] // g,), dtype=w.dtype)
+        return torch.zeros(w.shape[:-1] + (w.shape[-1] * b // 32,), dtype=torch.uint32), s, s.clone()
+
+    def gather_qmm(x, w, *args, rhs_indices=None, **kw):
+        calls.append("gather_qmm")
+        shape = torch.broadcast_shapes(x.shape[:-2], rhs_indices.shape)
+        return torch.ones(*shape, x.shape[-2], w.shape[-2], dtype=x.dtype)
+
+    class Fast:
+        def switch_glu(self, x, indices, *args):
+            calls.append("switch_glu")
+            return torch.zeros(*indices.shape, x.shape[-1], dtype=x.dtype)
+
+    monkeypatch.setattr(ops, "quantize", quantize)
+    monkeypatch.setattr(ops, "gather_qmm", gather_qmm)
+    monkeypatch.setattr(ops, "_fast", Fast())
+    return calls
+
+
+def _switch_glu():
+    return nn.SwitchGLU(D, F, E, dtype=torch.bfloat16, device="cpu")
+
+
+class _Adapter(nn.QuantizedSwitchLinear):
+    def forward(self, x, indices, sorted_indices=False):
+        return super().forward(x, indices, sorted_indices) + 1
+
+
+class _Wrapper(torch.nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, *args, **kwargs):
+        return self.inner(*args, **kwargs) + 1
+
+
+@pytest.mark.parametrize("name", ("gate_proj", "up_proj", "down_proj"))
+@pytest.mark.parametrize("how", ("subclass", "wrapper", "hook", "pre-hook", "forward"))
+def test_switch_glu_calls_projections_that_are_more_than_their_buffers(stubs, name, how):
+    x, indices = torch.ones(3, D, dtype=torch.bfloat16), torch.zeros(3, 2, dtype=torch.int64)
+    block = _switch_glu()
+    block(x, indices)
+    assert stubs == ["switch_glu"]
+    layer = getattr(block, name)
+    seen = []
+    if how == "subclass":
+        layer.__class__ = _Adapter
+    elif how == "wrapper":
+        setattr(block, name, _Wrapper(layer))
+    elif how == "hook":
+        layer.register_forward_hook(lambda *args: seen.append(name))
+    elif how == "pre-hook":
+        layer.register_forward_pre_hook(lambda *args: seen.append(name))
+    else:
+        inner = layer.forward
+        layer.forward = lambda *args, **kwargs: inner(*args, **kwargs) + 1
+    y = block(x, indices)
+    assert stubs[1:] == ["gather_qmm"] * 3
+    assert y.shape == (3, 2, D)
+    if "hook" in how:
+        assert seen == [name]
+    elif name == "down_proj":
+        assert bool((y == 2).all())

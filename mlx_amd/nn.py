@@ -232,9 +232,9 @@ class SwiGLU(torch.nn.Module):
     """Gated MLP block ``down(silu(gate(x)) * up(x))`` over three
     :class:`QuantizedLinear` layers (the MLP of Llama-style models built from
     ``nn.QuantizedLinear``, python/mlx/nn/layers/quantized.py:205-307).  With at
-    most 8 rows of x and no additive biases the gate and up projections and the
-    gate arithmetic run as one ``quantized_swiglu`` call; otherwise as the three
-    separate products."""
+    most 8 rows of x, no additive biases and projections that are nothing but that
+    layer (no subclass, no hooks) gate, up and the gate arithmetic run as one
+    ``quantized_swiglu`` call; otherwise as the three separate products."""
 
     def __init__(self, input_dims: int, hidden_dims: int, bias: bool = False,
                  group_size: Optional[int] = None, bits: Optional[int] = None,
@@ -249,14 +249,15 @@ class SwiGLU(torch.nn.Module):
         modules = self._modules
         g, u = modules["gate_proj"], modules["up_proj"]
         rows = x.numel() // max(x.shape[-1], 1)
-        *g_triplet, g_bias = _held(g, "weight", "scales", "biases", "bias")
-        *u_triplet, u_bias = _held(u, "weight", "scales", "biases", "bias")
-        fused = (0 < rows <= 8 and g_bias is None and u_bias is None
-                 and (g.group_size, g.bits, g.mode) == (u.group_size, u.bits, "affine")
-                 and u.mode == "affine")
-        if fused:
-            h = ops.quantized_swiglu(x, tuple(g_triplet), tuple(u_triplet), g.group_size, g.bits)
-        else:
+        h = None
+        if (0 < rows <= 8 and _passable(g, QuantizedLinear) and _passable(u, QuantizedLinear)
+                and (g.group_size, g.bits, g.mode) == (u.group_size, u.bits, "affine")
+                and u.mode == "affine"):
+            *g_triplet, g_bias = _held(g, "weight", "scales", "biases", "bias")
+            *u_triplet, u_bias = _held(u, "weight", "scales", "biases", "bias")
+            if g_bias is None and u_bias is None:
+                h = ops.quantized_swiglu(x, tuple(g_triplet), tuple(u_triplet), g.group_size, g.bits)
+        if h is None:
             h = torch.nn.functional.silu(g(x)) * u(x)
         return modules["down_proj"](h)
 

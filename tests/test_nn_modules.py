@@ -23,6 +23,14 @@ def stubs(monkeypatch):
         shape = torch.broadcast_shapes(x.shape[:-2], rhs_indices.shape)
         return torch.ones(*shape, x.shape[-2], w.shape[-2], dtype=x.dtype)
 
+    def quantized_matmul(x, w, *args, **kw):
+        calls.append("quantized_matmul")
+        return torch.ones(*x.shape[:-1], w.shape[-2], dtype=x.dtype)
+
+    def quantized_swiglu(x, gate, up, *args):
+        calls.append("quantized_swiglu")
+        return torch.ones(*x.shape[:-1], gate[0].shape[0], dtype=x.dtype)
+
     class Fast:
         def switch_glu(self, x, indices, *args):
             calls.append("switch_glu")
@@ -30,6 +38,8 @@ def stubs(monkeypatch):
 
     monkeypatch.setattr(ops, "quantize", quantize)
     monkeypatch.setattr(ops, "gather_qmm", gather_qmm)
+    monkeypatch.setattr(ops, "quantized_matmul", quantized_matmul)
+    monkeypatch.setattr(ops, "quantized_swiglu", quantized_swiglu)
     monkeypatch.setattr(ops, "_fast", Fast())
     return calls
 
@@ -41,6 +51,11 @@ def _switch_glu():
 class _Adapter(nn.QuantizedSwitchLinear):
     def forward(self, x, indices, sorted_indices=False):
         return super().forward(x, indices, sorted_indices) + 1
+
+
+class _LinearAdapter(nn.QuantizedLinear):
+    def forward(self, x):
+        return super().forward(x) + 1
 
 
 class _Wrapper(torch.nn.Module):
@@ -79,3 +94,24 @@ def test_switch_glu_calls_projections_that_are_more_than_their_buffers(stubs, na
         assert seen == [name]
     elif name == "down_proj":
         assert bool((y == 2).all())
+
+
+@pytest.mark.parametrize("rows", (1, 8, 9))
+@pytest.mark.parametrize("how", ("plain", "subclass", "wrapper", "hook", "other layer"))
+def test_swiglu_calls_projections_that_are_more_than_their_buffers(stubs, rows, how):
+    block = nn.SwiGLU(D, F, dtype=torch.bfloat16, device="cpu")
+    seen = []
+    if how == "subclass":
+        block.up_proj.__class__ = _LinearAdapter
+    elif how == "wrapper":
+        block.gate_proj, block.up_proj = _Wrapper(block.gate_proj), _Wrapper(block.up_proj)
+    elif how == "hook":
+        block.gate_proj.register_forward_hook(lambda *args: seen.append(1))
+    elif how == "other layer":  # (no scales)
+        block.gate_proj = torch.nn.Linear(D, F, dtype=torch.bfloat16)
+    y = block(torch.ones(rows, D, dtype=torch.bfloat16))
+    assert y.shape == (rows, D)
+    products = 2 if how == "other layer" else 3
+    assert stubs == (["quantized_swiglu", "quantized_matmul"] if how == "plain" and rows <= 8
+                     else ["quantized_matmul"] * products)
+    assert len(seen) == (how == "hook")

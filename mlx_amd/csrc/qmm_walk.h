@@ -26,7 +26,8 @@
 //     fp32.  What offset and biases add, sum_g X[m][g] * (bias[n][g] - offset *
 //     scale[n][g]), is one v_mfma_f32_16x16x4_f32 per tile and four groups; X, the
 //     sums of x over a group, come from a chain with a matrix of ones.  Nothing is
-//     rounded before the final conversion;
+//     rounded before the final conversion, but the offset is taken back in fp32, so
+//     its size against the codes matters (walk_offset);
 //   * scales and biases of the workgroup's rows go to LDS once, as [group][row]
 //     pairs.
 #pragma once
@@ -75,18 +76,38 @@ template <>
 struct WalkMagic<bf16_t> {
   static constexpr uint32_t kBits = 0x43004300u; // 128.0 twice: 4-bit codes fit below
   static constexpr float kOffset = 128.0f;
-  static constexpr int kCodeBits = 7; // widest code that fits beside the offset
+  static constexpr uint32_t kOnes = 0x3F803F80u; // 1.0 twice
+  static constexpr int kCodeBits = 7; // of the mantissa: widest code that fits beside an offset
 };
 template <>
 struct WalkMagic<f16_t> {
   static constexpr uint32_t kBits = 0x64006400u; // 1024.0 twice
   static constexpr float kOffset = 1024.0f;
+  static constexpr uint32_t kOnes = 0x3C003C00u;
   static constexpr int kCodeBits = 10;
 };
 
-// What the widened codes of a width are above the codes themselves.
+// A widened code is (code + offset) / unit.  At the bottom of the mantissa (unit 1) the
+// packed dwords of 4 and 8 bits need the fewest instructions; everything else lies at
+// its top, for an offset of 2^bits: the fp32 sums lose what the offset is above the
+// codes, and 1024 + c loses more of a narrow c than a float16 result hides (x of one
+// sign, K = 4096, error of the result at the bottom / at the top: 2 bits, group 64
+// 5.9e-4 / 2.1e-4; 3 bits 3.6e-4 / 2.1e-4; 4 bits, group 128 3.4e-4 / 2.1e-4; 2.1e-4 is
+// what rounding the exact result loses).  Both take the same time.
+template <typename T, int BITS>
+constexpr bool walk_at_top() {
+  constexpr bool f16 = std::is_same<T, f16_t>::value;
+  return BITS <= WalkMagic<T>::kCodeBits && BITS != 8 && (f16 || BITS != 4);
+}
+template <typename T, int BITS>
+constexpr float walk_unit() {
+  return walk_at_top<T, BITS>() ? static_cast<float>(1 << BITS) : 1.0f;
+}
 template <typename T, int BITS>
 constexpr float walk_offset() {
+  if (walk_at_top<T, BITS>()) {
+    return static_cast<float>(1 << BITS);
+  }
   return BITS <= WalkMagic<T>::kCodeBits ? WalkMagic<T>::kOffset : 0.0f;
 }
 
@@ -165,6 +186,11 @@ __device__ __forceinline__ void swap_quads(uint32_t& a, uint32_t& b) {
 template <typename T, int BITS, int GS>
 struct WalkCodes {
   static constexpr bool kMagic = BITS <= WalkMagic<T>::kCodeBits;
+  static constexpr bool kTop = walk_at_top<T, BITS>();
+  static constexpr uint32_t kOffsetBits = kTop ? WalkMagic<T>::kOnes : WalkMagic<T>::kBits;
+  static constexpr int kShift = kTop ? WalkMagic<T>::kCodeBits - BITS : 0; // of a code
+  static constexpr uint32_t kMask = // of a code in the low half (4 bits: in both)
+      (BITS == 4 ? 0x000f000fu : (1u << BITS) - 1u) << kShift;
 
   // first code (within the chunk) of the eight that quad q holds in operand i
   static __device__ __forceinline__ int k_of(int i, int q) {
@@ -188,11 +214,18 @@ struct WalkCodes {
   }
 
   static __device__ __forceinline__ uint32_t pair(uint32_t c0, uint32_t c1) {
-    if constexpr (kMagic) {
-      return (c0 | (c1 << 16)) | WalkMagic<T>::kBits;
-    } else {
-      return pack2<T>(static_cast<float>(c0), static_cast<float>(c1));
+    return pack2<T>(static_cast<float>(c0), static_cast<float>(c1));
+  }
+
+  // (codes that straddle dwords) code i of w with its lowest bit at bit `at`
+  static __device__ __forceinline__ uint32_t
+  placed(const uint32_t (&w)[BITS], int i, int at) {
+    const int d = i * BITS / 32;
+    const int b = i * BITS % 32;
+    if (b + BITS > 32) {
+      return __builtin_amdgcn_alignbit(w[d + 1 < BITS ? d + 1 : d], w[d], b - at);
     }
+    return b >= at ? w[d] >> (b - at) : w[d] << (at - b);
   }
 
   // The registers the operands of a stage are made from: the packed dwords with
@@ -201,7 +234,8 @@ struct WalkCodes {
   static constexpr bool kWhole = BITS == 4 || BITS == 8;
   static constexpr int kKept = kWhole ? BITS : 16;
 
-  static __device__ __forceinline__ void regroup(const uint32_t (&w)[BITS], uint32_t (&d)[kKept]) {
+  static __device__ __forceinline__ void
+  regroup(const uint32_t (&w)[BITS], uint32_t (&d)[kKept], uint32_t mask, uint32_t magic) {
     if constexpr (BITS == 4) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -229,7 +263,9 @@ struct WalkCodes {
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        d[i] = pair(code32<BITS>(w, 2 * i), code32<BITS>(w, 2 * i + 1));
+        d[i] = (placed(w, 2 * i, kShift) & mask) | magic;
+        asm("" : "+v"(d[i])); // (two v_and_or_b32, not regrouped into three instructions)
+        d[i] = (placed(w, 2 * i + 1, kShift + 16) & (mask << 16)) | d[i];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) { // d[4 i + j]: dword j of operand i
@@ -257,10 +293,13 @@ struct WalkCodes {
     uint4 o;
     if constexpr (BITS == 4) {
       // codes 0,4 1,5 2,6 3,7: x is staged in that order
-      o.x = (d[i] & mask) | magic;
-      o.y = ((d[i] >> 4) & mask) | magic;
-      o.z = ((d[i] >> 8) & mask) | magic;
-      o.w = ((d[i] >> 12) & mask) | magic;
+      const auto at = [&](int bit) { // the codes at `bit` and 16 on, in their place
+        return bit > kShift ? d[i] >> (bit - kShift) : d[i] << (kShift - bit);
+      };
+      o.x = (at(0) & mask) | magic;
+      o.y = (at(4) & mask) | magic;
+      o.z = (at(8) & mask) | magic;
+      o.w = (at(12) & mask) | magic;
     } else if constexpr (BITS == 8 && kMagic) {
       // byte, 0x64, byte, 0x64
       o.x = __builtin_amdgcn_perm(magic, d[2 * i], 0x07010700u);
@@ -507,7 +546,7 @@ void qmm_walk_kernel(WalkArgs wa) {
   const bool eights = FP == 0 && ((G | g0 | g_count) & 7) == 0;
   const auto put_group = [&](int g, uint32_t s, uint32_t b) { // 16 bits each
     const float sv = half_value<T>(s);
-    stab[g * kRows + trow] = sv;
+    stab[g * kRows + trow] = sv * walk_unit<T, BITS>();
     btab[g * kRows + trow] = fmaf(-kOff, sv, half_value<T>(b));
   };
   const auto put_eight = [&](int g, const uint4& s, const uint4& b) {
@@ -610,8 +649,8 @@ void qmm_walk_kernel(WalkArgs wa) {
   const uint32_t one2 = pack2<T>(1.0f, 1.0f);
   const uint4 ones = make_uint4(one2, one2, one2, one2);
 
-  uint32_t mask = 0x000f000fu;
-  uint32_t magic = WalkMagic<T>::kBits;
+  uint32_t mask = Codes::kMask;
+  uint32_t magic = Codes::kOffsetBits;
   asm("" : "+v"(mask));
   asm("" : "+v"(magic));
 
@@ -690,7 +729,7 @@ void qmm_walk_kernel(WalkArgs wa) {
             asm volatile("" : "+v"(kept[t][i]));
           }
         } else {
-          Codes::regroup(d, kept[t]);
+          Codes::regroup(d, kept[t], mask, magic);
         }
       }
       __builtin_amdgcn_sched_barrier(0);

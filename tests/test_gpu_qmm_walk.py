@@ -25,9 +25,11 @@ def _check(x, q, group, bits, mode, y):
         w = mlx_amd.dequantize(q[0], q[1], mode=mode, dtype=torch.float32).double()
     want = x.double() @ w.T
     size = x.double().abs() @ w.abs().T
-    # (codes are multiplied with an offset of at most 1024 that the biases take back,
-    # in fp32: 1024 / (2^bits - 1) times the size of the product at worst)
-    sums = 2e-6 * (1 if mode != "affine" else 1 + 1024 / (2 ** bits - 1) / 8)
+    # (codes are multiplied with an offset that the biases take back, in fp32: that adds
+    # offset / (2^bits - 1) times the size of the product at worst)
+    f16 = x.dtype == torch.float16
+    offset = {8: 1024 if f16 else 0, 4: 16 if f16 else 128}.get(bits, 2 ** (bits or 0))
+    sums = 2e-6 * (1 if mode != "affine" else 1 + offset / (2 ** bits - 1) / 8)
     half = 2.0 ** -8 if x.dtype == torch.bfloat16 else 2.0 ** -11
     err = (y.double() - want).abs()
     ok = bool((err <= half * want.abs() + sums * size).all())
@@ -58,6 +60,25 @@ def test_affine(bits, group):
             y = mlx_amd.quantized_matmul(x, *q, group_size=group, bits=bits)
             _check(x, q, group, bits, "affine", y)
     assert taken >= 18, taken
+
+
+@pytest.mark.parametrize("bits", (2, 3, 4, 5, 6, 8))
+def test_x_of_one_sign(bits):
+    """Where every x has one sign the codes' offset weighs most against the result.
+    float16 results may lose nothing to it: sums in fp32 within half of what rounding
+    the exact result loses (the two add up in squares: sqrt(1 + 1/4))."""
+    for group, N, K in ((64, 1024, 2048), (128, 4096, 4096), (64, 4096, 8192)):
+        for M in (3, 6, 20, 40):
+            if not _lib.load().mlxrocm_qmm_rows_supported(M, N, K, 1, group, bits, 1):
+                continue
+            x, w = _inputs(M, N, K, torch.float16, M)
+            x = x.abs()
+            q = mlx_amd.quantize(w, group, bits)
+            y = mlx_amd.quantized_matmul(x, *q, group_size=group, bits=bits)
+            exact = x.double() @ mlx_amd.dequantize(
+                q[0], q[1].float(), q[2].float(), group, bits).double().T
+            rounding = (exact.half().double() - exact).norm()
+            assert float((y.double() - exact).norm() / rounding) < 1.25 ** 0.5, (group, N, K, M)
 
 
 @pytest.mark.parametrize("mode", ("mxfp4", "mxfp8", "nvfp4"))

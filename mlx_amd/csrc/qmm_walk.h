@@ -387,6 +387,32 @@ __device__ __forceinline__ float half_value(uint32_t v) {
     return static_cast<float>(__builtin_bit_cast(f16_t, static_cast<uint16_t>(v)));
   }
 }
+// x . w over codes [k0, k1) of a row, term by term with the weights as dequantize gives
+// them.  Only for sums that did not come out finite: an infinite x, or one whose
+// products with the offset codes leave fp32, would otherwise turn every result of its
+// row into inf - inf.  One thread per result, some hundred microseconds (a NaN in x ends
+// it at once).
+template <typename T, int BITS, int GS>
+__device__ __forceinline__ float walk_terms(
+    const T* x, const uint32_t* w, const T* scales, const T* biases, int k0, int k1) {
+  float v = 0.0f;
+#pragma unroll 1
+  for (int k = k0; k < k1 && v == v; k += 32) {
+    const uint32_t* p = w + static_cast<size_t>(k / 32) * BITS;
+    const float s = to_f32(scales[k / GS]);
+    const float b = to_f32(biases[k / GS]);
+#pragma unroll 1
+    for (int i = 0; i < 32; ++i) {
+      const int d = i * BITS / 32;
+      const int at = i * BITS % 32;
+      const uint64_t high = at + BITS > 32 ? p[d + 1] : 0u; // the code goes on there
+      const uint32_t c = static_cast<uint32_t>((high << 32 | p[d]) >> at) & ((1u << BITS) - 1u);
+      v = fmaf(to_f32(x[k + i]), round_to<T>(fmaf(s, static_cast<float>(c), b)), v);
+    }
+  }
+  return v;
+}
+
 // LDS: the [group][row] tables, then two x stages, which the final sums reuse.
 template <int MR, int NW, int KW, int NPW>
 constexpr size_t walk_x_bytes() {
@@ -852,20 +878,49 @@ void qmm_walk_kernel(WalkArgs wa) {
       }
       return v * factor;
     };
-    for (int m = tid / kSumRows; m < M; m += kSumM) {
-      const float v = sum_of(t, m);
+    const auto finish = [&](int m, auto&& sum) {
+      const float v = sum(t, m);
       const size_t at = static_cast<size_t>(m) * N + n;
       if (glu) {
         // the roundings of the unfused chain: both products, the sigmoid, gate *
         // sigmoid and the result
         const float g = round_to<T>(v);
-        const float up = round_to<T>(sum_of(t + NT / 2, m));
+        const float up = round_to<T>(sum(t + NT / 2, m));
         const float sg = round_to<T>(1.0f / (1.0f + __expf(-g)));
         p.out[at] = from_f32<T>(round_to<T>(g * sg) * up);
       } else if (planes) {
         plane[at] = v;
       } else {
         p.out[at] = from_f32<T>(p.valid ? v : 0.0f);
+      }
+    };
+    bool finite = true;
+    for (int m = tid / kSumRows; m < M; m += kSumM) {
+      finish(m, [&](int tile, int row_of_x) {
+        const float v = sum_of(tile, row_of_x);
+        finite = finite && __builtin_isfinite(v);
+        return v;
+      });
+    }
+    if constexpr (FP == 0) {
+      if (!finite) { // (this thread's results alone)
+        const int k1 = s1 * KW * kWkChunk < K ? s1 * KW * kWkChunk : K;
+        for (int m = tid / kSumRows; m < M; m += kSumM) {
+          finish(m, [&](int tile, int row_of_x) {
+            const float v = sum_of(tile, row_of_x);
+            if (__builtin_isfinite(v)) {
+              return v;
+            }
+            const bool alt = tile >= tiles_n;
+            const size_t at = static_cast<size_t>(n);
+            return walk_terms<T, BITS, GS>(
+                p.x + static_cast<size_t>(row_of_x) * K,
+                (alt ? a.w_alt : reinterpret_cast<const uint32_t*>(p.w)) + at * (K / 32) * BITS,
+                (alt ? static_cast<const T*>(a.scales_alt) : p.scales) + at * G,
+                (alt ? static_cast<const T*>(a.biases_alt) : p.biases) + at * G,
+                s0 * KW * kWkChunk, k1);
+          });
+        }
       }
     }
   }

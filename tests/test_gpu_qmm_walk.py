@@ -81,6 +81,53 @@ def test_x_of_one_sign(bits):
             assert float((y.double() - exact).norm() / rounding) < 1.25 ** 0.5, (group, N, K, M)
 
 
+def _same_kind(y, want):
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isposinf(), want.isposinf())
+    assert torch.equal(y.isneginf(), want.isneginf())
+
+
+@pytest.mark.parametrize("bits", (2, 3, 4, 5, 6, 8))
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+def test_infinite_and_huge_x(bits, dtype):
+    """One x that is infinite, NaN or near the end of bfloat16 decides its row as a
+    product with the dequantized weights does, and leaves the other rows alone."""
+    taken = 0
+    for (N, K), M, group in ((SHAPES[1], 8, 32), (SHAPES[3], 16, 64), (SHAPES[3], 64, 128),
+                             (SHAPES[6], 40, 64), (SHAPES[5], 33, 64)):
+        if not _lib.load().mlxrocm_qmm_rows_supported(
+                M, N, K, 1, group, bits, 2 if dtype == torch.bfloat16 else 1):
+            continue
+        taken += 1
+        x, w = _inputs(M, N, K, dtype, M)
+        x[0, K // 3] = float("inf")
+        x[1, K - 1] = float("-inf")
+        x[2, 7] = float("nan")
+        x[3, 5], x[3, K - 3] = float("inf"), float("-inf")
+        x[4, K // 2] = torch.finfo(dtype).max  # (bfloat16: its products leave fp32)
+        q = mlx_amd.quantize(w, group, bits)
+        y = mlx_amd.quantized_matmul(x, *q, group_size=group, bits=bits)
+        wd = mlx_amd.dequantize(q[0], q[1].float(), q[2].float(), group, bits).to(dtype).double()
+        want = x.double() @ wd.T
+        _same_kind(y[:4], want[:4].to(dtype))
+        assert bool(y[4:].isfinite().all())
+        # against weights rounded to the type: that, the sums and the result
+        size = x[4:].double().abs() @ wd.abs().T
+        half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        assert bool(((y[4:].double() - want[4:]).abs() <= 2 * half * size).all())
+    assert taken >= 3
+
+
+def test_infinite_x_in_the_gated_form():
+    x, gate = _inputs(5, 18944, 3584, torch.bfloat16, 1)
+    _, up = _inputs(5, 18944, 3584, torch.bfloat16, 2)
+    x[1, 100], x[3, 3583] = float("inf"), float("-inf")
+    g, u = mlx_amd.quantize(gate, 128, 8), mlx_amd.quantize(up, 128, 8)
+    y = mlx_amd.quantized_swiglu(x, g, u, 128, 8)
+    a, b = (mlx_amd.quantized_matmul(x, *q, group_size=128, bits=8) for q in (g, u))
+    _same_kind(y, (a.float() * torch.sigmoid(a.float()).bfloat16()).bfloat16() * b)
+    assert bool(y[::2].isfinite().all()) and bool(a[1].isinf().any())
+
+
 @pytest.mark.parametrize("mode", ("mxfp4", "mxfp8", "nvfp4"))
 @pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
 def test_fp_modes(mode, dtype):

@@ -77,7 +77,8 @@ bool walk_fits(const QmmArgs& a, int gs, int bits, int dtype, bool transpose, bo
   const uint64_t limit = uint64_t{1} << 32; // operands are addressed by 32-bit byte offsets
   if (!transpose || dtype == MLXROCM_FLOAT32 || a.M < 1 || a.M > 64 || a.K % 32 != 0 || a.K < 128 ||
       a.group_tiles != nullptr || a.L > 65535 ||
-      static_cast<uint64_t>(a.N) * a.K / 8 * bits >= limit) {
+      static_cast<uint64_t>(a.N) * a.K / 8 * bits >= limit ||
+      static_cast<uint64_t>(a.M) * a.K * 2 >= limit) {
     return false;
   }
   const WalkPlan pl = walk_plan(a, gs, bits, fp);

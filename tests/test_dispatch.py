@@ -195,6 +195,18 @@ def test_fp_qmm_workspace_size_is_exact_and_plans_name_the_kernels():
         "fp_quantize_dequantize+fp_scale_image+fp_qmm_t_tile(nt=7)"
 
 
+def test_few_row_kernel_keeps_x_within_its_32_bit_offsets():
+    """The kernel of 2..64 rows reaches W and x through 32-bit byte offsets: a call
+    whose x takes 4 GiB (64 rows of 2^25) is not one of its own, one a step short is."""
+    lib = _lib.load()
+    for K, fits in (((1 << 25) - 128, 1), (1 << 25, 0), ((1 << 25) + 128, 0)):
+        for dtype in (F16, BF16):
+            assert lib.mlxrocm_qmm_rows_supported(64, 4, K, 1, 64, 4, dtype) == fits
+            for mode in FP_MODES.values():
+                assert lib.mlxrocm_fp_qmm_rows_supported(64, 4, K, 1, mode, dtype) == fits
+    assert lib.mlxrocm_qmm_rows_supported(32, 4, 1 << 25, 1, 64, 4, BF16)  # half of it
+
+
 def test_no_valid_shape_is_refused():
     """A seeded random walk over valid shapes -- rows of x from 1 to 300,000, N from
     1 to 70,001, ragged K with [K, N] weights, stacks of matrices, every width,

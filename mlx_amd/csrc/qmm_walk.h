@@ -569,7 +569,9 @@ void qmm_walk_kernel(WalkArgs wa) {
     srow += at;
     brow += at;
   }
-  const bool eights = FP == 0 && ((G | g0 | g_count) & 7) == 0;
+  // (the problem's own base counts: a stack's stride is the caller's)
+  const bool eights = FP == 0 && ((G | g0 | g_count) & 7) == 0 &&
+      ((reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.biases)) & 15) == 0;
   const auto put_group = [&](int g, uint32_t s, uint32_t b) { // 16 bits each
     const float sv = half_value<T>(s);
     stab[g * kRows + trow] = sv * walk_unit<T, BITS>();
@@ -592,18 +594,25 @@ void qmm_walk_kernel(WalkArgs wa) {
     b8 = *reinterpret_cast<const uint4*>(brow + g);
   }
   if constexpr (FP != 0) { // four scale bytes at a time (K is whole chunks), four loads at once
+    // (as dwords where they start at one: scales may be a view at any byte)
     const uint8_t* s_base = static_cast<const uint8_t*>(a.scales) +
         static_cast<int64_t>(blockIdx.z) * a.sb_batch_stride;
     constexpr int kBytes = 32 / GS; // per entry
     const uint32_t first =
         static_cast<uint32_t>(row_of(trow >> 4, trow & 15)) * (K / GS) + g0 * kBytes;
     const int bytes = g_count * kBytes;
+    const bool dwords = (reinterpret_cast<uintptr_t>(s_base) & 3) == 0;
     for (int g = trun * 4; g < bytes; g += 4 * 4 * kRuns) {
       uint32_t v[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int at = g + j * 4 * kRuns;
-        v[j] = *reinterpret_cast<const uint32_t*>(s_base + first + (at < bytes ? at : 0));
+        const uint8_t* four = s_base + first + (at < bytes ? at : 0);
+        if (dwords) { // uniform
+          v[j] = *reinterpret_cast<const uint32_t*>(four);
+        } else {
+          v[j] = four[0] | four[1] << 8 | four[2] << 16 | static_cast<uint32_t>(four[3]) << 24;
+        }
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {

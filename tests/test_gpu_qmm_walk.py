@@ -187,3 +187,49 @@ def test_gated_form(bits, group, N, K):
         want = ((a.float() * torch.sigmoid(a.float()).bfloat16()).bfloat16() * b).double()
         # same sums in another order, then the same four roundings: a few last places
         assert float((y - want).norm() / want.norm()) < 2.0 ** -7
+
+
+def _at_byte(t, offset):
+    """The same values in memory that starts `offset` bytes past an aligned address."""
+    flat = torch.empty(t.numel() * t.element_size() + offset, dtype=torch.uint8, device=t.device)
+    flat[offset:] = t.contiguous().view(torch.uint8).reshape(-1)
+    return flat[offset:].view(t.dtype).view(t.shape)
+
+
+@pytest.mark.parametrize("mode", ("mxfp4", "mxfp8", "nvfp4"))
+def test_scale_bytes_at_any_address(mode):
+    for M in (3, 16, 40):
+        x, w = _inputs(2 * M, 640, 4096, torch.bfloat16, M)
+        q = mlx_amd.quantize(w, mode=mode)
+        stack = mlx_amd.quantize(w.reshape(2, 320, 4096), mode=mode)
+        want = mlx_amd.quantized_matmul(x[:M], *q, mode=mode)
+        want2 = mlx_amd.quantized_matmul(x.reshape(2, M, 4096), *stack, mode=mode)
+        for offset in (1, 2, 4):
+            y = mlx_amd.quantized_matmul(x[:M], q[0], _at_byte(q[1], offset), mode=mode)
+            assert torch.equal(y, want)
+            y = mlx_amd.quantized_matmul(
+                x.reshape(2, M, 4096), stack[0], _at_byte(stack[1], offset), mode=mode)
+            assert torch.equal(y, want2)
+
+
+def test_a_stack_whose_scales_lie_at_odd_strides():
+    lib = _lib.load()
+    M, N, K, group, bits = 16, 320, 4096, 64, 8
+    x, w = _inputs(2 * M, 2 * N, K, torch.bfloat16, 7)
+    q = [mlx_amd.quantize(t, group, bits) for t in w.reshape(2, N, K)]
+    per = N * K // group
+    spread = [torch.zeros(2 * per + 8, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for which in range(2):
+        for i in range(2):
+            at = i * (per + 3)
+            spread[which][at:at + per] = q[i][1 + which].reshape(-1)
+    wq = torch.stack([t[0].view(torch.int32) for t in q])
+    out = torch.empty((2, M, N), dtype=torch.bfloat16, device="cuda")
+    need = lib.mlxrocm_qmm_rows_workspace_size(M, N, K, 2, group, bits, _lib.BFLOAT16)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.mlxrocm_qmm_rows(
+        x.data_ptr(), wq.data_ptr(), spread[0].data_ptr(), spread[1].data_ptr(), out.data_ptr(), M,
+        N, K, 2, M * K, N * K * bits // 32, per + 3, group, bits, _lib.BFLOAT16, ws.data_ptr(),
+        need, torch.cuda.current_stream().cuda_stream))
+    for i in range(2):
+        _check(x[i * M:(i + 1) * M], q[i], group, bits, "affine", out[i])

@@ -74,41 +74,55 @@ template <typename T>
 struct WalkMagic;
 template <>
 struct WalkMagic<bf16_t> {
-  static constexpr uint32_t kBits = 0x43004300u; // 128.0 twice: 4-bit codes fit below
-  static constexpr float kOffset = 128.0f;
+  static constexpr int kMantissa = 7; // bits: a code and an offset above it
   static constexpr uint32_t kOnes = 0x3F803F80u; // 1.0 twice
-  static constexpr int kCodeBits = 7; // of the mantissa: widest code that fits beside an offset
+  static constexpr uint32_t kBits4 = 0x43004300u; // 128.0 twice: 4-bit codes fit below
+  static constexpr int kShift4 = 0;
+  static constexpr float kOffset4 = 128.0f;
 };
 template <>
 struct WalkMagic<f16_t> {
-  static constexpr uint32_t kBits = 0x64006400u; // 1024.0 twice
-  static constexpr float kOffset = 1024.0f;
+  static constexpr int kMantissa = 10;
   static constexpr uint32_t kOnes = 0x3C003C00u;
-  static constexpr int kCodeBits = 10;
+  static constexpr uint32_t kBits4 = 0x54005400u; // 64.0 twice: 1 is bit 4
+  static constexpr int kShift4 = 4;
+  static constexpr float kOffset4 = 64.0f;
+  static constexpr uint32_t kBits8 = 0x64006400u; // 1024.0 twice: 1 is bit 0
 };
 
-// A widened code is (code + offset) / unit.  At the bottom of the mantissa (unit 1) the
-// packed dwords of 4 and 8 bits need the fewest instructions; everything else lies at
-// its top, for an offset of 2^bits: the fp32 sums lose what the offset is above the
-// codes, and 1024 + c loses more of a narrow c than a float16 result hides (x of one
-// sign, K = 4096, error of the result at the bottom / at the top: 2 bits, group 64
-// 5.9e-4 / 2.1e-4; 3 bits 3.6e-4 / 2.1e-4; 4 bits, group 128 3.4e-4 / 2.1e-4; 2.1e-4 is
-// what rounding the exact result loses).  Both take the same time.
-template <typename T, int BITS>
+// A widened code is (code + offset) / unit.  The offset costs the fp32 sums what it is
+// above the codes, so it is kept as small as the instructions allow.  2, 3, 5 and 6
+// bits, whose pairs are put together code by code: at the top of the mantissa, offset
+// 2^bits (1024 + c, in the same time, loses more than a float16 result hides: x of one
+// sign, K = 4096, error of the result 5.9e-4 / 3.6e-4 at 2 / 3 bits in groups of 64
+// against 2.1e-4, which is what rounding the exact result loses).  4 bits: where one of
+// the four shifts of a dword falls away (float16: 1024 + c loses 3.4e-4 in groups of
+// 128; at the top of the mantissa, one shift more, 16 rows of 14336 x 4096 take 13.9 us
+// instead of 13.3).  8 bits: a byte, against codes that reach 255.
+template <int BITS>
 constexpr bool walk_at_top() {
-  constexpr bool f16 = std::is_same<T, f16_t>::value;
-  return BITS <= WalkMagic<T>::kCodeBits && BITS != 8 && (f16 || BITS != 4);
+  return BITS < 8 && BITS != 4;
 }
-template <typename T, int BITS>
+template <int BITS>
 constexpr float walk_unit() {
-  return walk_at_top<T, BITS>() ? static_cast<float>(1 << BITS) : 1.0f;
+  return walk_at_top<BITS>() ? static_cast<float>(1 << BITS) : 1.0f;
 }
 template <typename T, int BITS>
 constexpr float walk_offset() {
-  if (walk_at_top<T, BITS>()) {
-    return static_cast<float>(1 << BITS);
+  if (BITS == 4) {
+    return WalkMagic<T>::kOffset4;
   }
-  return BITS <= WalkMagic<T>::kCodeBits ? WalkMagic<T>::kOffset : 0.0f;
+  if (BITS == 8) { // (bfloat16: no room, converted)
+    return WalkMagic<T>::kMantissa < 8 ? 0.0f : 1024.0f;
+  }
+  return static_cast<float>(1 << BITS);
+}
+template <typename T, int BITS>
+constexpr uint32_t walk_offset_bits() {
+  if constexpr (BITS == 8) {
+    return WalkMagic<f16_t>::kBits8;
+  }
+  return BITS == 4 ? WalkMagic<T>::kBits4 : WalkMagic<T>::kOnes;
 }
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -185,10 +199,10 @@ __device__ __forceinline__ void swap_quads(uint32_t& a, uint32_t& b) {
 // i * 32 / GS only; k_of() says which.
 template <typename T, int BITS, int GS>
 struct WalkCodes {
-  static constexpr bool kMagic = BITS <= WalkMagic<T>::kCodeBits;
-  static constexpr bool kTop = walk_at_top<T, BITS>();
-  static constexpr uint32_t kOffsetBits = kTop ? WalkMagic<T>::kOnes : WalkMagic<T>::kBits;
-  static constexpr int kShift = kTop ? WalkMagic<T>::kCodeBits - BITS : 0; // of a code
+  static constexpr bool kMagic = BITS <= WalkMagic<T>::kMantissa;
+  static constexpr uint32_t kOffsetBits = walk_offset_bits<T, BITS>();
+  static constexpr int kShift = // of a code
+      BITS == 4 ? WalkMagic<T>::kShift4 : (BITS == 8 ? 0 : WalkMagic<T>::kMantissa - BITS);
   static constexpr uint32_t kMask = // of a code in the low half (4 bits: in both)
       (BITS == 4 ? 0x000f000fu : (1u << BITS) - 1u) << kShift;
 
@@ -294,7 +308,7 @@ struct WalkCodes {
     if constexpr (BITS == 4) {
       // codes 0,4 1,5 2,6 3,7: x is staged in that order
       const auto at = [&](int bit) { // the codes at `bit` and 16 on, in their place
-        return bit > kShift ? d[i] >> (bit - kShift) : d[i] << (kShift - bit);
+        return bit >= kShift ? d[i] >> (bit - kShift) : d[i] << (kShift - bit);
       };
       o.x = (at(0) & mask) | magic;
       o.y = (at(4) & mask) | magic;
@@ -574,7 +588,7 @@ void qmm_walk_kernel(WalkArgs wa) {
       ((reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.biases)) & 15) == 0;
   const auto put_group = [&](int g, uint32_t s, uint32_t b) { // 16 bits each
     const float sv = half_value<T>(s);
-    stab[g * kRows + trow] = sv * walk_unit<T, BITS>();
+    stab[g * kRows + trow] = sv * walk_unit<BITS>();
     btab[g * kRows + trow] = fmaf(-kOff, sv, half_value<T>(b));
   };
   const auto put_eight = [&](int g, const uint4& s, const uint4& b) {

@@ -28,7 +28,7 @@ def _check(x, q, group, bits, mode, y):
     # (codes are multiplied with an offset that the biases take back, in fp32: that adds
     # offset / (2^bits - 1) times the size of the product at worst)
     f16 = x.dtype == torch.float16
-    offset = {8: 1024 if f16 else 0, 4: 16 if f16 else 128}.get(bits, 2 ** (bits or 0))
+    offset = {8: 1024 if f16 else 0, 4: 64 if f16 else 128}.get(bits, 2 ** (bits or 0))
     sums = 2e-6 * (1 if mode != "affine" else 1 + offset / (2 ** bits - 1) / 8)
     half = 2.0 ** -8 if x.dtype == torch.bfloat16 else 2.0 ** -11
     err = (y.double() - want).abs()

@@ -838,10 +838,12 @@ size_t round256(size_t n) {
 // Whether the scale bytes of w are rewritten as a step-major image first (a scale
 // dword per row and K-step is a cache line of its own in the caller's layout).  The
 // image of 14336 x 4096 takes 4 us and every 256 rows of x read it once; a call of 512
-// rows takes 100 us or more, one of 100 rows 32 with the caller's layout.
+// rows takes 100 us or more, one of 100 rows 32 with the caller's layout.  The caller's
+// layout is loaded to LDS by the dword: scales that start at no dword always go by the
+// image.
 constexpr int kQqImageMinM = 512;
-bool qq_ws_image(int M) {
-  return M >= kQqImageMinM;
+bool qq_ws_image(int M, const uint8_t* scales) {
+  return M >= kQqImageMinM || (reinterpret_cast<uintptr_t>(scales) & 3u) != 0;
 }
 
 } // namespace
@@ -919,7 +921,7 @@ extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, 
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     return round256(static_cast<size_t>(M) * K * bits / 8) +
         round256(static_cast<size_t>(M) * K / 32) +
-        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0) +
+        round256(static_cast<size_t>(N) * K / 32) +
         round256(qq_mfma_plane_bytes(M, N, K, mode));
   }
   return round256(static_cast<size_t>(M) * K * dtype_size(dtype)) +
@@ -973,15 +975,14 @@ extern "C" int mlxrocm_fp_qqmm(
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     void* codes = workspace;
     uint8_t* xs = static_cast<uint8_t*>(workspace) + round256(n_elems * bits / 8);
-    const bool image = qq_ws_image(M) && (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
+    const bool image = qq_ws_image(M, scales);
     uint8_t* ws = xs + round256(n_elems / 32);
     rc = fp_quantize_activations(
         x, codes, xs, M, K, scales, image ? ws : nullptr, N, mode, dtype, s);
     if (rc != MLXROCM_OK) {
       return rc;
     }
-    void* planes = xs + round256(n_elems / 32) +
-        (qq_ws_image(M) ? round256(static_cast<size_t>(N) * K / 32) : 0);
+    void* planes = ws + round256(static_cast<size_t>(N) * K / 32);
     return launch_qq_mfma(
         codes, xs, wq, image ? ws : scales, image, out, M, N, K, mode, dtype, planes, s);
   }

@@ -367,11 +367,12 @@ __global__ __launch_bounds__(kFpBlock) void fp_quantize_dequantize_kernel(
 // The operands of the block-scaled matrix instruction: the first q_blocks workgroups
 // quantize x [rows][32 row_groups]; the rest (if any) rewrite the scale bytes of w, as
 // dwords [w_rows][steps], to [steps][w_rows], 64 rows x 32 steps each through LDS.
-// One launch for both: the second would take as long to start as it runs (4 us).
+// One launch for both: the second would take as long to start as it runs (4 us).  The
+// bytes of w may start anywhere.
 template <typename T, int GS, int BITS>
 __global__ __launch_bounds__(kFpBlock) void fp_activations_kernel(
     const T* x, size_t n_units, uint8_t* xq, uint8_t* xs, uint32_t rows, uint32_t row_groups,
-    unsigned q_blocks, const uint32_t* ws, uint32_t* ws_image, int w_rows, int steps) {
+    unsigned q_blocks, const uint8_t* ws, uint32_t* ws_image, int w_rows, int steps) {
   __shared__ uint32_t tile[64][33];
   if (blockIdx.x < q_blocks) { // uniform
     quantize_dequantize_unit<T, GS, BITS, true>(
@@ -384,10 +385,14 @@ __global__ __launch_bounds__(kFpBlock) void fp_activations_kernel(
   const int r0 = static_cast<int>(t / across) * 64;
   const int s0 = static_cast<int>(t % across) * 32;
   const int sx = threadIdx.x & 31;
+  const bool dwords = (reinterpret_cast<uintptr_t>(ws) & 3) == 0; // uniform
 #pragma unroll
   for (int r = threadIdx.x >> 5; r < 64; r += kFpBlock / 32) {
     if (r0 + r < w_rows && s0 + sx < steps) {
-      tile[r][sx] = ws[static_cast<size_t>(r0 + r) * steps + s0 + sx];
+      const uint8_t* four = ws + (static_cast<size_t>(r0 + r) * steps + s0 + sx) * 4;
+      tile[r][sx] = dwords
+          ? *reinterpret_cast<const uint32_t*>(four)
+          : four[0] | four[1] << 8 | four[2] << 16 | static_cast<uint32_t>(four[3]) << 24;
     }
   }
   __syncthreads();
@@ -637,7 +642,7 @@ namespace mlxrocm {
 
 // x -> codes and scale bytes by the rules of fp_quantize_dequantize (what qqmm
 // applies to its first operand), in the MX modes.  x is [M][K], K % 128 == 0.  ws_image
-// not null: also the scale bytes ws of w, [N][K / 32] and 4-byte aligned, as the image
+// not null: also the scale bytes ws of w, [N][K / 32], as the image
 // [K / 128][N] of dwords.
 int fp_quantize_activations(
     const void* x, void* codes, uint8_t* scales, int M, int K, const uint8_t* ws, void* ws_image,
@@ -660,7 +665,7 @@ int fp_quantize_activations(
       fp_activations_kernel<T, 32, B><<<static_cast<unsigned>(blocks), kFpBlock, 0, s>>>(
           static_cast<const T*>(x), n_units, static_cast<uint8_t*>(codes), scales,
           static_cast<uint32_t>(M), static_cast<uint32_t>(K / 32), static_cast<unsigned>(q_blocks),
-          reinterpret_cast<const uint32_t*>(ws), static_cast<uint32_t*>(ws_image), N, steps);
+          ws, static_cast<uint32_t*>(ws_image), N, steps);
       MLXROCM_HIP_TRY(hipGetLastError());
       return static_cast<int>(MLXROCM_OK);
     };

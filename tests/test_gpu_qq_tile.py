@@ -45,3 +45,18 @@ def test_steps_tiles_and_scales(gpu, mode, dtype, M, N, K):
     sums = 2e-5 if mode == "mxfp8" and dtype != torch.float32 else 2e-6
     err = (y.double() - want).abs()
     assert bool((err <= half * want.abs() + sums * size).all()), float((err / size).max())
+
+
+@pytest.mark.parametrize("mode", ("mxfp8", "mxfp4"))
+@pytest.mark.parametrize("M", (8, 16, 100, 512))
+def test_scale_bytes_at_any_address(gpu, mode, M):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, 1152), generator=g, device="cuda").bfloat16()
+    wq, scales = mlx_amd.quantize(
+        torch.randn((300, 1152), generator=g, device="cuda").bfloat16(), mode=mode)
+    want = mlx_amd.qqmm(x, wq, scales, mode=mode)
+    for offset in (1, 2, 4):
+        flat = torch.empty(scales.numel() + offset, dtype=torch.uint8, device="cuda")
+        flat[offset:] = scales.reshape(-1)
+        moved = flat[offset:].view(scales.shape)
+        assert torch.equal(mlx_amd.qqmm(x, wq, moved, mode=mode), want)

@@ -613,8 +613,17 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
         )
         return out
     bb, _ = _dense_batches(biases, batch_shape)
-    if transpose and sb_image is None and lib.mlxrocm_qmm_rows_supported(
-            M, w_outer, K, L, group_size, bits, code):
+    if sb_image is not None:
+        want = lib.mlxrocm_qmm_sb_image_size(
+            w_outer, K, L if sb_stride else 1, group_size, code)
+        if (not transpose or sb_image.dtype != dtype or sb_image.device != x.device
+                or not sb_image.is_contiguous() or sb_image.numel() * sb_image.element_size() != want):
+            raise ValueError(
+                "[quantized_matmul] sb_image does not belong to these scales and biases "
+                "(quantized_matmul_sb_image with the same dtype, transpose=True)"
+            )
+    if transpose and lib.mlxrocm_qmm_rows_supported(M, w_outer, K, L, group_size, bits, code):
+        # the rows of a decode step of some sequences (an image is for prefill)
         ws_bytes = lib.mlxrocm_qmm_rows_workspace_size(M, w_outer, K, L, group_size, bits, code)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
         _lib.check(
@@ -630,15 +639,6 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
     )
     # a temporary of the call, like the ones eval_gpu hands to add_temporary
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-    if sb_image is not None:
-        want = lib.mlxrocm_qmm_sb_image_size(
-            w_outer, K, L if sb_stride else 1, group_size, code)
-        if (not transpose or sb_image.dtype != dtype or sb_image.device != x.device
-                or not sb_image.is_contiguous() or sb_image.numel() * sb_image.element_size() != want):
-            raise ValueError(
-                "[quantized_matmul] sb_image does not belong to these scales and biases "
-                "(quantized_matmul_sb_image with the same dtype, transpose=True)"
-            )
     _lib.check(
         lib.mlxrocm_qmm_prepacked(
             xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(),

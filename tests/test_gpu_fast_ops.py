@@ -81,6 +81,21 @@ def test_what_is_left_to_the_bodies(both):
     assert dx.shape == leaf.shape
 
 
+@pytest.mark.parametrize("rows", (1, 3, 16, 48, 600))
+def test_an_image_of_scales_and_biases(both, rows):
+    """Neither the host path nor an image decides which kernel multiplies."""
+    q = mlx_amd.quantize(_x(512, 4096), 64, 8)
+    image = mlx_amd.quantized_matmul_sb_image(q[1], q[2], 64)
+    x = _x(rows, 4096)
+    kw = dict(group_size=64, bits=8)
+    both(lambda: mlx_amd.quantized_matmul(x, *q, **kw, sb_image=image))
+    strided = torch.stack([x, x], dim=-1)[..., 0]
+    assert not strided.is_contiguous()
+    want = mlx_amd.quantized_matmul(x, *q, **kw)
+    assert torch.equal(mlx_amd.quantized_matmul(x, *q, **kw, sb_image=image), want)
+    assert torch.equal(mlx_amd.quantized_matmul(strided, *q, **kw, sb_image=image), want)
+
+
 def test_on_another_stream_and_thread():
     import threading
 

@@ -96,6 +96,36 @@ def test_switch_glu_calls_projections_that_are_more_than_their_buffers(stubs, na
         assert bool((y == 2).all())
 
 
+@pytest.mark.parametrize("dtype,width,pairs,ordered", (
+    (torch.float32, D, 1022, False), (torch.float32, D, 1024, True),
+    (torch.bfloat16, D, 4096, False), (torch.bfloat16, 96, 4094, False),
+    (torch.bfloat16, 96, 4096, True)))
+@pytest.mark.parametrize("threshold", (64, 5000))
+def test_switch_glu_orders_pairs_that_the_products_do_not_group(
+        stubs, monkeypatch, dtype, width, pairs, ordered, threshold):
+    seen = []
+
+    def gather_qmm(x, w, *args, rhs_indices=None, sorted_indices=False, **kw):
+        """Every result is its expert plus the sum of its row of x."""
+        seen.append((sorted_indices, bool((rhs_indices[1:] >= rhs_indices[:-1]).all())))
+        y = x.sum(-1, keepdim=True) + rhs_indices[..., None, None]
+        return y.expand(*y.shape[:-1], w.shape[-2])
+
+    monkeypatch.setattr(ops, "gather_qmm", gather_qmm)
+    block = nn.SwitchGLU(width, F, E, dtype=dtype, device="cpu", group_size=32,
+                         activation=lambda t: t, sort_threshold=threshold)
+    indices = torch.arange(pairs).reshape(-1, 2) * 7 % E
+    tokens = torch.arange(pairs // 2) % 5
+    x = torch.zeros(pairs // 2, width, dtype=dtype)
+    x[:, 0] = tokens
+    y = block(x, indices.int())
+    ordered = ordered and threshold == 64
+    assert [s for s, _ in seen] == [ordered] * 3 and (not ordered or all(o for _, o in seen))
+    want = F * (tokens[:, None] + indices).double() ** 2 + indices
+    assert y.shape == (pairs // 2, 2, width)
+    assert torch.equal(y.double(), want.to(dtype).double()[..., None].expand(y.shape))
+
+
 @pytest.mark.parametrize("rows", (1, 8, 9))
 @pytest.mark.parametrize("how", ("plain", "subclass", "wrapper", "hook", "other layer"))
 def test_swiglu_calls_projections_that_are_more_than_their_buffers(stubs, rows, how):

@@ -1,8 +1,7 @@
 // quantize.hip -- affine group-wise quantize / dequantize for gfx950.
 //
 // Streaming kernels, dequantize bound by HBM and quantize by its vector instructions.
-// A lane owns one "unit" of 8
-// consecutive elements: 8 codes are exactly BITS bytes of the packed stream for
+// A lane owns one "unit" of 8 consecutive elements: 8 codes are exactly BITS bytes of the packed stream for
 // every supported width, so a unit never shares a byte with its neighbour even
 // when 3/5/6-bit codes straddle uint32 words.  A quantization group is GS/8
 // adjacent lanes of one wavefront; its min/max is a butterfly over those lanes.
@@ -19,13 +18,13 @@ namespace {
 
 constexpr int kQuantBlock = 256;
 
-// The reference's arithmetic for one unit of a group, step by step, for every input.
-template <int BITS, int LPG>
-__device__ __forceinline__ void quantize_unit_exact(
-    const float (&v)[8], float& scale, float& bias, uint64_t& packed) {
+// Extremes of a unit's group as the reference finds them, for every input.
+template <int LPG>
+__device__ __forceinline__ void
+group_extremes_exact(const float (&v)[8], float& w_max, float& w_min) {
   // std::max / std::min semantics: keep the accumulator unless strictly beaten.
-  float w_max = v[0];
-  float w_min = v[0];
+  w_max = v[0];
+  w_min = v[0];
 #pragma unroll
   for (int i = 1; i < 8; ++i) {
     w_max = (w_max < v[i]) ? v[i] : w_max;
@@ -38,7 +37,12 @@ __device__ __forceinline__ void quantize_unit_exact(
     w_max = (w_max < o_max) ? o_max : w_max;
     w_min = (o_min < w_min) ? o_min : w_min;
   }
+}
 
+// The reference's arithmetic for one unit of a group, step by step, for every input.
+template <int BITS>
+__device__ __forceinline__ void quantize_unit_exact(
+    const float (&v)[8], float w_max, float w_min, float& scale, float& bias, uint64_t& packed) {
   constexpr float n_bins = static_cast<float>((1 << BITS) - 1);
   constexpr float eps = 1e-7f;
   const bool mask = fabsf(w_min) > fabsf(w_max);
@@ -85,11 +89,11 @@ __device__ __forceinline__ void quantize_unit_exact(
       packed |= static_cast<uint64_t>(static_cast<uint32_t>(q)) << (i * BITS);
     }
   }
-
 }
 
-// the value of lane ^ OFF (or one equal to it), of an operand that is the same within aligned runs of OFF lanes: data
-// parallel moves, no LDS (half_mirror and mirror reverse runs of 8 and 16)
+// the value of lane ^ OFF (or one equal to it), of an operand that is the same within
+// aligned runs of OFF lanes: data parallel moves, no LDS (half_mirror and mirror reverse
+// runs of 8 and 16)
 template <int OFF>
 __device__ __forceinline__ float dpp_xor(float x) {
   constexpr int ctrl = OFF == 1 ? 0xB1 : (OFF == 2 ? 0x4E : (OFF == 4 ? 0x141 : 0x140));
@@ -109,21 +113,15 @@ __device__ __forceinline__ float reciprocal(float d) {
   return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
 }
 
-// The same results in fewer instructions, which are what bounds the kernel
-// (14336 x 4096, 4-bit, bf16: 42 us, of which 32 were vector instructions at four
-// clocks each; now 34 us): minima and maxima three at a time, group exchanges
-// without LDS, divisions without range scaling, codes clamped and packed by one
-// instruction each.  `false`, and nothing decided, for a unit of a group with a NaN, a
-// range below 1e-4 (eps = 1e-7 acts on ranges below 1e-7 n_bins) or values past 1e30.
-template <int BITS, int LPG>
-__device__ __forceinline__ bool quantize_unit_fast(
-    const float (&v)[8], float& scale, float& bias, uint64_t& packed) {
-  constexpr float n_bins = static_cast<float>((1 << BITS) - 1);
-  bool plain = !__builtin_isunordered(v[0], v[1]) && !__builtin_isunordered(v[2], v[3]) &&
-      !__builtin_isunordered(v[4], v[5]) && !__builtin_isunordered(v[6], v[7]);
-  float w_max = fmaxf(
+// The same extremes in fewer instructions: three values at a time, group exchanges
+// without LDS.  `false` for a unit with a NaN, whose group's extremes are not the
+// reference's (neither may a zero's sign be, which no result depends on).
+template <int LPG>
+__device__ __forceinline__ bool
+group_extremes(const float (&v)[8], float& w_max, float& w_min) {
+  w_max = fmaxf(
       fmaxf(fmaxf(fmaxf(v[0], v[1]), v[2]), fmaxf(fmaxf(v[3], v[4]), v[5])), fmaxf(v[6], v[7]));
-  float w_min = fminf(
+  w_min = fminf(
       fminf(fminf(fminf(v[0], v[1]), v[2]), fminf(fminf(v[3], v[4]), v[5])), fminf(v[6], v[7]));
   w_max = fmaxf(w_max, dpp_xor<1>(w_max));
   w_min = fminf(w_min, dpp_xor<1>(w_min));
@@ -137,19 +135,41 @@ __device__ __forceinline__ bool quantize_unit_fast(
     w_max = fmaxf(w_max, dpp_xor<8>(w_max));
     w_min = fminf(w_min, dpp_xor<8>(w_min));
   }
+  return !__builtin_isunordered(v[0], v[1]) && !__builtin_isunordered(v[2], v[3]) &&
+      !__builtin_isunordered(v[4], v[5]) && !__builtin_isunordered(v[6], v[7]);
+}
+
+// The arithmetic of quantize_unit_exact() in fewer instructions, which are what bounds
+// the kernel (14336 x 4096, 4-bit, bf16: 42 us, of which 32 were vector instructions at
+// four clocks each; now 34 us): divisions without range scaling, codes clamped and packed
+// by one instruction each.  For extremes below 1e30; a range below 1e-4 needs SMALL, where
+// eps = 1e-7 may act (it does on ranges below 1e-7 n_bins) and the edge round to 0.
+// Quotients stay exact there: divisors are 5e-8 or more, and a numerator small enough to
+// lose its residuals gives a quotient that rounds to 0 either way.
+template <int BITS, bool SMALL>
+__device__ __forceinline__ void quantize_unit_short(
+    const float (&v)[8], float w_max, float w_min, float& scale, float& bias, uint64_t& packed) {
+  constexpr float n_bins = static_cast<float>((1 << BITS) - 1);
   const float range = w_max - w_min;
   const bool mask = fabsf(w_min) > fabsf(w_max);
   const float edge = mask ? w_min : w_max;
-  plain = plain && range > 1e-4f && fabsf(edge) < 1e30f;
   float s0 = quotient(range, n_bins, 1.0f / n_bins);
+  if constexpr (SMALL) {
+    s0 = fmaxf(s0, 1e-7f);
+  }
   s0 = mask ? s0 : -s0;
-  // |edge| >= range / 2, so this quotient is n_bins / 2 or more and never rounds to 0
+  // |edge| >= range / 2, so (but for eps) this quotient is n_bins / 2 or more and does
+  // not round to 0
   const float q0 = rintf(quotient(edge, s0, reciprocal(s0)));
   scale = quotient(edge, q0, reciprocal(q0));
   bias = edge;
+  if constexpr (SMALL) {
+    scale = q0 == 0.0f ? s0 : scale;
+    bias = q0 == 0.0f ? 0.0f : bias;
+  }
   const float r = reciprocal(scale);
   uint32_t even = 0, odd = 0, low = 0, high = 0;
-  packed = 0;
+  float lower = 0.0f, upper = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float c = __builtin_amdgcn_fmed3f(rintf(quotient(v[i] - bias, scale, r)), 0.0f, n_bins);
@@ -165,16 +185,19 @@ __device__ __forceinline__ bool quantize_unit_fast(
       } else {
         high = __builtin_amdgcn_cvt_pk_u8_f32(c, i - 4, high);
       }
-    } else {
-      packed |= static_cast<uint64_t>(static_cast<uint32_t>(c)) << (i * BITS);
+    } else { // four codes as one whole number below 2^24, exact in fp32
+      float& four = i < 4 ? lower : upper;
+      four = __builtin_fmaf(c, static_cast<float>(1 << (i % 4 * BITS)), i % 4 == 0 ? 0.0f : four);
     }
   }
   if constexpr (BITS == 4) {
     packed = even | odd << 4;
   } else if constexpr (BITS == 8) {
     packed = static_cast<uint64_t>(high) << 32 | low;
+  } else {
+    packed = static_cast<uint64_t>(static_cast<uint32_t>(upper)) << (4 * BITS) |
+        static_cast<uint32_t>(lower);
   }
-  return plain;
 }
 
 template <typename T, int BITS, int GS>
@@ -202,11 +225,24 @@ __global__ __launch_bounds__(kQuantBlock) void affine_quantize_kernel(
     }
   }
 
-  float scale, bias;
+  // One way for a wavefront, chosen before any division: groups of zeros or of tiny values
+  // (pruned or padded weights) take four instructions more than others; NaN and values past
+  // 1e30 the long way.  14336 x 4096, 4-bit g64, bf16, us a launch back to back: ordinary
+  // weights 28, one group of zeros per wavefront 29 (both ways in turn 40), a NaN in every
+  // wavefront 63.
+  float w_max, w_min, scale, bias;
   uint64_t packed = 0;
-  // (the lanes of a group take one path: the same group gives all of them one scale)
-  if (__any(!quantize_unit_fast<BITS, LPG>(v, scale, bias, packed))) {
-    quantize_unit_exact<BITS, LPG>(v, scale, bias, packed);
+  const bool ordered = group_extremes<LPG>(v, w_max, w_min);
+  const bool short_way = ordered && fmaxf(fabsf(w_max), fabsf(w_min)) < 1e30f;
+  if (__all(short_way && w_max - w_min > 1e-4f)) {
+    quantize_unit_short<BITS, false>(v, w_max, w_min, scale, bias, packed);
+  } else if (__all(short_way)) {
+    quantize_unit_short<BITS, true>(v, w_max, w_min, scale, bias, packed);
+  } else {
+    if (!__all(ordered)) {
+      group_extremes_exact<LPG>(v, w_max, w_min);
+    }
+    quantize_unit_exact<BITS>(v, w_max, w_min, scale, bias, packed);
   }
 
   if (active && (threadIdx.x % LPG) == 0) {

@@ -29,3 +29,28 @@ def test_ties_extremes_and_mixed_waves(oracle, gpu, dtype, bits, gs):
     spike[::gs] = 5.0
     rows.append(spike)
     _check_quantize(oracle, gpu, torch.stack(rows).to(dtype), gs, bits)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("bits", ALL_BITS)
+@pytest.mark.parametrize("gs", ALL_GROUPS)
+def test_small_groups(oracle, gpu, dtype, bits, gs):
+    """Ranges and edges about eps = 1e-7 and its multiples, far below it, constants, zeros of
+    both signs: the short way's form for them, bit for bit."""
+    g = torch.Generator().manual_seed(bits + gs)
+    n = 1 << 15
+    unit = torch.randn((n // gs, gs), generator=g)
+    power = torch.rand((n // gs, 1), generator=g)
+    near = torch.randint(1, 8, (n // gs, 1), generator=g) * 0.5e-7 * (1 + (power - 0.5) * 1e-3)
+    rows = [
+        unit * 10.0 ** (-12 * power),                                  # 1 .. 1e-12
+        unit * 10.0 ** (-45 + 8 * power),                              # about the end of fp32
+        unit.sign() * near,                                            # edges of some half eps
+        near + unit * 1e-9,
+        torch.where(unit > 0, near * (2 ** bits - 1), near * 0.0),     # ranges of some n_bins eps
+        near.expand_as(unit) * 1e7,                                    # constants
+        unit * 0.0,
+        torch.where(power < 0.3, unit * 0.0, unit),                    # some groups pruned
+    ]
+    w = torch.stack([r.reshape(-1) for r in rows]).to(dtype)
+    _check_quantize(oracle, gpu, w, gs, bits)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import mlx_amd
+from mlx_amd import _lib
 from tests.util import (
     ALL_BITS, ALL_GROUPS, DTYPES, activations, exact_affine_weights,
     exact_affine_weights_on, exact_product_error, exact_tolerance,
@@ -14,13 +15,34 @@ from tests.util import (
 pytestmark = pytest.mark.gpu
 
 
-def _check_qmm(oracle, gpu, x, w, gs, bits, transpose=True, rows=None, quantized=None):
+def _by_table(x, wq, s, b, transpose, gs, bits):
+    """mlxrocm_qmm, whose rule table the few-row kernels belong to: quantized_matmul
+    sends many of their shapes to mlxrocm_qmm_rows instead."""
+    lib = _lib.load()
+    *batch, M, K = x.shape
+    L = math.prod(batch)
+    code = {torch.float16: _lib.FLOAT16, torch.bfloat16: _lib.BFLOAT16}[x.dtype]
+    N = wq.shape[-2]
+    assert transpose and wq.shape[:-2] == x.shape[:-2]
+    out = torch.empty((*batch, M, N), dtype=x.dtype, device=x.device)
+    need = lib.mlxrocm_qmm_workspace_size(M, N, K, L, int(L > 1), gs, bits, code, 1)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.mlxrocm_qmm(
+        x.data_ptr(), wq.data_ptr(), s.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, L, M * K,
+        N * K * bits // 32 if L > 1 else 0, N * K // gs if L > 1 else 0, gs, bits, code, 1, ws.data_ptr(), need,
+        torch.cuda.current_stream().cuda_stream))
+    return out
+
+
+def _check_qmm(oracle, gpu, x, w, gs, bits, transpose=True, rows=None, quantized=None,
+               product=None):
     """x [M, K]; w dense weights (quantized on the CPU by the oracle) or a
     ready (wq, s, b) triple.  Every row of the result is compared with the fp64
     product of the exact affine weights (torch float64 on the GPU); `rows` is
-    the subset of x rows the scalar CPU oracle is run on (all rows if None)."""
+    the subset of x rows the scalar CPU oracle is run on (all rows if None);
+    `product` the call (quantized_matmul if None)."""
     wq, s, b = quantized if quantized is not None else oracle.quantize(w, gs, bits)
-    got = mlx_amd.quantized_matmul(
+    got = (product or mlx_amd.quantized_matmul)(
         x.to(gpu), wq.to(gpu), s.to(gpu), b.to(gpu), transpose, gs, bits
     )
     torch.cuda.synchronize()
@@ -233,7 +255,7 @@ def test_qmm_few_rows_kernels(oracle, gpu, dtype, bits):
                         (20, 8224, 384), (32, 8192, 128)):
             w = normal_weights((N, K), dtype, seed=bits + gs + M)
             x = activations((M, K), dtype, seed=M)
-            _check_qmm(oracle, gpu, x, w, gs, bits)
+            _check_qmm(oracle, gpu, x, w, gs, bits, product=_by_table)
 
 
 @pytest.mark.parametrize("dtype,gs", ((torch.bfloat16, 128), (torch.float16, 64)))
@@ -246,7 +268,8 @@ def test_qmm_few_rows_of_8_bit_over_many_bytes(oracle, gpu, dtype, gs):
     quantized = oracle.quantize(w, gs, 8)
     for M in (3, 8):
         x = activations((M, K), dtype, seed=M)
-        _check_qmm(oracle, gpu, x, None, gs, 8, rows=torch.tensor([0, M - 1]), quantized=quantized)
+        _check_qmm(oracle, gpu, x, None, gs, 8, rows=torch.tensor([0, M - 1]), quantized=quantized,
+                   product=_by_table)
 
 
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))

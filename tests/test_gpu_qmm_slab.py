@@ -1,17 +1,23 @@
 """GPU parity of the few-row kernel that streams packed 4-bit rows through LDS
 with x resident per K range (5..32 rows of a plain call, small expert groups of
 a gather): against the CPU oracle and the fp64 product of the exact weights."""
+import functools
+
 import pytest
 import torch
 
 import mlx_amd
 from mlx_amd import _lib
-from tests.test_gpu_qmm import _check_qmm
+from tests.test_gpu_qmm import _by_table, _check_qmm
 from tests.util import (
     activations, exact_affine_weights, exact_tolerance, matmul_tolerance, normal_weights,
 )
 
 pytestmark = pytest.mark.gpu
+
+# Through mlxrocm_qmm itself: quantized_matmul sends most of these shapes to the
+# kernel of mlxrocm_qmm_rows.
+_check_qmm = functools.partial(_check_qmm, product=_by_table)
 
 CODE = {torch.float16: 1, torch.bfloat16: 2}
 
@@ -32,6 +38,7 @@ def test_slab_rows_and_groups(oracle, gpu, dtype, gs, M):
     _check_qmm(oracle, gpu, x, w, gs, 4, rows=torch.tensor([0, M - 1]))
     if M >= 9 and (gs != 32 or M <= 16):  # (5..8 rows: only where the 4x4x4 kernel is not chosen)
         ws = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, gs, 4, CODE[dtype], 1)
+        assert "qmm_slab(" in _lib.qmm_plan(M, N, K, 1, False, gs, 4, CODE[dtype])[1]
         assert ws == _planes_bytes(M, N, K), "the shape did not take the slab kernel"
 
 
@@ -48,6 +55,7 @@ def test_slab_ragged_and_single_range(oracle, gpu, N, K):
         _check_qmm(oracle, gpu, x, w, 64, 4, rows=torch.tensor([M - 1]))
         ws = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, 2, 1)
         if M >= 9 or K >= 8192 or N >= 32000:  # (5..8 rows: a long K or many rows of W)
+            assert "qmm_slab(" in _lib.qmm_plan(M, N, K)[1]
             assert ws == _planes_bytes(M, N, K)
 
 
@@ -64,6 +72,7 @@ def test_slab_short_last_range(oracle, gpu, dtype, gs, N, K):
         x = activations((M, K), dtype, seed=M)
         _check_qmm(oracle, gpu, x, None, gs, 4, rows=torch.tensor([M - 1]), quantized=quantized)
         ws = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, gs, 4, CODE[dtype], 1)
+        assert "qmm_slab(" in _lib.qmm_plan(M, N, K, 1, False, gs, 4, CODE[dtype])[1]
         assert ws == _planes_bytes(M, N, K), "the shape did not take the slab kernel"
 
 
@@ -80,6 +89,7 @@ def test_slab_two_passes_for_33_to_64_rows(oracle, gpu, dtype, gs):
         _check_qmm(oracle, gpu, x, None, gs, 4, rows=torch.tensor([0, 31, 32, M - 1]),
                    quantized=quantized)
         ws = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, gs, 4, CODE[dtype], 1)
+        assert "[qmm_slab_twice]" in _lib.qmm_plan(M, N, K, 1, False, gs, 4, CODE[dtype])[1]
         assert ws == _planes_bytes(32, N, K), "the shape did not take the slab kernel twice"
     assert lib.mlxrocm_qmm_workspace_size(65, N, K, 1, 0, gs, 4, CODE[dtype], 1) != _planes_bytes(32, N, K)
     assert lib.mlxrocm_qmm_workspace_size(40, N, K, 1, 0, 32, 4, CODE[dtype], 1) != _planes_bytes(32, N, K)
@@ -116,7 +126,7 @@ def test_slab_batched_weights(oracle, gpu):
     w = normal_weights((L, N, K), dtype, std=0.05)
     wq, s, b = oracle.quantize(w, 64, 4)
     x = activations((L, M, K), dtype)
-    got = mlx_amd.quantized_matmul(x.to(gpu), wq.to(gpu), s.to(gpu), b.to(gpu), True, 64, 4).cpu()
+    got = _by_table(x.to(gpu), wq.to(gpu), s.to(gpu), b.to(gpu), True, 64, 4).cpu()
     ref = oracle.qmm_batched(x, wq, s, b, True, 64, 4)
     w_hat = exact_affine_weights(wq, s, b, 64, 4)
     exact = torch.einsum("lmk,lnk->lmn", x.double(), w_hat)
@@ -207,6 +217,7 @@ def test_rows8_all_of_k_resident(oracle, gpu, dtype, gs, K):
         x = activations((M, K), dtype, seed=M)
         _check_qmm(oracle, gpu, x, None, gs, 4, rows=torch.tensor([M - 1]), quantized=quantized)
         ws = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, gs, 4, CODE[dtype], 1)
+        assert "qmm_rows8(" in _lib.qmm_plan(M, N, K, 1, False, gs, 4, CODE[dtype])[1]
         assert ws == 0, "the shape did not take the kernel without K ranges"
 
 
@@ -216,7 +227,7 @@ def test_rows8_batched(oracle, gpu):
     w = normal_weights((L, N, K), dtype, std=0.05)
     wq, s, b = oracle.quantize(w, 64, 4)
     x = activations((L, M, K), dtype)
-    got = mlx_amd.quantized_matmul(x.to(gpu), wq.to(gpu), s.to(gpu), b.to(gpu), True, 64, 4).cpu()
+    got = _by_table(x.to(gpu), wq.to(gpu), s.to(gpu), b.to(gpu), True, 64, 4).cpu()
     w_hat = exact_affine_weights(wq, s, b, 64, 4)
     exact = torch.einsum("lmk,lnk->lmn", x.double(), w_hat)
     assert float((got.double() - exact).abs().max()) <= exact_tolerance(dtype, K, x, w_hat, exact)

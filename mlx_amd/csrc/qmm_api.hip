@@ -572,8 +572,10 @@ int two_passes(const Call& c, const QmmArgs& head, const QmmArgs& tail) {
 }
 
 // 3..64 rows of x (mlxrocm_qmm_rows), whatever regime of the table below they
-// belong to: where the kernel of qmm_walk.h (rows of W dealt out evenly to the compute units, the whole of K
-// each, x walking through LDS) is ahead of that regime's own.  Graph replays over
+// belong to: where the kernel of qmm_walk.h (rows of W dealt out evenly to the compute
+// units, mostly the whole of K each, x walking through LDS) is ahead of that regime's
+// own.  The table does not know it: a caller asks mlxrocm_qmm_rows_supported first, as
+// quantized_matmul does, and mlxrocm_qmm without asking runs the table.  Graph replays over
 // 15 shapes from 1024 x 1024 to 128256 x 4096, us against the regime's kernel: 4-bit
 // g64 14336 x 4096 16 rows 13.8 against 16.6, 48 rows 21.5 against 33.7, 4096 x 4096
 // 32 rows 9.8 against 14.7, 4096 x 14336 8 rows 13.9 against 15.6; 8-bit 14336 x 4096
@@ -744,7 +746,8 @@ const Rule kRules[] = {
        return slab_launch(c, tail, region);
      },
      "4-bit, 33..64 rows: the slab kernel twice (32 rows, the rest); the tile GEMM costs the "
-     "same whatever M. Graph replays, 64 rows: 14336x4096 34.4 against 37.0, 4096x14336 35.1 "
+     "same whatever M. Only for callers that do not ask mlxrocm_qmm_rows_supported (which "
+     "takes all of these, faster). Graph replays, 64 rows: 14336x4096 34.4 against 37.0, 4096x14336 35.1 "
      "against 46.5, 28672x4096 49.1 against 59.6, 128256x4096 180 against 270; from 65 rows "
      "on the tile GEMM is ahead"},
     {"qmv_wide_twice",

@@ -9,15 +9,22 @@
 // instructions.  What it takes to come near that with x of up to 64 rows:
 //   * every compute unit owns an equal number of rows of W (R = 4..64, chosen by
 //     the host as N / units, so that the last round of workgroups is full) and
-//     the whole of K: y is finished where it is computed, without fp32 planes;
-//   * W goes from memory to registers, four stages ahead of its use.  A lane
+//     the whole of K: y is finished where it is computed.  Only where 17 rows of x or
+//     more meet few rows of W per unit, or the tables of the whole of K do not fit LDS,
+//     is K cut into ranges with fp32 planes (walk_plan);
+//   * W goes from memory to registers, asked for four stages ahead of its use (two
+//     where registers are short: kAhead).  Loads arrive in order, so the wait for x
+//     (below) is one for the W asked for before it, too: across it only the newest
+//     stage of W is in flight where x has one set of registers (48 and 64 rows; 16 and
+//     32 rows with one tile of W), two where it has two.  A lane
 //     (r = lane % 16, q = lane / 16) holds 32 consecutive codes of row r, the
 //     quads side by side: 16 rows x 128 codes per wavefront and stage.  The matrix
 //     instruction sums over the four quads, and a sum may not leave a quantization
 //     group, so for groups of 32 or 64 the quads first exchange registers
 //     (v_permlane32_swap / v_permlane16_swap, one instruction per two dwords);
 //   * x walks through LDS in stages of KW x 128 codes, double-buffered, one
-//     barrier per stage, fetched two stages ahead through registers.  KW wavefronts
+//     barrier per stage, fetched through registers and asked for XD stages (one or
+//     two) before it is stored for the next.  KW wavefronts
 //     (times NW that share them) split the 128-code chunks of a stage, and add
 //     their sums up through LDS at the end;
 //   * codes are multiplied as they are (widened exactly into the 16-bit type, with
@@ -656,7 +663,7 @@ void qmm_walk_kernel(WalkArgs wa) {
   fetch_x(s0, xr[0]);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int u = 0; u < kAhead; ++u) { // in the loop's order: stage j asks for W (j + 4), x (j + 1 + XD)
+  for (int u = 0; u < kAhead; ++u) { // as in the loop: stage j asks for W (j + kAhead), x (j + 1 + XD)
     fetch_w(s0 + u, w[u]);
     if (u == 0) {
       __builtin_amdgcn_sched_barrier(0);
@@ -858,7 +865,7 @@ void qmm_walk_kernel(WalkArgs wa) {
       if (FP == 0 && (u + 1) * NG % 4 == 0) {
         add_biases(s + 1 - 4 / NG);
       }
-      // x of the next stage, late: it has had two stages to arrive
+      // x of the next stage, late: it has had XD stages to arrive
       put_x(s + 1, xr[(u + 1) % XD]);
       __builtin_amdgcn_sched_barrier(0);
       fetch_x(s + 1 + XD, xr[(u + 1) % XD]);

@@ -18,10 +18,9 @@
 // with all eight in step the two phases added up, and the matrix pipe was busy for
 // 35 % of the time.  Scale dwords come from step-major images, [K / 128][rows]: in the
 // caller's layout each is a cache line of its own, as many requests as the codes.
-// x [2048, 4096] x W [14336, 4096], bf16, quantizing x included: mxfp8 172 -> 143 us,
-// mxfp4 102 -> 95; 512 rows, 14336 -> 4096, mxfp8 129 -> 105.
-// 16-byte pieces of a row are
-// XOR-swizzled so that fragment reads hit every bank once.  Wavefront (wm, wn)
+// x [2048, 4096] x W [14336, 4096], bf16, quantizing x included: mxfp8 172 -> 146 us
+// (140..155 over the boxes), mxfp4 102 -> 95; 512 rows, 14336 -> 4096, mxfp8 129 -> 105.
+// 16-byte pieces of a row are XOR-swizzled so that fragment reads hit every bank once.  Wavefront (wm, wn)
 // owns a 64 x 64 block: W fragments are the instruction's A operand, x
 // fragments its B operand, so a lane holds four consecutive n of one row m of y.
 #include <type_traits>

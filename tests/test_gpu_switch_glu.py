@@ -59,3 +59,16 @@ def test_batched_tokens_and_what_is_left_to_the_layers():
     lib = _lib.load()
     assert lib.mlxrocm_switch_glu_workspace_size(8, 2, 256, 512, 4, 64, 4, 0) == 0  # float32
     assert lib.mlxrocm_switch_glu_workspace_size(8, 2, 250, 512, 4, 64, 4, 2) == 0
+
+
+@pytest.mark.parametrize("D,dtype,tokens", [(256, torch.float32, 512), (96, torch.bfloat16, 2048)])
+def test_pairs_ordered_by_expert_give_the_same_rows(D, dtype, tokens):
+    block = _block(D, 192, 8, 32, 4, dtype)
+    block.activation = torch.nn.functional.gelu  # (not one call)
+    x = torch.randn((tokens, D), device="cuda").to(dtype)
+    idx = torch.randint(0, 8, (tokens, 2), device="cuda").to(torch.int32)
+    assert block._sorts(x, idx)
+    y = block(x, idx)
+    block.sort_threshold = 1 << 20
+    assert not block._sorts(x, idx)
+    assert torch.equal(y, block(x, idx))

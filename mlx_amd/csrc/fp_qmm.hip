@@ -595,12 +595,12 @@ size_t fp_image_bytes(int N, int K, int batches) {
 
 // ranges of K for a launch whose tiles do not fill the compute units
 int fp_k_splits(int M, int N, int K, int L) {
-  return (static_cast<int64_t>(M) * N) % 4 == 0 ? qmm_mfma_k_splits(M, N, K, L) : 1;
+  return qmm_mfma_k_splits(M, N, K, L);
 }
 
 size_t fp_tile_workspace(int M, int N, int K, int L, int batches) {
   const int splits = fp_k_splits(M, N, K, L);
-  const size_t planes = splits > 1 ? static_cast<size_t>(M) * N * splits * sizeof(float) : 0;
+  const size_t planes = splits > 1 ? k_split_plane(M, N) * splits * sizeof(float) : 0;
   return fp_image_bytes(N, K, batches) + planes;
 }
 
@@ -780,7 +780,13 @@ int fp_qmm_entry(
   }
   if (fp_tile_applies(M, N, K, L, mode, dtype, transpose != 0)) {
     const int batches = scales_batch_stride != 0 ? L : 1;
-    const size_t need = fp_tile_workspace(M, N, K, L, batches);
+    size_t need = fp_tile_workspace(M, N, K, L, batches);
+    int splits = fp_k_splits(M, N, K, L);
+    if (N % 4 != 0 && workspace_bytes < need) {
+      // (padded planes: the plan without them is there for a caller with the image alone)
+      splits = 1;
+      need = fp_image_bytes(N, K, batches);
+    }
     if (workspace == nullptr || workspace_bytes < need ||
         (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) {
       return fail(
@@ -799,7 +805,6 @@ int fp_qmm_entry(
     a.sb_transposed = 2;
     // elements of T between the images of two batch entries
     a.sb_batch_stride = batches > 1 ? static_cast<int64_t>(N) * (K / 32) * 2 : 0;
-    const int splits = fp_k_splits(M, N, K, L);
     if (splits <= 1) {
       return launch_qmm_mfma_fp(a, mode, dtype, 1, s);
     }
@@ -809,7 +814,7 @@ int fp_qmm_entry(
     if (rc != MLXROCM_OK) {
       return rc;
     }
-    return reduce_k_splits(partial, out, static_cast<size_t>(M) * N, splits, dtype, s);
+    return reduce_k_splits(partial, out, M, N, splits, dtype, s);
   }
   return fp_launch(a, mode, dtype, transpose != 0, s);
 }

@@ -150,6 +150,13 @@ struct Scratch {
   // Optional: the caller's transposed image of scales and biases
   // (mlxrocm_qmm_sb_image); the prefill path then skips its pre-pass.
   const void* sb_image = nullptr;
+  // No plan may want more than this (the entry point with built-in scratch).
+  size_t most = SIZE_MAX;
+  // Is there room for `bytes`?  For plans that are an alternative to one with less
+  // scratch: workspace_size counts them, a caller with less runs the other one.
+  bool affords(size_t wanted) const {
+    return wanted <= most && (dry || (base != nullptr && bytes >= wanted));
+  }
 };
 
 constexpr size_t kScratchAlign = 256;
@@ -186,6 +193,17 @@ constexpr int kTransposeSbMinM = 512;
 // block runs on the bf16 matrix path with fp32 scales, biases and output.
 constexpr size_t kSplitScratchBytes = size_t(256) << 20;
 
+// fp32 planes of a K split.
+size_t plane_bytes(const QmmArgs& a, int k_splits) {
+  return k_split_plane(a.M, a.N) * k_splits * sizeof(float);
+}
+
+// Shapes whose planes are padded.  They are split like all others, but only where
+// scratch allows: the plan without planes is there for a caller that has none.
+bool ragged(const QmmArgs& a) {
+  return a.N % 4 != 0;
+}
+
 int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t s) {
   const size_t row_bytes = split_x_bytes(1, a.K);
   int rows_per_block = static_cast<int>(kSplitScratchBytes / row_bytes / 256 * 256);
@@ -201,18 +219,21 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
   }
   // few tiles: also cut K (one row block, one batch entry only)
   int k_splits = 1;
-  if (rows_per_block == a.M && a.L == 1 && (static_cast<int64_t>(a.M) * a.N) % 4 == 0) {
+  if (rows_per_block == a.M && a.L == 1) {
     k_splits = qmm_mfma_k_splits(a.M, a.N, a.K, 1, kSplitFp32Width);
   }
   const size_t x_bytes = (split_x_bytes(rows_per_block, a.K) + 255) / 256 * 256;
-  const size_t plane = static_cast<size_t>(a.M) * a.N;
-  const size_t partial_raw = k_splits > 1 ? plane * k_splits * sizeof(float) : 0;
-  const size_t partial_bytes = (partial_raw + 255) / 256 * 256;
   // scales / biases transposed to [K / group][N], as for the 16-bit prefill
   const int G = a.K / gs;
   const int sb_batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool sb_t = a.M >= kTransposeSbMinM;
   const size_t sb_bytes = sb_t ? qmm_n_sb_bytes(a.N, G, sb_batches, MLXROCM_FLOAT32) : 0;
+  size_t partial_bytes =
+      k_splits > 1 ? (plane_bytes(a, k_splits) + 255) / 256 * 256 : 0;
+  if (ragged(a) && !sc.affords(x_bytes + partial_bytes + sb_bytes)) {
+    k_splits = 1;
+    partial_bytes = 0;
+  }
   void* region = nullptr;
   int rc = claim(sc, x_bytes + partial_bytes + sb_bytes, &region);
   if (rc != MLXROCM_OK || sc.dry) {
@@ -260,7 +281,7 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
         return rc;
       }
       if (k_splits > 1) {
-        rc = reduce_k_splits(partial, out, plane, k_splits, MLXROCM_FLOAT32, s);
+        rc = reduce_k_splits(partial, out, a.M, a.N, k_splits, MLXROCM_FLOAT32, s);
         if (rc != MLXROCM_OK) {
           return rc;
         }
@@ -273,9 +294,8 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
 // 16-bit prefill whose tiles would leave most compute units idle: K is cut into
 // ranges, the fp32 partial tiles go to the workspace and are added up.
 int run_k_split(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scratch& sc, hipStream_t s) {
-  const size_t plane = static_cast<size_t>(a.M) * a.N;
   void* region = nullptr;
-  int rc = claim(sc, plane * k_splits * sizeof(float), &region);
+  int rc = claim(sc, plane_bytes(a, k_splits), &region);
   if (rc != MLXROCM_OK || sc.dry) {
     return rc;
   }
@@ -285,7 +305,7 @@ int run_k_split(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scr
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  return reduce_k_splits(region, a.out, plane, k_splits, dtype, s);
+  return reduce_k_splits(region, a.out, a.M, a.N, k_splits, dtype, s);
 }
 
 // Prefill (transpose=true, 16-bit types) from 512 rows of x on: the tile kernel
@@ -301,8 +321,7 @@ int run_qmm_t_transposed_sb(
   const bool prepacked = sc.sb_image != nullptr;
   const size_t sb_bytes =
       prepacked ? 0 : (qmm_n_sb_bytes(a.N, G, batches, dtype) + 255) / 256 * 256;
-  const size_t plane = static_cast<size_t>(a.M) * a.N;
-  const size_t partial_bytes = k_splits > 1 ? plane * k_splits * sizeof(float) : 0;
+  const size_t partial_bytes = k_splits > 1 ? plane_bytes(a, k_splits) : 0;
   void* region = nullptr;
   int rc = MLXROCM_OK;
   if (sb_bytes + partial_bytes != 0) {
@@ -336,7 +355,7 @@ int run_qmm_t_transposed_sb(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  return reduce_k_splits(partial, a.out, plane, k_splits, dtype, s);
+  return reduce_k_splits(partial, a.out, a.M, a.N, k_splits, dtype, s);
 }
 
 // transpose=false on the matrix cores.  The column loader wants the four
@@ -370,8 +389,7 @@ int run_qmm_n(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStr
   const TilePlan pl = qmm_n_plan(a.M, a.N, a.K, a.L);
   const int k_splits = pl.splits;
   const size_t sb_bytes = (qmm_n_sb_bytes(a.K, G, batches, dtype) + 255) / 256 * 256;
-  const size_t plane = static_cast<size_t>(a.M) * a.N;
-  const size_t partial_bytes = k_splits > 1 ? plane * k_splits * sizeof(float) : 0;
+  const size_t partial_bytes = k_splits > 1 ? plane_bytes(a, k_splits) : 0;
   void* region = nullptr;
   int rc = claim(sc, sb_bytes + partial_bytes, &region);
   if (rc != MLXROCM_OK || sc.dry) {
@@ -396,7 +414,7 @@ int run_qmm_n(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStr
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  return reduce_k_splits(partial, a.out, plane, k_splits, dtype, s);
+  return reduce_k_splits(partial, a.out, a.M, a.N, k_splits, dtype, s);
 }
 
 // Where the slab kernel is worth its launch: its units (K ranges x 256-row
@@ -552,10 +570,16 @@ Family family_of(const Call& c) {
 }
 
 int tile_k_splits(const Call& c) {
-  if (c.a.lhs_indices == nullptr && (static_cast<int64_t>(c.a.M) * c.a.N) % 4 == 0) {
-    return qmm_mfma_k_splits(c.a.M, c.a.N, c.a.K, c.a.L);
+  if (c.a.lhs_indices != nullptr) {
+    return 1;
   }
-  return 1;
+  const int splits = qmm_mfma_k_splits(c.a.M, c.a.N, c.a.K, c.a.L);
+  if (ragged(c.a) && splits > 1) {
+    const bool image = c.a.M >= kTransposeSbMinM && c.sc.sb_image == nullptr;
+    const size_t sb = image ? (qmm_n_sb_bytes(c.a.N, c.a.K / c.gs, 1, c.dtype) + 255) / 256 * 256 : 0;
+    return c.sc.affords(sb + plane_bytes(c.a, splits)) ? splits : 1;
+  }
+  return splits;
 }
 
 bool tile_t(const Call& c) {
@@ -848,7 +872,7 @@ const Rule kRules[] = {
      },
      "few tiles: K cut into up to 16 ranges of at least 8 steps, fp32 planes + reduction. "
      "M=512, N=4096: 75 -> 43; K=14336: 249 -> 92; 3584x18944, 128 rows: 45.6 (16 ranges) "
-     "against 57.5 (8)"},
+     "against 57.5 (8); odd N (padded planes) 775x4096, 255 rows: 79 -> 28"},
     {"qmm_t_tile",
      [](const Call& c) { return tile_t(c); },
      [](const Call& c) {
@@ -1144,6 +1168,36 @@ int qmm_entry(
 
 } // namespace
 
+namespace {
+
+// Scratch of a call whose plan wants no more than `most`; 0 for a call that is refused.
+size_t workspace_need(
+    int M,
+    int N,
+    int K,
+    int L,
+    int batched_weights,
+    int group_size,
+    int bits,
+    int dtype,
+    int transpose,
+    size_t most) {
+  Scratch sc;
+  sc.dry = true;
+  sc.most = most;
+  // the strides only say "one weight for every batch entry" or "one each"
+  const int64_t w_stride = batched_weights ? 4096 : 0;
+  const int64_t x_stride = static_cast<int64_t>(M) * K;
+  if (qmm_entry(
+          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
+          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
+    return 0;
+  }
+  return sc.need;
+}
+
+} // namespace
+
 extern "C" size_t mlxrocm_qmm_workspace_size(
     int M,
     int N,
@@ -1154,17 +1208,8 @@ extern "C" size_t mlxrocm_qmm_workspace_size(
     int bits,
     int dtype,
     int transpose) {
-  Scratch sc;
-  sc.dry = true;
-  // the strides only say "one weight for every batch entry" or "one each"
-  const int64_t w_stride = batched_weights ? 4096 : 0;
-  const int64_t x_stride = static_cast<int64_t>(M) * K;
-  if (qmm_entry(
-          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
-          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
-    return 0;
-  }
-  return sc.need;
+  return workspace_need(
+      M, N, K, L, batched_weights, group_size, bits, dtype, transpose, SIZE_MAX);
 }
 
 extern "C" int mlxrocm_qmm(
@@ -1426,8 +1471,9 @@ extern "C" int mlxrocm_qmm_static(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  const size_t need = mlxrocm_qmm_workspace_size(
-      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose);
+  const size_t need = workspace_need(
+      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose,
+      kStaticScratchBytes);
   if (need > kStaticScratchBytes) {
     return fail(
         MLXROCM_UNSUPPORTED,
@@ -1442,6 +1488,7 @@ extern "C" int mlxrocm_qmm_static(
   Scratch sc;
   sc.base = static_cast<char*>(region);
   sc.bytes = kStaticScratchBytes;
+  sc.most = kStaticScratchBytes;
   return qmm_entry(
       x, wq, scales, biases, out, M, N, K, L, x_batch_stride, w_batch_stride,
       sb_batch_stride, group_size, bits, dtype, transpose, sc,

@@ -224,6 +224,13 @@ int launch_qmm_mfma_split(const QmmArgs& a, int gs, int bits, hipStream_t s, int
 // Few tiles: K is cut into qmm_mfma_k_splits() ranges whose fp32 partial tiles
 // (k_splits planes of M x N behind a.out) reduce_k_splits() adds up.
 int qmm_mfma_k_splits(int M, int N, int K, int L, int nt = 7);
+// Elements of a row of such a plane and of a plane: rows start at 16 bytes.
+__host__ __device__ inline int k_split_row(int N) {
+  return (N + 3) / 4 * 4;
+}
+__host__ __device__ inline size_t k_split_plane(int M, int N) {
+  return static_cast<size_t>(M) * k_split_row(N);
+}
 constexpr int kSplitFp32Width = 6; // of launch_qmm_mfma_split's tiles, times 32 columns
 // transpose=false (w [K, N*bits/32]), 4/8-bit, 16-bit types, K % 64 == 0; with
 // k_splits > 1 `a.out` points at k_splits fp32 planes as for the k-split launch.
@@ -284,7 +291,8 @@ bool qmv_quad_supported(const QmmArgs& a, int gs, int bits, int dtype);
 int launch_qmv_quad(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 long qmv_quad_workgroups_two_sets(const QmmArgs& a, int bits);
 int launch_qmm_mfma_ksplit(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, hipStream_t s);
-int reduce_k_splits(const void* partial, void* out, size_t n, int k_splits, int dtype, hipStream_t s);
+int reduce_k_splits(
+    const void* partial, void* out, int M, int N, int k_splits, int dtype, hipStream_t s);
 // expert-routed gated MLP (qmm_mfma_experts.hip): pair images, launch_gather_group's tables
 int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 int launch_qmm_mfma_experts(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);

@@ -193,8 +193,12 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
     p.scales = static_cast<const TS*>(a.scales) + wb * a.sb_batch_stride;
     p.biases = static_cast<const TS*>(a.biases) + wb * a.sb_batch_stride;
     const int64_t plane = k_splits > 1 ? blockIdx.z : l;
-    p.out = static_cast<TO*>(a.out) + plane * a.M * static_cast<int64_t>(a.N);
+    p.out = static_cast<TO*>(a.out) +
+        (k_splits > 1 ? plane * static_cast<int64_t>(k_split_plane(a.M, a.N))
+                      : plane * a.M * static_cast<int64_t>(a.N));
   }
+  // elements between two rows of y, or of a plane of partial sums
+  const int ldy = k_splits > 1 ? k_split_row(a.N) : a.N;
   // x as the kernel sees it: three 64-wide blocks per block of K when split
   const int Kx = kSplit ? 3 * K : K;
 
@@ -718,7 +722,7 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
     constexpr int kRowsPerIter = kThreads / kLanesPerRow;
     const int c = tid % kLanesPerRow;
     const int r0 = tid / kLanesPerRow;
-    const bool vec_ok = (N % kPiece) == 0; // rows of y stay 16-byte aligned
+    const bool vec_ok = (ldy % kPiece) == 0; // rows of y stay 16-byte aligned
     if (c < kChunks) {
 #pragma unroll 4
       for (int r = r0; r < kPassRows; r += kRowsPerIter) {
@@ -745,7 +749,7 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
         }
         const size_t orow =
             GROUPED ? static_cast<size_t>(a.group_perm[row0 + mr]) : static_cast<size_t>(m);
-        TO* dst = p.out + orow * N + n;
+        TO* dst = p.out + orow * ldy + n;
         if (vec_ok && n + kPiece <= N) {
           *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
         } else {

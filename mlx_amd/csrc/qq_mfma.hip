@@ -82,7 +82,7 @@ struct QqArgs {
   void* out;             // [M][N]
   int M, N, K;
   uint32_t ws_row, ws_step; // bytes from a row of W, from a step, to the next
-  // K ranges (blockIdx.z): range z writes plane z of `out`, [splits][M][N]
+  // K ranges (blockIdx.z): range z writes plane z of `out` (k_split_plane())
   int splits;
 };
 
@@ -368,10 +368,11 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     k_loop(read_step, settle, multiply);
     // D[n][m] 32 x 32: register i of lane (col, half) holds n = 8 (i / 4) + 4 half
     // + i % 4, m = col
-    TO* out = static_cast<TO*>(a.out) + static_cast<size_t>(blockIdx.z) * M * N;
+    const int ldy = a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
+    TO* out = static_cast<TO*>(a.out) + blockIdx.z * k_split_plane(M, N);
     const int col = lane & 31;
     const int half = lane >> 5;
-    const bool vec_ok = (N % 4) == 0;
+    const bool vec_ok = (ldy % 4) == 0;
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       const int m = m0 + wm * 16 * MI + 32 * j + col;
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
           }
           const float v0 = acc[i][j][4 * g4 + 0], v1 = acc[i][j][4 * g4 + 1];
           const float v2 = acc[i][j][4 * g4 + 2], v3 = acc[i][j][4 * g4 + 3];
-          TO* dst = out + static_cast<size_t>(m) * N + n;
+          TO* dst = out + static_cast<size_t>(m) * ldy + n;
           if (vec_ok && n + 4 <= N) {
             if constexpr (sizeof(TO) == 4) {
               *reinterpret_cast<float4*>(dst) = make_float4(v0, v1, v2, v3);
@@ -522,10 +523,11 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #undef QQ_DMA4
 
   // D[n][m]: register r of lane (col, quad) holds n = 4 quad + r, m = col
-  TO* out = static_cast<TO*>(a.out) + static_cast<size_t>(blockIdx.z) * M * N;
+  const int ldy = a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
+  TO* out = static_cast<TO*>(a.out) + blockIdx.z * k_split_plane(M, N);
   const int col = lane & 15;
   const int quad = lane >> 4;
-  const bool vec_ok = (N % 4) == 0;
+  const bool vec_ok = (ldy % 4) == 0;
 #pragma unroll
   for (int j = 0; j < MI; ++j) {
     const int m = m0 + wm * 16 * MI + 16 * j + col;
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       if (n >= N) {
         continue;
       }
-      TO* dst = out + static_cast<size_t>(m) * N + n;
+      TO* dst = out + static_cast<size_t>(m) * ldy + n;
       if (vec_ok && n + 4 <= N) {
         if constexpr (sizeof(TO) == 4) {
           *reinterpret_cast<float4*>(dst) =
@@ -612,7 +614,7 @@ QqPlan qq_plan(int M, int N, int K, int mode) {
   const long wide_tiles = mt * ((N + 255) / 256);
   // (4-bit codes: the wide tile where it still fills the chip)
   QqPlan best = {mode == MLXROCM_MXFP4 && wide_tiles >= cus, 1};
-  if (best.wide || (static_cast<int64_t>(M) * N) % 4 != 0) {
+  if (best.wide) {
     return best;
   }
   const long tiles = mt * ((N + 127) / 128);
@@ -636,7 +638,7 @@ QqPlan qq_plan(int M, int N, int K, int mode) {
 
 size_t qq_mfma_plane_bytes(int M, int N, int K, int mode) {
   const int splits = qq_plan(M, N, K, mode).splits;
-  return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
+  return splits > 1 ? splits * k_split_plane(M, N) * sizeof(float) : 0;
 }
 
 int launch_qq_mfma(
@@ -678,7 +680,7 @@ int launch_qq_mfma(
   if (rc != MLXROCM_OK || pl.splits == 1) {
     return rc;
   }
-  return reduce_k_splits(planes, out, static_cast<size_t>(M) * N, pl.splits, dtype, s);
+  return reduce_k_splits(planes, out, M, N, pl.splits, dtype, s);
 }
 
 } // namespace mlxrocm

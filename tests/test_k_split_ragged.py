@@ -1,0 +1,87 @@
+"""K ranges where rows of y do not fill whole 16-byte pieces: the fp32 planes are
+padded, the sum of the planes is not."""
+import pytest
+import torch
+
+import mlx_amd
+from mlx_amd import _lib
+
+# N % 4 of 1, 2, 3 and 0; one and several tiles, rows past a tile, M * N odd and even
+SHAPES = ((255, 775, 4096), (66, 1001, 2048), (97, 222, 1536), (513, 803, 2048), (70, 449, 1024),
+          (130, 640, 1024))
+FP = {"mxfp4": _lib.MXFP4, "mxfp8": _lib.MXFP8, "nvfp4": _lib.NVFP4}
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("dtype", (_lib.FLOAT32, _lib.BFLOAT16))
+def test_split_with_scratch_and_plain_without(M, N, K, dtype):
+    need = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, dtype, 1)
+    rc, plan = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=need)
+    assert rc == _lib.OK and "reduce_k_splits" in plan, plan
+    if N % 4 and dtype != _lib.FLOAT32 and M < 512:  # (these took no workspace before)
+        rc, plan = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=0)
+        assert rc == _lib.OK and "reduce_k_splits" not in plan, plan
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("mode", ("affine", "mxfp4", "mxfp8", "nvfp4"))
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+def test_products(gpu, M, N, K, mode, dtype):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((N, K), generator=g, device="cuda") * K ** -0.5).to(dtype)
+    q = mlx_amd.quantize(w, mode=mode)
+    if mode == "affine":
+        w_hat = mlx_amd.dequantize(q[0], q[1].float(), q[2].float()).double()
+    else:
+        w_hat = mlx_amd.dequantize(*q, mode=mode, dtype=torch.float32).double()
+    y = mlx_amd.quantized_matmul(x, *q, mode=mode)
+    want = x.double() @ w_hat.T
+    size = x.double().abs() @ w_hat.abs().T
+    # half an ulp of the result; weights rounded to the type (16-bit affine) or products
+    # formed from bf16 halves (float32, 2**-16); fp32 sums over K terms
+    half = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    terms = 2.0 ** -16 if dtype == torch.float32 else (half if mode == "affine" else 0.0) + 2e-6
+    err = (y.double() - want).abs()
+    assert bool((err <= half * want.abs() + terms * size).all()), float((err / size).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("mode", ("mxfp4", "mxfp8"))
+def test_both_operands_quantized(gpu, M, N, K, mode):
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+
+    def grid(rows):  # numbers of the format, so that quantizing x changes nothing
+        table = torch.tensor((6.0, 3.0, 1.5, -0.5) if mode == "mxfp4" else (448.0, -256.0, 96.0, 3.5),
+                             device="cuda")
+        v = table[torch.randint(0, 4, (rows, K), generator=g, device="cuda")]
+        v[:, ::32] = table[0]
+        return (v / table[0].log2().floor().exp2()).bfloat16()
+
+    x, q = grid(M), mlx_amd.quantize(grid(N), mode=mode)
+    y = mlx_amd.qqmm(x, *q, mode=mode)
+    x_hat, w_hat = x.double(), mlx_amd.dequantize(*q, mode=mode, dtype=torch.float32).double()
+    want, size = x_hat @ w_hat.T, x_hat.abs() @ w_hat.abs().T
+    # (the e4m3 instruction keeps about 17 bits below a step's largest product)
+    err = (y.double() - want).abs()
+    assert bool((err <= 2.0 ** -8 * want.abs() + 2e-5 * size).all()), float((err / size).max())
+
+
+@pytest.mark.gpu
+def test_built_in_scratch_takes_what_it_took(gpu):
+    """mlxrocm_qmm_static plans within its 64 MiB: the call without planes, where planes
+    do not fit beside the split x."""
+    lib = _lib.load()
+    M, N, K = 255, 14333, 18944
+    assert lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.FLOAT32, 1) > 64 << 20
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    wq, s, b = mlx_amd.quantize(torch.randn((N, K), generator=g, device="cuda") * K ** -0.5)
+    y = torch.empty((M, N), device="cuda")
+    _lib.check(lib.mlxrocm_qmm_static(
+        x.data_ptr(), wq.data_ptr(), s.data_ptr(), b.data_ptr(), y.data_ptr(), M, N, K, 1, M * K,
+        0, 0, 64, 4, _lib.FLOAT32, 1, torch.cuda.current_stream().cuda_stream))
+    want = mlx_amd.quantized_matmul(x, wq, s, b)
+    assert float((y - want).norm() / want.norm()) < 1e-5

@@ -308,6 +308,26 @@ int run_k_split(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scr
   return reduce_k_splits(region, a.out, a.M, a.N, k_splits, dtype, s);
 }
 
+// Rows of x that are few for 256-row tiles (qmm_mid.h).
+int run_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStream_t s) {
+  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, bits);
+  if (pl.splits <= 1) {
+    return MLXROCM_LAUNCH(sc, launch_qmm_mid(a, gs, bits, dtype, pl, s));
+  }
+  void* region = nullptr;
+  int rc = claim(sc, plane_bytes(a, pl.splits), &region);
+  if (rc != MLXROCM_OK || sc.dry) {
+    return rc;
+  }
+  QmmArgs part = a;
+  part.out = region;
+  rc = launch_qmm_mid(part, gs, bits, dtype, pl, s);
+  if (rc != MLXROCM_OK) {
+    return rc;
+  }
+  return reduce_k_splits(region, a.out, a.M, a.N, pl.splits, dtype, s);
+}
+
 // Prefill (transpose=true, 16-bit types) from 512 rows of x on: the tile kernel
 // reads one scale and one bias per thread and K-step, and with the caller's
 // [N][K / group] layout every lane of such a load touches a line of its own
@@ -586,6 +606,32 @@ bool tile_t(const Call& c) {
   return family_of(c) == Family::QmmT && qmm_mfma_supported(c.a, c.gs, c.bits, c.dtype, c.transpose);
 }
 
+// Where the tiles of up to 128 rows (qmm_mid.h) are ahead of those of 256: up to 256 rows,
+// more where K is short, while one round of workgroups holds them.  us per call against the
+// tile kernel, bf16 4-bit g64, 66 / 128 / 256 rows: 4096 x 4096 16.3 / 20.3 / 22.3 against
+// 21.8 / 23.6 / 29.5; 4096 x 14336 25.3 / 29.2 / 44.2 against 36.1 / 39.0 / 50.6;
+// 14336 x 4096 25.7 / 30.4 / 41.9 against 30.0 / 33.6 / 46.9; 32000 x 4096 66 / 128 rows 39.7 / 44.0
+// against 51.8 / 52.6; 2048 x 2048, 256 / 2048 rows 16.0 / 27.4
+// against 24.2 / 39.3.  It is behind in a second round (18944 x 3584, 192 rows: 63 against
+// 45; 32000 x 4096, 192 rows: 76 against 66) and over a long K with more rows, where codes
+// dequantized once for 256 rows are dearer to do again for each 128 (4096 x 14336, 512
+// rows: 77.5 against 71.5).  Up to 64 rows other kernels are ahead of both.
+constexpr int kMidMinM = 65;
+constexpr int kMidMaxM = 256;
+constexpr int kMidMaxMShortK = 2048;
+constexpr int kMidShortK = 2048;
+bool mid_pays(const Call& c) {
+  const QmmArgs& a = c.a;
+  if (a.M < kMidMinM || a.M > (a.K <= kMidShortK ? kMidMaxMShortK : kMidMaxM) ||
+      !qmm_mid_supported(a, c.gs, c.bits, c.dtype, c.transpose)) {
+    return false;
+  }
+  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, c.bits);
+  // (a caller with less scratch than the planes take has what it had before)
+  return pl.groups <= compute_units() &&
+      (pl.splits == 1 || c.sc.affords(plane_bytes(a, pl.splits)));
+}
+
 // Two passes over the same scratch, one after the other on the stream.
 int two_passes(const Call& c, const QmmArgs& head, const QmmArgs& tail) {
   const int rc = run(head, c.gs, c.bits, c.dtype, c.transpose, c.sc, c.s);
@@ -854,6 +900,12 @@ const Rule kRules[] = {
      "float32, 9..16 rows: this table twice (8 rows, the rest); the split-bf16 matrix path "
      "costs the same whatever M. Graph replays, 14336x4096 4-bit: 89 at 9 rows, 132 at 16, "
      "against 155; 4096x14336: 76 / 117 against 171"},
+    {"qmm_mid",
+     [](const Call& c) { return tile_t(c) && mid_pays(c); },
+     [](const Call& c) { return run_qmm_mid(c.a, c.gs, c.bits, c.dtype, c.sc, c.s); },
+     "65..256 rows (..2048 at K <= 2048) in one round of 128 x 128 tiles: packed W and x both "
+     "by direct-to-LDS loads two or more K-steps of 128 ahead, W dequantized in registers. "
+     "4096x14336, 96 rows: 26.6 against 37.2 (tile kernel); 1024x1024, 512 rows: 13.5 against 23.8"},
     {"qmm_t_tile_sb_transposed",
      [](const Call& c) {
        return tile_t(c) && c.a.lhs_indices == nullptr && c.a.M >= kTransposeSbMinM;

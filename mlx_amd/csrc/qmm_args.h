@@ -291,6 +291,19 @@ bool qmv_quad_supported(const QmmArgs& a, int gs, int bits, int dtype);
 int launch_qmv_quad(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 long qmv_quad_workgroups_two_sets(const QmmArgs& a, int bits);
 int launch_qmm_mfma_ksplit(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, hipStream_t s);
+// Some tens to some hundreds of rows of x (qmm_mid.h): transpose=true, 16-bit types, one
+// problem, K % 128 == 0.  With pl.splits > 1 `a.out` points at that many fp32 planes.
+struct MidPlan {
+  int rows;   // of x per tile, at most 128
+  int tiles;  // of x
+  long groups; // workgroups of one range
+  int splits; // ranges of K
+};
+bool qmm_mid_supported(const QmmArgs& a, int gs, int bits, int dtype, bool transpose);
+MidPlan qmm_mid_plan(int M, int N, int K, int bits);
+int launch_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, const MidPlan& pl, hipStream_t s);
+int launch_qmm_mid_bf16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);
+int launch_qmm_mid_f16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);
 int reduce_k_splits(
     const void* partial, void* out, int M, int N, int k_splits, int dtype, hipStream_t s);
 // expert-routed gated MLP (qmm_mfma_experts.hip): pair images, launch_gather_group's tables

@@ -10,7 +10,7 @@
 // 1322-1356 -- quantize x, dequantize it, multiply by the dequantized w): the
 // codes are multiplied as they are, nothing is dequantized.
 //
-// Workgroup: 512 threads, tile 256 (m) x 128 (n), K-step 128 codes.  Both code
+// Workgroup: 512 threads, tile 256 (m) x 128 or 256 (n), K-step 128 codes.  Both code
 // tiles and their scale dwords go HBM -> LDS by DMA (global_load_lds) into a
 // ring of stages.  Reading a step's fragments takes about as long as multiplying
 // them (8-bit codes: 128 KB at 128 bytes a clock against 16 instructions of 32 to 40
@@ -19,9 +19,9 @@
 // 35 % of the time.  Scale dwords come from step-major images, [K / 128][rows]: in the
 // caller's layout each is a cache line of its own, as many requests as the codes.
 // x [2048, 4096] x W [14336, 4096], bf16, quantizing x included: mxfp8 172 -> 146 us
-// (140..155 over the boxes), mxfp4 102 -> 95; 512 rows, 14336 -> 4096, mxfp8 129 -> 105.
+// (140..155 over the boxes), in 256 x 256 tiles 120; mxfp4 102 -> 95; 512 rows, 14336 -> 4096, mxfp8 129 -> 105.
 // 16-byte pieces of a row are XOR-swizzled so that fragment reads hit every bank once.  Wavefront (wm, wn)
-// owns a 64 x 64 block: W fragments are the instruction's A operand, x
+// owns a 64 x 64 (or 128) block: W fragments are the instruction's A operand, x
 // fragments its B operand, so a lane holds four consecutive n of one row m of y.
 #include <type_traits>
 
@@ -41,7 +41,9 @@ constexpr int kQqBK = 128; // codes per step
 
 // Shape of a workgroup: WM x WN wavefronts, each with MI x NI tiles of 16 x 16
 // (m x n).
-//   <8, 4, 4, 4, 2>: 256 x 128, eight wavefronts  (8-bit codes: three stages fit)
+//   <8, 4, 4, 4, 2>: 256 x 128, eight wavefronts  (8-bit codes, few tiles: three stages fit)
+//   <8, 4, 8, 4, 2>: 256 x 256, eight wavefronts  (8-bit codes: two stages, 256 registers;
+//                    a step of twice the work takes 1.56 us against 0.91: 2.75 PFLOP/s)
 //   <4, 4, 8, 4, 2>: 256 x 256, eight wavefronts  (4-bit codes, enough tiles)
 //   <4, 4, 4, 4, 2>: 256 x 128                    (4-bit codes, few tiles)
 // What the shapes trade is bytes fetched per flop: measured at [8192, 4096] x
@@ -70,7 +72,7 @@ struct QqShape {
   static constexpr int kLoads = kXDma + kWDma + kSDma;
   static_assert(kBM % 64 == 0 && kBN % 64 == 0, "a wavefront's scale load stays on one operand");
   static_assert(kBM % (kRowsPerDma * kWaves) == 0 && kBN % (kRowsPerDma * kWaves) == 0, "DMA split");
-  static_assert(kStages >= 3, "the loop needs three stages");
+  static_assert(kStages >= 2, "the loop needs two stages");
   static_assert(MI % 4 == 0 && NI % 4 == 0, "scale bytes travel four to a register");
 };
 
@@ -223,8 +225,13 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   //   * In its read phase of step t a wavefront requests step t + kS - 1 into the stage
   //     of step t - 1, whose last reads (B's, phase 2 t - 1) were waited for before the
   //     barrier that ended them.
+  // With two stages half B would wait for step t + 1 in the phase that requested it, so
+  // it requests step t + 2 a phase later, ahead of its multiplication of step t: that
+  // stage's last reads are its own of the phase before.  Both halves then request a step
+  // in the same phase, two phases ahead of its first read.
   // Every wavefront passes 2 nk + 2 barriers.
   constexpr int kS = S::kStages;
+  constexpr bool kTwo = kS == 2;
   auto k_loop = [&](auto&& read_step, auto&& settle, auto&& multiply) {
     auto barrier = [] {
       __builtin_amdgcn_sched_barrier(0);
@@ -245,6 +252,9 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     auto half = [&](auto behind_c) {
       constexpr bool kBehind = decltype(behind_c)::value;
       if constexpr (kBehind) {
+        if constexpr (kTwo) {
+          issue(1, S::kStage);
+        }
         barrier();
       }
       int rd = 0;                    // stage of step t
@@ -252,7 +262,9 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
       for (int t = 0; t < nk; ++t) {
         read_step(smem + rd);
         __builtin_amdgcn_sched_barrier(0);
-        issue(t + kS - 1, wr);
+        if constexpr (!(kTwo && kBehind)) {
+          issue(t + kS - 1, wr);
+        }
         wr = rd;
         rd = rd + S::kStage < kS * S::kStage ? rd + S::kStage : 0;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -262,6 +274,9 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
           landed();
         }
         barrier();
+        if constexpr (kTwo && kBehind) {
+          issue(t + 2, wr); // (the stage of step t)
+        }
         __builtin_amdgcn_s_setprio(1);
         __builtin_amdgcn_sched_barrier(0);
         multiply();
@@ -599,14 +614,22 @@ bool qq_mfma_supported(int M, int N, int K, int mode) {
 
 // Tile width and K ranges of a launch, the ones that finish first.  A step of the
 // 256 x 128 tile takes 0.8..1 us with 8-bit codes and 0.6 with 4-bit ones (256 x 256:
-// 1.2), a tile some 4 us before and after its steps; ranges cost fp32 planes, written
+// 1.56 and 1.2), a tile some 4 us before and after its steps; ranges cost fp32 planes, written
 // and read again at about 5 TB/s, and a launch.  [512, 14336] x [4096, 14336] has 64
 // tiles for 256 compute units: mxfp8 105 -> 53 us in ranges, mxfp4 82 -> 49; 16 rows,
 // 4096 x 4096: 30 -> 14 and 24 -> 14.
 struct QqPlan {
-  bool wide; // 4-bit codes: 256 x 256
+  bool wide; // 256 x 256
   int splits;
 };
+// 8-bit codes in 256 x 256 tiles: ns a step with every compute unit at work.  Ahead where
+// it saves a round or its rounds are half as many; where 256 x 128 tiles fit one round, or
+// ranges fill it, those are.  us per call, quantizing x included, 256 x 128 (with ranges)
+// against 256 x 256: 14336 x 4096, 512 / 1024 / 2048 / 8192 rows 40 / 73 / 145 / 495
+// against 55 / 62 / 120 / 411; 4096 x 14336, 1024 / 2048 rows 77 / 125 against 151 / 161;
+// 8192 x 8192, 2048 rows 137 against 114; 2048 x 2048, 8192 rows 61 against 51; 1024 x 1024,
+// 8192 rows 29 against 32; 32000 x 4096, 128 / 300 rows 36 / 73 against 50 / 64.
+constexpr double kWideStep8 = 1560.0;
 QqPlan qq_plan(int M, int N, int K, int mode) {
   const long cus = compute_units();
   const long mt = (M + 255) / 256;
@@ -631,6 +654,13 @@ QqPlan qq_plan(int M, int N, int K, int mode) {
     if (ns < best_ns) {
       best.splits = static_cast<int>(splits);
       best_ns = ns;
+    }
+  }
+  if (mode == MLXROCM_MXFP8) {
+    const double ns = best.splits == 1 ? cost(1) : best_ns;
+    const double rounds = static_cast<double>((wide_tiles + cus - 1) / cus);
+    if (rounds * (static_cast<double>(steps) * kWideStep8 + 4000.0) < ns) {
+      best = {true, 1};
     }
   }
   return best;
@@ -672,7 +702,7 @@ int launch_qq_mfma(
   const int rc = dispatch_dtype(pl.splits > 1 ? MLXROCM_FLOAT32 : dtype, [&](auto tval) {
     using T = decltype(tval);
     if (mode == MLXROCM_MXFP8) {
-      return launch_qq<T, 8, 4, 4, 4, 2>(a, s);
+      return pl.wide ? launch_qq<T, 8, 4, 8, 4, 2>(a, s) : launch_qq<T, 8, 4, 4, 4, 2>(a, s);
     }
     return pl.wide ? launch_qq<T, 4, 4, 8, 4, 2, true>(a, s)
                    : launch_qq<T, 4, 4, 4, 4, 2, true>(a, s);

@@ -593,8 +593,9 @@ int mlxrocm_qmm_rows(
  * sb_batch_stride elements apart; image 16-byte aligned device memory).
  * mlxrocm_qmm_prepacked: mlxrocm_qmm with the image as an extra argument (NULL:
  * exactly mlxrocm_qmm).  Shapes that do not read an image ignore it; results
- * are those of mlxrocm_qmm bit for bit.  The workspace may then be smaller than
- * mlxrocm_qmm_workspace_size by mlxrocm_qmm_sb_image_size rounded up to 256.
+ * are those of mlxrocm_qmm bit for bit.  In such prefill calls the workspace may then
+ * be smaller than mlxrocm_qmm_workspace_size by mlxrocm_qmm_sb_image_size rounded up
+ * to 256.
  */
 size_t mlxrocm_qmm_sb_image_size(int N, int K, int batches, int group_size, int dtype);
 int mlxrocm_qmm_sb_image(

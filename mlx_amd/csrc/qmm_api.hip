@@ -308,16 +308,32 @@ int run_k_split(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scr
   return reduce_k_splits(region, a.out, a.M, a.N, k_splits, dtype, s);
 }
 
+// Bytes of the image of scales and biases that a prefill call makes (run_qmm_t_transposed_sb).
+size_t sb_image_bytes(const QmmArgs& a, int gs, int dtype) {
+  const int batches = a.sb_batch_stride == 0 ? 1 : a.L;
+  return (qmm_n_sb_bytes(a.N, a.K / gs, batches, dtype) + 255) / 256 * 256;
+}
+
+// Scratch of a call on qmm_mid_kernel: its planes and, from kTransposeSbMinM rows on, the
+// bytes of an image that it does not read -- a caller of mlxrocm_qmm_prepacked takes these
+// off what mlxrocm_qmm_workspace_size says, and has the planes and the same kernel then.
+size_t mid_bytes(const QmmArgs& a, int gs, int dtype, const MidPlan& pl, const Scratch& sc) {
+  const size_t planes = pl.splits > 1 ? plane_bytes(a, pl.splits) : 0;
+  const bool image = a.M >= kTransposeSbMinM && sc.sb_image == nullptr;
+  return planes + (image ? sb_image_bytes(a, gs, dtype) : 0);
+}
+
 // Rows of x that are few for 256-row tiles (qmm_mid.h).
 int run_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStream_t s) {
   const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, bits);
-  if (pl.splits <= 1) {
-    return MLXROCM_LAUNCH(sc, launch_qmm_mid(a, gs, bits, dtype, pl, s));
-  }
+  const size_t need = mid_bytes(a, gs, dtype, pl, sc);
   void* region = nullptr;
-  int rc = claim(sc, plane_bytes(a, pl.splits), &region);
+  int rc = need != 0 ? claim(sc, need, &region) : static_cast<int>(MLXROCM_OK);
   if (rc != MLXROCM_OK || sc.dry) {
     return rc;
+  }
+  if (pl.splits <= 1) {
+    return launch_qmm_mid(a, gs, bits, dtype, pl, s);
   }
   QmmArgs part = a;
   part.out = region;
@@ -339,8 +355,7 @@ int run_qmm_t_transposed_sb(
   const int G = a.K / gs;
   const int batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool prepacked = sc.sb_image != nullptr;
-  const size_t sb_bytes =
-      prepacked ? 0 : (qmm_n_sb_bytes(a.N, G, batches, dtype) + 255) / 256 * 256;
+  const size_t sb_bytes = prepacked ? 0 : sb_image_bytes(a, gs, dtype);
   const size_t partial_bytes = k_splits > 1 ? plane_bytes(a, k_splits) : 0;
   void* region = nullptr;
   int rc = MLXROCM_OK;
@@ -596,7 +611,7 @@ int tile_k_splits(const Call& c) {
   const int splits = qmm_mfma_k_splits(c.a.M, c.a.N, c.a.K, c.a.L);
   if (ragged(c.a) && splits > 1) {
     const bool image = c.a.M >= kTransposeSbMinM && c.sc.sb_image == nullptr;
-    const size_t sb = image ? (qmm_n_sb_bytes(c.a.N, c.a.K / c.gs, 1, c.dtype) + 255) / 256 * 256 : 0;
+    const size_t sb = image ? sb_image_bytes(c.a, c.gs, c.dtype) : 0;
     return c.sc.affords(sb + plane_bytes(c.a, splits)) ? splits : 1;
   }
   return splits;
@@ -627,9 +642,9 @@ bool mid_pays(const Call& c) {
     return false;
   }
   const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, c.bits);
-  // (a caller with less scratch than the planes take has what it had before)
-  return pl.groups <= compute_units() &&
-      (pl.splits == 1 || c.sc.affords(plane_bytes(a, pl.splits)));
+  // (a caller with less scratch has what it had before)
+  const size_t need = mid_bytes(a, c.gs, c.dtype, pl, c.sc);
+  return pl.groups <= compute_units() && (need == 0 || c.sc.affords(need));
 }
 
 // Two passes over the same scratch, one after the other on the stream.

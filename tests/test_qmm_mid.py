@@ -27,6 +27,42 @@ def test_less_scratch_keeps_the_other_plan():
     assert rc == _lib.OK and "qmm_mid(" not in plan, plan
 
 
+@pytest.mark.parametrize("bits,group", ((4, 64), (8, 32), (3, 128)))
+def test_workspace_counts_the_scale_image(bits, group):
+    """mlxrocm_qmm_prepacked takes a workspace that is smaller by the image: what is left
+    holds the planes of the same plan."""
+    lib = _lib.load()
+    for M in (512, 513, 700, 1024, 1500, 2048):
+        for N in (64, 222, 1024, 1401, 2048, 4096):
+            for K in (128, 640, 1024, 2048):
+                need = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, group, bits, _lib.BFLOAT16, 1)
+                image = lib.mlxrocm_qmm_sb_image_size(N, K, 1, group, _lib.BFLOAT16)
+                rc, plan = _lib.qmm_plan(M, N, K, group_size=group, bits=bits,
+                                         dtype=_lib.BFLOAT16, workspace_bytes=need)
+                planes = int(plan.split("reduce_k_splits(")[1][:-1]) if "reduce" in plan else 0
+                rest = planes * M * ((N + 3) // 4 * 4) * 4
+                assert rc == _lib.OK and need >= (image + 255) // 256 * 256 + rest, (M, N, K, plan)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", ((512, 1024, 2048), (2048, 1024, 2048), (600, 1024, 4096),
+                                   (600, 803, 4096)))
+def test_prepacked_with_the_smaller_workspace(gpu, M, N, K):
+    lib = _lib.load()
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+    wq, s, b = mlx_amd.quantize((torch.randn((N, K), device="cuda") / 64).to(torch.bfloat16))
+    image = mlx_amd.quantized_matmul_sb_image(s, b, 64)
+    room = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.BFLOAT16, 1)
+    room -= (lib.mlxrocm_qmm_sb_image_size(N, K, 1, 64, _lib.BFLOAT16) + 255) // 256 * 256
+    ws = torch.empty(max(room, 1), dtype=torch.uint8, device="cuda")
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    _lib.check(lib.mlxrocm_qmm_prepacked(
+        x.data_ptr(), wq.data_ptr(), s.data_ptr(), b.data_ptr(), image.data_ptr(), y.data_ptr(),
+        M, N, K, 1, M * K, 0, 0, 64, 4, _lib.BFLOAT16, 1, ws.data_ptr(), room,
+        torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(y, mlx_amd.quantized_matmul(x, wq, s, b))
+
+
 # (rows: one tile of 64, 96 and 128, several with a short last one; N: one row of W past a
 # tile, no whole 16-byte rows of y, less than a tile; K: one step, fewer steps than stages,
 # more than a table segment holds (2048 codes at groups of 32), many ranges)

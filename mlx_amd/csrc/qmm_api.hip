@@ -150,16 +150,18 @@ struct Scratch {
   // Optional: the caller's transposed image of scales and biases
   // (mlxrocm_qmm_sb_image); the prefill path then skips its pre-pass.
   const void* sb_image = nullptr;
-  // No plan may want more than this (the entry point with built-in scratch).
-  size_t most = SIZE_MAX;
-  // Is there room for `bytes`?  For plans that are an alternative to one with less
+  // Is there room for `wanted` bytes?  For plans that are an alternative to one with less
   // scratch: workspace_size counts them, a caller with less runs the other one.
   bool affords(size_t wanted) const {
-    return wanted <= most && (dry || (base != nullptr && bytes >= wanted));
+    return dry || (base != nullptr && bytes >= wanted);
   }
 };
 
 constexpr size_t kScratchAlign = 256;
+
+// Scratch of mlxrocm_qmm_static, which takes the plan of mlxrocm_qmm: a plan that is an
+// alternative to one with less scratch wants no more than this.
+constexpr size_t kStaticScratchBytes = size_t(64) << 20;
 
 int claim(Scratch& sc, size_t bytes, void** out) {
   *out = nullptr;
@@ -204,6 +206,16 @@ bool ragged(const QmmArgs& a) {
   return a.N % 4 != 0;
 }
 
+// K ranges of a ragged shape: `splits`, or as many of them as leave room for the `rest`
+// of the scratch in mlxrocm_qmm_static's.
+int ragged_splits(const QmmArgs& a, int splits, size_t rest) {
+  if (rest > kStaticScratchBytes) { // (refused there whatever the plan)
+    return splits;
+  }
+  const size_t most = (kStaticScratchBytes - rest) / plane_bytes(a, 1);
+  return most < static_cast<size_t>(splits) ? static_cast<int>(most) : splits;
+}
+
 int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t s) {
   const size_t row_bytes = split_x_bytes(1, a.K);
   int rows_per_block = static_cast<int>(kSplitScratchBytes / row_bytes / 256 * 256);
@@ -228,6 +240,9 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
   const int sb_batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool sb_t = a.M >= kTransposeSbMinM;
   const size_t sb_bytes = sb_t ? qmm_n_sb_bytes(a.N, G, sb_batches, MLXROCM_FLOAT32) : 0;
+  if (ragged(a) && k_splits > 1) {
+    k_splits = ragged_splits(a, k_splits, x_bytes + sb_bytes + 255); // (planes are rounded up)
+  }
   size_t partial_bytes =
       k_splits > 1 ? (plane_bytes(a, k_splits) + 255) / 256 * 256 : 0;
   if (ragged(a) && !sc.affords(x_bytes + partial_bytes + sb_bytes)) {
@@ -610,9 +625,10 @@ int tile_k_splits(const Call& c) {
   }
   const int splits = qmm_mfma_k_splits(c.a.M, c.a.N, c.a.K, c.a.L);
   if (ragged(c.a) && splits > 1) {
-    const bool image = c.a.M >= kTransposeSbMinM && c.sc.sb_image == nullptr;
-    const size_t sb = image ? sb_image_bytes(c.a, c.gs, c.dtype) : 0;
-    return c.sc.affords(sb + plane_bytes(c.a, splits)) ? splits : 1;
+    const size_t sb = c.a.M >= kTransposeSbMinM ? sb_image_bytes(c.a, c.gs, c.dtype) : 0;
+    const int room = ragged_splits(c.a, splits, sb);
+    const size_t own = c.sc.sb_image == nullptr ? sb : 0;
+    return room > 1 && c.sc.affords(own + plane_bytes(c.a, room)) ? room : 1;
   }
   return splits;
 }
@@ -644,7 +660,8 @@ bool mid_pays(const Call& c) {
   const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, c.bits);
   // (a caller with less scratch has what it had before)
   const size_t need = mid_bytes(a, c.gs, c.dtype, pl, c.sc);
-  return pl.groups <= compute_units() && (need == 0 || c.sc.affords(need));
+  return pl.groups <= compute_units() && plane_bytes(a, pl.splits) <= kStaticScratchBytes / 2 &&
+      (need == 0 || c.sc.affords(need));
 }
 
 // Two passes over the same scratch, one after the other on the stream.
@@ -1235,36 +1252,6 @@ int qmm_entry(
 
 } // namespace
 
-namespace {
-
-// Scratch of a call whose plan wants no more than `most`; 0 for a call that is refused.
-size_t workspace_need(
-    int M,
-    int N,
-    int K,
-    int L,
-    int batched_weights,
-    int group_size,
-    int bits,
-    int dtype,
-    int transpose,
-    size_t most) {
-  Scratch sc;
-  sc.dry = true;
-  sc.most = most;
-  // the strides only say "one weight for every batch entry" or "one each"
-  const int64_t w_stride = batched_weights ? 4096 : 0;
-  const int64_t x_stride = static_cast<int64_t>(M) * K;
-  if (qmm_entry(
-          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
-          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
-    return 0;
-  }
-  return sc.need;
-}
-
-} // namespace
-
 extern "C" size_t mlxrocm_qmm_workspace_size(
     int M,
     int N,
@@ -1275,8 +1262,17 @@ extern "C" size_t mlxrocm_qmm_workspace_size(
     int bits,
     int dtype,
     int transpose) {
-  return workspace_need(
-      M, N, K, L, batched_weights, group_size, bits, dtype, transpose, SIZE_MAX);
+  Scratch sc;
+  sc.dry = true;
+  // the strides only say "one weight for every batch entry" or "one each"
+  const int64_t w_stride = batched_weights ? 4096 : 0;
+  const int64_t x_stride = static_cast<int64_t>(M) * K;
+  if (qmm_entry(
+          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
+          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
+    return 0;
+  }
+  return sc.need;
 }
 
 extern "C" int mlxrocm_qmm(
@@ -1478,7 +1474,6 @@ extern "C" int mlxrocm_qmm_prepacked(
 // moment the code object is loaded until the process ends.  In host code the
 // name below is only a handle for hipGetSymbolAddress; the address a kernel
 // may use is looked up once per device and kept in g_static_scratch.
-constexpr size_t kStaticScratchBytes = size_t(64) << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -1538,9 +1533,8 @@ extern "C" int mlxrocm_qmm_static(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  const size_t need = workspace_need(
-      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose,
-      kStaticScratchBytes);
+  const size_t need = mlxrocm_qmm_workspace_size(
+      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose);
   if (need > kStaticScratchBytes) {
     return fail(
         MLXROCM_UNSUPPORTED,
@@ -1555,7 +1549,6 @@ extern "C" int mlxrocm_qmm_static(
   Scratch sc;
   sc.base = static_cast<char*>(region);
   sc.bytes = kStaticScratchBytes;
-  sc.most = kStaticScratchBytes;
   return qmm_entry(
       x, wq, scales, biases, out, M, N, K, L, x_batch_stride, w_batch_stride,
       sb_batch_stride, group_size, bits, dtype, transpose, sc,

@@ -917,22 +917,41 @@ extern "C" int mlxrocm_fp_qmm_rows(
       dtype, 1, workspace, workspace_bytes, stream, nullptr, true);
 }
 
-extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, int dtype) {
-  if (fp_check("qqmm", M, N, K, 1, mode, dtype, 1) != MLXROCM_OK ||
-      static_cast<int64_t>(M) * N == 0 || K == 0) {
-    return 0;
-  }
+namespace {
+
+// Scratch of qqmm, with the fp32 planes of K ranges or as much as the plan without them takes.
+size_t qqmm_bytes(int M, int N, int K, int mode, int dtype, bool planes) {
   if (qq_native(M, N, K, mode, dtype)) {
     const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
     return round256(static_cast<size_t>(M) * K * bits / 8) +
         round256(static_cast<size_t>(M) * K / 32) +
         round256(static_cast<size_t>(N) * K / 32) +
-        round256(qq_mfma_plane_bytes(M, N, K, mode));
+        (planes ? round256(qq_mfma_plane_bytes(M, N, K, mode)) : 0);
   }
-  return round256(static_cast<size_t>(M) * K * dtype_size(dtype)) +
-      (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)
-           ? mlxrocm_fp_qmm_rows_workspace_size(M, N, K, 1, mode, dtype)
-           : mlxrocm_fp_qmm_workspace_size(M, N, K, 1, 0, mode, dtype, 1));
+  const size_t xhat = round256(static_cast<size_t>(M) * K * dtype_size(dtype));
+  if (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)) {
+    return xhat + mlxrocm_fp_qmm_rows_workspace_size(M, N, K, 1, mode, dtype);
+  }
+  if (!planes && fp_tile_applies(M, N, K, 1, mode, dtype, true)) {
+    return xhat + fp_image_bytes(N, K, 1);
+  }
+  return xhat + mlxrocm_fp_qmm_workspace_size(M, N, K, 1, 0, mode, dtype, 1);
+}
+
+// What a call must have.  Planes of padded rows (N no multiple of four) are an alternative:
+// the plan without them is there for a caller with less.
+size_t qqmm_least_bytes(int M, int N, int K, int mode, int dtype) {
+  return qqmm_bytes(M, N, K, mode, dtype, N % 4 == 0);
+}
+
+} // namespace
+
+extern "C" size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, int dtype) {
+  if (fp_check("qqmm", M, N, K, 1, mode, dtype, 1) != MLXROCM_OK ||
+      static_cast<int64_t>(M) * N == 0 || K == 0) {
+    return 0;
+  }
+  return qqmm_bytes(M, N, K, mode, dtype, true);
 }
 
 extern "C" int mlxrocm_fp_qqmm(
@@ -963,7 +982,7 @@ extern "C" int mlxrocm_fp_qqmm(
   if (!x || !wq || !scales || !out) {
     return fail(MLXROCM_INVALID_ARGUMENT, "[qqmm] null device pointer");
   }
-  const size_t need = mlxrocm_fp_qqmm_workspace_size(M, N, K, mode, dtype);
+  const size_t need = qqmm_least_bytes(M, N, K, mode, dtype);
   if (workspace == nullptr || workspace_bytes < need ||
       (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) {
     return fail(
@@ -987,7 +1006,9 @@ extern "C" int mlxrocm_fp_qqmm(
     if (rc != MLXROCM_OK) {
       return rc;
     }
-    void* planes = ws + round256(static_cast<size_t>(N) * K / 32);
+    void* planes = workspace_bytes >= qqmm_bytes(M, N, K, mode, dtype, true)
+        ? ws + round256(static_cast<size_t>(N) * K / 32)
+        : nullptr;
     return launch_qq_mfma(
         codes, xs, wq, image ? ws : scales, image, out, M, N, K, mode, dtype, planes, s);
   }
@@ -1419,7 +1440,7 @@ extern "C" int mlxrocm_nvfp4_qqmm_global(
   if (!x || !wq || !scales || !out) {
     return fail(MLXROCM_INVALID_ARGUMENT, "[qqmm] null device pointer");
   }
-  const size_t need = mlxrocm_fp_qqmm_workspace_size(M, N, K, mode, dtype);
+  const size_t need = qqmm_least_bytes(M, N, K, mode, dtype);
   if (workspace == nullptr || workspace_bytes < need ||
       (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) {
     return fail(

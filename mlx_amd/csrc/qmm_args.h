@@ -142,9 +142,9 @@ int launch_qmm_mfma_fp_grouped(const QmmArgs& a, int mode, int dtype, hipStream_
 // qqmm in the MX modes on the block-scaled matrix instruction (qq_mfma.hip):
 // x as codes and an image of scale bytes (fp_quantize_activations, fp_quantize.hip)
 // times the quantized w, both [rows][K]; K % 128 == 0.  ws: the caller's scale bytes
-// [N][K / 32], or (ws_image) their image.
+// [N][K / 32], or (ws_image) their image.  planes: scratch for K ranges, or NULL for none.
 bool qq_mfma_supported(int M, int N, int K, int mode);
-size_t qq_mfma_plane_bytes(int M, int N, int K, int mode); // scratch for K ranges (planes)
+size_t qq_mfma_plane_bytes(int M, int N, int K, int mode);
 int launch_qq_mfma(
     const void* xq,
     const uint8_t* xs,

@@ -630,7 +630,7 @@ struct QqPlan {
 // 8192 x 8192, 2048 rows 137 against 114; 2048 x 2048, 8192 rows 61 against 51; 1024 x 1024,
 // 8192 rows 29 against 32; 32000 x 4096, 128 / 300 rows 36 / 73 against 50 / 64.
 constexpr double kWideStep8 = 1560.0;
-QqPlan qq_plan(int M, int N, int K, int mode) {
+QqPlan qq_plan(int M, int N, int K, int mode, bool planes = true) {
   const long cus = compute_units();
   const long mt = (M + 255) / 256;
   const long steps = K / kQqBK;
@@ -640,6 +640,7 @@ QqPlan qq_plan(int M, int N, int K, int mode) {
   if (best.wide) {
     return best;
   }
+  const long most = planes ? 16 : 1; // ranges
   const long tiles = mt * ((N + 127) / 128);
   const double step = mode == MLXROCM_MXFP8 ? 900.0 : 600.0; // ns
   auto cost = [&](long splits) -> double {
@@ -649,7 +650,7 @@ QqPlan qq_plan(int M, int N, int K, int mode) {
     return splits == 1 ? ns : ns + 4000.0 + static_cast<double>(splits) * M * N * 4.0 / 4000.0;
   };
   double best_ns = cost(1) / 1.08;
-  for (long splits = 2; splits <= 16 && splits * 4 <= steps && splits * tiles <= 2 * cus; ++splits) {
+  for (long splits = 2; splits <= most && splits * 4 <= steps && splits * tiles <= 2 * cus; ++splits) {
     const double ns = cost(splits);
     if (ns < best_ns) {
       best.splits = static_cast<int>(splits);
@@ -685,7 +686,7 @@ int launch_qq_mfma(
     int dtype,
     void* planes,
     hipStream_t s) {
-  const QqPlan pl = qq_plan(M, N, K, mode);
+  const QqPlan pl = qq_plan(M, N, K, mode, planes != nullptr);
   QqArgs a;
   a.splits = pl.splits;
   a.xq = static_cast<const uint8_t*>(xq);
@@ -698,7 +699,11 @@ int launch_qq_mfma(
   a.K = K;
   a.ws_row = ws_image ? 4u : static_cast<uint32_t>(K) / 32;
   a.ws_step = ws_image ? 4u * static_cast<uint32_t>(N) : 4u;
-  MLXROCM_REHEARSE("qq_mfma(%s)", mode == MLXROCM_MXFP8 ? "e4m3" : "e2m1");
+  if (rehearsing()) {
+    note_launch("qq_mfma(%s)", mode == MLXROCM_MXFP8 ? "e4m3" : "e2m1");
+    return pl.splits == 1 ? static_cast<int>(MLXROCM_OK)
+                          : reduce_k_splits(planes, out, M, N, pl.splits, dtype, s);
+  }
   const int rc = dispatch_dtype(pl.splits > 1 ? MLXROCM_FLOAT32 : dtype, [&](auto tval) {
     using T = decltype(tval);
     if (mode == MLXROCM_MXFP8) {

@@ -84,6 +84,48 @@ def test_built_in_scratch_takes_the_same_plan(dtype):
                 assert built_in == plan if rc == _lib.OK else need > 64 << 20, (M, N, K, plan)
 
 
+# (M, N, K), both modes of qqmm's own kernel and, at K % 128 != 0 or in nvfp4, the others
+QQ = ((96, 775, 4096), (300, 1001, 4096), (511, 222, 2048), (130, 803, 4160))
+
+
+def qqmm_bytes_without_planes(M, N, K, mode, dtype_size=2):
+    up = lambda n: (n + 255) // 256 * 256
+    if mode != _lib.NVFP4 and K % 128 == 0:  # codes and scales of x, scales of W
+        return up(M * K * (8 if mode == _lib.MXFP8 else 4) // 8) + up(M * K // 32) + up(N * K // 32)
+    return up(M * K * dtype_size) + up(N * (K // 32) * 4)  # x again, the scale image
+
+
+@pytest.mark.parametrize("M,N,K", QQ)
+@pytest.mark.parametrize("mode", FP.values(), ids=FP)
+def test_qqmm_without_room_for_planes(M, N, K, mode):
+    least = qqmm_bytes_without_planes(M, N, K, mode)
+    need = _lib.load().mlxrocm_fp_qqmm_workspace_size(M, N, K, mode, _lib.BFLOAT16)
+    rc, plan = _lib.fp_qqmm_plan(M, N, K, mode, _lib.BFLOAT16, need)
+    assert rc == _lib.OK and ("reduce_k_splits" in plan) == (need > least), plan
+    rc, plan = _lib.fp_qqmm_plan(M, N, K, mode, _lib.BFLOAT16, least)
+    assert rc == _lib.OK and "reduce_k_splits" not in plan, plan
+    rc, plan = _lib.fp_qqmm_plan(M, N, K, mode, _lib.BFLOAT16, least - 1)
+    assert rc == _lib.INVALID_ARGUMENT
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", QQ)
+@pytest.mark.parametrize("mode", FP)
+def test_qqmm_with_and_without_planes(gpu, M, N, K, mode):
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+    x = torch.randn((M, K), generator=g, device="cuda").bfloat16()
+    wq, s = mlx_amd.quantize(torch.randn((N, K), generator=g, device="cuda") * K ** -0.5, mode=mode)
+    ws = torch.empty(qqmm_bytes_without_planes(M, N, K, FP[mode]), dtype=torch.uint8, device="cuda")
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    _lib.check(lib.mlxrocm_fp_qqmm(
+        x.data_ptr(), wq.data_ptr(), s.data_ptr(), y.data_ptr(), M, N, K, FP[mode], _lib.BFLOAT16,
+        ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    want = mlx_amd.qqmm(x, wq, s, mode=mode)
+    # the same products in another order: an ulp of some results
+    assert float((y.double() - want.double()).norm() / want.double().norm()) < 2.0 ** -9
+
+
 @pytest.mark.gpu
 def test_built_in_scratch_takes_what_it_took(gpu):
     """mlxrocm_qmm_static plans within its 64 MiB: here two K ranges, where three fill the

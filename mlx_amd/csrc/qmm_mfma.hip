@@ -229,7 +229,21 @@ int qmm_mfma_k_splits(int M, int N, int K, int L, int nt) {
   if (s > 16) {
     s = 16;
   }
-  return s < 2 ? 1 : static_cast<int>(s);
+  if (s < 2) {
+    return 1;
+  }
+  // Results stored by the element (N no multiple of four), 16-bit tiles: ranges where the
+  // steps they save, some 0.4 us each beside narrower tiles without ranges, are worth more
+  // than the planes, written and read at about 10 GB/ms.  us without / with two ranges,
+  // bf16: 1495 x 4099 x 1024 38 / 44, 6334 x 1001 x 1344 (mxfp4) 41 / 46; 990 x 3001 x 1344
+  // (nvfp4) 42 / 37, 319 x 10762 x 2048 53 / 43.
+  if (nt != kSplitFp32Width && N % 4 != 0) {
+    const double saved = 0.4 * static_cast<double>(steps - (steps + s - 1) / s);
+    if (saved < 1.0 + static_cast<double>(k_split_plane(M, N)) * s * 4e-7) {
+      return 1;
+    }
+  }
+  return static_cast<int>(s);
 }
 
 // 16-bit operands with K cut into k_splits ranges: `a.out` points at k_splits
@@ -257,68 +271,56 @@ int launch_qmm_mfma_ksplit(
 
 namespace {
 
-// Four consecutive elements of y per thread, also where rows of y (N) are shorter than
-// rows of the planes (whole 16-byte pieces).  Before rows were padded a shape whose M N is
-// no multiple of four ran without K ranges, on a handful of compute units: 255 x 775 x 4096
-// bf16 79 us -> 28, float32 304 -> 62, 229 x 2735 x 13440 mxfp8 204 -> 50.
+// Four consecutive elements of a row of the planes per thread, with 16-byte loads: rows of
+// the planes are whole 16-byte pieces, also where rows of y (N) are not.  There the row is
+// found by one 32-bit division and the store starts at any element.  With four elements of
+// y per thread, each with a 64-bit division and loads of its own, whole calls took 2 to 10 %
+// longer: 1660 x 803 x 5888 mxfp4 48.5 us against 42.9, 1285 x 4099 x 8192 4-bit 122 against 116.
 template <typename TO>
 __global__ __launch_bounds__(256) void reduce_k_splits_kernel(
     const float* partial,
     TO* out,
-    size_t n, // elements of y
+    size_t pieces, // of a plane
     int N,
-    size_t plane,
     int k_splits) {
-  const size_t i = (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
-  if (i >= n) {
+  const size_t piece = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (piece >= pieces) {
     return;
   }
-  const int ld = k_split_row(N);
-  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (ld == N) { // (n is a multiple of 4)
-    float4 acc = *reinterpret_cast<const float4*>(partial + i);
-    for (int z = 1; z < k_splits; ++z) {
-      const float4 p = *reinterpret_cast<const float4*>(partial + z * plane + i);
-      acc.x += p.x;
-      acc.y += p.y;
-      acc.z += p.z;
-      acc.w += p.w;
-    }
-    v[0] = acc.x;
-    v[1] = acc.y;
-    v[2] = acc.z;
-    v[3] = acc.w;
-  } else {
-    size_t at[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const size_t j = i + e < n ? i + e : n - 1;
-      const size_t m = j / N;
-      at[e] = j + m * (ld - N);
-      v[e] = partial[at[e]];
-    }
-    for (int z = 1; z < k_splits; ++z) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] += partial[z * plane + at[e]];
-      }
-    }
+  const float4* p = reinterpret_cast<const float4*>(partial) + piece;
+  float4 acc = *p;
+  for (int z = 1; z < k_splits; ++z) {
+    const float4 v = p[z * pieces];
+    acc.x += v.x;
+    acc.y += v.y;
+    acc.z += v.z;
+    acc.w += v.w;
   }
-  if (i + 4 <= n) {
+  size_t at = piece * 4;
+  int n = 0;
+  if ((N & 3) != 0) {
+    const uint32_t row_pieces = static_cast<uint32_t>(k_split_row(N)) / 4;
+    const uint32_t m = static_cast<uint32_t>(piece) / row_pieces; // (the launcher checks the size)
+    n = static_cast<int>(static_cast<uint32_t>(piece) - m * row_pieces) * 4;
+    at = static_cast<size_t>(m) * N + n;
+  }
+  TO* y = out + at;
+  if (n + 4 <= N) {
+    // (one store, wherever an element may start)
     if constexpr (sizeof(TO) == 4) {
-      *reinterpret_cast<float4*>(out + i) = make_float4(v[0], v[1], v[2], v[3]);
+      typedef float __attribute__((ext_vector_type(4), aligned(4))) four;
+      *reinterpret_cast<four*>(y) = four{acc.x, acc.y, acc.z, acc.w};
     } else {
-      uint2 packed;
-      packed.x = pack2<TO>(v[0], v[1]);
-      packed.y = pack2<TO>(v[2], v[3]);
-      *reinterpret_cast<uint2*>(out + i) = packed;
+      typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) four;
+      *reinterpret_cast<four*>(y) = four{pack2<TO>(acc.x, acc.y), pack2<TO>(acc.z, acc.w)};
     }
-  } else {
+    return;
+  }
+  const float v[3] = {acc.x, acc.y, acc.z};
 #pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      if (i + e < n) {
-        out[i + e] = static_cast<TO>(v[e]);
-      }
+  for (int e = 0; e < 3; ++e) {
+    if (n + e < N) {
+      y[e] = static_cast<TO>(v[e]);
     }
   }
 }
@@ -329,9 +331,9 @@ __global__ __launch_bounds__(256) void reduce_k_splits_kernel(
 // y must be 16-byte aligned.
 int reduce_k_splits(
     const void* partial, void* out, int M, int N, int k_splits, int dtype, hipStream_t s) {
-  const size_t n = static_cast<size_t>(M) * N;
-  const size_t blocks = (n / 4 + 1 + 255) / 256;
-  if (blocks > 0x7fffffffull) {
+  const size_t pieces = k_split_plane(M, N) / 4;
+  const size_t blocks = (pieces + 255) / 256;
+  if (blocks > 0x7fffffffull || (N % 4 != 0 && pieces > 0xffffffffull)) {
     return fail(MLXROCM_UNSUPPORTED, "[qmm] output too large for the split-K reduction");
   }
   MLXROCM_REHEARSE("reduce_k_splits(%d)", k_splits);
@@ -340,7 +342,7 @@ int reduce_k_splits(
   return dispatch_dtype(dtype, [&](auto tval) {
     using T = decltype(tval);
     reduce_k_splits_kernel<T><<<g, 256, 0, s>>>(
-        p, static_cast<T*>(out), n, N, k_split_plane(M, N), k_splits);
+        p, static_cast<T*>(out), pieces, N, k_splits);
     MLXROCM_HIP_TRY(hipGetLastError());
     return static_cast<int>(MLXROCM_OK);
   });

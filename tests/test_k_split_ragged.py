@@ -23,6 +23,18 @@ def test_split_with_scratch_and_plain_without(M, N, K, dtype):
         assert rc == _lib.OK and "reduce_k_splits" not in plan, plan
 
 
+@pytest.mark.parametrize("M,N,K,split", (
+    (1495, 4099, 1024, False), (6334, 1001, 1344, False), (2195, 3001, 1344, False),
+    (990, 3001, 1344, True), (700, 6002, 2048, True), (1501, 1502, 4096, True),
+))
+def test_ranges_where_planes_cost_less_than_they_save(M, N, K, split):
+    need = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.BFLOAT16, 1)
+    rc, plan = _lib.qmm_plan(M, N, K, dtype=_lib.BFLOAT16, workspace_bytes=need)
+    assert rc == _lib.OK and "qmm_t_tile" in plan and ("reduce_k_splits" in plan) == split, plan
+    rc, plan = _lib.fp_qmm_plan(M, N, K)
+    assert rc == _lib.OK and ("reduce_k_splits" in plan) == split, plan
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("mode", ("affine", "mxfp4", "mxfp8", "nvfp4"))

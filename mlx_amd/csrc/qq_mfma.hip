@@ -107,6 +107,7 @@ template <typename TO, int BITS, int MI, int NI, int WM, int WN, bool BIG = fals
 __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   static_assert(!BIG || BITS == 4, "the 32 x 32 x 64 form pays for 4-bit codes only");
   using S = QqShape<BITS, MI, NI, WM, WN>;
+  constexpr bool kPlanes = sizeof(TO) == 4; // (planes are fp32: 16-bit results are y itself)
   constexpr int kBM = S::kBM;
   constexpr int kBN = S::kBN;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -383,8 +384,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     k_loop(read_step, settle, multiply);
     // D[n][m] 32 x 32: register i of lane (col, half) holds n = 8 (i / 4) + 4 half
     // + i % 4, m = col
-    const int ldy = a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
-    TO* out = static_cast<TO*>(a.out) + blockIdx.z * k_split_plane(M, N);
+    const int ldy = kPlanes && a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
+    TO* out = static_cast<TO*>(a.out) + (kPlanes ? blockIdx.z * k_split_plane(M, N) : 0);
     const int col = lane & 31;
     const int half = lane >> 5;
     const bool vec_ok = (ldy % 4) == 0;
@@ -538,8 +539,8 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #undef QQ_DMA4
 
   // D[n][m]: register r of lane (col, quad) holds n = 4 quad + r, m = col
-  const int ldy = a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
-  TO* out = static_cast<TO*>(a.out) + blockIdx.z * k_split_plane(M, N);
+  const int ldy = kPlanes && a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes
+  TO* out = static_cast<TO*>(a.out) + (kPlanes ? blockIdx.z * k_split_plane(M, N) : 0);
   const int col = lane & 15;
   const int quad = lane >> 4;
   const bool vec_ok = (ldy % 4) == 0;

@@ -630,7 +630,17 @@ struct QqPlan {
 // against 55 / 62 / 120 / 411; 4096 x 14336, 1024 / 2048 rows 77 / 125 against 151 / 161;
 // 8192 x 8192, 2048 rows 137 against 114; 2048 x 2048, 8192 rows 61 against 51; 1024 x 1024,
 // 8192 rows 29 against 32; 32000 x 4096, 128 / 300 rows 36 / 73 against 50 / 64.
+// Over a short K what a tile takes beside its steps decides: filling two stages, and, from
+// the second round on, results stored by the element (N no multiple of four), twice as many
+// to a tile.  256 x 256 against 256 x 128: 3920 x 4099 x 1024 67 against 56, 5285 x 4099 x 256
+// 63 against 55, 5083 x 4096 x 256 34 against 31; ahead in one round (1501 x 6002 x 256: 32
+// against 37) and at 3067 x 14336 x 256 (11 %).
 constexpr double kWideStep8 = 1560.0;
+double wide8_ns(long rounds, long steps, int N) {
+  const double k = static_cast<double>(steps);
+  const double ns = static_cast<double>(rounds) * (k * kWideStep8 + 4250.0 + 3000.0 / k);
+  return N % 4 == 0 ? ns : ns + static_cast<double>(rounds - 1) * 4000.0;
+}
 QqPlan qq_plan(int M, int N, int K, int mode, bool planes = true) {
   const long cus = compute_units();
   const long mt = (M + 255) / 256;
@@ -660,8 +670,7 @@ QqPlan qq_plan(int M, int N, int K, int mode, bool planes = true) {
   }
   if (mode == MLXROCM_MXFP8) {
     const double ns = best.splits == 1 ? cost(1) : best_ns;
-    const double rounds = static_cast<double>((wide_tiles + cus - 1) / cus);
-    if (rounds * (static_cast<double>(steps) * kWideStep8 + 4000.0) < ns) {
+    if (wide8_ns((wide_tiles + cus - 1) / cus, steps, N) < ns) {
       best = {true, 1};
     }
   }
@@ -701,14 +710,20 @@ int launch_qq_mfma(
   a.ws_row = ws_image ? 4u : static_cast<uint32_t>(K) / 32;
   a.ws_step = ws_image ? 4u * static_cast<uint32_t>(N) : 4u;
   if (rehearsing()) {
-    note_launch("qq_mfma(%s)", mode == MLXROCM_MXFP8 ? "e4m3" : "e2m1");
+    // (tiles of 256 columns go without saying, those of 128 by name for e4m3 alone)
+    note_launch("qq_mfma(%s)", mode == MLXROCM_MXFP4 ? "e2m1" : pl.wide ? "e4m3" : "e4m3,bn=128");
     return pl.splits == 1 ? static_cast<int>(MLXROCM_OK)
                           : reduce_k_splits(planes, out, M, N, pl.splits, dtype, s);
   }
   const int rc = dispatch_dtype(pl.splits > 1 ? MLXROCM_FLOAT32 : dtype, [&](auto tval) {
     using T = decltype(tval);
     if (mode == MLXROCM_MXFP8) {
-      return pl.wide ? launch_qq<T, 8, 4, 8, 4, 2>(a, s) : launch_qq<T, 8, 4, 4, 4, 2>(a, s);
+      if constexpr (sizeof(T) == 2) { // (wide tiles write no planes, and float32 x takes other kernels)
+        if (pl.wide) {
+          return launch_qq<T, 8, 4, 8, 4, 2>(a, s);
+        }
+      }
+      return launch_qq<T, 8, 4, 4, 4, 2>(a, s);
     }
     return pl.wide ? launch_qq<T, 4, 4, 8, 4, 2, true>(a, s)
                    : launch_qq<T, 4, 4, 4, 4, 2, true>(a, s);

@@ -3,12 +3,28 @@ import pytest
 import torch
 
 import mlx_amd
+from mlx_amd import _lib
 
-# more 256 x 128 tiles than a round holds (256), no more 256 x 256 tiles than that, so the
-# wide tile is chosen; one, two, three, five and nine steps; a row or column past a tile,
-# rows of y that are no whole 16-byte pieces, a last tile of one row of W, several rounds
+# fewer rounds of 256 x 256 tiles than of 256 x 128; one, two, three, five and nine steps; a
+# row or column past a tile, rows of y that are no whole 16-byte pieces, a last tile of one
+# row of W, one round and (531 tiles) three
 SHAPES = ((4111, 2503, 128), (4096, 2560, 256), (2049, 3841, 384), (300, 32001, 640),
           (257, 18002, 1152), (513, 45060, 512))
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES + ((8192, 14336, 4096), (2861, 11008, 2048)))
+def test_wide_tiles(M, N, K):
+    for dtype in (_lib.FLOAT16, _lib.BFLOAT16):
+        rc, plan = _lib.fp_qqmm_plan(M, N, K, _lib.MXFP8, dtype)
+        assert rc == _lib.OK and plan == "fp_quantize_activations+qq_mfma(e4m3)", plan
+
+
+# one round either way; K ranges fill the chip; a short K, results stored by the element
+@pytest.mark.parametrize("M,N,K", ((512, 14336, 4096), (1024, 4096, 14336), (5083, 4096, 256),
+                                   (3920, 4099, 1024), (2650, 6002, 768), (5285, 4099, 256)))
+def test_narrow_tiles(M, N, K):
+    rc, plan = _lib.fp_qqmm_plan(M, N, K, _lib.MXFP8, _lib.BFLOAT16)
+    assert rc == _lib.OK and "qq_mfma(e4m3,bn=128)" in plan, plan
 
 
 @pytest.mark.gpu

@@ -150,17 +150,21 @@ struct Scratch {
   // Optional: the caller's transposed image of scales and biases
   // (mlxrocm_qmm_sb_image); the prefill path then skips its pre-pass.
   const void* sb_image = nullptr;
-  // Is there room for `wanted` bytes?  For plans that are an alternative to one with less
-  // scratch: workspace_size counts them, a caller with less runs the other one.
+  // In a dry run: what the call is going to have (the entry point with built-in scratch).
+  size_t most = SIZE_MAX;
+  // For plans that are an alternative to one with less scratch: workspace_size counts
+  // them, a caller with less runs the other one.
+  size_t room() const {
+    return dry ? most : (base != nullptr ? bytes : 0);
+  }
   bool affords(size_t wanted) const {
-    return dry || (base != nullptr && bytes >= wanted);
+    return room() >= wanted;
   }
 };
 
 constexpr size_t kScratchAlign = 256;
 
-// Scratch of mlxrocm_qmm_static, which takes the plan of mlxrocm_qmm: a plan that is an
-// alternative to one with less scratch wants no more than this.
+// Scratch of mlxrocm_qmm_static.
 constexpr size_t kStaticScratchBytes = size_t(64) << 20;
 
 int claim(Scratch& sc, size_t bytes, void** out) {
@@ -200,20 +204,47 @@ size_t plane_bytes(const QmmArgs& a, int k_splits) {
   return k_split_plane(a.M, a.N) * k_splits * sizeof(float);
 }
 
-// Shapes whose planes are padded.  They are split like all others, but only where
-// scratch allows: the plan without planes is there for a caller that has none.
+// Shapes whose planes are padded.  They are split like all others, but the plan without
+// planes is there for a caller with next to no scratch, and one whose scratch is short of
+// the planes (mlxrocm_qmm_static) takes the rows of x in blocks: the same ranges, and so
+// the same bits.
 bool ragged(const QmmArgs& a) {
   return a.N % 4 != 0;
 }
 
-// K ranges of a ragged shape: `splits`, or as many of them as leave room for the `rest`
-// of the scratch in mlxrocm_qmm_static's.
-int ragged_splits(const QmmArgs& a, int splits, size_t rest) {
-  if (rest > kStaticScratchBytes) { // (refused there whatever the plan)
-    return splits;
+// Rows of x whose scratch, `fixed` bytes and `row` for each, there is room for: all, or for
+// ragged shapes whole 32s of them in up to eight blocks (0: fewer than that).
+int rows_with_room(const QmmArgs& a, size_t fixed, size_t row, const Scratch& sc) {
+  if (!ragged(a) || sc.affords(fixed + row * a.M)) {
+    return a.M;
   }
-  const size_t most = (kStaticScratchBytes - rest) / plane_bytes(a, 1);
-  return most < static_cast<size_t>(splits) ? static_cast<int>(most) : splits;
+  const size_t rows = sc.room() > fixed ? (sc.room() - fixed) / row / 32 * 32 : 0;
+  return rows * 8 >= static_cast<size_t>(a.M) ? static_cast<int>(rows) : 0;
+}
+
+// Planes of the K ranges of `a`, `rows` rows at a time, and their sum: launch(part) with
+// part.out at the planes.
+template <typename F>
+int by_row_blocks(
+    const QmmArgs& a, int rows, int dtype, int k_splits, void* planes, hipStream_t s, F&& launch) {
+  const size_t esize = dtype_size(dtype);
+  for (int m0 = 0; m0 < a.M; m0 += rows) {
+    QmmArgs part = a;
+    part.M = a.M - m0 < rows ? a.M - m0 : rows;
+    part.x = static_cast<const char*>(a.x) + static_cast<size_t>(m0) * a.K * esize;
+    part.out = planes;
+    int rc = launch(part);
+    if (rc != MLXROCM_OK) {
+      return rc;
+    }
+    rc = reduce_k_splits(
+        planes, static_cast<char*>(a.out) + static_cast<size_t>(m0) * a.N * esize, part.M, a.N,
+        k_splits, dtype, s);
+    if (rc != MLXROCM_OK) {
+      return rc;
+    }
+  }
+  return MLXROCM_OK;
 }
 
 int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t s) {
@@ -234,21 +265,25 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
   if (rows_per_block == a.M && a.L == 1) {
     k_splits = qmm_mfma_k_splits(a.M, a.N, a.K, 1, kSplitFp32Width);
   }
-  const size_t x_bytes = (split_x_bytes(rows_per_block, a.K) + 255) / 256 * 256;
   // scales / biases transposed to [K / group][N], as for the 16-bit prefill
   const int G = a.K / gs;
   const int sb_batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool sb_t = a.M >= kTransposeSbMinM;
   const size_t sb_bytes = sb_t ? qmm_n_sb_bytes(a.N, G, sb_batches, MLXROCM_FLOAT32) : 0;
-  if (ragged(a) && k_splits > 1) {
-    k_splits = ragged_splits(a, k_splits, x_bytes + sb_bytes + 255); // (planes are rounded up)
+  auto x_of = [&](int rows) { return (split_x_bytes(rows, a.K) + 255) / 256 * 256; };
+  auto partial_of = [&](int rows) {
+    return (k_split_plane(rows, a.N) * k_splits * sizeof(float) + 255) / 256 * 256;
+  };
+  if (k_splits > 1 && ragged(a) && !sc.affords(x_of(a.M) + partial_of(a.M) + sb_bytes)) {
+    const size_t row = row_bytes + plane_bytes(a, k_splits) / a.M;
+    const int rows = sc.affords(x_of(a.M) + sb_bytes)
+        ? rows_with_room(a, sb_bytes + 2 * 255, row, sc) // (both are rounded up)
+        : 0;
+    k_splits = rows > 0 ? k_splits : 1;
+    rows_per_block = rows > 0 ? rows : rows_per_block;
   }
-  size_t partial_bytes =
-      k_splits > 1 ? (plane_bytes(a, k_splits) + 255) / 256 * 256 : 0;
-  if (ragged(a) && !sc.affords(x_bytes + partial_bytes + sb_bytes)) {
-    k_splits = 1;
-    partial_bytes = 0;
-  }
+  const size_t x_bytes = x_of(rows_per_block);
+  const size_t partial_bytes = k_splits > 1 ? partial_of(rows_per_block) : 0;
   void* region = nullptr;
   int rc = claim(sc, x_bytes + partial_bytes + sb_bytes, &region);
   if (rc != MLXROCM_OK || sc.dry) {
@@ -296,7 +331,7 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
         return rc;
       }
       if (k_splits > 1) {
-        rc = reduce_k_splits(partial, out, a.M, a.N, k_splits, MLXROCM_FLOAT32, s);
+        rc = reduce_k_splits(partial, out, rows, a.N, k_splits, MLXROCM_FLOAT32, s);
         if (rc != MLXROCM_OK) {
           return rc;
         }
@@ -309,18 +344,16 @@ int run_split_fp32(const QmmArgs& a, int gs, int bits, Scratch& sc, hipStream_t 
 // 16-bit prefill whose tiles would leave most compute units idle: K is cut into
 // ranges, the fp32 partial tiles go to the workspace and are added up.
 int run_k_split(const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scratch& sc, hipStream_t s) {
+  const size_t row = plane_bytes(a, k_splits) / a.M;
+  const int rows = rows_with_room(a, 0, row, sc);
   void* region = nullptr;
-  int rc = claim(sc, plane_bytes(a, k_splits), &region);
+  int rc = claim(sc, row * rows, &region);
   if (rc != MLXROCM_OK || sc.dry) {
     return rc;
   }
-  QmmArgs part = a;
-  part.out = region;
-  rc = launch_qmm_mfma_ksplit(part, gs, bits, dtype, k_splits, s);
-  if (rc != MLXROCM_OK) {
-    return rc;
-  }
-  return reduce_k_splits(region, a.out, a.M, a.N, k_splits, dtype, s);
+  return by_row_blocks(a, rows, dtype, k_splits, region, s, [&](const QmmArgs& part) {
+    return launch_qmm_mfma_ksplit(part, gs, bits, dtype, k_splits, s);
+  });
 }
 
 // Bytes of the image of scales and biases that a prefill call makes (run_qmm_t_transposed_sb).
@@ -371,7 +404,9 @@ int run_qmm_t_transposed_sb(
   const int batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool prepacked = sc.sb_image != nullptr;
   const size_t sb_bytes = prepacked ? 0 : sb_image_bytes(a, gs, dtype);
-  const size_t partial_bytes = k_splits > 1 ? plane_bytes(a, k_splits) : 0;
+  const size_t row = k_splits > 1 ? plane_bytes(a, k_splits) / a.M : 0;
+  const int rows = k_splits > 1 ? rows_with_room(a, sb_bytes, row, sc) : a.M;
+  const size_t partial_bytes = row * rows;
   void* region = nullptr;
   int rc = MLXROCM_OK;
   if (sb_bytes + partial_bytes != 0) {
@@ -399,13 +434,11 @@ int run_qmm_t_transposed_sb(
   if (k_splits <= 1) {
     return launch_qmm_mfma_pairs(part, gs, bits, dtype, s);
   }
-  void* partial = static_cast<char*>(region) + sb_bytes;
-  part.out = partial;
-  rc = launch_qmm_mfma_ksplit_pairs(part, gs, bits, dtype, k_splits, s);
-  if (rc != MLXROCM_OK) {
-    return rc;
-  }
-  return reduce_k_splits(partial, a.out, a.M, a.N, k_splits, dtype, s);
+  return by_row_blocks(
+      part, rows, dtype, k_splits, static_cast<char*>(region) + sb_bytes, s,
+      [&](const QmmArgs& block) {
+        return launch_qmm_mfma_ksplit_pairs(block, gs, bits, dtype, k_splits, s);
+      });
 }
 
 // transpose=false on the matrix cores.  The column loader wants the four
@@ -624,11 +657,10 @@ int tile_k_splits(const Call& c) {
     return 1;
   }
   const int splits = qmm_mfma_k_splits(c.a.M, c.a.N, c.a.K, c.a.L);
-  if (ragged(c.a) && splits > 1) {
-    const size_t sb = c.a.M >= kTransposeSbMinM ? sb_image_bytes(c.a, c.gs, c.dtype) : 0;
-    const int room = ragged_splits(c.a, splits, sb);
-    const size_t own = c.sc.sb_image == nullptr ? sb : 0;
-    return room > 1 && c.sc.affords(own + plane_bytes(c.a, room)) ? room : 1;
+  if (splits > 1) {
+    const bool image = c.a.M >= kTransposeSbMinM && c.sc.sb_image == nullptr;
+    const size_t sb = image ? sb_image_bytes(c.a, c.gs, c.dtype) : 0;
+    return rows_with_room(c.a, sb, plane_bytes(c.a, splits) / c.a.M, c.sc) > 0 ? splits : 1;
   }
   return splits;
 }
@@ -1250,6 +1282,32 @@ int qmm_entry(
   return run(a, group_size, bits, dtype, transpose != 0, sc, s);
 }
 
+// Scratch of a call that is going to have `most` of it; 0 for a call that is refused.
+size_t workspace_need(
+    int M,
+    int N,
+    int K,
+    int L,
+    int batched_weights,
+    int group_size,
+    int bits,
+    int dtype,
+    int transpose,
+    size_t most) {
+  Scratch sc;
+  sc.dry = true;
+  sc.most = most;
+  // the strides only say "one weight for every batch entry" or "one each"
+  const int64_t w_stride = batched_weights ? 4096 : 0;
+  const int64_t x_stride = static_cast<int64_t>(M) * K;
+  if (qmm_entry(
+          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
+          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
+    return 0;
+  }
+  return sc.need;
+}
+
 } // namespace
 
 extern "C" size_t mlxrocm_qmm_workspace_size(
@@ -1262,17 +1320,8 @@ extern "C" size_t mlxrocm_qmm_workspace_size(
     int bits,
     int dtype,
     int transpose) {
-  Scratch sc;
-  sc.dry = true;
-  // the strides only say "one weight for every batch entry" or "one each"
-  const int64_t w_stride = batched_weights ? 4096 : 0;
-  const int64_t x_stride = static_cast<int64_t>(M) * K;
-  if (qmm_entry(
-          nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, L, x_stride, w_stride,
-          w_stride, group_size, bits, dtype, transpose, sc, nullptr) != MLXROCM_OK) {
-    return 0;
-  }
-  return sc.need;
+  return workspace_need(
+      M, N, K, L, batched_weights, group_size, bits, dtype, transpose, SIZE_MAX);
 }
 
 extern "C" int mlxrocm_qmm(
@@ -1533,8 +1582,9 @@ extern "C" int mlxrocm_qmm_static(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  const size_t need = mlxrocm_qmm_workspace_size(
-      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose);
+  const size_t need = workspace_need(
+      M, N, K, L, w_batch_stride != 0 || sb_batch_stride != 0, group_size, bits, dtype, transpose,
+      kStaticScratchBytes);
   if (need > kStaticScratchBytes) {
     return fail(
         MLXROCM_UNSUPPORTED,

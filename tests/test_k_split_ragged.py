@@ -93,7 +93,12 @@ def test_built_in_scratch_takes_the_same_plan(dtype):
                 rc, plan = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=need)
                 assert rc == _lib.OK
                 rc, built_in = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=64 << 20)
-                assert built_in == plan if rc == _lib.OK else need > 64 << 20, (M, N, K, plan)
+                # (the same kernels and ranges, with less scratch for some rows of x at a time)
+                if rc == _lib.OK:
+                    assert set(built_in.split("+")) == set(plan.split("+")), (M, N, K, built_in)
+                    assert built_in == plan or need > 64 << 20
+                else:
+                    assert need > 64 << 20
 
 
 # (M, N, K), both modes of qqmm's own kernel and, at K % 128 != 0 or in nvfp4, the others
@@ -139,12 +144,12 @@ def test_qqmm_with_and_without_planes(gpu, M, N, K, mode):
 
 
 @pytest.mark.gpu
-def test_built_in_scratch_takes_what_it_took(gpu):
-    """mlxrocm_qmm_static plans within its 64 MiB: here two K ranges, where three fill the
-    compute units."""
+@pytest.mark.parametrize("M,N,K", ((255, 14333, 18944), (600, 2735, 14336)))
+def test_built_in_scratch_takes_what_it_took(gpu, M, N, K):
+    """mlxrocm_qmm_static plans within its 64 MiB: the rows of x in blocks, where planes for
+    all of them do not fit beside the split x."""
     lib = _lib.load()
-    M, N, K = 255, 14333, 18944
-    assert lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.FLOAT32, 1) <= 64 << 20
+    assert lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.FLOAT32, 1) > 64 << 20
     g = torch.Generator(device="cuda").manual_seed(0)
     x = torch.randn((M, K), generator=g, device="cuda")
     wq, s, b = mlx_amd.quantize(torch.randn((N, K), generator=g, device="cuda") * K ** -0.5)

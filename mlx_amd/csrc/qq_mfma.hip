@@ -632,14 +632,14 @@ struct QqPlan {
 // 8192 rows 29 against 32; 32000 x 4096, 128 / 300 rows 36 / 73 against 50 / 64.
 // Over a short K what a tile takes beside its steps decides: filling two stages, and, from
 // the second round on, results stored by the element (N no multiple of four), twice as many
-// to a tile.  256 x 256 against 256 x 128: 3920 x 4099 x 1024 67 against 56, 5285 x 4099 x 256
+// to a tile (not seen over 2048 codes: 5530 x 6002 x 4096 211 against 225).  256 x 256 against 256 x 128: 3920 x 4099 x 1024 67 against 56, 5285 x 4099 x 256
 // 63 against 55, 5083 x 4096 x 256 34 against 31; ahead in one round (1501 x 6002 x 256: 32
 // against 37) and at 3067 x 14336 x 256 (11 %).
 constexpr double kWideStep8 = 1560.0;
 double wide8_ns(long rounds, long steps, int N) {
   const double k = static_cast<double>(steps);
   const double ns = static_cast<double>(rounds) * (k * kWideStep8 + 4250.0 + 3000.0 / k);
-  return N % 4 == 0 ? ns : ns + static_cast<double>(rounds - 1) * 4000.0;
+  return N % 4 == 0 || steps > 16 ? ns : ns + static_cast<double>(rounds - 1) * 4000.0;
 }
 QqPlan qq_plan(int M, int N, int K, int mode, bool planes = true) {
   const long cus = compute_units();

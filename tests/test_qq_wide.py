@@ -12,7 +12,7 @@ SHAPES = ((4111, 2503, 128), (4096, 2560, 256), (2049, 3841, 384), (300, 32001, 
           (257, 18002, 1152), (513, 45060, 512))
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES + ((8192, 14336, 4096), (2861, 11008, 2048)))
+@pytest.mark.parametrize("M,N,K", SHAPES + ((8192, 14336, 4096), (2861, 11008, 2048), (5530, 6002, 4096)))
 def test_wide_tiles(M, N, K):
     for dtype in (_lib.FLOAT16, _lib.BFLOAT16):
         rc, plan = _lib.fp_qqmm_plan(M, N, K, _lib.MXFP8, dtype)

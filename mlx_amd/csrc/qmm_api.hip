@@ -373,7 +373,7 @@ size_t mid_bytes(const QmmArgs& a, int gs, int dtype, const MidPlan& pl, const S
 
 // Rows of x that are few for 256-row tiles (qmm_mid.h).
 int run_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipStream_t s) {
-  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, bits);
+  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, gs, bits);
   const size_t need = mid_bytes(a, gs, dtype, pl, sc);
   void* region = nullptr;
   int rc = need != 0 ? claim(sc, need, &region) : static_cast<int>(MLXROCM_OK);
@@ -670,15 +670,17 @@ bool tile_t(const Call& c) {
 }
 
 // Where the tiles of up to 128 rows (qmm_mid.h) are ahead of those of 256: up to 256 rows,
-// more where K is short, while one round of workgroups holds them.  us per call against the
-// tile kernel, bf16 4-bit g64, 66 / 128 / 256 rows: 4096 x 4096 16.3 / 20.3 / 22.3 against
-// 21.8 / 23.6 / 29.5; 4096 x 14336 25.3 / 29.2 / 44.2 against 36.1 / 39.0 / 50.6;
-// 14336 x 4096 25.7 / 30.4 / 41.9 against 30.0 / 33.6 / 46.9; 32000 x 4096 66 / 128 rows 39.7 / 44.0
-// against 51.8 / 52.6; 2048 x 2048, 256 / 2048 rows 16.0 / 27.4
-// against 24.2 / 39.3.  It is behind in a second round (18944 x 3584, 192 rows: 63 against
-// 45; 32000 x 4096, 192 rows: 76 against 66) and over a long K with more rows, where codes
-// dequantized once for 256 rows are dearer to do again for each 128 (4096 x 14336, 512
-// rows: 77.5 against 71.5).  Up to 64 rows other kernels are ahead of both.
+// more where K is short, while one round of workgroups holds them and by the accounts of
+// both kernels.  us per call against the tile kernel, bf16 4-bit g64, 66 / 128 / 256 rows:
+// 4096 x 4096 16.3 / 20.3 / 22.3 against 21.8 / 23.6 / 29.5; 4096 x 14336 25.3 / 29.2 / 44.2
+// against 36.1 / 39.0 / 50.6; 2048 x 2048, 256 / 2048 rows 16.0 / 27.4 against 24.2 / 39.3.
+// Codes that are dearer to unpack, or three tiles of 96 rows at 8 bits, leave less: 4096 x
+// 14336, 193 rows 8-bit g32 73 against 50; 11008 x 4096, 129 rows 6-bit 52 against 36.  Without
+// the accounts 24 % of 5700 random calls were behind the tile kernel by more than 2 %, the
+// worst by 54 %; with them 1.7 % of 11800, the worst by 15 %.  It is behind in a second round (18944 x 3584, 192
+// rows: 63 against 45) and over a long K with more rows, where codes dequantized once for
+// 256 rows are dearer to do again for each 128 (4096 x 14336, 512 rows: 77.5 against 71.5).
+// Up to 64 rows other kernels are ahead of both.
 constexpr int kMidMinM = 65;
 constexpr int kMidMaxM = 256;
 constexpr int kMidMaxMShortK = 2048;
@@ -689,11 +691,11 @@ bool mid_pays(const Call& c) {
       !qmm_mid_supported(a, c.gs, c.bits, c.dtype, c.transpose)) {
     return false;
   }
-  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, c.bits);
+  const MidPlan pl = qmm_mid_plan(a.M, a.N, a.K, c.gs, c.bits);
   // (a caller with less scratch has what it had before)
   const size_t need = mid_bytes(a, c.gs, c.dtype, pl, c.sc);
-  return pl.groups <= compute_units() && plane_bytes(a, pl.splits) <= kStaticScratchBytes / 2 &&
-      (need == 0 || c.sc.affords(need));
+  return pl.groups <= compute_units() && pl.us < qmm_mfma_us(a.M, a.N, a.K, c.bits) &&
+      plane_bytes(a, pl.splits) <= kStaticScratchBytes / 2 && (need == 0 || c.sc.affords(need));
 }
 
 // Two passes over the same scratch, one after the other on the stream.

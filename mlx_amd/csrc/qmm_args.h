@@ -298,9 +298,18 @@ struct MidPlan {
   int tiles;  // of x
   long groups; // workgroups of one range
   int splits; // ranges of K
+  double us;  // what the call takes, by the plan's account
 };
 bool qmm_mid_supported(const QmmArgs& a, int gs, int bits, int dtype, bool transpose);
-MidPlan qmm_mid_plan(int M, int N, int K, int bits);
+MidPlan qmm_mid_plan(int M, int N, int K, int gs, int bits);
+// Groups whose scales and biases its table in LDS holds (mf: 16-row tiles of x); with more
+// in its range a workgroup starts anew.
+constexpr int mid_table_groups(int mf, int bits) {
+  return mf * bits >= 40 ? 32 : 64;
+}
+// What the 256-row tile kernel takes for the same call (transpose=true, 16-bit types, one
+// problem), us.
+double qmm_mfma_us(int M, int N, int K, int bits);
 int launch_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, const MidPlan& pl, hipStream_t s);
 int launch_qmm_mid_bf16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);
 int launch_qmm_mid_f16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);

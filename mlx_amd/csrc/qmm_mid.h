@@ -48,10 +48,7 @@ constexpr int mid_x_bytes(int mf) {
 constexpr int mid_w_bytes(int bits) {
   return kMidBN * kMidBK * bits / 8;
 }
-// groups of the table of (scale, bias) pairs in front of the stages
-constexpr int mid_table_groups(int mf, int bits) {
-  return mf * bits >= 40 ? 32 : 64;
-}
+// (the table of (scale, bias) pairs in front of the stages: mid_table_groups())
 constexpr int mid_table_bytes(int mf, int bits) {
   return mid_table_groups(mf, bits) * kMidBN * 4;
 }

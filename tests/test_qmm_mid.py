@@ -19,6 +19,23 @@ def test_rule(M, N, K, taken):
     assert rc == _lib.OK and ("qmm_mid(" in plan) == taken, plan
 
 
+# by the accounts of both kernels: three tiles of 96 rows at 8 bits and codes that are dear to
+# unpack leave the tile kernel ahead
+@pytest.mark.parametrize("bits,group,M,N,K,taken", (
+    (8, 32, 193, 4096, 14336, False), (8, 64, 224, 4096, 14336, False),
+    (8, 32, 193, 8192, 8192, False), (8, 64, 256, 8192, 8192, False),
+    (6, 128, 129, 11008, 4096, False), (6, 32, 193, 14336, 4096, False),
+    (3, 64, 129, 11008, 4096, False), (2, 32, 129, 11008, 4096, False),
+    (8, 32, 96, 4096, 4096, True), (8, 64, 256, 4096, 4096, True), (6, 64, 192, 4096, 4096, True),
+    (6, 32, 96, 4096, 14336, True), (4, 32, 128, 4096, 14336, True), (3, 32, 700, 2048, 2048, True),
+))
+def test_rule_of_every_width(bits, group, M, N, K, taken):
+    need = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, group, bits, _lib.BFLOAT16, 1)
+    rc, plan = _lib.qmm_plan(M, N, K, group_size=group, bits=bits, dtype=_lib.BFLOAT16,
+                             workspace_bytes=need)
+    assert rc == _lib.OK and ("qmm_mid(" in plan) == taken, plan
+
+
 def test_less_scratch_keeps_the_other_plan():
     M, N, K = 97, 222, 4096
     need = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, _lib.BFLOAT16, 1)

@@ -664,6 +664,18 @@ def test_qmm_prepacked_scale_image(gpu, dtype):
         plain = mlx_amd.quantized_matmul(x, wq, s, b, True, gs, 4)
         packed = mlx_amd.quantized_matmul(x, wq, s, b, True, gs, 4, sb_image=image)
         assert torch.equal(plain, packed), M
+    # (at K <= 2048 the prefill kernel reads no image; these do)
+    from mlx_amd import _lib
+    code = {torch.bfloat16: _lib.BFLOAT16, torch.float16: _lib.FLOAT16}[dtype]
+    long_w = mlx_amd.quantize(normal_weights((N, 2 * K), dtype, std=0.05).to(gpu), gs, 4)
+    long_image = mlx_amd.quantized_matmul_sb_image(*long_w[1:], gs)
+    for M in (600, 2048, 5000):
+        plan = _lib.qmm_plan(M, N, 2 * K, dtype=code, workspace_bytes=1 << 30)[1]
+        assert plan.startswith("[qmm_t_tile_sb_transposed]"), plan
+        long_x = activations((M, 2 * K), dtype).to(gpu)
+        plain = mlx_amd.quantized_matmul(long_x, *long_w, True, gs, 4)
+        packed = mlx_amd.quantized_matmul(long_x, *long_w, True, gs, 4, sb_image=long_image)
+        assert torch.equal(plain, packed), M
     with pytest.raises(ValueError):
         mlx_amd.quantized_matmul(x, wq, s, b, True, gs, 4, sb_image=image[:-8])
     # the layer keeps the image and drops it when the weights are replaced

@@ -6,9 +6,13 @@ import torch
 import mlx_amd
 from mlx_amd import _lib
 
-# N % 4 of 1, 2, 3 and 0; one and several tiles, rows past a tile, M * N odd and even
-SHAPES = ((255, 775, 4096), (66, 1001, 2048), (97, 222, 1536), (513, 803, 2048), (70, 449, 1024),
-          (130, 640, 1024))
+# N % 4 of 1, 2, 3 and 0; one and several tiles, rows past a tile, M * N odd and even; the
+# rule that the 16-bit types take in affine mode
+RULES = {(255, 775, 4096): "qmm_mid", (66, 1001, 2048): "qmm_mid", (97, 222, 1536): "qmm_mid",
+         (513, 803, 2048): "qmm_mid", (70, 449, 1024): "qmm_mid", (130, 640, 1024): "qmm_mid",
+         (300, 803, 4096): "qmm_t_tile_k_split", (265, 1002, 3520): "qmm_t_tile_k_split",
+         (600, 803, 4096): "qmm_t_tile_sb_transposed", (514, 229, 2112): "qmm_t_tile_sb_transposed"}
+SHAPES = tuple(RULES)
 FP = {"mxfp4": _lib.MXFP4, "mxfp8": _lib.MXFP8, "nvfp4": _lib.NVFP4}
 
 
@@ -18,6 +22,8 @@ def test_split_with_scratch_and_plain_without(M, N, K, dtype):
     need = _lib.load().mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, dtype, 1)
     rc, plan = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=need)
     assert rc == _lib.OK and "reduce_k_splits" in plan, plan
+    rule = RULES[M, N, K] if dtype != _lib.FLOAT32 else "qmm_t_split_fp32"
+    assert plan.startswith(f"[{rule}]"), plan
     if N % 4 and dtype != _lib.FLOAT32 and M < 512:  # (these took no workspace before)
         rc, plan = _lib.qmm_plan(M, N, K, dtype=dtype, workspace_bytes=0)
         assert rc == _lib.OK and "reduce_k_splits" not in plan, plan
@@ -141,6 +147,28 @@ def test_qqmm_with_and_without_planes(gpu, M, N, K, mode):
     want = mlx_amd.qqmm(x, wq, s, mode=mode)
     # the same products in another order: an ulp of some results
     assert float((y.double() - want.double()).norm() / want.double().norm()) < 2.0 ** -9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", ((300, 803, 4096), (265, 1002, 3520), (600, 803, 4096)))
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+def test_scratch_for_some_rows_gives_the_same_bits(gpu, M, N, K, dtype):
+    lib = _lib.load()
+    code = {torch.float32: _lib.FLOAT32, torch.bfloat16: _lib.BFLOAT16}[dtype]
+    x = torch.randn((M, K), device="cuda").to(dtype)
+    wq, s, b = mlx_amd.quantize((torch.randn((N, K), device="cuda") / 64).to(dtype))
+    want = mlx_amd.quantized_matmul(x, wq, s, b)
+    need = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, 4, code, 1)
+    for room in (need * 7 // 8, need * 2 // 3):
+        plan = _lib.qmm_plan(M, N, K, dtype=code, workspace_bytes=room)[1]
+        assert plan.count("reduce_k_splits") > 1, plan
+        ws = torch.empty(room, dtype=torch.uint8, device="cuda")
+        y = torch.full((M, N), -1.0, dtype=dtype, device="cuda")
+        _lib.check(lib.mlxrocm_qmm(
+            x.data_ptr(), wq.data_ptr(), s.data_ptr(), b.data_ptr(), y.data_ptr(), M, N, K, 1,
+            M * K, 0, 0, 64, 4, code, 1, ws.data_ptr(), room,
+            torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(y, want)
 
 
 @pytest.mark.gpu

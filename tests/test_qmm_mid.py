@@ -137,3 +137,13 @@ def test_replays_and_streams(gpu):
                 got.append(mlx_amd.quantized_matmul(x, *q))
     torch.cuda.synchronize()
     assert all(torch.equal(y, want) for y in got)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = mlx_amd.quantized_matmul(x, *q)
+    for i in range(4):
+        x.copy_(torch.randn((100, 4096), device="cuda"))
+        want = mlx_amd.quantized_matmul(x, *q)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), i

@@ -315,17 +315,8 @@ __global__ __launch_bounds__(256) void reduce_k_splits_kernel(
     acc.z += v.z;
     acc.w += v.w;
   }
-  size_t at = piece * 4;
-  int n = 0;
-  if ((N & 3) != 0) {
-    const uint32_t row_pieces = static_cast<uint32_t>(k_split_row(N)) / 4;
-    const uint32_t m = static_cast<uint32_t>(piece) / row_pieces; // (the launcher checks the size)
-    n = static_cast<int>(static_cast<uint32_t>(piece) - m * row_pieces) * 4;
-    at = static_cast<size_t>(m) * N + n;
-  }
-  TO* y = out + at;
-  if (n + 4 <= N) {
-    // (one store, wherever an element may start)
+  // (one store, wherever an element may start)
+  auto store = [&](TO* y) {
     if constexpr (sizeof(TO) == 4) {
       typedef float __attribute__((ext_vector_type(4), aligned(4))) four;
       *reinterpret_cast<four*>(y) = four{acc.x, acc.y, acc.z, acc.w};
@@ -333,6 +324,17 @@ __global__ __launch_bounds__(256) void reduce_k_splits_kernel(
       typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) four;
       *reinterpret_cast<four*>(y) = four{pack2<TO>(acc.x, acc.y), pack2<TO>(acc.z, acc.w)};
     }
+  };
+  if ((N & 3) == 0) {
+    store(out + piece * 4);
+    return;
+  }
+  const uint32_t row_pieces = static_cast<uint32_t>(k_split_row(N)) / 4;
+  const uint32_t m = static_cast<uint32_t>(piece) / row_pieces; // (the launcher checks the size)
+  const int n = static_cast<int>(static_cast<uint32_t>(piece) - m * row_pieces) * 4;
+  TO* y = out + static_cast<size_t>(m) * N + n;
+  if (n + 4 <= N) {
+    store(y);
     return;
   }
   const float v[3] = {acc.x, acc.y, acc.z};

@@ -750,7 +750,7 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
         const size_t orow =
             GROUPED ? static_cast<size_t>(a.group_perm[row0 + mr]) : static_cast<size_t>(m);
         TO* dst = p.out + orow * ldy + n;
-        if (vec_ok && n + kPiece <= N) {
+        if (vec_ok) { // (below N whole pieces fit: N or the planes' rows are made of them)
           *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
         } else {
           for (int e = 0; e < kPiece && n + e < N; ++e) {

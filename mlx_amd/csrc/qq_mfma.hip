@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     TO* out = static_cast<TO*>(a.out) + (kPlanes ? blockIdx.z * k_split_plane(M, N) : 0);
     const int col = lane & 31;
     const int half = lane >> 5;
-    const bool vec_ok = (ldy % 4) == 0;
+    const bool vec_ok = (ldy % 4) == 0; // (n is a multiple of four: below N whole fours fit)
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       const int m = m0 + wm * 16 * MI + 32 * j + col;
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
           const float v0 = acc[i][j][4 * g4 + 0], v1 = acc[i][j][4 * g4 + 1];
           const float v2 = acc[i][j][4 * g4 + 2], v3 = acc[i][j][4 * g4 + 3];
           TO* dst = out + static_cast<size_t>(m) * ldy + n;
-          if (vec_ok && n + 4 <= N) {
+          if (vec_ok) {
             if constexpr (sizeof(TO) == 4) {
               *reinterpret_cast<float4*>(dst) = make_float4(v0, v1, v2, v3);
             } else {
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
   TO* out = static_cast<TO*>(a.out) + (kPlanes ? blockIdx.z * k_split_plane(M, N) : 0);
   const int col = lane & 15;
   const int quad = lane >> 4;
-  const bool vec_ok = (ldy % 4) == 0;
+  const bool vec_ok = (ldy % 4) == 0; // (n is a multiple of four: below N whole fours fit)
 #pragma unroll
   for (int j = 0; j < MI; ++j) {
     const int m = m0 + wm * 16 * MI + 16 * j + col;
@@ -557,7 +557,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
         continue;
       }
       TO* dst = out + static_cast<size_t>(m) * ldy + n;
-      if (vec_ok && n + 4 <= N) {
+      if (vec_ok) {
         if constexpr (sizeof(TO) == 4) {
           *reinterpret_cast<float4*>(dst) =
               make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);

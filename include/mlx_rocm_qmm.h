@@ -246,7 +246,8 @@ int mlxrocm_fp_qmm_rows(
  * same real products, summed exactly for e2m1 codes and with about 17 bits
  * below the largest product of a 128-code step for e4m3 codes; otherwise x is
  * quantized and dequantized in dtype and takes the kernels of mlxrocm_fp_qmm.  workspace: mlxrocm_fp_qqmm_workspace_size bytes,
- * 256-byte aligned, used only during the call.
+ * 256-byte aligned, used only during the call (with N no multiple of four the fp32
+ * planes of K ranges may be missing from it).
  */
 size_t mlxrocm_fp_qqmm_workspace_size(int M, int N, int K, int mode, int dtype);
 int mlxrocm_fp_qqmm(
@@ -512,7 +513,9 @@ int mlxrocm_gguf_repack(
  * rows take the same path 32 rows at a time and need what 32 rows need).  Calls with one to
  * four rows of x and transpose != 0 never use one.  The call only enqueues work: it allocates
  * nothing, takes no lock and does not synchronize, so it can be captured in a
- * HIP graph.  A workspace that is too small is MLXROCM_INVALID_ARGUMENT.
+ * HIP graph.  A workspace that is too small is MLXROCM_INVALID_ARGUMENT; calls
+ * that only go faster with all of it (65..2048 rows of x where tiles are few, N
+ * no multiple of four) take another plan with less.
  */
 size_t mlxrocm_qmm_workspace_size(
     int M,
@@ -637,7 +640,8 @@ int mlxrocm_qmm_prepacked(
  * loops, harnesses that forbid hipMalloc).  It has no counterpart in the
  * reference.  The scratch the shapes listed above need comes from a 64 MiB
  * array inside the library's device image (one copy per GPU, held until the
- * process ends); a shape that needs more is refused with MLXROCM_UNSUPPORTED.
+ * process ends); a shape that needs more is refused with MLXROCM_UNSUPPORTED
+ * (with N no multiple of four, rows of x are taken in blocks where that fits).
  * The first call on a device looks the array's address up (no allocation; do
  * it once outside a graph capture -- an empty call, M == 0, is enough).  All
  * calls on one GPU share the array: calls that may overlap in time (different

@@ -574,8 +574,9 @@ int run_widened(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipS
 // ---------------------------------------------------------------------------
 // Kernel choice.  One call of the dispatcher is a `Call`; the table below is
 // walked top to bottom and the first rule whose predicate holds runs.  A
-// predicate reads the problem only (never the scratch), so a sizing run, a
-// rehearsal and the real call take the same rule.  Every threshold is a
+// predicate reads the problem, and of the scratch only whether it holds what the
+// rule would claim (qmm_mid, ragged K ranges), so a sizing run, a rehearsal and a
+// call with the scratch that the sizing run names take the same rule.  Every threshold is a
 // measurement on the 256-CU part; the rule's `evidence` string carries the
 // figures (microseconds per launch unless stated; "A against B" = this rule
 // against the rules below it).
@@ -969,9 +970,10 @@ const Rule kRules[] = {
     {"qmm_mid",
      [](const Call& c) { return tile_t(c) && mid_pays(c); },
      [](const Call& c) { return run_qmm_mid(c.a, c.gs, c.bits, c.dtype, c.sc, c.s); },
-     "65..256 rows (..2048 at K <= 2048) in one round of 128 x 128 tiles: packed W and x both "
-     "by direct-to-LDS loads two or more K-steps of 128 ahead, W dequantized in registers. "
-     "4096x14336, 96 rows: 26.6 against 37.2 (tile kernel); 1024x1024, 512 rows: 13.5 against 23.8"},
+     "65..256 rows (..2048 at K <= 2048) in one round of 128 x 128 tiles, where the accounts of "
+     "both kernels say so: packed W and x both by direct-to-LDS loads two or more K-steps of 128 "
+     "ahead, W dequantized in registers. 4096x14336, 96 rows: 27.9 against 38.0 (tile kernel); "
+     "1024x1024, 512 rows: 14.1 against 23.7. Not 8-bit g32 4096x14336, 193 rows (73 against 50)"},
     {"qmm_t_tile_sb_transposed",
      [](const Call& c) {
        return tile_t(c) && c.a.lhs_indices == nullptr && c.a.M >= kTransposeSbMinM;
@@ -988,9 +990,9 @@ const Rule kRules[] = {
      [](const Call& c) {
        return run_k_split(c.a, c.gs, c.bits, c.dtype, tile_k_splits(c), c.sc, c.s);
      },
-     "few tiles: K cut into up to 16 ranges of at least 8 steps, fp32 planes + reduction. "
-     "M=512, N=4096: 75 -> 43; K=14336: 249 -> 92; 3584x18944, 128 rows: 45.6 (16 ranges) "
-     "against 57.5 (8); odd N (padded planes) 775x4096, 255 rows: 79 -> 28"},
+     "fewer than 512 rows, few tiles: K cut into up to 16 ranges of at least 8 steps, fp32 planes "
+     "+ reduction. Against no ranges: 803x4096, 391 rows 3-bit 83 -> 31; 6002x8192, 471 rows "
+     "4-bit 146 -> 74; 2735x8192, 307 rows 8-bit 158 -> 43 (odd N: padded planes)"},
     {"qmm_t_tile",
      [](const Call& c) { return tile_t(c); },
      [](const Call& c) {

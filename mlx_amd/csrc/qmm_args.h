@@ -222,7 +222,7 @@ size_t split_x_bytes(size_t rows, int K);
 int split_x_for_mfma(const void* x, void* xs, size_t rows, int K, hipStream_t s);
 int launch_qmm_mfma_split(const QmmArgs& a, int gs, int bits, hipStream_t s, int k_splits);
 // Few tiles: K is cut into qmm_mfma_k_splits() ranges whose fp32 partial tiles
-// (k_splits planes of M x N behind a.out) reduce_k_splits() adds up.
+// (k_splits planes of k_split_plane(M, N) elements behind a.out) reduce_k_splits() adds up.
 int qmm_mfma_k_splits(int M, int N, int K, int L, int nt = 7);
 // Elements of a row of such a plane and of a plane: rows start at 16 bytes.
 __host__ __device__ inline int k_split_row(int N) {

@@ -266,7 +266,7 @@ double qmm_mfma_us(int M, int N, int K, int bits) {
 }
 
 // 16-bit operands with K cut into k_splits ranges: `a.out` points at k_splits
-// fp32 planes of M x N (reduce_k_splits adds them up into y).
+// fp32 planes (k_split_plane(); reduce_k_splits adds them up into y).
 int launch_qmm_mfma_ksplit(
     const QmmArgs& a,
     int gs,

@@ -172,8 +172,8 @@ int fp_scale_image_for_qmm_t(
 }
 
 // a.scales: the image above (a.sb_transposed == 2); K % 64 == 0.  k_splits > 1:
-// K is cut into that many ranges and a.out points at as many fp32 planes of
-// M x N, which reduce_k_splits adds up.
+// K is cut into that many ranges and a.out points at as many fp32 planes
+// (k_split_plane()), which reduce_k_splits adds up.
 int launch_qmm_mfma_fp(const QmmArgs& a, int mode, int dtype, int k_splits, hipStream_t s) {
   if (k_splits > 1) {
     constexpr int kNT = 7;

@@ -159,7 +159,7 @@ int launch_qmm_mfma_pairs(const QmmArgs& a, int gs, int bits, int dtype, hipStre
   return dtype == MLXROCM_BFLOAT16 ? run(bf16_t{}) : run(f16_t{});
 }
 
-// K cut into k_splits ranges: `a.out` points at k_splits fp32 planes of M x N.
+// K cut into k_splits ranges: `a.out` points at k_splits fp32 planes (k_split_plane()).
 int launch_qmm_mfma_ksplit_pairs(
     const QmmArgs& a, int gs, int bits, int dtype, int k_splits, hipStream_t s) {
   constexpr int kNT = 7;

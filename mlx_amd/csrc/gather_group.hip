@@ -13,7 +13,7 @@
 //            rows are zero-filled here;
 //   plan     one workgroup: exclusive scan of the counts -> first sorted
 //            position of every expert, and the list of tiles {expert, first
-//            position, rows} of up to tile_rows rows (256 for the tile GEMM, 32
+//            position, rows} of up to tile_rows rows (256 for the tile GEMMs, 32
 //            for the few-row kernel when the groups are small); the tile count
 //            stays on the device;
 //   scatter  perm[position] = pair: rank inside the workgroup from an LDS
@@ -64,6 +64,70 @@ __global__ __launch_bounds__(256) void group_count_kernel(
   }
 }
 
+// First sorted position of every expert and the list of tiles from the counts in LDS, by all
+// threads of the workgroup.  256-row tiles that are full come first, the others behind them by
+// eighths of their height, highest first: qmm_own_kernel deals tiles out in the order of the
+// list and multiplies as many rows as a tile has, so its time ends with the workgroup that got
+// most rows.  Tiles of 32 rows stay in the order of their experts.
+constexpr int kHeights = 8;
+__device__ __forceinline__ void plan_tiles(
+    int n_experts,
+    int tile_rows, // a power of two
+    const int32_t* cnt,
+    int32_t* first_pos,
+    int32_t* first_tile,
+    int32_t* offsets,
+    int32_t* tiles,
+    int32_t* n_tiles) {
+  __shared__ int32_t next[kHeights]; // of the tiles of a height: how many, then the next one
+  const bool by_height = tile_rows == kGroupLargeTile;
+  const int shift = __ffs(tile_rows) - 1;
+  auto height = [&](int rows) { return ((rows * kHeights - 1) >> shift); };
+  if (threadIdx.x < kHeights) {
+    next[threadIdx.x] = 0;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; by_height && e < n_experts; e += blockDim.x) {
+    const int rest = cnt[e] & (tile_rows - 1);
+    if (rest != 0) {
+      atomicAdd(&next[height(rest)], 1);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int pos = 0;
+    int tile = 0;
+    for (int e = 0; e < n_experts; ++e) {
+      first_pos[e] = pos;
+      first_tile[e] = tile;
+      pos += cnt[e];
+      tile += (cnt[e] + (by_height ? 0 : tile_rows - 1)) >> shift;
+    }
+    for (int h = kHeights - 1; h >= 0; --h) {
+      const int n = next[h];
+      next[h] = tile;
+      tile += n;
+    }
+    n_tiles[0] = tile;
+    n_tiles[1] = pos; // pairs with both indices in range
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) {
+    offsets[e] = first_pos[e];
+    const int c = cnt[e];
+    int t = first_tile[e];
+    for (int r = 0; r < c; r += tile_rows, ++t) {
+      const int rows = c - r < tile_rows ? c - r : tile_rows;
+      if (by_height && rows < tile_rows) {
+        t = atomicAdd(&next[height(rows)], 1); // (the expert's last)
+      }
+      tiles[3 * t + 0] = e;
+      tiles[3 * t + 1] = first_pos[e] + r;
+      tiles[3 * t + 2] = rows;
+    }
+  }
+}
+
 __global__ __launch_bounds__(256) void group_plan_kernel(
     int n_experts,
     int tile_rows,
@@ -78,29 +142,7 @@ __global__ __launch_bounds__(256) void group_plan_kernel(
     cnt[e] = counts[e];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int pos = 0;
-    int tile = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      first_pos[e] = pos;
-      first_tile[e] = tile;
-      pos += cnt[e];
-      tile += (cnt[e] + tile_rows - 1) / tile_rows;
-    }
-    n_tiles[0] = tile;
-    n_tiles[1] = pos; // pairs with both indices in range
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) {
-    offsets[e] = first_pos[e];
-    const int c = cnt[e];
-    int t = first_tile[e];
-    for (int r = 0; r < c; r += tile_rows, ++t) {
-      tiles[3 * t + 0] = e;
-      tiles[3 * t + 1] = first_pos[e] + r;
-      tiles[3 * t + 2] = (c - r < tile_rows) ? c - r : tile_rows;
-    }
-  }
+  plan_tiles(n_experts, tile_rows, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
 }
 
 __global__ __launch_bounds__(256) void group_scatter_kernel(
@@ -220,29 +262,7 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int pos = 0;
-    int tile = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      first_pos[e] = pos;
-      first_tile[e] = tile;
-      pos += cnt[e];
-      tile += (cnt[e] + tile_rows - 1) / tile_rows;
-    }
-    n_tiles[0] = tile;
-    n_tiles[1] = pos; // pairs with both indices in range
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < n_experts; e += kFusedThreads) {
-    offsets[e] = first_pos[e];
-    const int c = cnt[e];
-    int t = first_tile[e];
-    for (int r = 0; r < c; r += tile_rows, ++t) {
-      tiles[3 * t + 0] = e;
-      tiles[3 * t + 1] = first_pos[e] + r;
-      tiles[3 * t + 2] = (c - r < tile_rows) ? c - r : tile_rows;
-    }
-  }
+  plan_tiles(n_experts, tile_rows, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
   __syncthreads();
   for (int e = threadIdx.x; e < n_experts; e += kFusedThreads) {
     first_tile[e] = first_pos[e];

@@ -315,6 +315,12 @@ int launch_qmm_mid_bf16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, h
 int launch_qmm_mid_f16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);
 int reduce_k_splits(
     const void* partial, void* out, int M, int N, int k_splits, int dtype, hipStream_t s);
+// Tiles whose wavefronts own their rows of W (qmm_own.h): pair images, 16-bit types.
+bool qmm_own_experts_supported(const QmmArgs& a, int bits);
+int launch_qmm_own_experts(
+    const QmmArgs& a, int gs, int bits, int dtype, bool glu, hipStream_t s);
+int launch_qmm_own_experts_bf16(const QmmArgs& a, int gs, int bits, bool glu, hipStream_t s);
+int launch_qmm_own_experts_f16(const QmmArgs& a, int gs, int bits, bool glu, hipStream_t s);
 // expert-routed gated MLP (qmm_mfma_experts.hip): pair images, launch_gather_group's tables
 int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 int launch_qmm_mfma_experts(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);

@@ -210,7 +210,8 @@ int mlxrocm_fp_qmm(
 
 /*
  * mlxrocm_qmm_rows for the floating-point modes (2..64 rows per problem; 9..64 in
- * float16, whose range the scales could leave; K a multiple of 128).
+ * float16, whose range the scales could leave; more rows of one problem as there; K a
+ * multiple of 128).
  */
 int mlxrocm_fp_qmm_rows_supported(
     int M, int N, int K, int L, int mode, int dtype);
@@ -549,12 +550,14 @@ int mlxrocm_qmm(
     mlxrocm_stream_t stream);
 
 /*
- * mlxrocm_qmm with transpose != 0 for the rows of a decode step of some sequences
- * (3..64 rows per problem, 16-bit types, every width), on the kernel that walks x
- * through LDS: one pass over W whatever the rows, nothing rounded before the
- * result.  _supported: 1 where it takes a call and is ahead of mlxrocm_qmm, else 0;
+ * mlxrocm_qmm with transpose != 0 on the kernels that are ahead of its own, 16-bit types,
+ * every width.  3..64 rows per problem (a decode step of some sequences): the kernel
+ * that walks x through LDS, one pass over W whatever the rows, nothing rounded before the
+ * result.  More rows of one problem, K a multiple of 128: tiles whose wavefronts unpack
+ * their own rows of W (scratch: the image of mlxrocm_qmm_sb_image and the fp32 planes of K
+ * ranges).  _supported: 1 where it takes a call and is ahead of mlxrocm_qmm, else 0;
  * it looks at shapes only.  workspace: device scratch used only during the call,
- * 16-byte aligned, of _workspace_size bytes (mostly 0, and then it may be NULL).
+ * 16-byte aligned, of _workspace_size bytes (up to 64 rows mostly 0: it may be NULL then).
  */
 int mlxrocm_qmm_rows_supported(
     int M, int N, int K, int L, int group_size, int bits, int dtype);

@@ -598,6 +598,23 @@ int fp_k_splits(int M, int N, int K, int L) {
   return qmm_mfma_k_splits(M, N, K, L);
 }
 
+// More than 64 rows (mlxrocm_fp_qmm_rows): where tiles whose wavefronts own their rows of W
+// (qmm_own.h) are ahead of the tile kernel.
+bool fp_own_pays(int M, int N, int K, int L, int mode, int dtype, OwnPlan* pl) {
+  const int bits = mode == MLXROCM_MXFP8 ? 8 : 4;
+  if (!qmm_own_supported(M, N, K, L, bits, dtype) ||
+      !fp_tile_applies(M, N, K, L, mode, dtype, true)) {
+    return false;
+  }
+  *pl = qmm_own_plan(M, N, K, kOwnFpCodes + mode);
+  return qmm_own_pays(*pl, kOwnFpCodes + mode, qmm_mfma_us(M, N, K, 4));
+}
+
+size_t fp_own_bytes(int M, int N, int K, const OwnPlan& pl) {
+  return fp_image_bytes(N, K, 1) +
+      (pl.splits > 1 ? k_split_plane(M, N) * pl.splits * sizeof(float) : 0);
+}
+
 size_t fp_tile_workspace(int M, int N, int K, int L, int batches) {
   const int splits = fp_k_splits(M, N, K, L);
   const size_t planes = splits > 1 ? k_split_plane(M, N) * splits * sizeof(float) : 0;
@@ -718,7 +735,7 @@ int fp_qmm_entry(
     size_t workspace_bytes,
     mlxrocm_stream_t stream,
     const float* out_scale = nullptr,
-    bool rows = false) { // a call that fp_walk_applies() to
+    bool rows = false) { // a call that fp_walk_applies() or fp_own_pays() to
   int rc = fp_check("quantized_matmul", M, N, K, L, mode, dtype, transpose);
   if (rc != MLXROCM_OK) {
     return rc;
@@ -766,7 +783,9 @@ int fp_qmm_entry(
   a.n_experts = L;
   a.out_scale = out_scale;
   if (rows) {
-    const size_t need = qmm_walk_fp_plane_bytes(a, mode);
+    OwnPlan pl;
+    const bool own = M > 64 && fp_own_pays(M, N, K, L, mode, dtype, &pl);
+    const size_t need = own ? fp_own_bytes(M, N, K, pl) : qmm_walk_fp_plane_bytes(a, mode);
     if (need != 0 &&
         (workspace == nullptr || workspace_bytes < need ||
          (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0)) {
@@ -776,7 +795,23 @@ int fp_qmm_entry(
           "(mlxrocm_fp_qmm_rows_workspace_size); got %zu",
           need, workspace_bytes);
     }
-    return launch_qmm_walk_fp(a, mode, dtype, workspace, s);
+    if (!own) {
+      return launch_qmm_walk_fp(a, mode, dtype, workspace, s);
+    }
+    rc = fp_scale_image_for_qmm_t(scales, workspace, N, K, 1, 0, mode, dtype, s);
+    if (rc != MLXROCM_OK) {
+      return rc;
+    }
+    a.scales = workspace;
+    a.biases = workspace;
+    a.sb_batch_stride = 0;
+    a.sb_transposed = 2;
+    void* planes = static_cast<char*>(workspace) + fp_image_bytes(N, K, 1);
+    a.out = pl.splits > 1 ? planes : out;
+    rc = launch_qmm_own(a, 32, kOwnFpCodes + mode, dtype, pl, s);
+    return rc != MLXROCM_OK || pl.splits <= 1
+        ? rc
+        : reduce_k_splits(planes, out, M, N, pl.splits, dtype, s);
   }
   if (fp_tile_applies(M, N, K, L, mode, dtype, transpose != 0)) {
     const int batches = scales_batch_stride != 0 ? L : 1;
@@ -878,15 +913,20 @@ extern "C" int mlxrocm_fp_qmm(
 }
 
 extern "C" int mlxrocm_fp_qmm_rows_supported(int M, int N, int K, int L, int mode, int dtype) {
+  OwnPlan pl;
   return M >= 2 && fp_check("quantized_matmul", M, N, K, L, mode, dtype, 1) == MLXROCM_OK &&
-      N > 0 && L > 0 && fp_walk_applies(fp_shape(M, N, K, L), mode, dtype);
+      N > 0 && L > 0 &&
+      (M > 64 ? fp_own_pays(M, N, K, L, mode, dtype, &pl)
+              : fp_walk_applies(fp_shape(M, N, K, L), mode, dtype));
 }
 
 extern "C" size_t mlxrocm_fp_qmm_rows_workspace_size(
     int M, int N, int K, int L, int mode, int dtype) {
-  return mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)
-      ? qmm_walk_fp_plane_bytes(fp_shape(M, N, K, L), mode)
-      : 0;
+  if (!mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)) {
+    return 0;
+  }
+  return M > 64 ? fp_own_bytes(M, N, K, qmm_own_plan(M, N, K, kOwnFpCodes + mode))
+                : qmm_walk_fp_plane_bytes(fp_shape(M, N, K, L), mode);
 }
 
 extern "C" int mlxrocm_fp_qmm_rows(
@@ -919,6 +959,12 @@ extern "C" int mlxrocm_fp_qmm_rows(
 
 namespace {
 
+// Rows of x_hat that take mlxrocm_fp_qmm_rows (more of them keep the plan, and the scratch, of
+// mlxrocm_fp_qmm).
+bool qqmm_rows(int M, int N, int K, int mode, int dtype) {
+  return M <= 64 && mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype);
+}
+
 // Scratch of qqmm, with the fp32 planes of K ranges or as much as the plan without them takes.
 size_t qqmm_bytes(int M, int N, int K, int mode, int dtype, bool planes) {
   if (qq_native(M, N, K, mode, dtype)) {
@@ -929,7 +975,7 @@ size_t qqmm_bytes(int M, int N, int K, int mode, int dtype, bool planes) {
         (planes ? round256(qq_mfma_plane_bytes(M, N, K, mode)) : 0);
   }
   const size_t xhat = round256(static_cast<size_t>(M) * K * dtype_size(dtype));
-  if (mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype)) {
+  if (qqmm_rows(M, N, K, mode, dtype)) {
     return xhat + mlxrocm_fp_qmm_rows_workspace_size(M, N, K, 1, mode, dtype);
   }
   if (!planes && fp_tile_applies(M, N, K, 1, mode, dtype, true)) {
@@ -1021,7 +1067,7 @@ extern "C" int mlxrocm_fp_qqmm(
   return fp_qmm_entry(
       workspace, wq, scales, out, M, N, K, 1, 0, 0, 0, mode, dtype, 1,
       static_cast<char*>(workspace) + xhat_bytes, workspace_bytes - xhat_bytes, stream, nullptr,
-      mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype) != 0);
+      qqmm_rows(M, N, K, mode, dtype));
 }
 
 namespace {
@@ -1461,5 +1507,5 @@ extern "C" int mlxrocm_nvfp4_qqmm_global(
   return fp_qmm_entry(
       workspace, wq, scales, out, M, N, K, 1, 0, 0, 0, mode, dtype, 1,
       static_cast<char*>(workspace) + xhat_bytes, workspace_bytes - xhat_bytes, stream,
-      global_scale_w, mlxrocm_fp_qmm_rows_supported(M, N, K, 1, mode, dtype) != 0);
+      global_scale_w, qqmm_rows(M, N, K, mode, dtype));
 }

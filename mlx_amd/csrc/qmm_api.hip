@@ -699,6 +699,44 @@ bool mid_pays(const Call& c) {
       plane_bytes(a, pl.splits) <= kStaticScratchBytes / 2 && (need == 0 || c.sc.affords(need));
 }
 
+// More than 64 rows of x (mlxrocm_qmm_rows): where tiles whose wavefronts own their rows of W
+// (qmm_own.h) are ahead of the tile kernel and of qmm_mid, by the accounts of all three.
+bool own_pays(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* pl) {
+  // (ragged rows with K ranges: mlxrocm_qmm sums the same ranges for a caller short of scratch,
+  // a block of rows at a time, and so has the bits of this call whatever the scratch)
+  if (!qmm_own_supported(M, N, K, L, bits, dtype) ||
+      (N % 4 != 0 && qmm_mfma_k_splits(M, N, K, 1) > 1)) {
+    return false;
+  }
+  double other = qmm_mfma_us(M, N, K, bits);
+  if (M <= (K <= kMidShortK ? kMidMaxMShortK : kMidMaxM)) {
+    const MidPlan mid = qmm_mid_plan(M, N, K, gs, bits);
+    other = mid.groups <= compute_units() && mid.us < other ? mid.us : other;
+  }
+  *pl = qmm_own_plan(M, N, K, bits);
+  return qmm_own_pays(*pl, bits, other);
+}
+
+size_t own_plane_bytes(int M, int N, const OwnPlan& pl) {
+  return pl.splits > 1 ? k_split_plane(M, N) * pl.splits * sizeof(float) : 0;
+}
+
+// image: pairs of scales and biases (interleave_sb_for_qmm_t).
+int run_qmm_own(
+    const QmmArgs& a, int gs, int bits, int dtype, const OwnPlan& pl, const void* image,
+    void* planes, hipStream_t s) {
+  QmmArgs part = a;
+  part.scales = image;
+  part.biases = image; // (unused: a pair holds both)
+  part.sb_transposed = 2;
+  if (pl.splits <= 1) {
+    return launch_qmm_own(part, gs, bits, dtype, pl, s);
+  }
+  part.out = planes;
+  const int rc = launch_qmm_own(part, gs, bits, dtype, pl, s);
+  return rc != MLXROCM_OK ? rc : reduce_k_splits(planes, a.out, a.M, a.N, pl.splits, dtype, s);
+}
+
 // Two passes over the same scratch, one after the other on the stream.
 int two_passes(const Call& c, const QmmArgs& head, const QmmArgs& tail) {
   const int rc = run(head, c.gs, c.bits, c.dtype, c.transpose, c.sc, c.s);
@@ -1283,6 +1321,12 @@ int qmm_entry(
           kScratchAlign);
     }
   }
+  // (the kernel, and so the bits, of mlxrocm_qmm_rows where the scratch holds its planes)
+  OwnPlan pl;
+  if (sc.sb_image != nullptr &&
+      own_pays(M, N, K, L, group_size, bits, dtype, &pl) && sc.affords(own_plane_bytes(M, N, pl))) {
+    return run_qmm_own(a, group_size, bits, dtype, pl, sc.sb_image, sc.base, s);
+  }
   return run(a, group_size, bits, dtype, transpose != 0, sc, s);
 }
 
@@ -1377,15 +1421,24 @@ extern "C" int mlxrocm_qmm_rows_supported(
       check_shape("quantized_matmul", M, N, K, L, group_size, bits, dtype, 1) != MLXROCM_OK) {
     return 0;
   }
+  OwnPlan pl;
+  if (own_pays(M, N, K, L, group_size, bits, dtype, &pl)) {
+    return 1;
+  }
   const QmmArgs a = rows_shape(M, N, K, L);
   return walk_pays(a, group_size, bits) && qmm_walk_supported(a, group_size, bits, dtype, true);
 }
 
 extern "C" size_t mlxrocm_qmm_rows_workspace_size(
     int M, int N, int K, int L, int group_size, int bits, int dtype) {
-  return mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)
-      ? qmm_walk_plane_bytes(rows_shape(M, N, K, L), group_size, bits)
-      : 0;
+  if (!mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)) {
+    return 0;
+  }
+  if (M > 64) {
+    const OwnPlan pl = qmm_own_plan(M, N, K, bits);
+    return sb_image_bytes(rows_shape(M, N, K, L), group_size, dtype) + own_plane_bytes(M, N, pl);
+  }
+  return qmm_walk_plane_bytes(rows_shape(M, N, K, L), group_size, bits);
 }
 
 extern "C" int mlxrocm_qmm_rows(
@@ -1434,7 +1487,10 @@ extern "C" int mlxrocm_qmm_rows(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  const size_t need = qmm_walk_plane_bytes(a, group_size, bits);
+  const size_t image = M > 64 ? sb_image_bytes(a, group_size, dtype) : 0;
+  const OwnPlan pl = M > 64 ? qmm_own_plan(M, N, K, bits) : OwnPlan{};
+  const size_t need =
+      M > 64 ? image + own_plane_bytes(M, N, pl) : qmm_walk_plane_bytes(a, group_size, bits);
   if (need != 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {
     return fail(
         MLXROCM_INVALID_ARGUMENT,
@@ -1442,8 +1498,14 @@ extern "C" int mlxrocm_qmm_rows(
         "(mlxrocm_qmm_rows_workspace_size); got %zu",
         need, workspace_bytes);
   }
-  return launch_qmm_walk(
-      a, group_size, bits, dtype, workspace, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (M > 64) {
+    const int made = interleave_sb_for_qmm_t(scales, biases, workspace, N, K / group_size, 1, 0, s);
+    return made != MLXROCM_OK ? made
+                              : run_qmm_own(a, group_size, bits, dtype, pl, workspace,
+                                            static_cast<char*>(workspace) + image, s);
+  }
+  return launch_qmm_walk(a, group_size, bits, dtype, workspace, s);
 }
 
 extern "C" size_t mlxrocm_qmm_sb_image_size(int N, int K, int batches, int group_size, int dtype) {

@@ -315,7 +315,25 @@ int launch_qmm_mid_bf16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, h
 int launch_qmm_mid_f16(const QmmArgs& a, int gs, int bits, const MidPlan& pl, hipStream_t s);
 int reduce_k_splits(
     const void* partial, void* out, int M, int N, int k_splits, int dtype, hipStream_t s);
-// Tiles whose wavefronts own their rows of W (qmm_own.h): pair images, 16-bit types.
+// Tiles whose wavefronts own their rows of W (qmm_own.h): pair images, 16-bit types.  One
+// product, more than 64 rows of x.  With pl.splits > 1 `a.out` points at that many planes.
+struct OwnPlan {
+  int mt;     // tiles of 16 mt rows of x
+  int splits; // ranges of K
+  double us;  // what the call takes, by the plan's account
+};
+// codes: the width of affine codes, or kOwnFpCodes + mlxrocm_fp_mode
+constexpr int kOwnFpCodes = 16;
+bool qmm_own_supported(int M, int N, int K, int L, int bits, int dtype);
+OwnPlan qmm_own_plan(int M, int N, int K, int codes);
+// Whether it is ahead of the kernel that takes the call otherwise (`other`: us).
+bool qmm_own_pays(const OwnPlan& pl, int codes, double other);
+int launch_qmm_own(
+    const QmmArgs& a, int gs, int codes, int dtype, const OwnPlan& pl, hipStream_t s);
+int launch_qmm_own_bf16(const QmmArgs& a, int gs, int bits, const OwnPlan& pl, hipStream_t s);
+int launch_qmm_own_f16(const QmmArgs& a, int gs, int bits, const OwnPlan& pl, hipStream_t s);
+int launch_qmm_own_fp_bf16(const QmmArgs& a, int mode, const OwnPlan& pl, hipStream_t s);
+int launch_qmm_own_fp_f16(const QmmArgs& a, int mode, const OwnPlan& pl, hipStream_t s);
 bool qmm_own_experts_supported(const QmmArgs& a, int bits);
 int launch_qmm_own_experts(
     const QmmArgs& a, int gs, int bits, int dtype, bool glu, hipStream_t s);

@@ -55,6 +55,25 @@ __device__ __forceinline__ void own_unroll(F&& f) {
 
 #define OWN_INLINE __attribute__((always_inline))
 
+// Lanes 16 g + i, g = 0..3, as a 4 x 4 matrix of registers v[0..3]: transposed, so that
+// lanes of g hold in v[j] what lanes of j held in v[g].
+__device__ __forceinline__ void transpose_rows(uint32_t& v0, uint32_t& v1, uint32_t& v2, uint32_t& v3) {
+  auto swap32 = [](uint32_t& a, uint32_t& b) { // a's lanes 32.. for b's lanes 0..31
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  auto swap16 = [](uint32_t& a, uint32_t& b) { // a's odd 16s of lanes for b's even ones
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  swap32(v0, v2);
+  swap32(v1, v3);
+  swap16(v0, v1);
+  swap16(v2, v3);
+}
+
 // out = x W^T.  MT: tiles have 16 MT rows of x (4..16, even; grouped: 0, as many as the tile list says, in
 // steps of 32).  TO float with k_splits > 1: planes (k_split_plane()) of K ranges.  FP: the
 // modes of FpPairDequant.  GLU: gated pairs of columns of W and a.w_alt, 128 to a tile.
@@ -65,6 +84,13 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   using DQ = std::conditional_t<FP != 0, FpPairDequant<T, (FP != 0 ? FP : 1)>, PairDequant<T, BITS>>;
   constexpr int kStage = own_stage_bytes(MT_);
   constexpr int kTileRows = GROUPED ? kOwnBM : 16 * MT_;
+  // A product of 4-bit codes without ranges of K: the matrix instructions of a step take its
+  // codes 32 by 32 in their order, as those of the tile kernel do, so that mlxrocm_qmm, a graph
+  // that holds it and mlxrocm_qmm_rows return the same bits.  A lane loads 32 codes in a row
+  // and gives 24 of them to the three lanes that hold the same row of W (swaps of registers
+  // between lanes, with scales and biases 24 vector instructions a step: 8192 x 14336 x 4096
+  // 685 -> 712 us).  Everywhere else the codes stay where they were loaded.
+  constexpr bool kInOrder = BITS == 4 && FP == 0 && !GROUPED && sizeof(TO) == 2;
   constexpr int kCols = GLU ? kOwnBN / 2 : kOwnBN; // columns of y of a tile
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x;
@@ -80,7 +106,7 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   const int ny = __builtin_amdgcn_readfirstlane(
       GROUPED ? *a.group_ntiles : (a.M + kTileRows - 1) / kTileRows);
   const int plane = nx * ny;
-  const int tiles = plane * (GROUPED ? 1 : (k_splits > 1 ? k_splits : a.L));
+  const int tiles = plane * (GROUPED ? 1 : k_splits);
   // Rounds of gridDim.x tiles.  Workgroups b, b + 8, .. share an XCD: they take neighbouring
   // tiles, and what is left for the last round is dealt out evenly to the XCDs.
   const int stride = gridDim.x;
@@ -137,17 +163,16 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     const int col = uniform(in_band / high);
     const int ty = 4 * band + in_band - col * high;
     n0 = col * kCols + wave * (kCols / 8);
-    int64_t xb = 0, wb = 0;
+    int64_t wb = 0;
     if constexpr (GROUPED) {
       wb = uniform(a.group_tiles[3 * ty]);
       row0 = uniform(a.group_tiles[3 * ty + 1]);
       rows = uniform(a.group_tiles[3 * ty + 2]);
     } else {
-      xb = wb = k_splits > 1 ? 0 : z;
       m0 = ty * kTileRows;
       rows = a.M - m0 < kTileRows ? a.M - m0 : kTileRows;
     }
-    px = static_cast<const uint8_t*>(a.x) + xb * a.x_batch_stride * 2;
+    px = static_cast<const uint8_t*>(a.x);
     const int64_t wo = wb * a.w_batch_stride * 4;
     const int64_t so = wb * a.sb_batch_stride * 2;
     pw[0] = reinterpret_cast<const uint8_t*>(a.w) + wo;
@@ -165,12 +190,15 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
       sb_voff[j] = (static_cast<uint32_t>((32 * wk) >> gs_shift) * N + nc) * 4u;
     }
     // x: load i of wavefront w moves rows 32 i + 4 w .. + 3, the 16 pieces of a row in 16
-    // lanes.  Piece 4 k + s of row r (k: which 32 of the step's 128 columns, s: which 8 of
-    // them) sits at 8 (k % 2) + ((4 (k / 2) + s) ^ (r % 8)): the 64 lanes of a fragment
-    // read, 16 rows by four k, then hit every bank of LDS once in each quarter.
+    // lanes.  Piece p of row r (eight columns) is read in slice s by the lanes of k, p = 4 s + k
+    // in order and 4 k + s otherwise.  It sits at 8 (k % 2) + (q ^ (r % 8)), q being what
+    // else there is of p: the 64 lanes of a fragment read, 16 rows by four k, then hit every
+    // bank of LDS once in each quarter.
     const int xr0 = 4 * wave + (at >> 4);
     const uint32_t xlow = static_cast<uint32_t>((at ^ xr0) & 7);
-    const uint32_t xpiece = ((xlow >> 2) * 2 + ((at >> 3) & 1)) * 4 + (xlow & 3);
+    const uint32_t odd = (at >> 3) & 1;
+    const uint32_t xpiece =
+        kInOrder ? 2 * xlow + odd : ((xlow >> 2) * 2 + odd) * 4 + (xlow & 3);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int r = 32 * i + xr0;
@@ -191,14 +219,17 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   };
 
   uint32_t wreg[2][BITS];
-  float sf[2], bf[2];
+  constexpr int kScales = kInOrder ? 4 : 1; // of a row in a step: of each 32 codes
+  uint32_t sb[2][kScales]; // pairs of scale and bias
+  float sf[2], bf[2];      // those of the codes being unpacked
   RawWords<BITS> wnext[2];
   RawTuple<1> snext[2];
   uint32_t rd[4]; // byte offset of this lane's piece of slice s in a row block
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int fi = lane & 15, fk = lane >> 4;
-    rd[s] = fi * 256 + (8 * (fk & 1) + ((4 * (fk >> 1) + s) ^ (fi & 7))) * 16;
+    const int of_half = kInOrder ? 2 * s + (fk >> 1) : 4 * (fk >> 1) + s;
+    rd[s] = fi * 256 + (8 * (fk & 1) + (of_half ^ (fi & 7))) * 16;
   }
 
   auto load_w = [&](int k) OWN_INLINE {
@@ -212,21 +243,20 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     }
   };
   // behind the wait that covers the loads of load_w()
-  auto take_w = [&]() OWN_INLINE {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      wnext[j].pin();
-      snext[j].pin();
-    }
+  auto take_w = [&](auto jval) OWN_INLINE {
+    constexpr int j = decltype(jval)::value;
+    wnext[j].pin();
+    snext[j].pin();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int i = 0; i < BITS; ++i) {
-        wreg[j][i] = wnext[j].get(i);
-      }
-      sf[j] = raw_value<T>(snext[j].get(0)) * DQ::kCodeScale;
-      bf[j] = raw_value<T>(snext[j].get(0) >> 16);
+    for (int i = 0; i < BITS; ++i) {
+      wreg[j][i] = wnext[j].get(i);
+    }
+    sb[j][0] = snext[j].get(0);
+    if constexpr (kInOrder) {
+      transpose_rows(wreg[j][0], wreg[j][1], wreg[j][2], wreg[j][3]);
+      sb[j][1] = sb[j][2] = sb[j][3] = sb[j][0];
+      transpose_rows(sb[j][0], sb[j][1], sb[j][2], sb[j][3]);
     }
   };
   auto dma_x = [&](int stage, int k, auto i) OWN_INLINE {
@@ -262,6 +292,11 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     auto pair = [&](auto s, auto q) OWN_INLINE {
       constexpr int j = decltype(q)::value / 4;
       constexpr int i = decltype(q)::value % 4;
+      if constexpr (i == 0 && (kInOrder || decltype(s)::value == 0)) {
+        constexpr int g = kInOrder ? decltype(s)::value : 0;
+        sf[j] = raw_value<T>(sb[j][g]) * DQ::kCodeScale;
+        bf[j] = raw_value<T>(sb[j][g] >> 16);
+      }
       wf[s % 2][j][i] = dq[j].template pair<4 * decltype(s)::value + i>(wreg[j], sf[j], bf[j]);
     };
     own_unroll<8>([&](auto q) OWN_INLINE { pair(std::integral_constant<int, 0>{}, q); });
@@ -293,7 +328,10 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
         if constexpr (m == 6 * MT) {
           // the packed W asked for in slot 0 is older than the loads of x
           asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma) : "memory");
-          take_w();
+          take_w(std::integral_constant<int, 0>{});
+        }
+        if constexpr (m == 7 * MT - 1) { // before the first pair of the second row
+          take_w(std::integral_constant<int, 1>{});
         }
         if constexpr (m == kBarrier) {
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -436,7 +474,8 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   own_unroll<kLoads>([&](auto i) OWN_INLINE { dma_x(0, kbeg, i); });
   load_w(kbeg);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  take_w();
+  take_w(std::integral_constant<int, 0>{});
+  take_w(std::integral_constant<int, 1>{});
   __syncthreads();
   __builtin_amdgcn_s_setprio(3);
   if constexpr (!GROUPED) {

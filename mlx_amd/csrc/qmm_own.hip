@@ -8,10 +8,32 @@ namespace {
 constexpr uint64_t k32Bit = uint64_t{1} << 32;
 
 // Whole steps of K; operands within the kernel's 32-bit byte offsets.
-bool own_addresses(const QmmArgs& a, int bits) {
-  return a.K % kOwnBK == 0 && a.K >= kOwnBK &&
-      static_cast<uint64_t>(a.N) * a.K * bits / 8 < k32Bit;
+bool own_addresses(int N, int K, int bits) {
+  return K % kOwnBK == 0 && K >= kOwnBK && static_cast<uint64_t>(N) * K * bits / 8 < k32Bit;
 }
+
+// us of a step of 128 codes: fixed + 16-row blocks of the tile * (each + busy * share of the
+// compute units at work, by which the clock gives way).
+struct Step {
+  double fixed, each, busy;
+};
+constexpr Step kSteps[] = {
+    {0.73, 0.0845, 0.0263}, // 2-bit
+    {0.77, 0.0876, 0.0326}, // 3-bit
+    {0.62, 0.0817, 0.0398}, // 4-bit
+    {1.13, 0.0851, 0.0215}, // 5-bit
+    {1.16, 0.0830, 0.0229}, // 6-bit
+    {1.11, 0.0652, 0.0287}, // 8-bit
+    {0.59, 0.0720, 0.0337}, // mxfp4
+    {1.14, 0.0574, 0.0184}, // mxfp8
+    {0.64, 0.0794, 0.0388}, // nvfp4
+};
+const Step& step_of(int codes) {
+  return kSteps[codes >= kOwnFpCodes ? 6 + codes - kOwnFpCodes : codes == 8 ? 5 : codes - 2];
+}
+
+// Scratch of ranges of K that a plan may ask for.
+constexpr size_t kOwnMostPlanes = size_t(128) << 20;
 
 } // namespace
 
@@ -22,7 +44,76 @@ bool own_addresses(const QmmArgs& a, int bits) {
 // -> 310, 8-bit 438 -> 382, 800 tokens 283 -> 264.
 bool qmm_own_experts_supported(const QmmArgs& a, int bits) {
   // (x: the callers check it for every grouped kernel)
-  return own_addresses(a, bits) && static_cast<uint64_t>(a.L) * a.N * 2 < kNoStore;
+  return own_addresses(a.N, a.K, bits) && static_cast<uint64_t>(a.L) * a.N * 2 < kNoStore;
+}
+
+bool qmm_own_supported(int M, int N, int K, int L, int bits, int dtype) {
+  return M > 64 && L == 1 && dtype != MLXROCM_FLOAT32 && own_addresses(N, K, bits) &&
+      static_cast<uint64_t>(M) * K * 2 < k32Bit &&
+      static_cast<uint64_t>(kOwnBM) * (N + 3) * 4 < kNoStore;
+}
+
+// The height of the tiles and the number of K ranges with the least time by this account,
+// fitted to 27000 calls of 65..8192 rows on 14 shapes, every width and mode, each in every
+// height and several numbers of ranges (errors of 5 %; the choice takes 1.2 % longer than the
+// best one on average): the launches and the image of scales, rounds of tiles, planes written
+// and added up.  Ranges are cut only while one round of workgroups holds their tiles.
+OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
+  const Step& step = step_of(codes);
+  const long cus = compute_units();
+  const long nx = (N + kOwnBN - 1) / kOwnBN;
+  const int steps = K / kOwnBK;
+  const double plane = 1e-6 * static_cast<double>(k_split_plane(M, N));
+  OwnPlan pl{};
+  for (int mt = 4; mt <= 16; mt += 2) {
+    if (mt > 4 && 16 * mt > (M + 31) / 32 * 32) {
+      break;
+    }
+    const long tiles = nx * ((M + 16 * mt - 1) / (16 * mt));
+    for (int s = 1; s <= 16; ++s) {
+      if (s > 1 &&
+          (tiles * s > cus || 2 * s > steps ||
+           k_split_plane(M, N) * s * sizeof(float) > kOwnMostPlanes)) {
+        break;
+      }
+      const long rounds = (tiles * s + cus - 1) / cus;
+      const double busy = static_cast<double>(tiles * s) / static_cast<double>(rounds * cus);
+      // (4-bit codes in one range are put in order: kInOrder)
+      const double fixed = step.fixed + (codes == 4 && s == 1 ? 0.12 : 0.0);
+      const double each = (steps + s - 1) / s * (fixed + mt * (step.each + busy * step.busy));
+      const double us = 5.9 + rounds * (0.36 * mt - 1.1 + each) +
+          (s > 1 ? 6.6 + (0.89 * s + 0.15) * plane : 0.34 * plane);
+      if (pl.mt == 0 || us < pl.us) {
+        pl = {mt, s, us};
+      }
+    }
+  }
+  return pl;
+}
+
+// With the accounts of both sides, which err by 5 and 7..15 %, these margins leave 1.8 % of the
+// 2000 calls taken (of 3000 timed) behind by more than 3 %, the worst by 12 %, the others 18 %
+// shorter on average.  us against the tile kernel, bf16 g64 4-bit: 2048 x 4096 x 14336 198 / 243,
+// 2048 x 8192 x 8192 198 / 275, 2048 x 4096 x 4096 66 / 78, 320 x 14336 x 4096 51 / 60, 320 x 8192 x
+// 8192 54 / 80; the tile kernel stays ahead where its widths make whole rounds: 1024 x 14336 x
+// 4096 8-bit 102 / 99, 512 x 18944 x 3584 8-bit 77 / 72.  Less is to be gained where its
+// unpacking is one convert for two codes (mxfp8: 512 x 18944 x 3584 75 / 66) or this kernel
+// has to put the codes in order (4-bit, one range: 5291 x 6853 x 8192 557 / 553).
+bool qmm_own_pays(const OwnPlan& pl, int codes, double other) {
+  const bool less = codes == kOwnFpCodes + MLXROCM_MXFP8 || (codes == 4 && pl.splits == 1);
+  return pl.us < (less ? 0.82 : 0.88) * other;
+}
+
+int launch_qmm_own(
+    const QmmArgs& a, int gs, int codes, int dtype, const OwnPlan& pl, hipStream_t s) {
+  MLXROCM_REHEARSE("qmm_own(rows=%d,ksplit=%d)", 16 * pl.mt, pl.splits);
+  if (codes >= kOwnFpCodes) {
+    const int mode = codes - kOwnFpCodes;
+    return dtype == MLXROCM_BFLOAT16 ? launch_qmm_own_fp_bf16(a, mode, pl, s)
+                                     : launch_qmm_own_fp_f16(a, mode, pl, s);
+  }
+  return dtype == MLXROCM_BFLOAT16 ? launch_qmm_own_bf16(a, gs, codes, pl, s)
+                                   : launch_qmm_own_f16(a, gs, codes, pl, s);
 }
 
 int launch_qmm_own_experts(

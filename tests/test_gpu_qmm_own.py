@@ -62,3 +62,88 @@ def test_experts(D, F, bits):
     # and row by row: a row of another expert or of another position is no near miss
     r = (y.double() - want).norm(dim=-1) / want.norm(dim=-1)
     assert float(r.max()) < (2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -9)
+
+
+# heights of a tile from 64 to 256 rows with a short last one, one and several rounds of tiles,
+# ranges of K (the odd step among them), rows of y of any number of elements
+SHAPES = ((321, 8191, 2176), (300, 2736, 8192), (257, 14337, 4096), (511, 4098, 4224),
+          (1537, 4099, 4096), (3000, 1023, 1024), (4097, 2050, 256),
+          (66, 18944, 3584), (2048, 4096, 14336))
+FP = {"mxfp4": (_lib.MXFP4, 32, 4), "mxfp8": (_lib.MXFP8, 32, 8), "nvfp4": (_lib.NVFP4, 16, 4)}
+CODE = {torch.float16: _lib.FLOAT16, torch.bfloat16: _lib.BFLOAT16}
+
+
+def _relative(y, want, dtype):
+    # results rounded once (half an ulp of 2**-7 / 2**-10 of the value), sums in 32 bits of
+    # another order (2**-24 each, some tens of roundings)
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    d = y.double() - want
+    rms = want.pow(2).mean().sqrt()
+    assert float(d.norm() / want.norm()) < half
+    assert bool((d.abs() <= half * want.abs() * 1.001 + 2.0 ** -17 * rms).all())
+
+
+@pytest.mark.parametrize("bits", BITS)
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+def test_products(bits, dtype):
+    taken = 0
+    for M, N, K in SHAPES:
+        group = (32, 64, 128)[(M + bits) % 3]
+        if not _lib.load().mlxrocm_qmm_rows_supported(M, N, K, 1, group, bits, CODE[dtype]):
+            continue
+        taken += 1
+        g = torch.Generator(device="cuda").manual_seed(M)
+        x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+        w = (torch.randn((N, K), generator=g, device="cuda") / K ** 0.5).to(dtype)
+        wq, s, b = mlx_amd.quantize(w, group, bits)
+        y = mlx_amd.quantized_matmul(x, wq, s, b, group_size=group, bits=bits)
+        codes = mlx_amd.dequantize(wq, torch.ones_like(s, dtype=torch.float32),
+                                   torch.zeros_like(s, dtype=torch.float32), group, bits).double()
+        w_hat = codes.unflatten(1, (-1, group)) * s.double()[..., None] + b.double()[..., None]
+        w_hat = w_hat.flatten(1).to(dtype).double()
+        _relative(y, x.double() @ w_hat.T, dtype)
+        # the image made beforehand, and rows that are no numbers stay by themselves
+        image = mlx_amd.quantized_matmul_sb_image(s, b, group)
+        assert torch.equal(y, mlx_amd.quantized_matmul(x, wq, s, b, group_size=group, bits=bits,
+                                                       sb_image=image))
+        x[M - 1] = float("nan")
+        z = mlx_amd.quantized_matmul(x, wq, s, b, group_size=group, bits=bits)
+        assert torch.equal(z[:-1], y[:-1]) and bool(z[-1].isnan().all())
+    assert taken >= 5
+
+
+@pytest.mark.parametrize("mode", FP)
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+def test_floating_point_codes(mode, dtype):
+    code, group, bits = FP[mode]
+    taken = 0
+    for M, N, K in SHAPES:
+        if not _lib.load().mlxrocm_fp_qmm_rows_supported(M, N, K, 1, code, CODE[dtype]):
+            continue
+        taken += 1
+        g = torch.Generator(device="cuda").manual_seed(M)
+        x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+        w = (torch.randn((N, K), generator=g, device="cuda")).to(dtype)
+        wq, s = mlx_amd.quantize(w, mode=mode)[:2]
+        y = mlx_amd.quantized_matmul(x, wq, s, None, mode=mode)
+        w_hat = mlx_amd.dequantize(wq, s, None, mode=mode, dtype=dtype).double()
+        _relative(y, x.double() @ w_hat.T, dtype)
+    assert taken >= 4
+
+
+def test_replayed_from_a_graph():
+    M, N, K = 300, 2736, 8192
+    wq, s, b = mlx_amd.quantize((torch.randn((N, K), device="cuda") / 64).bfloat16())
+    x = torch.randn((M, K), device="cuda").bfloat16()
+    assert _lib.load().mlxrocm_qmm_rows_supported(M, N, K, 1, 64, 4, _lib.BFLOAT16)
+    mlx_amd.quantized_matmul(x, wq, s, b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = mlx_amd.quantized_matmul(x, wq, s, b)
+    for seed in range(4):
+        torch.manual_seed(seed)
+        x.copy_(torch.randn((M, K), device="cuda"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, mlx_amd.quantized_matmul(x, wq, s, b)), seed

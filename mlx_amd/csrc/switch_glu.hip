@@ -4,8 +4,8 @@
 // block issues them).  What the call saves over those: the pairs are grouped by
 // expert once instead of three times (and instead of being sorted beforehand), the
 // indices are read as they come, the gate is applied where its operands are, and
-// from 64 pairs per expert on the two first products run as one launch of the tile
-// kernel whose epilogue writes the gated result -- 8 experts of [14336, 4096], 4096
+// from 64 pairs per expert on (fewer: least_pairs) the two first products run as one launch
+// of a tile kernel whose epilogue writes the gated result -- 8 experts of [14336, 4096], 4096
 // pairs: 2 x 117 MB written and read again are left out, and one pass over x.
 #include "qmm_args.h"
 
@@ -55,12 +55,32 @@ size_t round256(size_t n) {
   return (n + 255) / 256 * 256;
 }
 
-// The tile kernel's grouped form: as many pairs per expert as mlxrocm_gather_qmm
-// asks for, and operands within 32-bit byte offsets.
-bool tiled(int tokens, int top, int D, int F, int E) {
+// Pairs per expert from which the tiles are ahead: as many as mlxrocm_gather_qmm asks for of
+// the tile kernel, fewer where qmm_own_kernel takes both products and the products one by one
+// would run on the staged kernel of 32 rows (4-bit codes have one that rounds no weight, and
+// keep it).  us per call, products / tiles, 8-bit, by pairs per expert: 4096 x 14336, 8
+// experts 24 525 / 529, 32 546 / 532, 44 707 / 554, 64 876 / 580; 2048 x 1408, 64 experts 12
+// 189 / 194, 16 226 / 216, 32 246 / 201, 64 375 / 248; 1024 x 1024, 32 experts 16 75 / 64, 64
+// 109 / 82 (3-bit: 28 458 / 469, 28 238 / 185, 28 70 / 57).
+int least_pairs(int64_t pairs, int D, int F, int bits) {
+  QmmArgs in{};
+  in.N = F;
+  in.K = D;
+  in.L = static_cast<int>(pairs);
+  QmmArgs out = in;
+  out.N = D;
+  out.K = F;
+  if (bits == 4 || !qmm_own_experts_supported(in, bits) || !qmm_own_experts_supported(out, bits)) {
+    return 64;
+  }
+  return D <= 2048 && F <= 2048 ? 16 : 32;
+}
+
+// The tile kernels' grouped form: operands within 32-bit byte offsets.
+bool tiled(int tokens, int top, int D, int F, int E, int least) {
   const int64_t pairs = static_cast<int64_t>(tokens) * top;
   const int64_t limit = int64_t{1} << 32;
-  return pairs > 64 * static_cast<int64_t>(E) && D % 64 == 0 &&
+  return pairs > least * static_cast<int64_t>(E) && D % 64 == 0 &&
       F % 64 == 0 && static_cast<int64_t>(tokens) * D * 2 < limit && pairs * F * 2 < limit &&
       gather_group_max_tiles(static_cast<int>(pairs), E, kGroupLargeTile) <= 65535 &&
       gather_group_workspace_bytes(static_cast<int>(pairs), E) > 0;
@@ -75,7 +95,11 @@ struct Layout {
   size_t total;
 };
 
-Layout layout_of(int tokens, int top, int D, int F, int E, int gs, int bits, int dtype) {
+// room: what the caller has.  One with too little for tiles of few pairs has the products one
+// by one.
+Layout layout_of(
+    int tokens, int top, int D, int F, int E, int gs, int bits, int dtype, bool* tiles,
+    size_t room = SIZE_MAX, int least = 0) {
   const size_t pairs = static_cast<size_t>(tokens) * top;
   Layout l{};
   size_t at = 0;
@@ -88,7 +112,9 @@ Layout layout_of(int tokens, int top, int D, int F, int E, int gs, int bits, int
   l.row = take(pairs * 4);
   l.self = take(pairs * 4);
   l.h = take(pairs * F * dtype_size(dtype));
-  if (tiled(tokens, top, D, F, E)) {
+  const int fewest = least_pairs(pairs, D, F, bits);
+  *tiles = tiled(tokens, top, D, F, E, least > fewest ? least : fewest);
+  if (*tiles) {
     l.rest = take(gather_group_workspace_bytes(static_cast<int>(pairs), E));
     l.gate_image = take(qmm_n_sb_bytes(F, D / gs, E, dtype));
     l.up_image = take(qmm_n_sb_bytes(F, D / gs, E, dtype));
@@ -102,7 +128,9 @@ Layout layout_of(int tokens, int top, int D, int F, int E, int gs, int bits, int
     l.rest = take(in > out ? in : out);
   }
   l.total = at;
-  return l;
+  return l.total > room && *tiles && least == 0
+      ? layout_of(tokens, top, D, F, E, gs, bits, dtype, tiles, room, 64)
+      : l;
 }
 
 bool good_shape(int tokens, int top, int D, int F, int E, int gs, int bits, int dtype) {
@@ -123,7 +151,8 @@ extern "C" size_t mlxrocm_switch_glu_workspace_size(
   if (!good_shape(tokens, top, D, F, n_experts, group_size, bits, dtype)) {
     return 0;
   }
-  return layout_of(tokens, top, D, F, n_experts, group_size, bits, dtype).total;
+  bool tiles;
+  return layout_of(tokens, top, D, F, n_experts, group_size, bits, dtype, &tiles).total;
 }
 
 extern "C" int mlxrocm_switch_glu(
@@ -172,7 +201,9 @@ extern "C" int mlxrocm_switch_glu(
       return fail(MLXROCM_UNSUPPORTED, "[switch_glu] operands must be 16-byte aligned");
     }
   }
-  const Layout l = layout_of(tokens, top, D, F, E, group_size, bits, dtype);
+  bool tiles;
+  const Layout l =
+      layout_of(tokens, top, D, F, E, group_size, bits, dtype, &tiles, workspace_bytes);
   if (workspace_bytes < l.total) {
     return fail(
         MLXROCM_INVALID_ARGUMENT,
@@ -201,7 +232,7 @@ extern "C" int mlxrocm_switch_glu(
   const int64_t sb_out = static_cast<int64_t>(D) * (F / group_size);
   void* h = ws + l.h;
 
-  if (!tiled(tokens, top, D, F, E)) {
+  if (!tiles) {
     void* up = ws + l.up;
     void* rest = ws + l.rest;
     const size_t rest_bytes = workspace_bytes - l.rest;

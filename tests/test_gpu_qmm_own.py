@@ -147,3 +147,34 @@ def test_replayed_from_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, mlx_amd.quantized_matmul(x, wq, s, b)), seed
+
+
+@pytest.mark.parametrize("bits", (3, 8))
+@pytest.mark.parametrize("E,D,F,tokens", ((8, 512, 384, 70), (4, 2176, 256, 70)))
+def test_few_pairs_of_an_expert(bits, E, D, F, tokens):
+    """Tiles of 17 and 33 pairs per expert and more, with the scratch the call names, and the
+    products one by one with less: the same roundings."""
+    lib = _lib.load()
+    torch.manual_seed(bits)
+    block = nn.SwitchGLU(D, F, E, group_size=64, bits=bits, dtype=torch.bfloat16)
+    x = torch.randn((tokens, D), device="cuda").bfloat16()
+    idx = torch.randint(0, E, (tokens, 2), device="cuda")
+    idx[3, 1] = E + 2  # no such expert: a row of zeros
+    y = block(x, idx)
+    assert not y[3, 1].any()
+    need = lib.mlxrocm_switch_glu_workspace_size(tokens, 2, D, F, E, 64, bits, _lib.BFLOAT16)
+    ops = [t for layer in (block.gate_proj, block.up_proj, block.down_proj)
+           for t in (layer.weight, layer.scales, layer.biases)]
+    plain = tokens * 2 * F * 2 * 2 + 3 * 4 * tokens * 2  # h, up and the pairs
+    got = {}
+    for room in (need, need - 1):
+        ws = torch.empty(room, dtype=torch.uint8, device="cuda")
+        out = torch.empty((tokens, 2, D), dtype=torch.bfloat16, device="cuda")
+        _lib.check(lib.mlxrocm_switch_glu(
+            x.data_ptr(), idx.data_ptr(), 8, *[t.data_ptr() for t in ops], out.data_ptr(), tokens,
+            2, D, F, E, 64, bits, _lib.BFLOAT16, ws.data_ptr(), room,
+            torch.cuda.current_stream().cuda_stream))
+        got[room] = out
+    assert need > plain and torch.equal(got[need], y)
+    d = (got[need - 1].double() - y.double()).norm() / y.double().norm()
+    assert float(d) < 2.0 ** -8

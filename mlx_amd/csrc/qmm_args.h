@@ -335,13 +335,25 @@ int launch_qmm_own_f16(const QmmArgs& a, int gs, int bits, const OwnPlan& pl, hi
 int launch_qmm_own_fp_bf16(const QmmArgs& a, int mode, const OwnPlan& pl, hipStream_t s);
 int launch_qmm_own_fp_f16(const QmmArgs& a, int mode, const OwnPlan& pl, hipStream_t s);
 bool qmm_own_experts_supported(const QmmArgs& a, int bits);
+// K ranges of a product of routed rows whose fp32 planes, a.L x a.N each, `room` bytes hold;
+// with more than one a.out points at the planes (reduce_grouped_planes adds them up).
+int qmm_own_experts_splits(const QmmArgs& a, int bits, size_t room);
 int launch_qmm_own_experts(
-    const QmmArgs& a, int gs, int bits, int dtype, bool glu, hipStream_t s);
-int launch_qmm_own_experts_bf16(const QmmArgs& a, int gs, int bits, bool glu, hipStream_t s);
-int launch_qmm_own_experts_f16(const QmmArgs& a, int gs, int bits, bool glu, hipStream_t s);
+    const QmmArgs& a, int gs, int bits, int dtype, bool glu, int k_splits, hipStream_t s);
+int launch_qmm_own_experts_bf16(
+    const QmmArgs& a, int gs, int bits, bool glu, int k_splits, hipStream_t s);
+int launch_qmm_own_experts_f16(
+    const QmmArgs& a, int gs, int bits, bool glu, int k_splits, hipStream_t s);
+// a.out (rows through a.group_perm) = sum of the planes, rows in sorted order; N % 4 == 0
+int reduce_grouped_planes(
+    const QmmArgs& a, const float* planes, int ranges, int64_t plane_elems, int dtype,
+    hipStream_t s);
 // expert-routed gated MLP (qmm_mfma_experts.hip): pair images, launch_gather_group's tables
 int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
-int launch_qmm_mfma_experts(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
+// planes: scratch of `room` bytes for K ranges
+int launch_qmm_mfma_experts(
+    const QmmArgs& a, int gs, int bits, int dtype, void* planes, size_t room, hipStream_t s);
+int expected_tiles(int pairs, int experts);
 int launch_qmm_mfma_grouped(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 // transpose=false form: scales / biases are the [group][k] images of all experts
 int launch_qmm_mfma_grouped_n(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);

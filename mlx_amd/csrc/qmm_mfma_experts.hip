@@ -15,7 +15,7 @@ int expected_tiles(int pairs, int experts) {
 // images, a.w_alt / a.scales_alt the up weights.  256-column tiles, 128 of each.
 int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s) {
   if (qmm_own_experts_supported(a, bits)) { // (K a multiple of 128)
-    return launch_qmm_own_experts(a, gs, bits, dtype, true, s);
+    return launch_qmm_own_experts(a, gs, bits, dtype, true, 1, s);
   }
   constexpr int kNT = 8;
   MLXROCM_REHEARSE("qmm_t_tile_experts_glu(nt=%d)", kNT);
@@ -32,13 +32,24 @@ int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, h
   return dtype == MLXROCM_BFLOAT16 ? run(bf16_t{}) : run(f16_t{});
 }
 
-int launch_qmm_mfma_experts(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s) {
+int launch_qmm_mfma_experts(
+    const QmmArgs& a, int gs, int bits, int dtype, void* planes, size_t room, hipStream_t s) {
   // Tiles of 256 columns that leave half of the compute units idle over a short K are behind
   // the narrower ones here: 2400 pairs of 32 experts, 1024 x 1024, whole call 82.8 us against 81.1.
   const long own_tiles =
       static_cast<long>(expected_tiles(a.L, a.n_experts)) * ((a.N + 255) / 256);
   if (qmm_own_experts_supported(a, bits) && (2 * own_tiles > compute_units() || a.K > 2048)) {
-    return launch_qmm_own_experts(a, gs, bits, dtype, false, s);
+    const int splits = qmm_own_experts_splits(a, bits, room);
+    if (splits <= 1) {
+      return launch_qmm_own_experts(a, gs, bits, dtype, false, 1, s);
+    }
+    QmmArgs part = a;
+    part.out = planes;
+    const int rc = launch_qmm_own_experts(part, gs, bits, dtype, false, splits, s);
+    return rc != MLXROCM_OK
+        ? rc
+        : reduce_grouped_planes(
+              a, static_cast<const float*>(planes), splits, static_cast<int64_t>(a.L) * a.N, dtype, s);
   }
   const int gs_shift = shift_of(gs);
   // the tile count is on the device: the width that suits the expected one

@@ -75,7 +75,8 @@ __device__ __forceinline__ void transpose_rows(uint32_t& v0, uint32_t& v1, uint3
 }
 
 // out = x W^T.  MT: tiles have 16 MT rows of x (4..16, even; grouped: 0, as many as the tile list says, in
-// steps of 32).  TO float with k_splits > 1: planes (k_split_plane()) of K ranges.  FP: the
+// steps of 32).  TO float with k_splits > 1: planes (k_split_plane(); grouped: of a.L rows in
+// the order of a.group_perm, N % 4 == 0) of K ranges.  FP: the
 // modes of FpPairDequant.  GLU: gated pairs of columns of W and a.w_alt, 128 to a tile.
 template <typename T, typename TO, int BITS, int MT_, int FP = 0, bool GLU = false>
 __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   const int ny = __builtin_amdgcn_readfirstlane(
       GROUPED ? *a.group_ntiles : (a.M + kTileRows - 1) / kTileRows);
   const int plane = nx * ny;
-  const int tiles = plane * (GROUPED ? 1 : k_splits);
+  const int tiles = plane * k_splits;
   // Rounds of gridDim.x tiles.  Workgroups b, b + 8, .. share an XCD: they take neighbouring
   // tiles, and what is left for the last round is dealt out evenly to the XCDs.
   const int stride = gridDim.x;
@@ -396,6 +397,7 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     TO* out = static_cast<TO*>(a.out);
     uint32_t bytes; // behind `out`: what lies past it is not stored
     if constexpr (GROUPED) {
+      out += static_cast<int64_t>(my_z) * a.L * ldy; // (of a plane)
       bytes = static_cast<uint32_t>(a.L) * static_cast<uint32_t>(ldy) * sizeof(TO);
     } else {
       out += (static_cast<int64_t>(my_z) * a.M + my_m0) * ldy;
@@ -414,7 +416,9 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     own_unroll<MT>([&](auto f) OWN_INLINE {
       const int mr = 16 * f + fi;
       if constexpr (GROUPED) {
-        const uint32_t row = a.group_perm[my_row0 + (mr < my_rows ? mr : my_rows - 1)];
+        // (planes: rows in their sorted order)
+        const int pos = my_row0 + (mr < my_rows ? mr : my_rows - 1);
+        const uint32_t row = sizeof(TO) == 4 ? pos : a.group_perm[pos];
         off[f] = mr < my_rows ? (row * static_cast<uint32_t>(ldy) + n) * sizeof(TO) : kNoStore;
       } else {
         off[f] = (static_cast<uint32_t>(mr) * static_cast<uint32_t>(ldy) + n) * sizeof(TO);

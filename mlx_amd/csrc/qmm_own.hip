@@ -116,11 +116,47 @@ int launch_qmm_own(
                                    : launch_qmm_own_f16(a, gs, codes, pl, s);
 }
 
+// Tiles that leave units idle over a long K: ranges of 1024 codes or more, up to four, with the
+// least time by qmm_own_plan's account of a step, of planes and their sum.  8 experts, 4096 x
+// 14336 4-bit, 300 tokens to 2 experts each: the product 231 us without ranges, the whole call
+// 486 / 407 (600 tokens, by scratch without: 643 against 692 of the tile kernel).  From a round
+// of tiles on the order of the list evens the workgroups' shares out, and ranges gain nothing
+// (2048 tokens, two ranges: 1.07 of the tile kernel, 1.07..1.12 without).
+int qmm_own_experts_splits(const QmmArgs& a, int bits, size_t room) {
+  const size_t plane = static_cast<size_t>(a.L) * a.N * sizeof(float);
+  if (a.N % 4 != 0 || plane >= kNoStore) {
+    return 1;
+  }
+  const long cus = compute_units();
+  const long expected = expected_tiles(a.L, a.n_experts);
+  const long least = a.n_experts < a.L ? a.n_experts : a.L;
+  const long high = expected > least ? expected : least;
+  const long tiles = high * ((a.N + kOwnBN - 1) / kOwnBN);
+  if (tiles >= cus) {
+    return 1;
+  }
+  const int mt = static_cast<int>((a.L / high + 31) / 32 * 2);
+  const Step& step = step_of(bits);
+  const double each =
+      a.K / kOwnBK * (step.fixed + (mt < 4 ? 4 : mt > 16 ? 16 : mt) * (step.each + step.busy));
+  int best = 1;
+  double best_us = 0.0;
+  for (int s = 1; s <= 4 && (s == 1 || (s * 1024 <= a.K && s * plane <= room)); ++s) {
+    const double us = each / s * static_cast<double>((tiles * s + cus - 1) / cus) +
+        (s > 1 ? 6.6 + (0.89 * s + 0.15) * 1e-6 / sizeof(float) * static_cast<double>(plane) : 0.0);
+    if (s == 1 || us < 0.95 * best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 int launch_qmm_own_experts(
-    const QmmArgs& a, int gs, int bits, int dtype, bool glu, hipStream_t s) {
-  MLXROCM_REHEARSE("qmm_own_experts%s", glu ? "_glu" : "");
-  return dtype == MLXROCM_BFLOAT16 ? launch_qmm_own_experts_bf16(a, gs, bits, glu, s)
-                                   : launch_qmm_own_experts_f16(a, gs, bits, glu, s);
+    const QmmArgs& a, int gs, int bits, int dtype, bool glu, int k_splits, hipStream_t s) {
+  MLXROCM_REHEARSE("qmm_own_experts%s(ksplit=%d)", glu ? "_glu" : "", k_splits);
+  return dtype == MLXROCM_BFLOAT16 ? launch_qmm_own_experts_bf16(a, gs, bits, glu, k_splits, s)
+                                   : launch_qmm_own_experts_f16(a, gs, bits, glu, k_splits, s);
 }
 
 } // namespace mlxrocm

@@ -3,8 +3,9 @@
 
 namespace mlxrocm {
 
-int launch_qmm_own_experts_bf16(const QmmArgs& a, int gs, int bits, bool glu, hipStream_t s) {
-  return glu ? own_experts<bf16_t, true>(a, gs, bits, s) : own_experts<bf16_t, false>(a, gs, bits, s);
+int launch_qmm_own_experts_bf16(
+    const QmmArgs& a, int gs, int bits, bool glu, int k_splits, hipStream_t s) {
+  return own_experts<bf16_t>(a, gs, bits, glu, k_splits, s);
 }
 
 } // namespace mlxrocm

@@ -1345,15 +1345,21 @@ int launch_qmm_slab_grouped(
   if (rc != MLXROCM_OK || pl.ranges <= 1) {
     return rc;
   }
+  return reduce_grouped_planes(a, pl.planes, pl.ranges, pl.plane_elems, dtype, s);
+}
+
+int reduce_grouped_planes(
+    const QmmArgs& a, const float* planes, int ranges, int64_t plane_elems, int dtype,
+    hipStream_t s) {
   const int64_t threads = static_cast<int64_t>(a.L) * (a.N / 4);
   const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
   if (dtype == MLXROCM_BFLOAT16) {
     slab_reduce_grouped_kernel<bf16_t><<<blocks, 256, 0, s>>>(
-        pl.planes, pl.ranges, pl.plane_elems, a.group_perm, a.group_ntiles + 1,
+        planes, ranges, plane_elems, a.group_perm, a.group_ntiles + 1,
         static_cast<bf16_t*>(a.out), a.N);
   } else {
     slab_reduce_grouped_kernel<f16_t><<<blocks, 256, 0, s>>>(
-        pl.planes, pl.ranges, pl.plane_elems, a.group_perm, a.group_ntiles + 1,
+        planes, ranges, plane_elems, a.group_perm, a.group_ntiles + 1,
         static_cast<f16_t*>(a.out), a.N);
   }
   MLXROCM_HIP_TRY(hipGetLastError());

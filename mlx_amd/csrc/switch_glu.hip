@@ -323,5 +323,7 @@ extern "C" int mlxrocm_switch_glu(
   o.w_batch_stride = w_out;
   o.sb_batch_stride = 2 * sb_out;
   o.sb_transposed = 2;
-  return launch_qmm_mfma_experts(o, group_size, bits, dtype, s);
+  // (planes of K ranges where the images of the first two products were: side by side, done with)
+  return launch_qmm_mfma_experts(
+      o, group_size, bits, dtype, ws + l.gate_image, l.down_image - l.gate_image, s);
 }

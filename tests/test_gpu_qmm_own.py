@@ -14,23 +14,24 @@ BITS = (2, 3, 4, 5, 6, 8)
 ROWS = (1, 16, 17, 63, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 255, 256, 257, 0, 600)
 
 
-def _indices(tokens, dtype=torch.int64):
-    e = torch.cat([torch.full((n,), i) for i, n in enumerate(ROWS)])
+def _indices(rows):
+    e = torch.cat([torch.full((n,), i) for i, n in enumerate(rows)])
     g = torch.Generator().manual_seed(5)
-    return e[torch.randperm(len(e), generator=g)].reshape(tokens, -1).to("cuda", dtype)
+    return e[torch.randperm(len(e), generator=g)].reshape(-1, 1).to("cuda")
 
 
 @pytest.mark.parametrize("bits", BITS)
-@pytest.mark.parametrize("D,F", [
-    (128, 1664),  # one step of K, 13 tiles of gated columns: more tiles than workgroups
-    (2944, 128),  # 23 steps, one of the second product; 11.5 tiles of columns
+@pytest.mark.parametrize("D,F,rows,group", [
+    (128, 1664, ROWS, 64),  # one step of K, 13 tiles of gated columns: more tiles than workgroups
+    (2944, 128, ROWS, 128), # 23 steps, one of the second product; 11.5 tiles of columns
+    (384, 2432, (1, 0, 97, 182), 32),  # the second product in ranges of 9 and 10 steps
+    (128, 5248, (2, 65, 0, 199), 32),  # the same, in four
 ])
-def test_experts(D, F, bits):
+def test_experts(D, F, rows, group, bits):
     dtype = torch.bfloat16 if (bits + D) % 2 else torch.float16
-    group = (32, 64, 128)[bits % 3]
     torch.manual_seed(bits)
-    block = nn.SwitchGLU(D, F, len(ROWS), group_size=group, bits=bits, dtype=dtype)
-    idx = _indices(sum(ROWS))
+    block = nn.SwitchGLU(D, F, len(rows), group_size=group, bits=bits, dtype=dtype)
+    idx = _indices(rows)
     x = torch.randn((idx.shape[0], D), device="cuda").to(dtype)
     assert block._in_one_call(x, idx) is not None
     y = block(x, idx)
@@ -45,7 +46,7 @@ def test_experts(D, F, bits):
         return w.flatten(1).to(dtype).double()
 
     want = torch.empty(y.shape, device="cuda", dtype=torch.float64)
-    for e, n in enumerate(ROWS):
+    for e, n in enumerate(rows):
         at = idx == e
         assert int(at.sum()) == n
         if n:

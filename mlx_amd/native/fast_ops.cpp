@@ -275,22 +275,26 @@ PyObject* quantized_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor out = new_tensor(with_last(*x, N), x->scalar_type(), device);
   void* stream = stream_of(device);
   int rc = 0;
-  if (mode == kAffine && transpose && abi.rows_supported(M, N, K, 1, gs, bits, code)) {
-    const Workspace ws(abi.rows_workspace_size(M, N, K, 1, gs, bits, code), device);
-    Py_BEGIN_ALLOW_THREADS;
-    rc = abi.rows(
-        x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
-        biases->data_ptr(), out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code, ws.ptr(),
-        ws.bytes, stream);
-    Py_END_ALLOW_THREADS;
-  } else if (mode == kAffine) {
+  if (mode == kAffine) {
+    const bool rows = transpose && abi.rows_supported(M, N, K, 1, gs, bits, code);
     const Workspace ws(
-        abi.qmm_workspace_size(M, N, K, 1, 0, gs, bits, code, transpose), device);
+        rows ? abi.rows_workspace_size(M, N, K, 1, gs, bits, code)
+             : abi.qmm_workspace_size(M, N, K, 1, 0, gs, bits, code, transpose),
+        device);
     Py_BEGIN_ALLOW_THREADS;
-    rc = abi.qmm_prepacked(
-        x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
-        biases->data_ptr(), image, out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code,
-        transpose, ws.ptr(), ws.bytes, stream);
+    // (up to 64 rows no kernel of qmm_rows reads an image; beyond, qmm_prepacked with its
+    // scratch runs the same kernel on the caller's image)
+    if (rows && (image == nullptr || M <= 64)) {
+      rc = abi.rows(
+          x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
+          biases->data_ptr(), out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code, ws.ptr(),
+          ws.bytes, stream);
+    } else {
+      rc = abi.qmm_prepacked(
+          x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
+          biases->data_ptr(), image, out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code,
+          transpose, ws.ptr(), ws.bytes, stream);
+    }
     Py_END_ALLOW_THREADS;
   } else if (transpose && abi.fp_rows_supported(M, N, K, 1, mode, code)) {
     const Workspace ws(abi.fp_rows_workspace_size(M, N, K, 1, mode, code), device);

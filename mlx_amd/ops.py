@@ -622,10 +622,18 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
                 "[quantized_matmul] sb_image does not belong to these scales and biases "
                 "(quantized_matmul_sb_image with the same dtype, transpose=True)"
             )
-    if transpose and lib.mlxrocm_qmm_rows_supported(M, w_outer, K, L, group_size, bits, code):
-        # the rows of a decode step of some sequences (an image is for prefill)
+    rows = transpose and lib.mlxrocm_qmm_rows_supported(M, w_outer, K, L, group_size, bits, code)
+    if rows:
         ws_bytes = lib.mlxrocm_qmm_rows_workspace_size(M, w_outer, K, L, group_size, bits, code)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    else:
+        ws_bytes = lib.mlxrocm_qmm_workspace_size(
+            M, w_outer, K, L, int(w_stride != 0), group_size, bits, code, int(bool(transpose))
+        )
+    # a temporary of the call, like the ones eval_gpu hands to add_temporary
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    # (up to 64 rows no kernel of qmm_rows reads an image; beyond, qmm_prepacked with its scratch
+    # runs the same kernel on the caller's image)
+    if rows and (sb_image is None or M <= 64):
         _lib.check(
             lib.mlxrocm_qmm_rows(
                 xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(), out.data_ptr(),
@@ -634,11 +642,6 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
             )
         )
         return out
-    ws_bytes = lib.mlxrocm_qmm_workspace_size(
-        M, w_outer, K, L, int(w_stride != 0), group_size, bits, code, int(bool(transpose))
-    )
-    # a temporary of the call, like the ones eval_gpu hands to add_temporary
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     _lib.check(
         lib.mlxrocm_qmm_prepacked(
             xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(),

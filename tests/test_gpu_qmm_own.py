@@ -150,6 +150,28 @@ def test_replayed_from_a_graph():
         assert torch.equal(y, mlx_amd.quantized_matmul(x, wq, s, b)), seed
 
 
+@pytest.mark.parametrize("N,K,bits", ((1024, 4096, 8), (1024, 4096, 4), (2048, 1024, 2)))
+def test_a_kept_image_is_read(N, K, bits):
+    """The caller's image of scales and biases takes the place of one made in the call, with
+    and without K ranges, on the host path and beside it."""
+    lib = _lib.load()
+    wq, s, b = mlx_amd.quantize((torch.randn((N, K), device="cuda") / 64).bfloat16(), 64, bits)
+    taken = [M for M in (200, 640, 1500, 4096)
+             if lib.mlxrocm_qmm_rows_supported(M, N, K, 1, 64, bits, _lib.BFLOAT16)]
+    assert taken
+    kw = dict(group_size=64, bits=bits)
+    image = mlx_amd.quantized_matmul_sb_image(s, b, 64)
+    for M in taken:
+        x = torch.randn((M, K), device="cuda").bfloat16()
+        strided = torch.stack([x, x], dim=-1)[..., 0]
+        want = mlx_amd.quantized_matmul(x, wq, s, b, **kw)
+        for rows in (x, strided):
+            assert torch.equal(mlx_amd.quantized_matmul(rows, wq, s, b, **kw, sb_image=image), want)
+            # (doubling is exact: a call that makes its own image gives `want` here as well)
+            twice = mlx_amd.quantized_matmul(rows, wq, s, b, **kw, sb_image=2 * image)
+            assert torch.equal(twice, 2 * want), M
+
+
 @pytest.mark.parametrize("bits", (3, 8))
 @pytest.mark.parametrize("E,D,F,tokens", ((8, 512, 384, 70), (4, 2176, 256, 70)))
 def test_few_pairs_of_an_expert(bits, E, D, F, tokens):

@@ -589,7 +589,7 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
     if not affine:
         fp = _MODE_CODE[mode]
         if transpose and lib.mlxrocm_fp_qmm_rows_supported(M, w_outer, K, L, fp, code):
-            # the rows of a decode step of some sequences
+            # a decode step of some sequences, or many rows where other tiles are ahead
             ws_bytes = lib.mlxrocm_fp_qmm_rows_workspace_size(M, w_outer, K, L, fp, code)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
             _lib.check(

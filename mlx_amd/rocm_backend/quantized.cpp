@@ -160,7 +160,7 @@ void QuantizedMatmul::eval_gpu(const std::vector<array>& inputs, array& out) {
   if (!affine) {
     // inputs are {x, w, scales}: no biases (mlx/ops.cpp:4816-4821)
     const int mode = fp_mode_code(mode_);
-    // the rows of a decode step of some sequences have a kernel of their own
+    // kernels beside the table of mlxrocm_qmm: a decode step of some sequences, many rows
     const bool rows = transpose_ && mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dt) != 0;
     const size_t ws_bytes = rows
         ? mlxrocm_fp_qmm_rows_workspace_size(M, N, K, L, mode, dt)
@@ -213,7 +213,7 @@ void QuantizedMatmul::eval_gpu(const std::vector<array>& inputs, array& out) {
   }
   array biases = ensure_row_contiguous(inputs[3], enc, s);
 
-  // the rows of a decode step of some sequences have a kernel of their own
+  // kernels beside the table of mlxrocm_qmm: a decode step of some sequences, many rows
   const bool rows = transpose_ &&
       mlxrocm_qmm_rows_supported(M, N, K, L, group_size_, bits_, dt) != 0;
   // device scratch of the call: a temporary like any other

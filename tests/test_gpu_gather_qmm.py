@@ -276,6 +276,28 @@ def test_gather_qmm_grouped_matches_ungrouped(gpu):
     assert float(diff) <= 2 ** -7 * float(scale)
 
 
+@pytest.mark.parametrize("E,T", ((1, 700), (64, 5000), (65, 2500), (200, 16384), (130, 16385), (9, 1024)))
+def test_gather_qmm_many_experts(gpu, E, T):
+    """Grouping over more experts than a wavefront has lanes and as many pairs as one workgroup
+    takes (and one more), half of the experts unused, some pairs without an expert."""
+    N, K, dtype = 64, 128, torch.bfloat16
+    assert _grouped_ws_bytes(1, N, K, T, E, 64, 8) > 0
+    wq, s, b = mlx_amd.quantize(normal_weights((E, N, K), dtype, std=0.5).to(gpu), 64, 8)
+    x = activations((32, 1, K), dtype).to(gpu)
+    g = torch.Generator().manual_seed(E + T)
+    used = torch.randperm(E, generator=g)[:(E + 1) // 2]
+    rhs = used[torch.randint(0, len(used), (T,), generator=g) ** 2 % len(used)].to(gpu)
+    lhs = torch.randint(0, 32, (T,), generator=g).to(gpu)
+    rhs[3::97] = E
+    got = mlx_amd.gather_qmm(x, wq, s, b, lhs, rhs, True, 64, 8)
+    lhs, rhs, x = lhs.cpu(), rhs.cpu(), x.cpu()
+    w_hat = exact_affine_weights(wq.cpu(), s.cpu(), b.cpu(), 64, 8)
+    every = (x.reshape(32, K).double() @ w_hat.reshape(E * N, K).T).reshape(32, E, N)
+    exact = every[lhs, rhs.clamp(max=E - 1)] * (rhs < E)[:, None]
+    err = float((got.cpu().reshape(T, N).double() - exact).abs().max())
+    assert err <= exact_tolerance(dtype, K, x, w_hat, exact)
+
+
 @pytest.mark.parametrize("bits,gs", ((4, 64), (5, 32), (8, 128)))
 def test_gather_qmm_small_groups(oracle, gpu, bits, gs):
     """A few index pairs per expert (at most 64 on average): the pairs are

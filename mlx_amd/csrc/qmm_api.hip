@@ -1802,6 +1802,39 @@ int gather_entry(
     size_t workspace_bytes, hipStream_t s);
 } // namespace
 
+namespace mlxrocm {
+
+size_t gather_gated_bytes(
+    int N, int K, int n_indices, int n_experts, int x_batches, int64_t x_batch_stride, int gs,
+    int bits, int dtype) {
+  if (!group_gather(
+          1, N, K, n_indices, n_experts, x_batches, x_batch_stride, gs, bits, dtype, true) ||
+      !group_gather_slab(N, K, n_indices, n_experts, gs, bits) ||
+      !qmm_slab_plans_in_kernel(n_indices, n_experts)) {
+    return 0;
+  }
+  const size_t planes = qmm_slab_grouped_plane_bytes(n_indices, N, K);
+  return planes == 0 ? 0 : gather_group_workspace_bytes(n_indices, n_experts) + 2 * planes;
+}
+
+int gather_gated(
+    const QmmArgs& gate, const QmmArgs& up, int gs, int bits, int dtype, void* workspace,
+    hipStream_t s) {
+  QmmArgs both[2] = {gate, up};
+  for (QmmArgs& a : both) {
+    const int rc = check_alignment("switch_glu", a, dtype, true, bits);
+    if (rc != MLXROCM_OK) {
+      return rc;
+    }
+    bind_gather_group(a, kGroupSmallTile, workspace);
+  }
+  return launch_qmm_slab_grouped_gated(
+      both[0], both[1], gs, dtype,
+      static_cast<char*>(workspace) + gather_group_workspace_bytes(gate.L, gate.n_experts), s);
+}
+
+} // namespace mlxrocm
+
 extern "C" int mlxrocm_gather_qmm(
     const void* x,
     const uint32_t* wq,

@@ -215,6 +215,17 @@ bool qmm_slab_plans_in_kernel(int n_indices, int n_experts);
 int launch_qmm_slab_grouped(
     const QmmArgs& a, int gs, int bits, int dtype, void* planes, bool plan_in_kernel,
     hipStream_t s);
+int launch_qmm_slab_grouped_gated(
+    const QmmArgs& gate, const QmmArgs& up, int gs, int dtype, void* planes, hipStream_t s);
+// Scratch (qmm_api.hip) of h = silu(x Wg^T) * (x Wu^T) over index pairs, one row of x each, on
+// that kernel; 0: mlxrocm_gather_qmm takes the two products elsewhere.
+size_t gather_gated_bytes(
+    int N, int K, int n_indices, int n_experts, int x_batches, int64_t x_batch_stride, int gs,
+    int bits, int dtype);
+// gate.out and up.out are h; a scratch of that many bytes, 16-byte aligned.
+int gather_gated(
+    const QmmArgs& gate, const QmmArgs& up, int gs, int bits, int dtype, void* workspace,
+    hipStream_t s);
 // fp32 operands on the bf16 matrix path: x is first split into bf16 high and
 // low parts (split_x_for_mfma into a buffer of split_x_bytes), then
 // launch_qmm_mfma_split runs with a.x pointing at that buffer.

@@ -1200,6 +1200,45 @@ __global__ __launch_bounds__(256) void slab_reduce_grouped_kernel(
   *reinterpret_cast<uint2*>(out + static_cast<int64_t>(perm[pos]) * N + n) = packed;
 }
 
+// h[perm[pos]] = silu(gate) * up, both the sums of their K ranges rounded to T as
+// slab_reduce_grouped_kernel does.  Bound by its launch: 8 tokens to 2 of 8 experts, 4096 x
+// 14336, two reductions and a pass over their results took 4.8 us each under a trace, this one
+// 4.8 in the place of all three.
+template <typename T>
+__global__ __launch_bounds__(256) void slab_reduce_gated_kernel(
+    const float* gate,
+    const float* up,
+    int ranges,
+    int64_t plane_elems,
+    const int32_t* perm,
+    const int32_t* n_rows,
+    T* h,
+    int N) {
+  const int rows = *n_rows;
+  const int quads = N / 4;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t pos = i / quads;
+  if (pos >= rows) {
+    return;
+  }
+  const int n = static_cast<int>(i - pos * quads) * 4;
+  floatx4 g = {0.0f, 0.0f, 0.0f, 0.0f};
+  floatx4 u = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int r = 0; r < ranges; ++r) {
+    g += *reinterpret_cast<const floatx4*>(gate + r * plane_elems + pos * N + n);
+    u += *reinterpret_cast<const floatx4*>(up + r * plane_elems + pos * N + n);
+  }
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = gated<T>(round_to<T>(g[e]), round_to<T>(u[e]));
+  }
+  uint2 packed;
+  packed.x = pack2<T>(v[0], v[1]);
+  packed.y = pack2<T>(v[2], v[3]);
+  *reinterpret_cast<uint2*>(h + static_cast<int64_t>(perm[pos]) * N + n) = packed;
+}
+
 template <typename T, int GS, int MT, int MODE>
 int launch_one(const QmmArgs& a, const SlabPlan& pl, hipStream_t s) {
   constexpr size_t smem = slab_smem_bytes<GS, MT, MODE>();
@@ -1322,20 +1361,32 @@ bool qmm_slab_plans_in_kernel(int n_indices, int n_experts) {
   return n_indices <= kSlPlanPairs && n_experts <= kSlPlanExperts;
 }
 
+namespace {
+
+// 16-row tiles: few pairs per expert (8 on average at most) and the kernel's own grouping.  They
+// leave LDS for a third ring slot; an expert that does get more than 16 rows is then read once per
+// tile.  32-wide groups have no two-tile form at all.
+bool slab_one_tile(const QmmArgs& a, int gs, bool plan_in_kernel) {
+  return plan_in_kernel &&
+      (gs == 32 || static_cast<int64_t>(a.L) <= 8 * static_cast<int64_t>(a.n_experts));
+}
+
+SlabPlan slab_grouped_plan(const QmmArgs& a, int tile_rows, void* planes) {
+  SlabPlan pl = make_plan(a.N, a.K, gather_group_max_tiles(a.L, a.n_experts, tile_rows));
+  pl.planes = static_cast<float*>(planes);
+  pl.plane_elems = static_cast<int64_t>(a.L) * a.N;
+  return pl;
+}
+
+} // namespace
+
 int launch_qmm_slab_grouped(
     const QmmArgs& a, int gs, int bits, int dtype, void* planes, bool plan_in_kernel,
     hipStream_t s) {
   (void)bits;
-  // Few pairs per expert (8 on average at most) and the kernel's own grouping:
-  // 16-row tiles, which leave LDS for a third ring slot; an expert that does get
-  // more than 16 rows is then read once per tile.  32-wide groups have no
-  // two-tile form at all.
-  const bool one_tile = plan_in_kernel &&
-      (gs == 32 || static_cast<int64_t>(a.L) <= 8 * static_cast<int64_t>(a.n_experts));
+  const bool one_tile = slab_one_tile(a, gs, plan_in_kernel);
   const int tile_rows = one_tile ? 16 : kGroupSmallTile;
-  SlabPlan pl = make_plan(a.N, a.K, gather_group_max_tiles(a.L, a.n_experts, tile_rows));
-  pl.planes = static_cast<float*>(planes);
-  pl.plane_elems = static_cast<int64_t>(a.L) * a.N;
+  const SlabPlan pl = slab_grouped_plan(a, tile_rows, planes);
   MLXROCM_REHEARSE(
       "qmm_slab_grouped(%s,tile=%d,ranges=%d)", plan_in_kernel ? "plans" : "planned", tile_rows,
       pl.ranges);
@@ -1346,6 +1397,39 @@ int launch_qmm_slab_grouped(
     return rc;
   }
   return reduce_grouped_planes(a, pl.planes, pl.ranges, pl.plane_elems, dtype, s);
+}
+
+// h = silu(gate) * up for two products over the same pairs, in more than one K range; the order
+// of the pairs that the kernel finds depends on them alone, so the planes of both agree.
+// planes: twice qmm_slab_grouped_plane_bytes().
+int launch_qmm_slab_grouped_gated(
+    const QmmArgs& gate, const QmmArgs& up, int gs, int dtype, void* planes, hipStream_t s) {
+  const bool one_tile = slab_one_tile(gate, gs, true);
+  const int tile_rows = one_tile ? 16 : kGroupSmallTile;
+  const SlabPlan of_gate = slab_grouped_plan(gate, tile_rows, planes);
+  const SlabPlan of_up = slab_grouped_plan(
+      up, tile_rows, of_gate.planes + of_gate.ranges * of_gate.plane_elems);
+  MLXROCM_REHEARSE("qmm_slab_grouped_gated(tile=%d,ranges=%d)", tile_rows, of_gate.ranges);
+  int rc = launch_any<2>(gate, of_gate, gs, dtype, one_tile ? 1 : 2, s);
+  if (rc == MLXROCM_OK) {
+    rc = launch_any<2>(up, of_up, gs, dtype, one_tile ? 1 : 2, s);
+  }
+  if (rc != MLXROCM_OK) {
+    return rc;
+  }
+  const int64_t threads = static_cast<int64_t>(gate.L) * (gate.N / 4);
+  const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
+  if (dtype == MLXROCM_BFLOAT16) {
+    slab_reduce_gated_kernel<bf16_t><<<blocks, 256, 0, s>>>(
+        of_gate.planes, of_up.planes, of_gate.ranges, of_gate.plane_elems, gate.group_perm,
+        gate.group_ntiles + 1, static_cast<bf16_t*>(gate.out), gate.N);
+  } else {
+    slab_reduce_gated_kernel<f16_t><<<blocks, 256, 0, s>>>(
+        of_gate.planes, of_up.planes, of_gate.ranges, of_gate.plane_elems, gate.group_perm,
+        gate.group_ntiles + 1, static_cast<f16_t*>(gate.out), gate.N);
+  }
+  MLXROCM_HIP_TRY(hipGetLastError());
+  return MLXROCM_OK;
 }
 
 int reduce_grouped_planes(

@@ -89,14 +89,15 @@ bool tiled(int tokens, int top, int D, int F, int E, int least) {
 struct Layout {
   size_t expert, row, self; // u32 [pairs] each
   size_t h;                 // [pairs, F]
-  size_t up;                // [pairs, F] (not tiled)
+  size_t up;                // [pairs, F] (products one by one)
+  bool gated;               // not tiled: the first two products meet in h (gather_gated)
   size_t rest;              // workspace of the products (tables and images: tiled)
   size_t gate_image, up_image, down_image;
   size_t total;
 };
 
-// room: what the caller has.  One with too little for tiles of few pairs has the products one
-// by one.
+// room: what the caller has.  One with too little for tiles of few pairs, or for the planes of
+// two products, has the products one by one.
 Layout layout_of(
     int tokens, int top, int D, int F, int E, int gs, int bits, int dtype, bool* tiles,
     size_t room = SIZE_MAX, int least = 0) {
@@ -120,12 +121,16 @@ Layout layout_of(
     l.up_image = take(qmm_n_sb_bytes(F, D / gs, E, dtype));
     l.down_image = take(qmm_n_sb_bytes(D, F / gs, E, dtype));
   } else {
-    l.up = take(pairs * F * dtype_size(dtype));
     const size_t in = mlxrocm_gather_qmm_workspace_size(
         1, F, D, static_cast<int>(pairs), E, gs, bits, dtype, 1, 0);
     const size_t out = mlxrocm_gather_qmm_workspace_size(
         1, D, F, static_cast<int>(pairs), E, gs, bits, dtype, 1, 0);
-    l.rest = take(in > out ? in : out);
+    const size_t both = gather_gated_bytes(
+        F, D, static_cast<int>(pairs), E, tokens, D, gs, bits, dtype);
+    l.gated = both != 0 && at + round256(both > out ? both : out) <= room;
+    l.up = l.gated ? 0 : take(pairs * F * dtype_size(dtype));
+    const size_t first = l.gated ? both : in;
+    l.rest = take(first > out ? first : out);
   }
   l.total = at;
   return l.total > room && *tiles && least == 0
@@ -236,7 +241,40 @@ extern "C" int mlxrocm_switch_glu(
     void* up = ws + l.up;
     void* rest = ws + l.rest;
     const size_t rest_bytes = workspace_bytes - l.rest;
-    int rc = mlxrocm_gather_qmm(
+    int rc;
+    if (l.gated) {
+      // two launches less: 8 tokens to 2 of 8 experts, 4096 x 14336, 190.3 -> 185.3 us
+      // (64 tokens 236 -> 231, 256 tokens 555 -> 549; 64 experts 2048 x 1408, 32 tokens to 6
+      // 114 -> 109)
+      QmmArgs gate{};
+      gate.x = x;
+      gate.w = gate_w;
+      gate.scales = gate_scales;
+      gate.biases = gate_biases;
+      gate.out = h;
+      gate.M = 1;
+      gate.N = F;
+      gate.K = D;
+      gate.L = pairs;
+      gate.x_batch_stride = D;
+      gate.w_batch_stride = w_in;
+      gate.sb_batch_stride = sb_in;
+      gate.lhs_indices = row;
+      gate.rhs_indices = expert;
+      gate.x_batches = tokens;
+      gate.n_experts = E;
+      QmmArgs other = gate;
+      other.w = up_w;
+      other.scales = up_scales;
+      other.biases = up_biases;
+      rc = gather_gated(gate, other, group_size, bits, dtype, rest, s);
+      return rc != MLXROCM_OK
+          ? rc
+          : mlxrocm_gather_qmm(
+                h, down_w, down_scales, down_biases, self, expert, out, 1, D, F, pairs, pairs, E, F,
+                w_out, sb_out, group_size, bits, dtype, 1, 0, rest, rest_bytes, stream);
+    }
+    rc = mlxrocm_gather_qmm(
         x, gate_w, gate_scales, gate_biases, row, expert, h, 1, F, D, pairs, tokens, E, D, w_in,
         sb_in, group_size, bits, dtype, 1, 0, rest, rest_bytes, stream);
     if (rc == MLXROCM_OK) {

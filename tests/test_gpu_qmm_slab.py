@@ -231,3 +231,36 @@ def test_rows8_batched(oracle, gpu):
     w_hat = exact_affine_weights(wq, s, b, 64, 4)
     exact = torch.einsum("lmk,lnk->lmn", x.double(), w_hat)
     assert float((got.double() - exact).abs().max()) <= exact_tolerance(dtype, K, x, w_hat, exact)
+
+
+@pytest.mark.parametrize("E,D,F,tokens,top,gs", (
+    (8, 2048, 4096, 4, 2, 64),     # as few pairs as are grouped
+    (3, 2560, 4096, 9, 2, 32),  # a short last K range, 16-row tiles
+    (64, 1536, 2304, 85, 6, 128),  # 510 pairs, more than one tile of an expert
+))
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+def test_gated_planes(E, D, F, tokens, top, gs, dtype):
+    """The two first products of a routed MLP whose planes meet in the gate: with the scratch the
+    call names, and one by one with less, the same bits; a pair without an expert is zero."""
+    lib = _lib.load()
+    torch.manual_seed(tokens)
+    block = mlx_amd.nn.SwitchGLU(D, F, E, group_size=gs, bits=4, dtype=dtype)
+    x = torch.randn((tokens, D), device="cuda").to(dtype)
+    idx = torch.randint(0, E, (tokens, top), device="cuda")
+    idx[2, 1] = E
+    need = lib.mlxrocm_switch_glu_workspace_size(tokens, top, D, F, E, gs, 4, CODE[dtype])
+    planes = -(-D // 1024) * tokens * top * F * 4
+    assert need > 2 * planes  # both at once
+    ops = [t for layer in (block.gate_proj, block.up_proj, block.down_proj)
+           for t in (layer.weight, layer.scales, layer.biases)]
+    got = []
+    for room in (need, need - 1):
+        ws = torch.full((room,), 0x7f, dtype=torch.uint8, device="cuda")
+        out = torch.full((tokens, top, D), 7.0, dtype=dtype, device="cuda")
+        _lib.check(lib.mlxrocm_switch_glu(
+            x.data_ptr(), idx.data_ptr(), 8, *[t.data_ptr() for t in ops], out.data_ptr(), tokens,
+            top, D, F, E, gs, 4, CODE[dtype], ws.data_ptr(), room,
+            torch.cuda.current_stream().cuda_stream))
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(block(x, idx), got[0])
+    assert not got[0][2, 1].any() and float(got[0].float().abs().sum()) > 0

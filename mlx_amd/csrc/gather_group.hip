@@ -232,9 +232,9 @@ __device__ __forceinline__ int wave_counter_add(
 // What bounds it: the vector instructions of one compute unit, about 70 per wavefront and call of
 // wave_counter_add.  A pair's expert, and its rank among that expert's, which the count gives by the
 // way, stay in registers: the scatter adds them to the expert's first position and counts nothing
-// again.us of a routed MLP whose pairs it groups, counting twice -> once: 64 experts 2048 x 1408,
-// 2048 tokens to 6 265 -> 260 (the kernel under a trace 23.0 -> 19.4), 32 experts 1024 x 1024,
-// 900 tokens to 4 69.2 -> 67.3; 8 experts 552 -> 553 (10.6 -> 10.2).
+// again.  us of a routed MLP whose pairs it groups, counting twice -> once: 64 experts 2048 x
+// 1408, 2048 tokens to 6 265 -> 260 (this kernel under a trace 23.0 -> 19.4), 32 experts 1024 x
+// 1024, 900 tokens to 4 69.2 -> 67.3; 8 experts 4096 x 14336, 600 tokens 552 -> 553.
 template <typename T>
 __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     const uint32_t* lhs,

@@ -85,13 +85,15 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
   using DQ = std::conditional_t<FP != 0, FpPairDequant<T, (FP != 0 ? FP : 1)>, PairDequant<T, BITS>>;
   constexpr int kStage = own_stage_bytes(MT_);
   constexpr int kTileRows = GROUPED ? kOwnBM : 16 * MT_;
-  // A product of 4-bit codes without ranges of K: the matrix instructions of a step take its
-  // codes 32 by 32 in their order, as those of the tile kernel do, so that mlxrocm_qmm, a graph
-  // that holds it and mlxrocm_qmm_rows return the same bits.  A lane loads 32 codes in a row
-  // and gives 24 of them to the three lanes that hold the same row of W (swaps of registers
-  // between lanes, with scales and biases 24 vector instructions a step: 8192 x 14336 x 4096
-  // 685 -> 712 us).  Everywhere else the codes stay where they were loaded.
-  constexpr bool kInOrder = BITS == 4 && FP == 0 && !GROUPED && sizeof(TO) == 2;
+  // Without ranges of K the matrix instructions of a step take its 4-bit codes 32 by 32 in their
+  // order, and those of routed rows at 8 bits too: a result has the bits that the tile kernel
+  // gives in one range, so that which of the two runs does not show.  A lane loads 32 codes in a
+  // row and gives 24 of them to the three lanes that hold the same row of W (swaps of registers
+  // between lanes, with scales and biases 24 vector instructions a step, 32 at 8 bits: 8192 x
+  // 14336 x 4096 685 -> 712 us; routed, 2048 tokens to 2 of 8 experts, 4096 x 14336, the call 1401
+  // -> 1454.  Loads of a lane's own 8 codes instead, four for one: 1791).  Everywhere else the
+  // codes stay where they were loaded.
+  constexpr bool kInOrder = (BITS == 4 || (BITS == 8 && GROUPED)) && FP == 0 && sizeof(TO) == 2;
   constexpr int kCols = GLU ? kOwnBN / 2 : kOwnBN; // columns of y of a tile
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x;
@@ -255,7 +257,12 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     }
     sb[j][0] = snext[j].get(0);
     if constexpr (kInOrder) {
-      transpose_rows(wreg[j][0], wreg[j][1], wreg[j][2], wreg[j][3]);
+      constexpr int each = BITS / 4; // dwords of eight codes
+#pragma unroll
+      for (int i = 0; i < each; ++i) {
+        transpose_rows(
+            wreg[j][i], wreg[j][each + i], wreg[j][2 * each + i], wreg[j][3 * each + i]);
+      }
       sb[j][1] = sb[j][2] = sb[j][3] = sb[j][0];
       transpose_rows(sb[j][0], sb[j][1], sb[j][2], sb[j][3]);
     }

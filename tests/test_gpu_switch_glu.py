@@ -72,3 +72,24 @@ def test_pairs_ordered_by_expert_give_the_same_rows(D, dtype, tokens):
     block.sort_threshold = 1 << 20
     assert not block._sorts(x, idx)
     assert torch.equal(y, block(x, idx))
+
+
+@pytest.mark.parametrize("tokens,top,E,D,F,group", [
+    (700, 2, 4, 512, 1664, 64),    # the second product in one round of tiles
+    (3000, 4, 9, 1280, 640, 32),   # more rounds than one; 11 tiles of up to 256 rows an expert
+    (300, 2, 3, 1920, 1024, 128),  # few tiles
+])
+@pytest.mark.parametrize("bits", (4, 8))
+def test_the_bits_of_the_three_products(tokens, top, E, D, F, group, bits):
+    """Many rows, no ranges of K: whatever kernel takes a product sums its codes in their order,
+    as gather_qmm's tiles do, and the results agree to the bit (bfloat16: in float16 the gate of
+    torch and that of the one call round here and there differently)."""
+    dtype = torch.bfloat16
+    block = _block(D, F, E, group, bits, dtype)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn((tokens, D), generator=g, device="cuda").to(dtype)
+    idx = torch.randint(0, E, (tokens, top), generator=g, device="cuda")
+    y = block(x, idx)
+    block.activation = lambda t: torch.nn.functional.silu(t)
+    assert block._in_one_call(x, idx) is None
+    assert torch.equal(y, block(x, idx))

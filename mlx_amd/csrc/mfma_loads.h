@@ -105,6 +105,30 @@ struct RawWords {
   }
 };
 
+// ---- direct-to-LDS loads --------------------------------------------------------
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
+}
+
+// 64 lanes x 16 bytes from sbase + voff to LDS, lane by lane from `at` (uniform); vmcnt counts
+// them.  A load that takes its LDS address from M0 has to keep one wait state behind the write of
+// M0, or it may read the address before: the compiler, which keeps it for its own loads, does
+// not look into inline assembly.
+__device__ __forceinline__ void dma16(uint32_t at, uint32_t voff, const void* sbase) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(voff), "s"(sbase), "s"(at)
+               : "memory");
+}
+// 64 lanes x 4 bytes
+__device__ __forceinline__ void dma4(uint32_t at, uint32_t voff, const void* sbase) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+               :
+               : "v"(voff), "s"(sbase), "s"(at)
+               : "memory");
+}
+
 // One scale or bias value as loaded: 16 bits in the low half, or a float.
 template <typename TS>
 __device__ __forceinline__ void raw_load_value(uint32_t& v, uint32_t voff, const void* sbase) {

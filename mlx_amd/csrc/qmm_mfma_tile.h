@@ -302,15 +302,7 @@ __global__ __launch_bounds__(kThreads) void qmm_t_mfma_kernel(
 // x rows 32 w + 8 i .. + 7 of the tile at k0, straight into LDS stage `xs`
 // (element offset of the stage); completion is counted by vmcnt.
 #define QMM_DMA_X1(xs, k0, i, xoff)                                              \
-  do {                                                                           \
-    const T* g__ = p.x + (k0); /* uniform */                                     \
-    const uint32_t m0__ = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(     \
-        (__attribute__((address_space(3))) char*)(lds + (xs) + (wave * 32 + 8 * (i)) * kBK))); \
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"            \
-                 :                                                               \
-                 : "v"(xoff), "s"(g__), "s"(m0__)                                \
-                 : "memory");                                                    \
-  } while (0)
+  dma16(lds_address(lds + (xs) + (wave * 32 + 8 * (i)) * kBK), xoff, p.x + (k0))
 #define QMM_DMA_X(xs, k0)                                                        \
   do {                                                                           \
     QMM_DMA_X1(xs, k0, 0, xoff0);                                                \

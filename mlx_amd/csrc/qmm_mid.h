@@ -63,19 +63,6 @@ constexpr size_t mid_stage_bytes(int mf, int bits) {
       static_cast<size_t>(mid_stages(mf, bits) + 1) * mid_w_bytes(bits);
 }
 
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
-}
-
-// 64 lanes x 16 bytes from sbase + voff to LDS, lane by lane from `at`; vmcnt counts them.
-__device__ __forceinline__ void dma16(uint32_t at, uint32_t voff, const void* sbase) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(voff), "s"(sbase), "s"(at)
-               : "memory");
-}
-
 // Lets all but the `LEFT` newest loads of this wavefront land and its LDS reads end (the
 // stage they read is filled again behind the barrier), then meets the others.
 template <int LEFT>

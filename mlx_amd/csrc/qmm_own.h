@@ -268,14 +268,8 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     }
   };
   auto dma_x = [&](int stage, int k, auto i) OWN_INLINE {
-    const uint8_t* g = px + static_cast<size_t>(k) * 2;
-    const uint32_t voff = xoff[decltype(i)::value];
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-        (__attribute__((address_space(3))) char*)(smem + stage + (32 * i + 4 * wave) * 256)));
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(g), "s"(lds0)
-                 : "memory");
+    dma16(lds_address(smem + stage + (32 * i + 4 * wave) * 256), xoff[decltype(i)::value],
+          px + static_cast<size_t>(k) * 2);
   };
   int cur = 0; // stage of the step being multiplied
 

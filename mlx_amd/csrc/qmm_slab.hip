@@ -36,6 +36,7 @@
 // weight row are stored at piece ^ (row / 2 % 8), rows of x are 16 bytes longer
 // than a power of two.
 #include "mfma_dequant.h"
+#include "mfma_loads.h"
 #include "qmm_args.h"
 
 namespace mlxrocm {
@@ -130,11 +131,6 @@ __device__ __forceinline__ uint4 widen8(uint32_t w, uint32_t mask, uint32_t magi
   return r;
 }
 
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (__attribute__((address_space(3))) const char*)p));
-}
-
 // A wave-uniform pointer, in scalar registers whatever the compiler believes
 // about its uniformity.
 __device__ __forceinline__ const void* uniform_ptr(const void* p) {
@@ -144,14 +140,9 @@ __device__ __forceinline__ const void* uniform_ptr(const void* p) {
   return reinterpret_cast<const void*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// 16 bytes per lane from base + voff to LDS at m0 + 16 * lane.
-__device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t m0) {
-  base = uniform_ptr(base);
-  m0 = __builtin_amdgcn_readfirstlane(m0);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(voff), "s"(base), "s"(m0)
-               : "memory");
+// dma16() with a base and an address that the compiler need not know to be uniform.
+__device__ __forceinline__ void dma16_to(uint32_t at, uint32_t voff, const void* base) {
+  dma16(__builtin_amdgcn_readfirstlane(at), voff, uniform_ptr(base));
 }
 
 // 16 bytes per lane into registers, completion counted by vmcnt like the DMAs
@@ -402,7 +393,7 @@ __global__ __launch_bounds__(kSlThreads, 2) void qmm_slab_kernel(const QmmArgs a
     const uint32_t m0 = ring_lds + slot * kSlSlotBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      dma16(wb, w_off[i], m0 + i * 1024);
+      dma16_to(m0 + i * 1024, w_off[i], wb);
     }
   };
   InFlight4 sbq[kSbInstrs]; // in flight within one loop iteration only
@@ -951,8 +942,8 @@ __global__ __launch_bounds__(64 * kR8Tiles * KW) void qmm_rows8_kernel(const Qmm
       int n = n0 + r;
       n = n < N ? n : N - 1;
       const uint32_t off = static_cast<uint32_t>(n) * static_cast<uint32_t>(rbk) + c * 16;
-      dma16(p.scales, off, sb_lds + i * 1024);
-      dma16(p.biases, off, sb_lds + 16 * rbk + i * 1024);
+      dma16_to(sb_lds + i * 1024, off, p.scales);
+      dma16_to(sb_lds + 16 * rbk + i * 1024, off, p.biases);
     }
   }
   // ---- W: DMA i of a step fetches tile row 8 i + lane / 8, LDS piece lane % 8
@@ -970,8 +961,8 @@ __global__ __launch_bounds__(64 * kR8Tiles * KW) void qmm_rows8_kernel(const Qmm
     const int jc = step0 + (j < nsteps ? j : nsteps - 1); // past the end: again, into a free slot
     const uint8_t* wb = p.w + jc * (kSlStep / 2);
     const uint32_t m0 = ring_lds + slot * kR8SlotBytes;
-    dma16(wb, w_off[0], m0);
-    dma16(wb, w_off[1], m0 + 1024);
+    dma16_to(m0, w_off[0], wb);
+    dma16_to(m0 + 1024, w_off[1], wb);
   };
 #pragma unroll
   for (int i = 0; i < kR8Stages - 1; ++i) {

@@ -172,26 +172,9 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     }
   }
 
-  auto lds_addr = [&](int byte_off) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-        (__attribute__((address_space(3))) char*)(smem + byte_off)));
+  auto lds_at = [&](int byte_off) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(lds_address(smem + byte_off)));
   };
-#define QQ_DMA16(voff, gbase, lds_byte)                                          \
-  do {                                                                           \
-    const uint32_t m0__ = __builtin_amdgcn_readfirstlane(lds_addr(lds_byte));    \
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"            \
-                 :                                                               \
-                 : "v"(voff), "s"(gbase), "s"(m0__)                              \
-                 : "memory");                                                    \
-  } while (0)
-#define QQ_DMA4(voff, gbase, lds_byte)                                           \
-  do {                                                                           \
-    const uint32_t m0__ = __builtin_amdgcn_readfirstlane(lds_addr(lds_byte));    \
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"              \
-                 :                                                               \
-                 : "v"(voff), "s"(gbase), "s"(m0__)                              \
-                 : "memory");                                                    \
-  } while (0)
 
   // all loads of step t (clamped to the last step: the counts stay the same), into
   // the stage at byte `stage`
@@ -201,17 +184,17 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
     const uint8_t* wg = wq + static_cast<size_t>(tc) * S::kRowBytes;
 #pragma unroll
     for (int j = 0; j < S::kXDma; ++j) {
-      QQ_DMA16(xoff[j], xg, stage + (wave * S::kXDma + j) * 1024);
+      dma16(lds_at(stage + (wave * S::kXDma + j) * 1024), xoff[j], xg);
     }
 #pragma unroll
     for (int j = 0; j < S::kWDma; ++j) {
-      QQ_DMA16(woff[j], wg, stage + S::kXTile + (wave * S::kWDma + j) * 1024);
+      dma16(lds_at(stage + S::kXTile + (wave * S::kWDma + j) * 1024), woff[j], wg);
     }
 #pragma unroll
     for (int j = 0; j < S::kSDma; ++j) {
       const int first = (j * S::kWaves + wave) * 64; // uniform
-      QQ_DMA4(soff[j], sbase[j] + static_cast<size_t>(tc) * sstep[j],
-              stage + S::kXTile + S::kWTile + first * 4);
+      dma4(lds_at(stage + S::kXTile + S::kWTile + first * 4), soff[j],
+           sbase[j] + static_cast<size_t>(tc) * sstep[j]);
     }
   };
 
@@ -535,8 +518,6 @@ __global__ __launch_bounds__(64 * WM * WN) void qq_mfma_kernel(const QqArgs a) {
 #undef QQ_MMA
 
   k_loop(read_step, settle, multiply);
-#undef QQ_DMA16
-#undef QQ_DMA4
 
   // D[n][m]: register r of lane (col, quad) holds n = 4 quad + r, m = col
   const int ldy = kPlanes && a.splits > 1 ? k_split_row(N) : N; // rows of a plane start at 16 bytes

@@ -584,10 +584,10 @@ int mlxrocm_qmm_rows(
     mlxrocm_stream_t stream);
 
 /*
- * Prefill calls (16-bit types, transpose != 0, M >= 512) first transpose scales
- * and biases to [K / group_size][N] (scale, bias) pairs so that consecutive rows
- * of W read consecutive values, both with one load (a few MB, about 5 us per
- * call).  Weights do not change
+ * Prefill calls (16-bit types, transpose != 0, M >= 512; mlxrocm_qmm_rows from 65 rows
+ * on) first transpose scales and biases to [K / group_size][N] (scale, bias) pairs so that
+ * consecutive rows of W read consecutive values, both with one load (a few MB, about 5 us
+ * per call).  Weights do not change
  * between calls: a caller that keeps that image beside a weight skips the
  * pre-pass.  The reference has no such cache -- its GPU backends read scales in
  * the caller's layout (mlx/backend/cuda/quantized/qmm/qmm.cu:143-146,
@@ -602,6 +602,8 @@ int mlxrocm_qmm_rows(
  * are those of mlxrocm_qmm bit for bit.  In such prefill calls the workspace may then
  * be smaller than mlxrocm_qmm_workspace_size by mlxrocm_qmm_sb_image_size rounded up
  * to 256.
+ * mlxrocm_qmm_rows_prepacked: the same for mlxrocm_qmm_rows (its shapes, its bits; up to 64 rows
+ * the image is ignored), with a workspace smaller by as much from 65 rows on.
  */
 size_t mlxrocm_qmm_sb_image_size(int N, int K, int batches, int group_size, int dtype);
 int mlxrocm_qmm_sb_image(
@@ -633,6 +635,26 @@ int mlxrocm_qmm_prepacked(
     int bits,
     int dtype,
     int transpose,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream);
+int mlxrocm_qmm_rows_prepacked(
+    const void* x,
+    const uint32_t* wq,
+    const void* scales,
+    const void* biases,
+    const void* sb_image,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t sb_batch_stride,
+    int group_size,
+    int bits,
+    int dtype,
     void* workspace,
     size_t workspace_bytes,
     mlxrocm_stream_t stream);

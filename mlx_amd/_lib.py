@@ -45,6 +45,10 @@ SIGNATURES = {
         _i,
         [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _i, _p, _sz, _p],
     ),
+    "mlxrocm_qmm_rows_prepacked": (
+        _i,
+        [_p] * 6 + [_i] * 4 + [_i64] * 3 + [_i] * 3 + [_p, _sz, _p],
+    ),
     "mlxrocm_qmm_static": (
         _i,
         [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _i, _p],

@@ -1321,12 +1321,6 @@ int qmm_entry(
           kScratchAlign);
     }
   }
-  // (the kernel, and so the bits, of mlxrocm_qmm_rows where the scratch holds its planes)
-  OwnPlan pl;
-  if (sc.sb_image != nullptr &&
-      own_pays(M, N, K, L, group_size, bits, dtype, &pl) && sc.affords(own_plane_bytes(M, N, pl))) {
-    return run_qmm_own(a, group_size, bits, dtype, pl, sc.sb_image, sc.base, s);
-  }
   return run(a, group_size, bits, dtype, transpose != 0, sc, s);
 }
 
@@ -1441,11 +1435,15 @@ extern "C" size_t mlxrocm_qmm_rows_workspace_size(
   return qmm_walk_plane_bytes(rows_shape(M, N, K, L), group_size, bits);
 }
 
-extern "C" int mlxrocm_qmm_rows(
+namespace {
+
+// sb_image: the caller's image of scales and biases, or null.
+int rows_entry(
     const void* x,
     const uint32_t* wq,
     const void* scales,
     const void* biases,
+    const void* sb_image,
     void* out,
     int M,
     int N,
@@ -1459,8 +1457,7 @@ extern "C" int mlxrocm_qmm_rows(
     int dtype,
     void* workspace,
     size_t workspace_bytes,
-    mlxrocm_stream_t stream) {
-  mlxrocm::ApiRange api_range("mlxrocm_qmm_rows");
+    hipStream_t s) {
   if (!mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)) {
     return fail(
         MLXROCM_UNSUPPORTED, "[quantized_matmul] M=%d N=%d K=%d: not a shape of the few-row kernel",
@@ -1487,7 +1484,7 @@ extern "C" int mlxrocm_qmm_rows(
   if (rc != MLXROCM_OK) {
     return rc;
   }
-  const size_t image = M > 64 ? sb_image_bytes(a, group_size, dtype) : 0;
+  const size_t image = M > 64 && sb_image == nullptr ? sb_image_bytes(a, group_size, dtype) : 0;
   const OwnPlan pl = M > 64 ? qmm_own_plan(M, N, K, bits) : OwnPlan{};
   const size_t need =
       M > 64 ? image + own_plane_bytes(M, N, pl) : qmm_walk_plane_bytes(a, group_size, bits);
@@ -1498,14 +1495,76 @@ extern "C" int mlxrocm_qmm_rows(
         "(mlxrocm_qmm_rows_workspace_size); got %zu",
         need, workspace_bytes);
   }
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (M > 64) {
-    const int made = interleave_sb_for_qmm_t(scales, biases, workspace, N, K / group_size, 1, 0, s);
-    return made != MLXROCM_OK ? made
-                              : run_qmm_own(a, group_size, bits, dtype, pl, workspace,
-                                            static_cast<char*>(workspace) + image, s);
+  if (M <= 64) {
+    return launch_qmm_walk(a, group_size, bits, dtype, workspace, s); // (reads no image)
   }
-  return launch_qmm_walk(a, group_size, bits, dtype, workspace, s);
+  if (sb_image == nullptr) {
+    const int made = interleave_sb_for_qmm_t(scales, biases, workspace, N, K / group_size, 1, 0, s);
+    if (made != MLXROCM_OK) {
+      return made;
+    }
+    sb_image = workspace;
+  }
+  return run_qmm_own(
+      a, group_size, bits, dtype, pl, sb_image, static_cast<char*>(workspace) + image, s);
+}
+
+} // namespace
+
+extern "C" int mlxrocm_qmm_rows(
+    const void* x,
+    const uint32_t* wq,
+    const void* scales,
+    const void* biases,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t sb_batch_stride,
+    int group_size,
+    int bits,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream) {
+  mlxrocm::ApiRange api_range("mlxrocm_qmm_rows");
+  return rows_entry(
+      x, wq, scales, biases, nullptr, out, M, N, K, L, x_batch_stride, w_batch_stride,
+      sb_batch_stride, group_size, bits, dtype, workspace, workspace_bytes,
+      static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mlxrocm_qmm_rows_prepacked(
+    const void* x,
+    const uint32_t* wq,
+    const void* scales,
+    const void* biases,
+    const void* sb_image,
+    void* out,
+    int M,
+    int N,
+    int K,
+    int L,
+    int64_t x_batch_stride,
+    int64_t w_batch_stride,
+    int64_t sb_batch_stride,
+    int group_size,
+    int bits,
+    int dtype,
+    void* workspace,
+    size_t workspace_bytes,
+    mlxrocm_stream_t stream) {
+  mlxrocm::ApiRange api_range("mlxrocm_qmm_rows_prepacked");
+  if ((reinterpret_cast<uintptr_t>(sb_image) & 15u) != 0) {
+    return fail(MLXROCM_INVALID_ARGUMENT, "[quantized_matmul] the image must be 16-byte aligned");
+  }
+  return rows_entry(
+      x, wq, scales, biases, sb_image, out, M, N, K, L, x_batch_stride, w_batch_stride,
+      sb_batch_stride, group_size, bits, dtype, workspace, workspace_bytes,
+      static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t mlxrocm_qmm_sb_image_size(int N, int K, int batches, int group_size, int dtype) {

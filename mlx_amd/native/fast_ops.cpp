@@ -40,7 +40,7 @@ struct Abi {
   decltype(&mlxrocm_qmm_sb_image_size) qmm_sb_image_size;
   decltype(&mlxrocm_qmm_rows_supported) rows_supported;
   decltype(&mlxrocm_qmm_rows_workspace_size) rows_workspace_size;
-  decltype(&mlxrocm_qmm_rows) rows;
+  decltype(&mlxrocm_qmm_rows_prepacked) rows_prepacked;
   decltype(&mlxrocm_fp_qmm_workspace_size) fp_qmm_workspace_size;
   decltype(&mlxrocm_fp_qmm) fp_qmm;
   decltype(&mlxrocm_fp_qmm_rows_supported) fp_rows_supported;
@@ -282,13 +282,11 @@ PyObject* quantized_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
              : abi.qmm_workspace_size(M, N, K, 1, 0, gs, bits, code, transpose),
         device);
     Py_BEGIN_ALLOW_THREADS;
-    // (up to 64 rows no kernel of qmm_rows reads an image; beyond, qmm_prepacked with its
-    // scratch runs the same kernel on the caller's image)
-    if (rows && (image == nullptr || M <= 64)) {
-      rc = abi.rows(
+    if (rows) {
+      rc = abi.rows_prepacked(
           x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
-          biases->data_ptr(), out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code, ws.ptr(),
-          ws.bytes, stream);
+          biases->data_ptr(), image, out.data_ptr(), M, N, K, 1, M * K, 0, 0, gs, bits, code,
+          ws.ptr(), ws.bytes, stream);
     } else {
       rc = abi.qmm_prepacked(
           x->data_ptr(), static_cast<const uint32_t*>(w->data_ptr()), scales->data_ptr(),
@@ -673,7 +671,7 @@ PyObject* bind(PyObject*, PyObject* table) {
       take("mlxrocm_qmm_sb_image_size", abi.qmm_sb_image_size) &&
       take("mlxrocm_qmm_rows_supported", abi.rows_supported) &&
       take("mlxrocm_qmm_rows_workspace_size", abi.rows_workspace_size) &&
-      take("mlxrocm_qmm_rows", abi.rows) &&
+      take("mlxrocm_qmm_rows_prepacked", abi.rows_prepacked) &&
       take("mlxrocm_fp_qmm_workspace_size", abi.fp_qmm_workspace_size) &&
       take("mlxrocm_fp_qmm", abi.fp_qmm) &&
       take("mlxrocm_fp_qmm_rows_supported", abi.fp_rows_supported) &&

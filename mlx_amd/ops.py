@@ -631,12 +631,11 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
         )
     # a temporary of the call, like the ones eval_gpu hands to add_temporary
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-    # (up to 64 rows no kernel of qmm_rows reads an image; beyond, qmm_prepacked with its scratch
-    # runs the same kernel on the caller's image)
-    if rows and (sb_image is None or M <= 64):
+    image = sb_image.data_ptr() if sb_image is not None else None
+    if rows:
         _lib.check(
-            lib.mlxrocm_qmm_rows(
-                xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(), out.data_ptr(),
+            lib.mlxrocm_qmm_rows_prepacked(
+                xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(), image, out.data_ptr(),
                 M, w_outer, K, L, M * K, w_stride, sb_stride, group_size, bits, code,
                 ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(x),
             )
@@ -645,7 +644,7 @@ def _quantized_matmul(x, w, scales, biases, transpose, group_size, bits, mode, s
     _lib.check(
         lib.mlxrocm_qmm_prepacked(
             xb.data_ptr(), wb.data_ptr(), sb.data_ptr(), bb.data_ptr(),
-            sb_image.data_ptr() if sb_image is not None else None, out.data_ptr(),
+            image, out.data_ptr(),
             M, w_outer, K, L, M * K, w_stride, sb_stride, group_size, bits,
             code, int(bool(transpose)),
             ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(x),

@@ -201,3 +201,67 @@ def test_few_pairs_of_an_expert(bits, E, D, F, tokens):
     assert need > plain and torch.equal(got[need], y)
     d = (got[need - 1].double() - y.double()).norm() / y.double().norm()
     assert float(d) < 2.0 ** -8
+
+
+def _weights(N, K, bits, dtype, group=64):
+    g = torch.Generator(device="cuda").manual_seed(N + K + bits)
+    w = (torch.randn((N, K), generator=g, device="cuda") / K ** 0.5).to(dtype)
+    return mlx_amd.quantize(w, group, bits)
+
+
+def _c_call(entry, x, q, image, N, bits, code, transpose, workspace_bytes, group=64):
+    """A call at the C boundary on one product; image: None, or a 1-tuple with it or None."""
+    (M, K), (wq, s, b) = x.shape, q
+    out = torch.full((M, N), 7.0, dtype=x.dtype, device="cuda")
+    ws = torch.full((workspace_bytes,), 0x7f, dtype=torch.uint8, device="cuda")
+    between = [] if image is None else [image[0].data_ptr() if image[0] is not None else None]
+    _lib.check(entry(
+        x.data_ptr(), wq.data_ptr(), s.data_ptr(), b.data_ptr(), *between, out.data_ptr(), M, N, K,
+        1, M * K, 0, 0, group, bits, code, *transpose,
+        ws.data_ptr() if workspace_bytes else None, workspace_bytes,
+        torch.cuda.current_stream().cuda_stream))
+    return out
+
+
+# mlxrocm_qmm in one range of the tile kernel and in several, in front of shapes that the tiles of
+# this file take (first four) and of shapes that they leave to the tile kernel
+TABLE = ((2048, 4096, 4096, 8), (1024, 4096, 4096, 4), (300, 14336, 4096, 2), (5000, 1024, 4096, 4),
+         (600, 803, 4096, 4), (1024, 14336, 4096, 8), (1792, 7168, 4096, 4))
+
+
+@pytest.mark.parametrize("M,N,K,bits", TABLE)
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+def test_prepacked_calls_have_the_bits_of_plain_ones(M, N, K, bits, dtype):
+    """mlxrocm_qmm_prepacked those of mlxrocm_qmm and mlxrocm_qmm_rows_prepacked those of
+    mlxrocm_qmm_rows, with the scratch of the plain call and without the image's share of it;
+    quantized_matmul those of the entry that it takes, with an image and without."""
+    lib, code = _lib.load(), CODE[dtype]
+    q = _weights(N, K, bits, dtype)
+    x = torch.randn((M, K), device="cuda").to(dtype)
+    image = mlx_amd.quantized_matmul_sb_image(q[1], q[2], 64)
+    share = -(-lib.mlxrocm_qmm_sb_image_size(N, K, 1, 64, code) // 256) * 256
+    rows = bool(lib.mlxrocm_qmm_rows_supported(M, N, K, 1, 64, bits, code))
+    assert rows == ((M, N, K, bits) in TABLE[:4])
+
+    need = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, bits, code, 1)
+    plan = _lib.qmm_plan(M, N, K, bits=bits, dtype=code)[1]
+    share = share if "interleave_sb" in plan else 0
+    plain = _c_call(lib.mlxrocm_qmm, x, q, None, N, bits, code, (1,), need)
+    for room in (need, need - share):
+        for kept in (image, None) if room == need else (image,):
+            y = _c_call(lib.mlxrocm_qmm_prepacked, x, q, (kept,), N, bits, code, (1,), room)
+            assert torch.equal(y, plain), (room, kept is None)
+    if rows:
+        need = lib.mlxrocm_qmm_rows_workspace_size(M, N, K, 1, 64, bits, code)
+        share = -(-lib.mlxrocm_qmm_sb_image_size(N, K, 1, 64, code) // 256) * 256
+        plain = _c_call(lib.mlxrocm_qmm_rows, x, q, None, N, bits, code, (), need)
+        for room in (need, need - share):
+            for kept in (image, None) if room == need else (image,):
+                y = _c_call(lib.mlxrocm_qmm_rows_prepacked, x, q, (kept,), N, bits, code, (), room)
+                assert torch.equal(y, plain), (room, kept is None)
+    # (native host path, then the Python one)
+    strided = torch.stack([x, x], dim=-1)[..., 0]
+    for t in (x, strided):
+        for kept in (image, None):
+            y = mlx_amd.quantized_matmul(t, *q, group_size=64, bits=bits, sb_image=kept)
+            assert torch.equal(y, plain), kept is None

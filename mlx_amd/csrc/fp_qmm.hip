@@ -1244,7 +1244,9 @@ int fp_gather_entry(
     a.n_experts = n_experts;
     a.out_scale = out_scale;
     // pairs with an index out of range are zero-filled by the grouping kernels
-    rc = launch_gather_group(a, dtype, kGroupLargeTile, workspace, s);
+    rc = launch_gather_group(
+        a, dtype, kGroupLargeTile, gather_tiles_by_height(N, K, mode == MLXROCM_MXFP8 ? 8 : 4),
+        workspace, s);
     if (rc != MLXROCM_OK) {
       return rc;
     }

@@ -65,14 +65,13 @@ __global__ __launch_bounds__(256) void group_count_kernel(
 }
 
 // First sorted position of every expert and the list of tiles from the counts in LDS, by all
-// threads of the workgroup.  256-row tiles that are full come first, the others behind them by
-// eighths of their height, highest first: qmm_own_kernel deals tiles out in the order of the
-// list and multiplies as many rows as a tile has, so its time ends with the workgroup that got
-// most rows.  Tiles of 32 rows stay in the order of their experts.
+// threads of the workgroup: in the order of their experts, or (by_height) those that are full
+// first and the others behind them by eighths of their height, highest first.
 constexpr int kHeights = 8;
 __device__ __forceinline__ void plan_tiles(
     int n_experts,
     int tile_rows, // a power of two
+    bool by_height,
     const int32_t* cnt,
     int32_t* first_pos,
     int32_t* first_tile,
@@ -80,7 +79,6 @@ __device__ __forceinline__ void plan_tiles(
     int32_t* tiles,
     int32_t* n_tiles) {
   __shared__ int32_t next[kHeights]; // of the tiles of a height: how many, then the next one
-  const bool by_height = tile_rows == kGroupLargeTile;
   const int shift = __ffs(tile_rows) - 1;
   auto height = [&](int rows) { return ((rows * kHeights - 1) >> shift); };
   if (threadIdx.x < kHeights) {
@@ -149,6 +147,7 @@ __device__ __forceinline__ void plan_tiles(
 __global__ __launch_bounds__(256) void group_plan_kernel(
     int n_experts,
     int tile_rows,
+    bool by_height,
     const int32_t* counts,
     int32_t* offsets,
     int32_t* tiles,
@@ -160,7 +159,7 @@ __global__ __launch_bounds__(256) void group_plan_kernel(
     cnt[e] = counts[e];
   }
   __syncthreads();
-  plan_tiles(n_experts, tile_rows, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
+  plan_tiles(n_experts, tile_rows, by_height, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
 }
 
 __global__ __launch_bounds__(256) void group_scatter_kernel(
@@ -244,6 +243,7 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     int n_experts,
     int key_bits,
     int tile_rows,
+    bool by_height,
     int32_t* offsets,
     int32_t* tiles,
     int32_t* n_tiles,
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kFusedThreads) void group_fused_kernel(
     }
   }
   __syncthreads();
-  plan_tiles(n_experts, tile_rows, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
+  plan_tiles(n_experts, tile_rows, by_height, cnt, first_pos, first_tile, offsets, tiles, n_tiles);
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     if (i * kFusedThreads < n_indices && key[i] < static_cast<uint32_t>(n_experts)) {
@@ -335,7 +335,8 @@ void bind_gather_group(QmmArgs& a, int tile_rows, void* workspace) {
 }
 
 // Fills the workspace and points the grouped-mode fields of `a` into it.
-int launch_gather_group(QmmArgs& a, int dtype, int tile_rows, void* workspace, hipStream_t s) {
+int launch_gather_group(
+    QmmArgs& a, int dtype, int tile_rows, bool by_height, void* workspace, hipStream_t s) {
   const int E = a.n_experts;
   const int n = a.L;
   int32_t* ws = static_cast<int32_t*>(workspace);
@@ -358,12 +359,12 @@ int launch_gather_group(QmmArgs& a, int dtype, int tile_rows, void* workspace, h
     }
     if (dtype == MLXROCM_BFLOAT16) {
       group_fused_kernel<bf16_t><<<1, kFusedThreads, 0, s>>>(
-          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, offsets, tiles, n_tiles,
-          perm, static_cast<bf16_t*>(a.out), a.N);
+          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, by_height, offsets, tiles,
+          n_tiles, perm, static_cast<bf16_t*>(a.out), a.N);
     } else {
       group_fused_kernel<f16_t><<<1, kFusedThreads, 0, s>>>(
-          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, offsets, tiles, n_tiles,
-          perm, static_cast<f16_t*>(a.out), a.N);
+          a.lhs_indices, a.rhs_indices, n, a.x_batches, E, key_bits, tile_rows, by_height, offsets, tiles,
+          n_tiles, perm, static_cast<f16_t*>(a.out), a.N);
     }
     MLXROCM_HIP_TRY(hipGetLastError());
     return MLXROCM_OK;
@@ -384,7 +385,7 @@ int launch_gather_group(QmmArgs& a, int dtype, int tile_rows, void* workspace, h
         static_cast<f16_t*>(a.out), a.N);
   }
   MLXROCM_HIP_TRY(hipGetLastError());
-  group_plan_kernel<<<1, 256, 0, s>>>(E, tile_rows, counts, offsets, tiles, n_tiles);
+  group_plan_kernel<<<1, 256, 0, s>>>(E, tile_rows, by_height, counts, offsets, tiles, n_tiles);
   MLXROCM_HIP_TRY(hipGetLastError());
   group_scatter_kernel<<<blocks, 256, 0, s>>>(
       a.lhs_indices, a.rhs_indices, n, a.x_batches, E, offsets, cursor, perm);

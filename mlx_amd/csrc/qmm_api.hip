@@ -2015,7 +2015,9 @@ int gather_entry(
       return launch_qmm_slab_grouped(
           a, group_size, bits, dtype, static_cast<char*>(workspace) + tables, true, s);
     }
-    rc = launch_gather_group(a, dtype, small ? kGroupSmallTile : kGroupLargeTile, workspace, s);
+    rc = launch_gather_group(
+        a, dtype, small ? kGroupSmallTile : kGroupLargeTile,
+        !small && gather_tiles_by_height(N, K, bits), workspace, s);
     if (rc != MLXROCM_OK) {
       return rc;
     }
@@ -2033,7 +2035,8 @@ int gather_entry(
     const int images = sb_expert_stride == 0 ? 1 : n_experts;
     const size_t tables = group_gather_n_tables(n_indices, n_experts);
     if (workspace_bytes >= tables + qmm_n_sb_bytes(K, G, images, dtype)) {
-      rc = launch_gather_group(a, dtype, kGroupLargeTile, workspace, s);
+      rc = launch_gather_group(
+          a, dtype, kGroupLargeTile, gather_tiles_by_height(N, K, bits), workspace, s);
       if (rc != MLXROCM_OK) {
         return rc;
       }

@@ -311,7 +311,7 @@ extern "C" int mlxrocm_switch_glu(
   a.M = 1;
   a.out = out;
   a.N = D;
-  int rc = launch_gather_group(a, dtype, kGroupLargeTile, ws + l.rest, s);
+  int rc = launch_gather_group(a, dtype, kGroupLargeTile, true, ws + l.rest, s);
   const struct {
     const void *scales, *biases;
     size_t image;

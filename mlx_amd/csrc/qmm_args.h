@@ -372,10 +372,18 @@ int reduce_grouped_planes(
     const QmmArgs& a, const float* planes, int ranges, int64_t plane_elems, int dtype,
     hipStream_t s);
 // expert-routed gated MLP (qmm_mfma_experts.hip): pair images, launch_gather_group's tables
-int launch_qmm_mfma_experts_glu(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
-// planes: scratch of `room` bytes for K ranges
+struct ExpertsPlan {
+  bool own_first;  // both first products on qmm_own_kernel, else on the tile kernel
+  bool own_second; // the last one, `splits` ranges of K
+  int splits;
+};
+// in, out: N, K, L and n_experts of the first products and of the last; planes: `room` bytes.
+ExpertsPlan qmm_experts_plan(const QmmArgs& in, const QmmArgs& out, int bits, size_t room);
+int launch_qmm_mfma_experts_glu(
+    const QmmArgs& a, int gs, int bits, int dtype, const ExpertsPlan& pl, hipStream_t s);
 int launch_qmm_mfma_experts(
-    const QmmArgs& a, int gs, int bits, int dtype, void* planes, size_t room, hipStream_t s);
+    const QmmArgs& a, int gs, int bits, int dtype, const ExpertsPlan& pl, void* planes,
+    hipStream_t s);
 int expected_tiles(int pairs, int experts);
 int launch_qmm_mfma_grouped(const QmmArgs& a, int gs, int bits, int dtype, hipStream_t s);
 // transpose=false form: scales / biases are the [group][k] images of all experts

@@ -37,11 +37,7 @@ constexpr size_t kOwnMostPlanes = size_t(128) << 20;
 
 } // namespace
 
-// Ahead of the tile kernel wherever it can run and tiles are many, by its unpacking and by the rows that an
-// expert's last tile has not got.  us per call of the gated MLP, start -> this kernel: 2048
-// tokens to 2 of 8 experts, 4096 x 14336 4-bit 1498 -> 1377 (1300 tokens 1122 -> 930, 300
-// tokens 511 -> 486, 700 at 8 bits 837 -> 841); 6 of 64, 2048 x 1408 4-bit, 2048 tokens 387
-// -> 310, 8-bit 438 -> 382, 800 tokens 283 -> 264.
+// (which products it takes: qmm_experts_plan)
 bool qmm_own_experts_supported(const QmmArgs& a, int bits) {
   // (x: the callers check it for every grouped kernel)
   return own_addresses(a.N, a.K, bits) && static_cast<uint64_t>(a.L) * a.N * 2 < kNoStore;
@@ -121,14 +117,18 @@ int launch_qmm_own(
 // 14336 4-bit, 300 tokens to 2 experts each: the product 231 us without ranges, the whole call
 // 486 / 407 (600 tokens, by scratch without: 643 against 692 of the tile kernel).  From a round
 // of tiles on the order of the list evens the workgroups' shares out, and ranges gain nothing
-// (2048 tokens, two ranges: 1.07 of the tile kernel, 1.07..1.12 without).
+// (2048 tokens, two ranges: 1.07 of the tile kernel, 1.07..1.12 without).  One expert more with a
+// second tile may start a second round of ranges, which codes that are dear to unpack feel: 8-bit,
+// 493 tokens, 9 tiles of rows instead of 8, 595 us on the tile kernel, 717 in two ranges (4-bit,
+// 489 tokens: 614 / 523).  So more than half a tile is counted there beyond the full ones.
 int qmm_own_experts_splits(const QmmArgs& a, int bits, size_t room) {
   const size_t plane = static_cast<size_t>(a.L) * a.N * sizeof(float);
   if (a.N % 4 != 0 || plane >= kNoStore) {
     return 1;
   }
   const long cus = compute_units();
-  const long expected = expected_tiles(a.L, a.n_experts);
+  const long expected =
+      bits == 4 ? expected_tiles(a.L, a.n_experts) : (5L * a.L / 256 + 3L * a.n_experts + 4) / 5;
   const long least = a.n_experts < a.L ? a.n_experts : a.L;
   const long high = expected > least ? expected : least;
   const long tiles = high * ((a.N + kOwnBN - 1) / kOwnBN);

@@ -55,25 +55,36 @@ size_t round256(size_t n) {
   return (n + 255) / 256 * 256;
 }
 
+// The first products and the last, as plans look at them.
+struct Shapes {
+  QmmArgs in, out;
+};
+Shapes shapes_of(int pairs, int D, int F, int E) {
+  Shapes s{};
+  s.in.N = F;
+  s.in.K = D;
+  s.in.L = pairs;
+  s.in.n_experts = E;
+  s.out = s.in;
+  s.out.N = D;
+  s.out.K = F;
+  return s;
+}
+
 // Pairs per expert from which the tiles are ahead: as many as mlxrocm_gather_qmm asks for of
 // the tile kernel, fewer where qmm_own_kernel takes both products and the products one by one
 // would run on the staged kernel of 32 rows (4-bit codes have one that rounds no weight, and
 // keep it).  us per call, products / tiles, 8-bit, by pairs per expert: 4096 x 14336, 8
 // experts 24 525 / 529, 32 546 / 532, 44 707 / 554, 64 876 / 580; 2048 x 1408, 64 experts 12
-// 189 / 194, 16 226 / 216, 32 246 / 201, 64 375 / 248; 1024 x 1024, 32 experts 16 75 / 64, 64
-// 109 / 82 (3-bit: 28 458 / 469, 28 238 / 185, 28 70 / 57).
-int least_pairs(int64_t pairs, int D, int F, int bits) {
-  QmmArgs in{};
-  in.N = F;
-  in.K = D;
-  in.L = static_cast<int>(pairs);
-  QmmArgs out = in;
-  out.N = D;
-  out.K = F;
-  if (bits == 4 || !qmm_own_experts_supported(in, bits) || !qmm_own_experts_supported(out, bits)) {
+// 189 / 194, 17 193 / 204, 22 217 / 209, 32 246 / 201, 64 375 / 248; 1024 x 1024, 32 experts 16 75
+// / 64, 64 109 / 82 (3-bit: 28 458 / 469, 28 238 / 185, 28 70 / 57; 2048 x 1408 16 173 / 140).
+int least_pairs(const Shapes& s, int bits) {
+  if (bits == 4 || !qmm_own_experts_supported(s.in, bits) ||
+      !qmm_own_experts_supported(s.out, bits)) {
     return 64;
   }
-  return D <= 2048 && F <= 2048 ? 16 : 32;
+  const int widest = s.in.N > s.in.K ? s.in.N : s.in.K;
+  return widest > 2048 ? 32 : widest > 1024 && bits == 8 ? 20 : 16;
 }
 
 // The tile kernels' grouped form: operands within 32-bit byte offsets.
@@ -113,7 +124,7 @@ Layout layout_of(
   l.row = take(pairs * 4);
   l.self = take(pairs * 4);
   l.h = take(pairs * F * dtype_size(dtype));
-  const int fewest = least_pairs(pairs, D, F, bits);
+  const int fewest = least_pairs(shapes_of(static_cast<int>(pairs), D, F, E), bits);
   *tiles = tiled(tokens, top, D, F, E, least > fewest ? least : fewest);
   if (*tiles) {
     l.rest = take(gather_group_workspace_bytes(static_cast<int>(pairs), E));
@@ -311,7 +322,13 @@ extern "C" int mlxrocm_switch_glu(
   a.M = 1;
   a.out = out;
   a.N = D;
-  int rc = launch_gather_group(a, dtype, kGroupLargeTile, true, ws + l.rest, s);
+  // (planes of K ranges where the images of the first two products were: side by side, done with)
+  const Shapes shapes = shapes_of(pairs, D, F, E);
+  const ExpertsPlan pl =
+      qmm_experts_plan(shapes.in, shapes.out, bits, l.down_image - l.gate_image);
+  int rc = launch_gather_group(
+      a, dtype, kGroupLargeTile,
+      pl.own_first || pl.own_second || gather_tiles_by_height(D, F, bits), ws + l.rest, s);
   const struct {
     const void *scales, *biases;
     size_t image;
@@ -343,7 +360,7 @@ extern "C" int mlxrocm_switch_glu(
   in.w_batch_stride = w_in;
   in.sb_batch_stride = 2 * sb_in; // pairs
   in.sb_transposed = 2;
-  rc = launch_qmm_mfma_experts_glu(in, group_size, bits, dtype, s);
+  rc = launch_qmm_mfma_experts_glu(in, group_size, bits, dtype, pl, s);
   if (rc != MLXROCM_OK) {
     return rc;
   }
@@ -361,7 +378,5 @@ extern "C" int mlxrocm_switch_glu(
   o.w_batch_stride = w_out;
   o.sb_batch_stride = 2 * sb_out;
   o.sb_transposed = 2;
-  // (planes of K ranges where the images of the first two products were: side by side, done with)
-  return launch_qmm_mfma_experts(
-      o, group_size, bits, dtype, ws + l.gate_image, l.down_image - l.gate_image, s);
+  return launch_qmm_mfma_experts(o, group_size, bits, dtype, pl, ws + l.gate_image, s);
 }

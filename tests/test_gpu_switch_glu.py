@@ -93,3 +93,25 @@ def test_the_bits_of_the_three_products(tokens, top, E, D, F, group, bits):
     block.activation = lambda t: torch.nn.functional.silu(t)
     assert block._in_one_call(x, idx) is None
     assert torch.equal(y, block(x, idx))
+
+
+@pytest.mark.parametrize("bits", (4, 8))
+@pytest.mark.parametrize("tokens,top,E,D,F,group", [
+    (700, 1, 2, 4096, 4352, 64),   # experts of more than 16 MB at 8 bits, the last product in one round
+    (900, 2, 8, 2048, 2304, 64),   # the last product in one round of the narrowest tiles
+    (1900, 3, 5, 4096, 4224, 32),  # experts of more than 16 MB at 8 bits, two rounds
+])
+def test_the_bits_of_the_three_products_large_experts(tokens, top, E, D, F, group, bits):
+    """The same where the tile kernel takes the last product, or all of them with tiles in the
+    order of their experts; an expert without rows, and pairs without an expert."""
+    block = _block(D, F, E, group, bits, torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn((tokens, D), generator=g, device="cuda").bfloat16()
+    idx = torch.randint(0, E, (tokens, top), generator=g, device="cuda")
+    idx[idx == 1] = 0
+    idx[5, 0] = E
+    y = block(x, idx)
+    assert not y[5, 0].any()
+    block.activation = lambda t: torch.nn.functional.silu(t)
+    assert block._in_one_call(x, idx) is None
+    assert torch.equal(y, block(x, idx))

@@ -53,7 +53,9 @@ bool qmm_own_supported(int M, int N, int K, int L, int bits, int dtype) {
 // fitted to 27000 calls of 65..8192 rows on 14 shapes, every width and mode, each in every
 // height and several numbers of ranges (errors of 5 %; the choice takes 1.2 % longer than the
 // best one on average): the launches and the image of scales, rounds of tiles, planes written
-// and added up.  Ranges are cut only while one round of workgroups holds their tiles.
+// and added up.  Ranges are cut only while one round of workgroups holds their tiles.  Rows of y
+// of an odd number of elements are stored element by element: 17 us a tile of 256 rows (planes
+// have whole pieces).
 OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
   const Step& step = step_of(codes);
   const long cus = compute_units();
@@ -78,7 +80,8 @@ OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
       const double fixed = step.fixed + (codes == 4 && s == 1 ? 0.12 : 0.0);
       const double each = (steps + s - 1) / s * (fixed + mt * (step.each + busy * step.busy));
       const double us = 5.9 + rounds * (0.36 * mt - 1.1 + each) +
-          (s > 1 ? 6.6 + (0.89 * s + 0.15) * plane : 0.34 * plane);
+          (s > 1 ? 6.6 + (0.89 * s + 0.15) * plane
+                 : 0.34 * plane + (N % 2 != 0 ? 1.05 * rounds * mt : 0.0));
       if (pl.mt == 0 || us < pl.us) {
         pl = {mt, s, us};
       }
@@ -87,17 +90,21 @@ OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
   return pl;
 }
 
-// With the accounts of both sides, which err by 5 and 7..15 %, these margins leave 1.8 % of the
-// 2000 calls taken (of 3000 timed) behind by more than 3 %, the worst by 12 %, the others 18 %
-// shorter on average.  us against the tile kernel, bf16 g64 4-bit: 2048 x 4096 x 14336 198 / 243,
+// With the accounts of both sides, which err by 5 and 7..15 %, these margins leave 1.0 % of the
+// 7000 calls taken behind by more than 3 %, the worst by 11 %; the mean takes 0.84 of the time.  us against the tile kernel, bf16 g64 4-bit: 2048 x 4096 x 14336 198 / 243,
 // 2048 x 8192 x 8192 198 / 275, 2048 x 4096 x 4096 66 / 78, 320 x 14336 x 4096 51 / 60, 320 x 8192 x
 // 8192 54 / 80; the tile kernel stays ahead where its widths make whole rounds: 1024 x 14336 x
 // 4096 8-bit 102 / 99, 512 x 18944 x 3584 8-bit 77 / 72.  Less is to be gained where its
-// unpacking is one convert for two codes (mxfp8: 512 x 18944 x 3584 75 / 66) or this kernel
-// has to put the codes in order (4-bit, one range: 5291 x 6853 x 8192 557 / 553).
+// unpacking is one convert for two codes (mxfp8: 512 x 18944 x 3584 75 / 66), its steps are cheap
+// (8-bit, one range: 1921 x 5120 x 13824 313 / 280) or this kernel has to put the codes in order
+// (4-bit, one range: 5291 x 6853 x 8192 557 / 553).
 bool qmm_own_pays(const OwnPlan& pl, int codes, double other) {
-  const bool less = codes == kOwnFpCodes + MLXROCM_MXFP8 || (codes == 4 && pl.splits == 1);
-  return pl.us < (less ? 0.82 : 0.88) * other;
+  const bool one = pl.splits == 1;
+  const double margin = codes == kOwnFpCodes + MLXROCM_MXFP8 ? (one ? 0.80 : 0.82)
+      : one && (codes == 4 || codes == 8)                    ? 0.82
+      : one && codes == kOwnFpCodes + MLXROCM_MXFP4          ? 0.85
+                                                             : 0.88;
+  return pl.us < margin * other;
 }
 
 int launch_qmm_own(

@@ -383,15 +383,6 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
       k2 = kbeg - kOwnBK;
     }
 
-    if constexpr (FP == 3) {
-      if (a.out_scale != nullptr) {
-        const float factor = *a.out_scale / (448.0f * 6.0f);
-        own_unroll<MT>([&](auto f) OWN_INLINE {
-          acc[0][f] *= factor;
-          acc[1][f] *= factor;
-        });
-      }
-    }
     // lane (fi, fk) holds row fi of x and rows 4 fk + r of both tiles of W
     const int at = lane_here();
     const int fi = at & 15, fk = at >> 4;
@@ -487,38 +478,38 @@ __global__ __launch_bounds__(kOwnThreads) void qmm_own_kernel(
     while (tile < tiles) {
       run_tile(std::integral_constant<int, MT_>{});
     }
-    return;
-  }
-  int have = 16; // 16-row blocks of the current tile that its first stage holds
-  while (tile < tiles) {
-    const int need = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
-    if (need > have) {
-      // the tile before was lower: its last step fetched too few rows
-      own_unroll<kLoads>([&](auto i) OWN_INLINE { dma_x(cur, kbeg, i); });
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-    }
-    if (need > 14) {
-      run_tile(std::integral_constant<int, 16>{});
-      have = 16;
-    } else if (need > 12) {
-      run_tile(std::integral_constant<int, 14>{});
-      have = 14;
-    } else if (need > 10) {
-      run_tile(std::integral_constant<int, 12>{});
-      have = 12;
-    } else if (need > 8) {
-      run_tile(std::integral_constant<int, 10>{});
-      have = 10;
-    } else if (need > 6) {
-      run_tile(std::integral_constant<int, 8>{});
-      have = 8;
-    } else if (need > 4) {
-      run_tile(std::integral_constant<int, 6>{});
-      have = 6;
-    } else {
-      run_tile(std::integral_constant<int, 4>{});
-      have = 4;
+  } else {
+    int have = 16; // 16-row blocks of the current tile that its first stage holds
+    while (tile < tiles) {
+      const int need = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
+      if (need > have) {
+        // the tile before was lower: its last step fetched too few rows
+        own_unroll<kLoads>([&](auto i) OWN_INLINE { dma_x(cur, kbeg, i); });
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      }
+      if (need > 14) {
+        run_tile(std::integral_constant<int, 16>{});
+        have = 16;
+      } else if (need > 12) {
+        run_tile(std::integral_constant<int, 14>{});
+        have = 14;
+      } else if (need > 10) {
+        run_tile(std::integral_constant<int, 12>{});
+        have = 12;
+      } else if (need > 8) {
+        run_tile(std::integral_constant<int, 10>{});
+        have = 10;
+      } else if (need > 6) {
+        run_tile(std::integral_constant<int, 8>{});
+        have = 8;
+      } else if (need > 4) {
+        run_tile(std::integral_constant<int, 6>{});
+        have = 6;
+      } else {
+        run_tile(std::integral_constant<int, 4>{});
+        have = 4;
+      }
     }
   }
 }

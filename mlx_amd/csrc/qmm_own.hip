@@ -109,6 +109,9 @@ bool qmm_own_pays(const OwnPlan& pl, int codes, double other) {
 
 int launch_qmm_own(
     const QmmArgs& a, int gs, int codes, int dtype, const OwnPlan& pl, hipStream_t s) {
+  if (a.out_scale != nullptr) {
+    return fail(MLXROCM_UNSUPPORTED, "[qmm_own] a scale of the results"); // (mlxrocm_fp_qmm takes it)
+  }
   MLXROCM_REHEARSE("qmm_own(rows=%d,ksplit=%d)", 16 * pl.mt, pl.splits);
   if (codes >= kOwnFpCodes) {
     const int mode = codes - kOwnFpCodes;

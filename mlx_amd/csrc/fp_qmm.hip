@@ -735,7 +735,8 @@ int fp_qmm_entry(
     size_t workspace_bytes,
     mlxrocm_stream_t stream,
     const float* out_scale = nullptr,
-    bool rows = false) { // a call that fp_walk_applies() or fp_own_pays() to
+    bool rows = false, // a call that fp_rows_plan() takes,
+    const OwnPlan& pl = {}) { // with this plan beyond 64 rows
   int rc = fp_check("quantized_matmul", M, N, K, L, mode, dtype, transpose);
   if (rc != MLXROCM_OK) {
     return rc;
@@ -783,8 +784,7 @@ int fp_qmm_entry(
   a.n_experts = L;
   a.out_scale = out_scale;
   if (rows) {
-    OwnPlan pl;
-    const bool own = M > 64 && fp_own_pays(M, N, K, L, mode, dtype, &pl);
+    const bool own = M > 64;
     const size_t need = own ? fp_own_bytes(M, N, K, pl) : qmm_walk_fp_plane_bytes(a, mode);
     if (need != 0 &&
         (workspace == nullptr || workspace_bytes < need ||
@@ -912,21 +912,29 @@ extern "C" int mlxrocm_fp_qmm(
       dtype, transpose, workspace, workspace_bytes, stream);
 }
 
-extern "C" int mlxrocm_fp_qmm_rows_supported(int M, int N, int K, int L, int mode, int dtype) {
-  OwnPlan pl;
+namespace {
+
+// Whether mlxrocm_fp_qmm_rows takes a call; more than 64 rows: *pl is its plan.
+bool fp_rows_plan(int M, int N, int K, int L, int mode, int dtype, OwnPlan* pl) {
   return M >= 2 && fp_check("quantized_matmul", M, N, K, L, mode, dtype, 1) == MLXROCM_OK &&
       N > 0 && L > 0 &&
-      (M > 64 ? fp_own_pays(M, N, K, L, mode, dtype, &pl)
+      (M > 64 ? fp_own_pays(M, N, K, L, mode, dtype, pl)
               : fp_walk_applies(fp_shape(M, N, K, L), mode, dtype));
+}
+
+} // namespace
+
+extern "C" int mlxrocm_fp_qmm_rows_supported(int M, int N, int K, int L, int mode, int dtype) {
+  OwnPlan pl;
+  return fp_rows_plan(M, N, K, L, mode, dtype, &pl);
 }
 
 extern "C" size_t mlxrocm_fp_qmm_rows_workspace_size(
     int M, int N, int K, int L, int mode, int dtype) {
-  if (!mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)) {
-    return 0;
-  }
-  return M > 64 ? fp_own_bytes(M, N, K, qmm_own_plan(M, N, K, kOwnFpCodes + mode))
-                : qmm_walk_fp_plane_bytes(fp_shape(M, N, K, L), mode);
+  OwnPlan pl;
+  return !fp_rows_plan(M, N, K, L, mode, dtype, &pl) ? 0
+      : M > 64 ? fp_own_bytes(M, N, K, pl)
+               : qmm_walk_fp_plane_bytes(fp_shape(M, N, K, L), mode);
 }
 
 extern "C" int mlxrocm_fp_qmm_rows(
@@ -947,14 +955,15 @@ extern "C" int mlxrocm_fp_qmm_rows(
     size_t workspace_bytes,
     mlxrocm_stream_t stream) {
   mlxrocm::ApiRange api_range("mlxrocm_fp_qmm_rows");
-  if (!mlxrocm_fp_qmm_rows_supported(M, N, K, L, mode, dtype)) {
+  OwnPlan pl{};
+  if (!fp_rows_plan(M, N, K, L, mode, dtype, &pl)) {
     return fail(
         MLXROCM_UNSUPPORTED, "[quantized_matmul] M=%d N=%d K=%d: not a shape of the few-row kernel",
         M, N, K);
   }
   return fp_qmm_entry(
       x, wq, scales, out, M, N, K, L, x_batch_stride, w_batch_stride, scales_batch_stride, mode,
-      dtype, 1, workspace, workspace_bytes, stream, nullptr, true);
+      dtype, 1, workspace, workspace_bytes, stream, nullptr, true, pl);
 }
 
 namespace {

@@ -708,13 +708,15 @@ bool own_pays(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* 
       (N % 4 != 0 && qmm_mfma_k_splits(M, N, K, 1) > 1)) {
     return false;
   }
-  double other = qmm_mfma_us(M, N, K, bits);
+  *pl = qmm_own_plan(M, N, K, bits);
+  if (!qmm_own_pays(*pl, bits, qmm_mfma_us(M, N, K, bits))) {
+    return false;
+  }
   if (M <= (K <= kMidShortK ? kMidMaxMShortK : kMidMaxM)) {
     const MidPlan mid = qmm_mid_plan(M, N, K, gs, bits);
-    other = mid.groups <= compute_units() && mid.us < other ? mid.us : other;
+    return mid.groups > compute_units() || qmm_own_pays(*pl, bits, mid.us);
   }
-  *pl = qmm_own_plan(M, N, K, bits);
-  return qmm_own_pays(*pl, bits, other);
+  return true;
 }
 
 size_t own_plane_bytes(int M, int N, const OwnPlan& pl) {
@@ -1407,32 +1409,36 @@ QmmArgs rows_shape(int M, int N, int K, int L) {
   return a;
 }
 
+// Whether mlxrocm_qmm_rows takes a call; more than 64 rows: *pl is its plan.
+bool rows_plan(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* pl) {
+  if (M <= 0 || N <= 0 || L <= 0 ||
+      check_shape("quantized_matmul", M, N, K, L, gs, bits, dtype, 1) != MLXROCM_OK) {
+    return false;
+  }
+  if (M > 64) {
+    return own_pays(M, N, K, L, gs, bits, dtype, pl);
+  }
+  const QmmArgs a = rows_shape(M, N, K, L);
+  return walk_pays(a, gs, bits) && qmm_walk_supported(a, gs, bits, dtype, true);
+}
+
 } // namespace
 
 extern "C" int mlxrocm_qmm_rows_supported(
     int M, int N, int K, int L, int group_size, int bits, int dtype) {
-  if (M <= 0 || N <= 0 || L <= 0 ||
-      check_shape("quantized_matmul", M, N, K, L, group_size, bits, dtype, 1) != MLXROCM_OK) {
-    return 0;
-  }
   OwnPlan pl;
-  if (own_pays(M, N, K, L, group_size, bits, dtype, &pl)) {
-    return 1;
-  }
-  const QmmArgs a = rows_shape(M, N, K, L);
-  return walk_pays(a, group_size, bits) && qmm_walk_supported(a, group_size, bits, dtype, true);
+  return rows_plan(M, N, K, L, group_size, bits, dtype, &pl);
 }
 
 extern "C" size_t mlxrocm_qmm_rows_workspace_size(
     int M, int N, int K, int L, int group_size, int bits, int dtype) {
-  if (!mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)) {
+  OwnPlan pl;
+  if (!rows_plan(M, N, K, L, group_size, bits, dtype, &pl)) {
     return 0;
   }
-  if (M > 64) {
-    const OwnPlan pl = qmm_own_plan(M, N, K, bits);
-    return sb_image_bytes(rows_shape(M, N, K, L), group_size, dtype) + own_plane_bytes(M, N, pl);
-  }
-  return qmm_walk_plane_bytes(rows_shape(M, N, K, L), group_size, bits);
+  const QmmArgs a = rows_shape(M, N, K, L);
+  return M > 64 ? sb_image_bytes(a, group_size, dtype) + own_plane_bytes(M, N, pl)
+                : qmm_walk_plane_bytes(a, group_size, bits);
 }
 
 namespace {
@@ -1458,7 +1464,8 @@ int rows_entry(
     void* workspace,
     size_t workspace_bytes,
     hipStream_t s) {
-  if (!mlxrocm_qmm_rows_supported(M, N, K, L, group_size, bits, dtype)) {
+  OwnPlan pl;
+  if (!rows_plan(M, N, K, L, group_size, bits, dtype, &pl)) {
     return fail(
         MLXROCM_UNSUPPORTED, "[quantized_matmul] M=%d N=%d K=%d: not a shape of the few-row kernel",
         M, N, K);
@@ -1485,7 +1492,6 @@ int rows_entry(
     return rc;
   }
   const size_t image = M > 64 && sb_image == nullptr ? sb_image_bytes(a, group_size, dtype) : 0;
-  const OwnPlan pl = M > 64 ? qmm_own_plan(M, N, K, bits) : OwnPlan{};
   const size_t need =
       M > 64 ? image + own_plane_bytes(M, N, pl) : qmm_walk_plane_bytes(a, group_size, bits);
   if (need != 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {

@@ -58,32 +58,38 @@ bool qmm_own_supported(int M, int N, int K, int L, int bits, int dtype) {
 // have whole pieces).
 OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
   const Step& step = step_of(codes);
-  const long cus = compute_units();
-  const long nx = (N + kOwnBN - 1) / kOwnBN;
+  const int cus = static_cast<int>(compute_units());
+  const int nx = (N + kOwnBN - 1) / kOwnBN;
   const int steps = K / kOwnBK;
-  const double plane = 1e-6 * static_cast<double>(k_split_plane(M, N));
+  const size_t plane_size = k_split_plane(M, N) * sizeof(float);
+  const double plane = 1e-6 / sizeof(float) * static_cast<double>(plane_size);
+  // (4-bit codes in one range are put in order: kInOrder)
+  const double in_order = codes == 4 ? 0.12 : 0.0;
+  size_t most = kOwnMostPlanes / plane_size;
+  most = most > 16 ? 16 : most;
+  const int ranges = static_cast<int>(most) * 2 > steps ? steps / 2 : static_cast<int>(most);
   OwnPlan pl{};
   for (int mt = 4; mt <= 16; mt += 2) {
     if (mt > 4 && 16 * mt > (M + 31) / 32 * 32) {
       break;
     }
-    const long tiles = nx * ((M + 16 * mt - 1) / (16 * mt));
-    for (int s = 1; s <= 16; ++s) {
-      if (s > 1 &&
-          (tiles * s > cus || 2 * s > steps ||
-           k_split_plane(M, N) * s * sizeof(float) > kOwnMostPlanes)) {
-        break;
-      }
-      const long rounds = (tiles * s + cus - 1) / cus;
-      const double busy = static_cast<double>(tiles * s) / static_cast<double>(rounds * cus);
-      // (4-bit codes in one range are put in order: kInOrder)
-      const double fixed = step.fixed + (codes == 4 && s == 1 ? 0.12 : 0.0);
-      const double each = (steps + s - 1) / s * (fixed + mt * (step.each + busy * step.busy));
-      const double us = 5.9 + rounds * (0.36 * mt - 1.1 + each) +
-          (s > 1 ? 6.6 + (0.89 * s + 0.15) * plane
-                 : 0.34 * plane + (N % 2 != 0 ? 1.05 * rounds * mt : 0.0));
-      if (pl.mt == 0 || us < pl.us) {
-        pl = {mt, s, us};
+    const long tiles = static_cast<long>(nx) * ((M + 16 * mt - 1) / (16 * mt));
+    const double tile = 0.36 * mt - 1.1;
+    const long rounds = (tiles + cus - 1) / cus;
+    const double busy = static_cast<double>(tiles) / static_cast<double>(rounds * cus);
+    const double us = 5.9 + 0.34 * plane +
+        rounds * (tile + steps * (step.fixed + in_order + mt * (step.each + busy * step.busy)) +
+                  (N % 2 != 0 ? 1.05 * mt : 0.0));
+    if (pl.mt == 0 || us < pl.us) {
+      pl = {mt, 1, us};
+    }
+    for (int s = 2; s <= ranges && tiles * s <= cus; ++s) { // (one round)
+      const double share = static_cast<double>(tiles * s) / cus;
+      const double each =
+          (steps + s - 1) / s * (step.fixed + mt * (step.each + share * step.busy));
+      const double cut = 5.9 + tile + each + 6.6 + (0.89 * s + 0.15) * plane;
+      if (cut < pl.us) {
+        pl = {mt, s, cut};
       }
     }
   }

@@ -865,6 +865,28 @@ int mlxrocm_qmm_plan(
     char* plan,
     size_t plan_bytes);
 
+/* The same for mlxrocm_qmm_rows and mlxrocm_fp_qmm_rows with the workspace that they name: where
+ * _supported answers 0, MLXROCM_UNSUPPORTED. */
+int mlxrocm_qmm_rows_plan(
+    int M,
+    int N,
+    int K,
+    int L,
+    int group_size,
+    int bits,
+    int dtype,
+    char* plan,
+    size_t plan_bytes);
+int mlxrocm_fp_qmm_rows_plan(
+    int M,
+    int N,
+    int K,
+    int L,
+    int mode,
+    int dtype,
+    char* plan,
+    size_t plan_bytes);
+
 /* The same for mlxrocm_gather_qmm. */
 int mlxrocm_gather_qmm_plan(
     int M,

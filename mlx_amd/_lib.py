@@ -86,6 +86,8 @@ SIGNATURES = {
     "mlxrocm_from_fp8": (_i, [_p, _p, _sz, _i, _p]),
     "mlxrocm_qmm_kernel_name": (ctypes.c_char_p, [_i] * 8),
     "mlxrocm_qmm_plan": (_i, [_i] * 9 + [_sz, ctypes.c_char_p, _sz]),
+    "mlxrocm_qmm_rows_plan": (_i, [_i] * 7 + [ctypes.c_char_p, _sz]),
+    "mlxrocm_fp_qmm_rows_plan": (_i, [_i] * 6 + [ctypes.c_char_p, _sz]),
     "mlxrocm_gather_qmm_plan": (_i, [_i] * 10 + [_sz, ctypes.c_char_p, _sz]),
     "mlxrocm_qmm_rule_count": (_i, []),
     "mlxrocm_qmm_rule_name": (ctypes.c_char_p, [_i]),
@@ -195,6 +197,20 @@ def qmm_plan(M, N, K, L=1, batched_weights=False, group_size=64, bits=4, dtype=B
         workspace_bytes = lib.mlxrocm_qmm_workspace_size(*args)
     buf = ctypes.create_string_buffer(1024)
     rc = lib.mlxrocm_qmm_plan(*args, workspace_bytes, buf, len(buf))
+    return rc, buf.value.decode()
+
+
+def qmm_rows_plan(M, N, K, L=1, group_size=64, bits=4, dtype=BFLOAT16):
+    """The same for mlxrocm_qmm_rows with its own workspace, e.g.
+    "interleave_sb+qmm_own(rows=256,ksplit=1)"."""
+    buf = ctypes.create_string_buffer(512)
+    rc = load().mlxrocm_qmm_rows_plan(M, N, K, L, group_size, bits, dtype, buf, len(buf))
+    return rc, buf.value.decode()
+
+
+def fp_qmm_rows_plan(M, N, K, L=1, mode=MXFP4, dtype=BFLOAT16):
+    buf = ctypes.create_string_buffer(512)
+    rc = load().mlxrocm_fp_qmm_rows_plan(M, N, K, L, mode, dtype, buf, len(buf))
     return rc, buf.value.decode()
 
 

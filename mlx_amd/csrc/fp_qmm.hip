@@ -1109,6 +1109,17 @@ extern "C" int mlxrocm_fp_qmm_plan(
       workspace_bytes != 0 ? fake_pointer(4) : nullptr, workspace_bytes, nullptr);
 }
 
+extern "C" int mlxrocm_fp_qmm_rows_plan(
+    int M, int N, int K, int L, int mode, int dtype, char* plan, size_t plan_bytes) {
+  RehearsalScope rehearsal(plan, plan_bytes);
+  const int64_t w_stride = L > 1 ? int64_t{1} << 28 : 0;
+  return mlxrocm_fp_qmm_rows(
+      fake_pointer(0), static_cast<const uint32_t*>(fake_pointer(1)),
+      static_cast<const uint8_t*>(fake_pointer(2)), fake_pointer(3), M, N, K, L,
+      static_cast<int64_t>(M) * K, w_stride, w_stride, mode, dtype, fake_pointer(4),
+      mlxrocm_fp_qmm_rows_workspace_size(M, N, K, L, mode, dtype), nullptr);
+}
+
 extern "C" int mlxrocm_fp_qqmm_plan(
     int M,
     int N,

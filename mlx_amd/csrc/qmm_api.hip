@@ -2113,6 +2113,19 @@ extern "C" int mlxrocm_qmm_plan(
       nullptr);
 }
 
+extern "C" int mlxrocm_qmm_rows_plan(
+    int M, int N, int K, int L, int group_size, int bits, int dtype, char* plan,
+    size_t plan_bytes) {
+  RehearsalScope rehearsal(plan, plan_bytes);
+  const int64_t w_stride = L > 1 ? int64_t{1} << 28 : 0;
+  return rows_entry(
+      fake_device_pointer(0), static_cast<const uint32_t*>(fake_device_pointer(1)),
+      fake_device_pointer(2), fake_device_pointer(3), nullptr, fake_device_pointer(4), M, N, K, L,
+      static_cast<int64_t>(M) * K, w_stride, w_stride, group_size, bits, dtype,
+      fake_device_pointer(5),
+      mlxrocm_qmm_rows_workspace_size(M, N, K, L, group_size, bits, dtype), nullptr);
+}
+
 extern "C" int mlxrocm_gather_qmm_plan(
     int M,
     int N,

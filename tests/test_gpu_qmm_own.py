@@ -265,3 +265,55 @@ def test_prepacked_calls_have_the_bits_of_plain_ones(M, N, K, bits, dtype):
         for kept in (image, None):
             y = mlx_amd.quantized_matmul(t, *q, group_size=64, bits=bits, sb_image=kept)
             assert torch.equal(y, plain), kept is None
+
+
+# the smallest calls found of every height of the tiles, in one range of K and in several:
+# (rows of a tile, M, N, K, ranges)
+HEIGHTS = {
+    3: ((64, 327, 1314, 128, 1), (64, 314, 476, 2176, 6), (96, 197, 17868, 128, 1),
+        (96, 2123, 404, 2048, 4), (128, 295, 16506, 256, 1), (128, 678, 528, 8192, 13),
+        (160, 706, 10790, 128, 1), (160, 262, 7404, 3072, 4), (192, 650, 13474, 256, 1),
+        (192, 518, 2096, 8192, 8), (224, 770, 15378, 256, 1), (224, 1292, 1184, 8192, 8),
+        (256, 1573, 8292, 384, 1), (256, 1154, 2748, 8192, 4)),
+    4: ((64, 2125, 424, 128, 1), (64, 279, 552, 2176, 6), (96, 195, 16420, 128, 1),
+        (96, 1888, 524, 2176, 4), (128, 300, 17312, 256, 1), (128, 2252, 532, 4096, 4),
+        (160, 515, 14652, 256, 1), (160, 2945, 524, 4096, 4), (192, 515, 19196, 256, 1),
+        (192, 331, 8228, 4224, 3), (224, 582, 19046, 384, 1), (224, 398, 9600, 4224, 3),
+        (256, 680, 19184, 640, 1), (256, 2776, 1136, 8192, 4)),
+    8: ((64, 2614, 404, 128, 1), (64, 316, 500, 2176, 6), (96, 199, 16414, 128, 1),
+        (96, 1241, 532, 2176, 6), (128, 2748, 2050, 128, 1), (128, 1156, 540, 4096, 8),
+        (160, 546, 13156, 256, 1), (160, 2819, 604, 2048, 4), (192, 523, 19880, 256, 1),
+        (192, 526, 4492, 3072, 4), (224, 578, 19098, 256, 1), (224, 587, 6436, 3072, 3),
+        (256, 1360, 9476, 384, 1), (256, 2320, 1824, 4224, 3)),
+    "mxfp8": ((64, 103, 462, 128, 1), (64, 208, 412, 1024, 4), (96, 257, 13206, 128, 1),
+              (96, 596, 516, 4224, 11), (128, 674, 8400, 128, 1), (128, 1169, 456, 8192, 11),
+              (160, 514, 13456, 256, 1), (160, 534, 1824, 6144, 8), (192, 515, 19906, 256, 1),
+              (192, 322, 9960, 3072, 3), (224, 590, 19148, 384, 1), (224, 769, 4712, 4096, 3),
+              (256, 1384, 9598, 640, 1), (256, 1806, 2412, 6144, 3)),
+}
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("codes", HEIGHTS)
+def test_every_height(codes, dtype):
+    """Every height of the tiles with and without K ranges, named by the plan of the call: no
+    constant of the rule drops one from the tests unseen."""
+    for rows, M, N, K, ranges in HEIGHTS[codes]:
+        kernel = f"qmm_own(rows={rows},ksplit={ranges})"
+        g = torch.Generator(device="cuda").manual_seed(M)
+        x = torch.randn((M, K), generator=g, device="cuda").to(dtype)
+        if codes == "mxfp8":
+            assert kernel in _lib.fp_qmm_rows_plan(M, N, K, 1, _lib.MXFP8, CODE[dtype])[1]
+            w = torch.randn((N, K), generator=g, device="cuda").to(dtype)
+            wq, s = mlx_amd.quantize(w, mode=codes)[:2]
+            y = mlx_amd.quantized_matmul(x, wq, s, None, mode=codes)
+            w_hat = mlx_amd.dequantize(wq, s, None, mode=codes, dtype=dtype).double()
+        else:
+            assert kernel in _lib.qmm_rows_plan(M, N, K, 1, 64, codes, CODE[dtype])[1]
+            wq, s, b = _weights(N, K, codes, dtype)
+            y = mlx_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=codes)
+            w_hat = mlx_amd.dequantize(wq, torch.ones_like(s, dtype=torch.float32),
+                                       torch.zeros_like(s, dtype=torch.float32), 64, codes).double()
+            w_hat = w_hat.unflatten(1, (-1, 64)) * s.double()[..., None] + b.double()[..., None]
+            w_hat = w_hat.flatten(1).to(dtype).double()
+        _relative(y, x.double() @ w_hat.T, dtype)

@@ -607,7 +607,7 @@ bool fp_own_pays(int M, int N, int K, int L, int mode, int dtype, OwnPlan* pl) {
     return false;
   }
   *pl = qmm_own_plan(M, N, K, kOwnFpCodes + mode);
-  return qmm_own_pays(*pl, kOwnFpCodes + mode, qmm_mfma_us(M, N, K, 4));
+  return qmm_own_pays(*pl, M, kOwnFpCodes + mode, qmm_mfma_us(M, N, K, 4));
 }
 
 size_t fp_own_bytes(int M, int N, int K, const OwnPlan& pl) {

@@ -709,12 +709,12 @@ bool own_pays(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* 
     return false;
   }
   *pl = qmm_own_plan(M, N, K, bits);
-  if (!qmm_own_pays(*pl, bits, qmm_mfma_us(M, N, K, bits))) {
+  if (!qmm_own_pays(*pl, M, bits, qmm_mfma_us(M, N, K, bits))) {
     return false;
   }
   if (M <= (K <= kMidShortK ? kMidMaxMShortK : kMidMaxM)) {
     const MidPlan mid = qmm_mid_plan(M, N, K, gs, bits);
-    return mid.groups > compute_units() || qmm_own_pays(*pl, bits, mid.us);
+    return mid.groups > compute_units() || qmm_own_pays(*pl, M, bits, mid.us);
   }
   return true;
 }

@@ -350,7 +350,7 @@ constexpr int kOwnFpCodes = 16;
 bool qmm_own_supported(int M, int N, int K, int L, int bits, int dtype);
 OwnPlan qmm_own_plan(int M, int N, int K, int codes);
 // Whether it is ahead of the kernel that takes the call otherwise (`other`: us).
-bool qmm_own_pays(const OwnPlan& pl, int codes, double other);
+bool qmm_own_pays(const OwnPlan& pl, int M, int codes, double other);
 int launch_qmm_own(
     const QmmArgs& a, int gs, int codes, int dtype, const OwnPlan& pl, hipStream_t s);
 int launch_qmm_own_bf16(const QmmArgs& a, int gs, int bits, const OwnPlan& pl, hipStream_t s);

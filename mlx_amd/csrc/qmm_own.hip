@@ -97,19 +97,21 @@ OwnPlan qmm_own_plan(int M, int N, int K, int codes) {
 }
 
 // With the accounts of both sides, which err by 5 and 7..15 %, these margins leave 1.0 % of the
-// 7000 calls taken behind by more than 3 %, the worst by 11 %; the mean takes 0.84 of the time.  us against the tile kernel, bf16 g64 4-bit: 2048 x 4096 x 14336 198 / 243,
+// 4000 calls taken behind by more than 3 %, the worst by 15 %; the mean takes 0.85 of the time.  us against the tile kernel, bf16 g64 4-bit: 2048 x 4096 x 14336 198 / 243,
 // 2048 x 8192 x 8192 198 / 275, 2048 x 4096 x 4096 66 / 78, 320 x 14336 x 4096 51 / 60, 320 x 8192 x
 // 8192 54 / 80; the tile kernel stays ahead where its widths make whole rounds: 1024 x 14336 x
 // 4096 8-bit 102 / 99, 512 x 18944 x 3584 8-bit 77 / 72.  Less is to be gained where its
-// unpacking is one convert for two codes (mxfp8: 512 x 18944 x 3584 75 / 66), its steps are cheap
-// (8-bit, one range: 1921 x 5120 x 13824 313 / 280) or this kernel has to put the codes in order
-// (4-bit, one range: 5291 x 6853 x 8192 557 / 553).
-bool qmm_own_pays(const OwnPlan& pl, int codes, double other) {
+// unpacking is one convert for two codes (mxfp8: 512 x 18944 x 3584 75 / 66; mxfp4 in one tile of
+// rows, 103 x 18944 x 3584 42 / 38), its steps are cheap (8-bit, one range: 1921 x 5120 x 13824 313
+// / 280) or this kernel has to put the codes in order (4-bit, one range: 5291 x 6853 x 8192 557 /
+// 553).
+bool qmm_own_pays(const OwnPlan& pl, int M, int codes, double other) {
   const bool one = pl.splits == 1;
-  const double margin = codes == kOwnFpCodes + MLXROCM_MXFP8 ? (one ? 0.80 : 0.82)
-      : one && (codes == 4 || codes == 8)                    ? 0.82
-      : one && codes == kOwnFpCodes + MLXROCM_MXFP4          ? 0.85
-                                                             : 0.88;
+  const double margin = codes == kOwnFpCodes + MLXROCM_MXFP8      ? 0.82
+      : one && codes == 4                                         ? 0.82
+      : one && codes == 8                                         ? 0.84
+      : one && codes == kOwnFpCodes + MLXROCM_MXFP4 && M <= 256 ? 0.82
+                                                                  : 0.88;
   return pl.us < margin * other;
 }
 

@@ -555,8 +555,9 @@ int mlxrocm_qmm(
  * that walks x through LDS, one pass over W whatever the rows, nothing rounded before the
  * result.  More rows of one problem, K a multiple of 128: tiles whose wavefronts unpack
  * their own rows of W (scratch: the image of mlxrocm_qmm_sb_image and the fp32 planes of K
- * ranges).  The order of the sums is these kernels' own: the last bits may be others than
- * mlxrocm_qmm's.  _supported: 1 where it takes a call and is ahead of mlxrocm_qmm, else 0;
+ * ranges).  The order of the sums is these kernels' own: where mlxrocm_qmm does not run the
+ * same one (mlxrocm_qmm_plan) the last bits may be others.  _supported: 1 where it takes a
+ * call and is level with mlxrocm_qmm or ahead of it, else 0;
  * it looks at shapes only.  workspace: device scratch used only during the call,
  * 16-byte aligned, of _workspace_size bytes (up to 64 rows mostly 0: it may be NULL then).
  */

@@ -392,21 +392,77 @@ int run_qmm_mid(const QmmArgs& a, int gs, int bits, int dtype, Scratch& sc, hipS
   return reduce_k_splits(region, a.out, a.M, a.N, pl.splits, dtype, s);
 }
 
+// (mid_pays)
+constexpr int kMidMinM = 65;
+constexpr int kMidMaxM = 256;
+constexpr int kMidMaxMShortK = 2048;
+constexpr int kMidShortK = 2048;
+
+// More than 64 rows of x (mlxrocm_qmm_rows): where tiles whose wavefronts own their rows of W
+// (qmm_own.h) are ahead of the tile kernel and of qmm_mid, by the accounts of all three.
+bool own_pays(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* pl) {
+  // (ragged rows with K ranges: mlxrocm_qmm sums the same ranges for a caller short of scratch,
+  // a block of rows at a time, and so has the bits of this call whatever the scratch)
+  if (!qmm_own_supported(M, N, K, L, bits, dtype) ||
+      (N % 4 != 0 && qmm_mfma_k_splits(M, N, K, 1) > 1)) {
+    return false;
+  }
+  *pl = qmm_own_plan(M, N, K, bits);
+  if (!qmm_own_pays(*pl, M, bits, qmm_mfma_us(M, N, K, bits))) {
+    return false;
+  }
+  if (M <= (K <= kMidShortK ? kMidMaxMShortK : kMidMaxM)) {
+    const MidPlan mid = qmm_mid_plan(M, N, K, gs, bits);
+    return mid.groups > compute_units() || qmm_own_pays(*pl, M, bits, mid.us);
+  }
+  return true;
+}
+
+size_t own_plane_bytes(int M, int N, const OwnPlan& pl) {
+  return pl.splits > 1 ? k_split_plane(M, N) * pl.splits * sizeof(float) : 0;
+}
+
+// image: pairs of scales and biases (interleave_sb_for_qmm_t).
+int run_qmm_own(
+    const QmmArgs& a, int gs, int bits, int dtype, const OwnPlan& pl, const void* image,
+    void* planes, hipStream_t s) {
+  QmmArgs part = a;
+  part.scales = image;
+  part.biases = image; // (unused: a pair holds both)
+  part.sb_transposed = 2;
+  if (pl.splits <= 1) {
+    return launch_qmm_own(part, gs, bits, dtype, pl, s);
+  }
+  part.out = planes;
+  const int rc = launch_qmm_own(part, gs, bits, dtype, pl, s);
+  return rc != MLXROCM_OK ? rc : reduce_k_splits(planes, a.out, a.M, a.N, pl.splits, dtype, s);
+}
+
 // Prefill (transpose=true, 16-bit types) from 512 rows of x on: the tile kernel
 // reads one scale and one bias per thread and K-step, and with the caller's
 // [N][K / group] layout every lane of such a load touches a line of its own
 // (measured: 15 % of the kernel's time).  A pre-pass transposes both arrays to
 // [K / group][N] in the workspace (a few MB, ~5 us), after which
 // a wavefront's 32 rows read 64 contiguous bytes.
+// Where the tiles that own their rows of W are ahead (own_pays) they take the call, so that it has
+// the bits of mlxrocm_qmm_rows, with a kept image or without -- but for planes beyond what every
+// entry has (mlxrocm_qmm_static), and the codes whose bits are the tile kernel's (kInOrder).
 int run_qmm_t_transposed_sb(
     const QmmArgs& a, int gs, int bits, int dtype, int k_splits, Scratch& sc, hipStream_t s) {
   const int G = a.K / gs;
   const int batches = a.sb_batch_stride == 0 ? 1 : a.L;
   const bool prepacked = sc.sb_image != nullptr;
   const size_t sb_bytes = prepacked ? 0 : sb_image_bytes(a, gs, dtype);
+  OwnPlan own;
+  const bool owns = own_pays(a.M, a.N, a.K, a.L, gs, bits, dtype, &own) &&
+      !(bits == 4 && own.splits <= 1 && k_splits <= 1) &&
+      sb_image_bytes(a, gs, dtype) + own_plane_bytes(a.M, a.N, own) <= kStaticScratchBytes;
+  if (owns) {
+    k_splits = 1; // (the tile kernel's)
+  }
   const size_t row = k_splits > 1 ? plane_bytes(a, k_splits) / a.M : 0;
   const int rows = k_splits > 1 ? rows_with_room(a, sb_bytes, row, sc) : a.M;
-  const size_t partial_bytes = row * rows;
+  const size_t partial_bytes = owns ? own_plane_bytes(a.M, a.N, own) : row * rows;
   void* region = nullptr;
   int rc = MLXROCM_OK;
   if (sb_bytes + partial_bytes != 0) {
@@ -424,6 +480,9 @@ int run_qmm_t_transposed_sb(
       return rc;
     }
     sb = region;
+  }
+  if (owns) {
+    return run_qmm_own(a, gs, bits, dtype, own, sb, static_cast<char*>(region) + sb_bytes, s);
   }
   const size_t image = static_cast<size_t>(a.N) * G; // pairs of one weight matrix
   QmmArgs part = a;
@@ -682,10 +741,6 @@ bool tile_t(const Call& c) {
 // rows: 63 against 45) and over a long K with more rows, where codes dequantized once for
 // 256 rows are dearer to do again for each 128 (4096 x 14336, 512 rows: 77.5 against 71.5).
 // Up to 64 rows other kernels are ahead of both.
-constexpr int kMidMinM = 65;
-constexpr int kMidMaxM = 256;
-constexpr int kMidMaxMShortK = 2048;
-constexpr int kMidShortK = 2048;
 bool mid_pays(const Call& c) {
   const QmmArgs& a = c.a;
   if (a.M < kMidMinM || a.M > (a.K <= kMidShortK ? kMidMaxMShortK : kMidMaxM) ||
@@ -697,46 +752,6 @@ bool mid_pays(const Call& c) {
   const size_t need = mid_bytes(a, c.gs, c.dtype, pl, c.sc);
   return pl.groups <= compute_units() && pl.us < qmm_mfma_us(a.M, a.N, a.K, c.bits) &&
       plane_bytes(a, pl.splits) <= kStaticScratchBytes / 2 && (need == 0 || c.sc.affords(need));
-}
-
-// More than 64 rows of x (mlxrocm_qmm_rows): where tiles whose wavefronts own their rows of W
-// (qmm_own.h) are ahead of the tile kernel and of qmm_mid, by the accounts of all three.
-bool own_pays(int M, int N, int K, int L, int gs, int bits, int dtype, OwnPlan* pl) {
-  // (ragged rows with K ranges: mlxrocm_qmm sums the same ranges for a caller short of scratch,
-  // a block of rows at a time, and so has the bits of this call whatever the scratch)
-  if (!qmm_own_supported(M, N, K, L, bits, dtype) ||
-      (N % 4 != 0 && qmm_mfma_k_splits(M, N, K, 1) > 1)) {
-    return false;
-  }
-  *pl = qmm_own_plan(M, N, K, bits);
-  if (!qmm_own_pays(*pl, M, bits, qmm_mfma_us(M, N, K, bits))) {
-    return false;
-  }
-  if (M <= (K <= kMidShortK ? kMidMaxMShortK : kMidMaxM)) {
-    const MidPlan mid = qmm_mid_plan(M, N, K, gs, bits);
-    return mid.groups > compute_units() || qmm_own_pays(*pl, M, bits, mid.us);
-  }
-  return true;
-}
-
-size_t own_plane_bytes(int M, int N, const OwnPlan& pl) {
-  return pl.splits > 1 ? k_split_plane(M, N) * pl.splits * sizeof(float) : 0;
-}
-
-// image: pairs of scales and biases (interleave_sb_for_qmm_t).
-int run_qmm_own(
-    const QmmArgs& a, int gs, int bits, int dtype, const OwnPlan& pl, const void* image,
-    void* planes, hipStream_t s) {
-  QmmArgs part = a;
-  part.scales = image;
-  part.biases = image; // (unused: a pair holds both)
-  part.sb_transposed = 2;
-  if (pl.splits <= 1) {
-    return launch_qmm_own(part, gs, bits, dtype, pl, s);
-  }
-  part.out = planes;
-  const int rc = launch_qmm_own(part, gs, bits, dtype, pl, s);
-  return rc != MLXROCM_OK ? rc : reduce_k_splits(planes, a.out, a.M, a.N, pl.splits, dtype, s);
 }
 
 // Two passes over the same scratch, one after the other on the stream.
@@ -1024,7 +1039,8 @@ const Rule kRules[] = {
      "prefill from 512 rows: scales and biases transposed to [K/group][N] first (5.2 us at "
      "14336x4096), after which a wavefront's 32 rows read 64 contiguous bytes; with the "
      "caller's layout those loads were 15 % of the tile kernel's time. M=2048, 14336x4096: "
-     "199.5 per call, 1206 TFLOP/s"},
+     "199.5 per call, 1206 TFLOP/s. Tiles that own their rows of W where ahead: 2048x8192x8192 "
+     "198 against 275"},
     {"qmm_t_tile_k_split",
      [](const Call& c) { return tile_t(c) && tile_k_splits(c) > 1; },
      [](const Call& c) {

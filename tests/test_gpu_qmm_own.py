@@ -223,10 +223,10 @@ def _c_call(entry, x, q, image, N, bits, code, transpose, workspace_bytes, group
     return out
 
 
-# mlxrocm_qmm in one range of the tile kernel and in several, in front of shapes that the tiles of
-# this file take (first four) and of shapes that they leave to the tile kernel
-TABLE = ((2048, 4096, 4096, 8), (1024, 4096, 4096, 4), (300, 14336, 4096, 2), (5000, 1024, 4096, 4),
-         (600, 803, 4096, 4), (1024, 14336, 4096, 8), (1792, 7168, 4096, 4))
+# shapes that the tiles of this file take (the first three in mlxrocm_qmm too; then fewer than 512
+# rows, and planes of more than 64 MB) and shapes that they leave to the tile kernel
+TABLE = ((2048, 4096, 4096, 8), (1024, 4096, 4096, 4), (5000, 1024, 4096, 4), (300, 14336, 4096, 2),
+         (2048, 4096, 14336, 4), (600, 803, 4096, 4), (1024, 14336, 4096, 8), (1792, 7168, 4096, 4))
 
 
 @pytest.mark.parametrize("M,N,K,bits", TABLE)
@@ -241,10 +241,11 @@ def test_prepacked_calls_have_the_bits_of_plain_ones(M, N, K, bits, dtype):
     image = mlx_amd.quantized_matmul_sb_image(q[1], q[2], 64)
     share = -(-lib.mlxrocm_qmm_sb_image_size(N, K, 1, 64, code) // 256) * 256
     rows = bool(lib.mlxrocm_qmm_rows_supported(M, N, K, 1, 64, bits, code))
-    assert rows == ((M, N, K, bits) in TABLE[:4])
+    assert rows == ((M, N, K, bits) in TABLE[:5])
 
     need = lib.mlxrocm_qmm_workspace_size(M, N, K, 1, 0, 64, bits, code, 1)
     plan = _lib.qmm_plan(M, N, K, bits=bits, dtype=code)[1]
+    assert ("qmm_own" in plan) == ((M, N, K, bits) in TABLE[:3])
     share = share if "interleave_sb" in plan else 0
     plain = _c_call(lib.mlxrocm_qmm, x, q, None, N, bits, code, (1,), need)
     for room in (need, need - share):
@@ -254,7 +255,8 @@ def test_prepacked_calls_have_the_bits_of_plain_ones(M, N, K, bits, dtype):
     if rows:
         need = lib.mlxrocm_qmm_rows_workspace_size(M, N, K, 1, 64, bits, code)
         share = -(-lib.mlxrocm_qmm_sb_image_size(N, K, 1, 64, code) // 256) * 256
-        plain = _c_call(lib.mlxrocm_qmm_rows, x, q, None, N, bits, code, (), need)
+        table, plain = plain, _c_call(lib.mlxrocm_qmm_rows, x, q, None, N, bits, code, (), need)
+        assert torch.equal(table, plain) or "qmm_own" not in plan
         for room in (need, need - share):
             for kept in (image, None) if room == need else (image,):
                 y = _c_call(lib.mlxrocm_qmm_rows_prepacked, x, q, (kept,), N, bits, code, (), room)

@@ -87,7 +87,7 @@ class QuantizedLinear(torch.nn.Module):
 
     def prepack(self) -> "QuantizedLinear":
         """Keeps the transposed image of scales and biases that prefill calls
-        (512 rows of x and more) would otherwise rebuild on every call.  Not in
+        (more than 64 rows of x) would otherwise rebuild on every call.  Not in
         the reference; call again after changing the weights."""
         if self.mode != "affine":
             return self  # no biases, nothing to transpose
